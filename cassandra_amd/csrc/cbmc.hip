@@ -1,21 +1,6 @@
-// cbmc.hip -- configurational-bias growth of flexible molecules on the device.
-//
-// One workgroup grows one molecule fragment by fragment as Build_Molecule
-// does (fragment_growth.f90:72-707, Fragment_Order :1317-1446,
-// Fragment_Placement :1449-2132): thread 0 makes the reference's random
-// draws (rranf, random_generators.f90:51-122) and the rigid-body geometry,
-// and the whole workgroup scores every trial of a stage at once -- kappa_ins
-// placements of the first fragment, kappa_dih rotations of each further
-// fragment -- against every molecule of the box (lanes split over (trial,
-// molecule)), with the intramolecular and dihedral terms of each trial on
-// one lane.  Two drivers use it:
-//   k_gcmc_chain: one workgroup per box runs that box's whole sequence of
-//     GCMC insertions and deletions (gcmc_driver.f90:90-200,
-//     move_insert.f90:22-424, move_delete.f90:22-416) in one launch, so every
-//     box of a multi-box run advances in the same persistent kernel;
-//   k_widom_cbmc: one workgroup per Widom insertion of a grown species
-//     (widom_insert.f90:22-594), or one workgroup walking all insertions on
-//     the reference's single stream.
+// cbmc.hip -- the growth kernels' host side (cbmc_grow.h has the kernels):
+// species set-up, the batches of CBMC Widom insertions, the GCMC, GEMC and
+// regrowth chains, and the est_emax / est_atompair_rminsq estimators.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -23,1276 +8,17 @@
 #include <cstring>
 #include <vector>
 
+#include "cbmc_grow.h"
 #include "engine.h"
 #include "kernels.h"
 
 namespace cass {
 
-constexpr int kCbA = 16;    // atoms of a grown species
-constexpr int kCbF = 8;     // fragments
-constexpr int kCbK = 32;    // trials per stage
-constexpr int kCbAng = 32;  // angles
-constexpr int kCbDih = 32;  // dihedrals
-
-// Growth description of one species (cass_cbmc_species plus what the
-// reference derives from it), in device memory.
-struct CbmcSpeciesDev {
-  int species, natoms, nfrag, spa0, coul_cbmc;
-  int frag_natoms[kCbF], frag_atoms[kCbF][kCbA];
-  int frag_nconnect[kCbF], frag_connect[kCbF][kCbF];
-  int frag_anchor[kCbF];
-  double prob_ins[kCbF], cum_prob_ins[kCbF];
-  int nconfig[kCbF];
-  long long lib_off[kCbF];
-  int nangles, angle[kCbAng][3];
-  double angle_k[kCbAng], angle_t0[kCbAng];
-  int ndihed, dihed[kCbDih][4];
-  double rb[kCbDih][6];
-  int kappa_ins, kappa_rot, kappa_dih;
-  // fragment bonds (Fragment_Connectivity order) and the probability of
-  // cutting off fragment1's side of each (prob_del1)
-  int nfbond, fbond[kCbF][2];
-  double prob_del1[kCbF];
-  // per atom and atom pair of the species (nonbond_list, intra scaling)
-  int type[kCbA];
-  double q[kCbA], mass[kCbA];
-  double vs[kCbA * kCbA], qs[kCbA * kCbA];
-  int bonded[kCbA * kCbA];
-  const double *lib;  // conformation libraries, lib_off[f] doubles in
-};
-
-// The topology's type and site tables in LDS, for the stage sums of the
-// growth kernels (ok = 0 when the topology is larger than these arrays: the
-// sums then read the device tables).
-constexpr int kCtSp = 8, kCtAt = 128, kCtT = 16;
-struct ChainTopo {
-  int ok, ntypes, njmax;
-  int sp_natoms[kCtSp], sp_atom_off[kCtSp];
-  int atom_type[kCtAt];
-  double atom_charge[kCtAt];
-  double eps[kCtT * kCtT], sig[kCtT * kCtT], mn[kCtT * kCtT], mm[kCtT * kCtT];
-};
-
-// LDS state of one growing molecule (these_atoms / this_molecule) and of
-// the current stage's trials.
-template <int NT>
-struct GrowLds {
-  double x[kCbA], y[kCbA], z[kCbA];
-  int exist[kCbA];
-  double4 com;  // (xcom, ycom, zcom, max_dcom)
-  // trial coordinates of the stage's atoms (first fragment: all its atoms;
-  // later fragments: the atoms it adds), per trial
-  double tx[kCbK][kCbA], ty[kCbK][kCbA], tz[kCbK][kCbA];
-  double4 tcom[kCbK];
-  int tatom[kCbA], tspa[kCbA], ntatom;  // the stage's atoms and species-atom ids
-  int tpos[kCbA];                        // position of an atom in tatom, -1 if absent
-  double theta[kCbK];
-  double sv[kCbK], sq[kCbK];
-  int sov[kCbK];
-  double ndih[kCbK];
-  double pv[NT], pq[NT];
-  int pov[NT];
-  double pem[NT / 64], sem;  // Eij_max of the full-cutoff pass: per wave, whole
-  double *rsq;               // closest r^2 per (species site, stage atom) of the
-                             // full-cutoff pass, global memory; null: not kept
-  int order[kCbF], placed[kCbF], ntotal;
-  int flag, trial;
-  double ln_pbias, ln_pseq;
-  // the rotated library conformation of the fragment being added (config_list)
-  double cx[kCbA], cy[kCbA], cz[kCbA];
-  double ha[3][3];
-  int anc_i, anc_c;
-  unsigned mask_new, mask_old;  // atoms the fragment adds / atoms placed before it
-  int64_t rng[5];
-  // the growth description and the topology tables, copied from device
-  // memory at kernel start: the one-lane bookkeeping between stages and the
-  // stage sums read them from LDS
-  CbmcSpeciesDev sp;
-  ChainTopo ct;
-  // the molecules in range of a stage's trials, one chunk of NT slots at a
-  // time: first site, site count, species' first site-type index and the
-  // mask of the trials in range
-  int cand_first[NT], cand_nj[NT], cand_oj[NT];
-  unsigned cand_mask[NT];
-  int wcnt[NT / 64];
-};
-
-// Copies the growth description into S.sp and the topology tables into
-// S.ct (every thread; a barrier must follow before either is read).
-template <int NT>
-__device__ inline void load_tables(GrowLds<NT> &S, const CbmcSpeciesDev *src, const TopoDev &tp) {
-  static_assert(sizeof(CbmcSpeciesDev) % 8 == 0, "8-byte words");
-  const uint64_t *s = (const uint64_t *)src;
-  uint64_t *d = (uint64_t *)&S.sp;
-  const int lane = threadIdx.x;
-  for (int i = lane; i < (int)(sizeof(CbmcSpeciesDev) / 8); i += NT) d[i] = s[i];
-  const bool ok = tp.nspecies <= kCtSp && tp.natoms_total <= kCtAt && tp.ntypes <= kCtT;
-  if (lane == 0) {
-    S.ct.ok = ok;
-    S.ct.ntypes = tp.ntypes;
-    int m = 0;
-    if (ok)
-      for (int i = 0; i < tp.nspecies; ++i) m = max(m, tp.sp_natoms[i]);
-    S.ct.njmax = m;
-  }
-  if (!ok) return;
-  for (int i = lane; i < tp.nspecies; i += NT) {
-    S.ct.sp_natoms[i] = tp.sp_natoms[i];
-    S.ct.sp_atom_off[i] = tp.sp_atom_off[i];
-  }
-  for (int i = lane; i < tp.natoms_total; i += NT) {
-    S.ct.atom_type[i] = tp.atom_type[i];
-    S.ct.atom_charge[i] = tp.atom_charge[i];
-  }
-  for (int i = lane; i < tp.ntypes * tp.ntypes; i += NT) {
-    S.ct.eps[i] = tp.eps[i];
-    S.ct.sig[i] = tp.sig[i];
-    S.ct.mn[i] = tp.mn ? tp.mn[i] : 0.0;
-    S.ct.mm[i] = tp.mm ? tp.mm[i] : 0.0;
-  }
-}
-
-
-__device__ inline int64_t cb_lsl(int64_t v, int k) { return (int64_t)((uint64_t)v << k); }
-__device__ inline int64_t cb_lsr(int64_t v, int k) { return (int64_t)((uint64_t)v >> k); }
-
-// rranf (random_generators.f90:97-120)
-__device__ inline double cb_uniform(int64_t *s) {
-  int64_t b;
-  b = cb_lsr(cb_lsl(s[0], 1) ^ s[0], 53);
-  s[0] = cb_lsl(s[0] & -2, 10) ^ b;
-  b = cb_lsr(cb_lsl(s[1], 24) ^ s[1], 50);
-  s[1] = cb_lsl(s[1] & -512, 5) ^ b;
-  b = cb_lsr(cb_lsl(s[2], 3) ^ s[2], 23);
-  s[2] = cb_lsl(s[2] & -4096, 29) ^ b;
-  b = cb_lsr(cb_lsl(s[3], 5) ^ s[3], 24);
-  s[3] = cb_lsl(s[3] & -131072, 23) ^ b;
-  b = cb_lsr(cb_lsl(s[4], 3) ^ s[4], 33);
-  s[4] = cb_lsl(s[4] & -8388608, 8) ^ b;
-  return (double)(s[0] ^ s[1] ^ s[2] ^ s[3] ^ s[4]) * 5.4210108624275221E-20 + 0.5;
-}
-
-__device__ inline double readlane_f64(double v, int l) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-  return __hiloint2double(hi, lo);
-}
-
-__device__ inline double readfirstlane_f64(double v) {
-  const int lo = __builtin_amdgcn_readfirstlane(__double2loint(v));
-  const int hi = __builtin_amdgcn_readfirstlane(__double2hiint(v));
-  return __hiloint2double(hi, lo);
-}
-
-// The selection among ntrial weighted trials (fragment_growth.f90:529-620,
-// 2044-2099), by the whole of wave 0: lane t < ntrial holds its trial's
-// weight w and kind wk (0 a weight; 1 none: an overlap or beta E >= max_kBT;
-// 2 an intramolecular overlap, whose cumulative weight repeats the previous
-// one).  The cumulative weights are summed in trial order as the reference
-// sums them, and the pick u W selects the first trial whose cumulative
-// weight exceeds it (without del_flag; with it trial 1 is kept).  Returns,
-// uniform over the wave, the trial, or -1 (cbmc_overlap) when no trial has a
-// weight or the pick passes the last; wsum = W.
-__device__ inline int select_trial(int ntrial, double w, int wk, bool del_flag, int64_t *rng, double &wsum) {
-  const int lane = threadIdx.x;
-  double run = 0.0, mycum = 0.0;
-  int all = 1;
-  for (int ii = 0; ii < ntrial; ++ii) {
-    const int k = __builtin_amdgcn_readlane(wk, ii);
-    if (k != 2) {
-      const double wi = readlane_f64(w, ii);
-      all = all && (k != 0);
-      run = ii > 0 ? __dadd_rn(run, wi) : wi;
-    }
-    if (lane == ii) mycum = run;
-  }
-  wsum = run;
-  if (all) return -1;
-  if (del_flag) return 0;
-  double u = 0.0;
-  if (lane == 0) u = cb_uniform(rng);
-  const double pick = __dmul_rn(readfirstlane_f64(u), run);
-  const uint64_t b = __builtin_amdgcn_ballot_w64(lane < ntrial && pick < mycum);
-  return b ? __builtin_ctzll(b) : -1;
-}
-
-// reads of device memory this kernel also writes go through vector loads
-template <typename T>
-__device__ inline T vld(const T *p) {
-  return *(const volatile T *)p;
-}
-
-// Arguments common to both drivers.
-struct GrowArgs {
-  BoxDev b;
-  TopoDev tp;
-  PairConst<double> cd;
-  PairConst<float> cf;
-  const CbmcSpeciesDev *sp;
-  double beta;
-};
-
-// The stage atoms at trial t against one site (xj, yj, zj) of type tj and
-// charge qj: the pair terms of Compute_MoleculePair_Energy
-// (energy_routines.f90:1589-1730) with the tables in LDS, added to ev / eq;
-// returns overlap (the caller discards the energies then).  EM: em is
-// raised to each in-cutoff pair's Eij_inter_vdw plus its bare q-q energy
-// (the Eij_max of energy_routines.f90:1702-1705; bare q-q per style as
-// Compute_AtomPair_Energy returns it, Ewald :2119, DSF :2074-2081, cut and
-// minimum image :2036-2046), in FP64 from the pair's vdW term; and with
-// S.rsq set, S.rsq[site_j * natoms + atom] is lowered to the pair's r^2
-// (swi_atompair_rsqmin, energy_routines.f90:1636-1643, 1700).
-template <typename P, int NT, bool EM = false>
-__device__ inline bool stage_site(const GrowArgs &a, const GrowLds<NT> &S, bool cbmc, int t, double xj, double yj,
-                                  double zj, int tj, double qj, int site_j, double &ev, double &eq, double &em) {
-  using TV = typename P::V;
-  using TQ = typename P::Q;
-  const BoxDev &b = a.b;
-  const ChainTopo &ct = S.ct;
-  const PairConst<double> &cd = a.cd;
-  const PairConst<TV> &cv = pconst<TV>(a.cd, a.cf);
-  const PairConst<TQ> &cq = pconst<TQ>(a.cd, a.cf);
-  const bool coul_cbmc = S.sp.coul_cbmc != 0;
-  bool ov = false;
-  for (int ia = 0; ia < S.ntatom; ++ia) {
-    double dx = S.tx[t][ia] - xj, dy = S.ty[t][ia] - yj, dz = S.tz[t][ia] - zj;
-    min_image(b, dx, dy, dz);
-    const double r2d = dx * dx + dy * dy + dz * dz;
-    if (r2d < cd.rc_low2) {
-      ov = true;
-      continue;
-    }
-    bool gv, gq;
-    pair_cutoff(cd, cbmc, r2d, gv, gq);
-    if (cbmc && !coul_cbmc) gq = false;
-    if (!(gv || gq)) continue;
-    const int sa = S.tspa[ia];
-    const int ti = ct.atom_type[sa];
-    TV e_v = (TV)0;
-    TQ e_q = (TQ)0;
-    if (ti >= 0 && tj >= 0 && gv) {
-      const int k = ti * ct.ntypes + tj;
-      e_v = vdw_inter<TV, typename P::M>(cv, (TV)r2d, (TV)ct.eps[k], (TV)ct.sig[k], (TV)ct.mn[k], (TV)ct.mm[k]);
-    }
-    const double qi = ct.atom_charge[sa];
-    const bool any_q = cd.q_style != CASS_Q_NONE && qi != 0.0 && qj != 0.0;
-    if (any_q && gq) e_q = qq_inter<TQ, typename P::M>(cq, (TQ)r2d, (TQ)(qi * qj));
-    if (gv) ev += (double)e_v;
-    if (gq) eq += (double)e_q;
-    if (EM) {
-      double bare = 0.0;
-      if (any_q && gq) {
-        const double rij = sqrt(r2d);
-        if (cd.q_style == CASS_Q_EWALD)
-          bare = qi * qj / rij * kChargeFactor;
-        else if (cd.q_style == CASS_Q_DSF)
-          bare = qi * qj * kChargeFactor / rij;
-        else
-          bare = kChargeFactor * (qi * qj) / rij;
-      }
-      const double eij = (gv ? (double)e_v : 0.0) + bare;
-      if (eij > em) em = eij;
-      if (S.rsq) {
-        double *m = S.rsq + site_j * S.sp.natoms + S.tatom[ia];
-        if (r2d < *m) atomicMin(m, r2d);
-      }
-    }
-  }
-  return ov;
-}
-
-// The molecule walk of stage_inter with the tables in LDS, one chunk of NT
-// molecule slots at a time.  Pass 1: one lane per slot tests the slot
-// against every trial's centre (Check_MoleculePair_Cutoff) and the slots in
-// range of some trial are listed in slot order (wave ballots).  Pass 2: the
-// (listed molecule, site) items of trial t are spread over its G lanes, each
-// item the stage atoms against one site.  Every thread calls it; the lane's
-// sums are added to ev / eq and an overlap sets ov.
-template <typename P, int NT, bool EM = false>
-__device__ void stage_items(const GrowArgs &a, GrowLds<NT> &S, int ntrial, int self, bool cbmc, int t, int r,
-                            int G, double &ev, double &eq, int &ov, double &em) {
-  const BoxDev &b = a.b;
-  const int lane = threadIdx.x, wave = lane >> 6;
-  const int njmax = S.ct.njmax;
-  for (int s0 = 0; s0 < b.nmols; s0 += NT) {
-    const int j = s0 + lane;
-    unsigned mask = 0;
-    int fj = 0, nj = 0, oj = 0;
-    if (j < b.nmols && j != self && b.live[j]) {
-      const double4 cj = b.comd[j];
-      for (int tt = 0; tt < ntrial; ++tt)
-        if (molpair_in_range(b, cbmc, S.tcom[tt], cj)) mask |= 1u << tt;
-      if (mask) {
-        const int sj = b.species[j];
-        fj = b.first[j];
-        nj = S.ct.sp_natoms[sj];
-        oj = S.ct.sp_atom_off[sj];
-      }
-    }
-    const uint64_t bal = __ballot(mask != 0);
-    if ((lane & 63) == 0) S.wcnt[wave] = __popcll(bal);
-    __syncthreads();
-    int base = 0, nc = 0;
-    for (int w = 0; w < NT / 64; ++w) {
-      if (w < wave) base += S.wcnt[w];
-      nc += S.wcnt[w];
-    }
-    if (mask) {
-      const int pos = base + __popcll(bal & ((1ull << (lane & 63)) - 1ull));
-      S.cand_first[pos] = fj;
-      S.cand_nj[pos] = nj;
-      S.cand_oj[pos] = oj;
-      S.cand_mask[pos] = mask;
-    }
-    __syncthreads();
-    if (t < ntrial && !ov) {
-      const int nitems = nc * njmax;
-      for (int k = r; k < nitems; k += G) {
-        const int c = k / njmax, ja = k - c * njmax;
-        if (!((S.cand_mask[c] >> t) & 1u) || ja >= S.cand_nj[c]) continue;
-        const int f = S.cand_first[c] + ja, o = S.cand_oj[c] + ja;
-        if (stage_site<P, NT, EM>(a, S, cbmc, t, b.x[f], b.y[f], b.z[f], S.ct.atom_type[o], S.ct.atom_charge[o], o,
-                                  ev, eq, em)) {
-          ov = 1;
-          break;
-        }
-      }
-    }
-    __syncthreads();  // the list is rebuilt for the next chunk
-  }
-}
-
-// ------------------------------------------------------------ stage scoring
-// Compute_Molecule_Nonbond_Inter_Energy (energy_routines.f90:1088-1206) of
-// the stage's atoms (tatom) at each of ntrial placements against every live
-// molecule but `self`: lanes are split into ntrial groups, each walking the
-// box's molecules with the COM prefilter (Check_MoleculePair_Cutoff) and
-// Compute_MoleculePair_Energy / Estimate_MoleculePair_Energy; the partials of
-// a group are summed in lane order.  Results in sv / sq / sov.  EM (one
-// trial, the LDS tables): also the largest pair term Eij_max in sem.
-template <typename P, int NT, bool EM = false>
-__device__ __attribute__((always_inline)) void stage_inter(const GrowArgs &a, GrowLds<NT> &S, int ntrial, int self,
-                                                           bool cbmc) {
-  const int lane = threadIdx.x;
-  const int G = NT / ntrial;
-  const int t = lane / G, r = lane - t * G;
-  double ev = 0.0, eq = 0.0, em = 0.0;
-  int ov = 0;
-  if (S.ct.ok && !(cbmc && a.b.apt_res > 0)) {
-    stage_items<P, NT, EM>(a, S, ntrial, self, cbmc, t, r, G, ev, eq, ov, em);
-  } else if (t < ntrial) {
-    // the device tables (a topology beyond the LDS arrays, or the CBMC
-    // energy table): G lanes of trial t walk the slots
-    const double4 ci = S.tcom[t];
-    const int na = S.ntatom;
-    for (int j = r; j < a.b.nmols; j += G) {
-      if (j == self || !a.b.live[j]) continue;
-      if (!molpair_in_range(a.b, cbmc, ci, a.b.comd[j])) continue;
-      if (molpair_energy<P>(a.b, a.tp, a.cd, a.cf, cbmc, S.sp.coul_cbmc != 0, na, S.tx[t], S.ty[t], S.tz[t],
-                            S.tspa, j, ev, eq, nullptr)) {
-        ov = 1;
-        break;
-      }
-    }
-  }
-  // the partials of each trial's G lanes summed in a fixed order
-  if (G % 64 == 0) {
-    // whole waves per trial: each wave by xor shuffles, then the trial's
-    // waves in order
-    double v = ev, q = eq, m = em;
-    int o = ov;
-    for (int off = 32; off > 0; off >>= 1) {
-      v += __shfl_xor(v, off);
-      q += __shfl_xor(q, off);
-      o |= __shfl_xor(o, off);
-      if (EM) m = fmax(m, __shfl_xor(m, off));
-    }
-    if ((lane & 63) == 0) {
-      S.pv[lane >> 6] = v;
-      S.pq[lane >> 6] = q;
-      S.pov[lane >> 6] = o;
-      if (EM) S.pem[lane >> 6] = m;
-    }
-    __syncthreads();
-    if (lane < ntrial) {
-      const int W = G >> 6;
-      double sv = 0.0, sq = 0.0, sm = 0.0;
-      int so = 0;
-      for (int k = lane * W; k < lane * W + W; ++k) {
-        sv += S.pv[k];
-        sq += S.pq[k];
-        so |= S.pov[k];
-        if (EM) sm = fmax(sm, S.pem[k]);
-      }
-      S.sv[lane] = sv;
-      S.sq[lane] = sq;
-      S.sov[lane] = so;
-      if (EM) S.sem = sm;
-    }
-  } else {
-    // a pairwise tree over each trial's lanes in LDS
-    S.pv[lane] = ev;
-    S.pq[lane] = eq;
-    S.pov[lane] = ov;
-    for (int off = 1; off < G; off <<= 1) {
-      __syncthreads();
-      if (t < ntrial && (r & (2 * off - 1)) == 0 && r + off < G) {
-        S.pv[lane] += S.pv[lane + off];
-        S.pq[lane] += S.pq[lane + off];
-        S.pov[lane] |= S.pov[lane + off];
-      }
-    }
-    __syncthreads();
-    if (lane < ntrial) {
-      S.sv[lane] = S.pv[lane * G];
-      S.sq[lane] = S.pq[lane * G];
-      S.sov[lane] = S.pov[lane * G];
-    }
-  }
-  __syncthreads();
-}
-
-// ------------------------------------------------------- per-trial helpers
-// Coordinates of atom k for trial t: the stage's atoms from the trial, the
-// others from the grown molecule.
-template <int NT>
-__device__ inline void atom_xyz(const GrowLds<NT> &S, int t, int k, double &x, double &y, double &z) {
-  const int p = t >= 0 ? S.tpos[k] : -1;
-  if (p >= 0) {
-    x = S.tx[t][p];
-    y = S.ty[t][p];
-    z = S.tz[t][p];
-  } else {
-    x = S.x[k];
-    y = S.y[k];
-    z = S.z[k];
-  }
-}
-
-// Dihedral d of Compute_Molecule_Dihedral_Energy (energy_routines.f90:350-447),
-// RB form, with trial t's coordinates; Get_Dihedral_Angle_COS
-// (internal_coordinate_routines.f90:305-410).
-template <int NT>
-__device__ inline double dihedral_term(const CbmcSpeciesDev &c, const GrowLds<NT> &S, int t, int d) {
-  const int *q = c.dihed[d];
-  double x1, y1, z1, x2, y2, z2, x3, y3, z3, x4, y4, z4;
-  atom_xyz(S, t, q[0], x1, y1, z1);
-  atom_xyz(S, t, q[1], x2, y2, z2);
-  atom_xyz(S, t, q[2], x3, y3, z3);
-  atom_xyz(S, t, q[3], x4, y4, z4);
-  const double rx12 = __dsub_rn(x1, x2), ry12 = __dsub_rn(y1, y2), rz12 = __dsub_rn(z1, z2);
-  const double rx32 = __dsub_rn(x3, x2), ry32 = __dsub_rn(y3, y2), rz32 = __dsub_rn(z3, z2);
-  const double rx34 = __dsub_rn(x3, x4), ry34 = __dsub_rn(y3, y4), rz34 = __dsub_rn(z3, z4);
-  const double mx = __dsub_rn(__dmul_rn(ry12, rz32), __dmul_rn(ry32, rz12));
-  const double my = __dadd_rn(-__dmul_rn(rx12, rz32), __dmul_rn(rz12, rx32));
-  const double mz = __dsub_rn(__dmul_rn(rx12, ry32), __dmul_rn(ry12, rx32));
-  const double nx = __dsub_rn(__dmul_rn(ry32, rz34), __dmul_rn(rz32, ry34));
-  const double ny = __dadd_rn(-__dmul_rn(rx32, rz34), __dmul_rn(rz32, rx34));
-  const double nz = __dsub_rn(__dmul_rn(rx32, ry34), __dmul_rn(ry32, rx34));
-  const double msq = __dadd_rn(__dadd_rn(__dmul_rn(mx, mx), __dmul_rn(my, my)), __dmul_rn(mz, mz));
-  const double nsq = __dadd_rn(__dadd_rn(__dmul_rn(nx, nx), __dmul_rn(ny, ny)), __dmul_rn(nz, nz));
-  const double mdn = __dadd_rn(__dadd_rn(__dmul_rn(mx, nx), __dmul_rn(my, ny)), __dmul_rn(mz, nz));
-  const double c1 = __ddiv_rn(mdn, __dsqrt_rn(__dmul_rn(msq, nsq)));
-  const double c2 = __dmul_rn(c1, c1), c3 = __dmul_rn(c1, c2), c4 = __dmul_rn(c2, c2), c5 = __dmul_rn(c2, c3);
-  const double *rb = c.rb[d];
-  double dot = __dmul_rn(1.0, rb[0]);
-  dot = __dadd_rn(dot, __dmul_rn(c1, rb[1]));
-  dot = __dadd_rn(dot, __dmul_rn(c2, rb[2]));
-  dot = __dadd_rn(dot, __dmul_rn(c3, rb[3]));
-  dot = __dadd_rn(dot, __dmul_rn(c4, rb[4]));
-  dot = __dadd_rn(dot, __dmul_rn(c5, rb[5]));
-  return dot;
-}
-
-// Compute_Molecule_Dihedral_Energy: the dihedrals whose four atoms exist
-// (exist[] per atom supplied by the caller), summed in order.
-template <int NT>
-__device__ double dihedral_energy(const CbmcSpeciesDev &c, const GrowLds<NT> &S, int t, const int *exist) {
-  double e = 0.0;
-  for (int d = 0; d < c.ndihed; ++d) {
-    const int *q = c.dihed[d];
-    if (!(exist[q[0]] && exist[q[1]] && exist[q[2]] && exist[q[3]])) continue;
-    e = __dadd_rn(e, dihedral_term(c, S, t, d));
-  }
-  return e;
-}
-
-// Angle k of Compute_Molecule_Angle_Energy (energy_routines.f90:283-347) of
-// the grown molecule, harmonic (0 for a fixed angle); Get_Bond_Angle
-// (internal_coordinate_routines.f90:188-272).
-template <int NT>
-__device__ inline double angle_term(const CbmcSpeciesDev &c, const GrowLds<NT> &S, int k) {
-  if (c.angle_k[k] == 0.0) return 0.0;
-  const int *q = c.angle[k];
-  const double rx21 = __dsub_rn(S.x[q[1]], S.x[q[0]]), ry21 = __dsub_rn(S.y[q[1]], S.y[q[0]]),
-               rz21 = __dsub_rn(S.z[q[1]], S.z[q[0]]);
-  const double rx32 = __dsub_rn(S.x[q[2]], S.x[q[1]]), ry32 = __dsub_rn(S.y[q[2]], S.y[q[1]]),
-               rz32 = __dsub_rn(S.z[q[2]], S.z[q[1]]);
-  const double c23 = __dadd_rn(__dadd_rn(__dmul_rn(rx21, rx32), __dmul_rn(ry21, ry32)), __dmul_rn(rz21, rz32));
-  const double c22 = __dadd_rn(__dadd_rn(__dmul_rn(rx21, rx21), __dmul_rn(ry21, ry21)), __dmul_rn(rz21, rz21));
-  const double c33 = __dadd_rn(__dadd_rn(__dmul_rn(rx32, rx32), __dmul_rn(ry32, ry32)), __dmul_rn(rz32, rz32));
-  const double inv = __ddiv_rn(1.0, __dsqrt_rn(__dmul_rn(c33, c22)));
-  double ct = __dmul_rn(c23, inv);
-  ct = fmin(ct, 0.999999);
-  ct = fmax(ct, -0.999999);
-  const double th = __dsub_rn(kPi, acos(ct));
-  const double d = __dsub_rn(th, c.angle_t0[k]);
-  return __dmul_rn(c.angle_k[k], __dmul_rn(d, d));
-}
-
-// One intramolecular site pair of Compute_AtomPair_Energy's intra branch
-// (energy_routines.f90:1831-2053, Ewald :2115-2135, DSF :2056-2082) with
-// the scaling of the pair; adds E_intra_vdw, E_intra_qq and the periodic
-// E_inter_qq.
-__device__ inline void intra_pair(const GrowArgs &a, const CbmcSpeciesDev &c, int i, int j, double r2, bool gv,
-                                  bool gq, double &ev, double &eq, double &eqi) {
-  const int n = c.natoms;
-  const double vs = c.vs[i * n + j], qs = c.qs[i * n + j];
-  const int ti = c.type[i], tj = c.type[j];
-  if (gv && ti >= 0 && tj >= 0) {
-    const int k = ti * a.tp.ntypes + tj;
-    const double eps = __dmul_rn(a.tp.eps[k], vs);
-    ev = __dadd_rn(ev, vdw_inter<double>(a.cd, r2, eps, a.tp.sig[k], a.tp.mn[k], a.tp.mm[k]));
-  }
-  if (gq) {
-    const double qi = c.q[i], qj = c.q[j];
-    if (a.cd.q_style == CASS_Q_EWALD) {
-      const double rij = __dsqrt_rn(r2);
-      const double erf_val = __dsub_rn(1.0, erfc_as<double>(__dmul_rn((double)a.cd.alpha, rij)));
-      const double eij = __dmul_rn(__ddiv_rn(__dmul_rn(qi, qj), rij), kChargeFactor);
-      eq = __dadd_rn(eq, __dmul_rn(qs, eij));
-      eqi = __dadd_rn(eqi, __dsub_rn(0.0, __dmul_rn(erf_val, eij)));
-    } else if (a.cd.q_style == CASS_Q_DSF) {
-      const double rij = __dsqrt_rn(r2);
-      const double cfqq = __dmul_rn(__dmul_rn(qi, qj), kChargeFactor);
-      double eij = __dadd_rn(__dsub_rn(__dmul_rn((double)a.cd.dsf2, __dsub_rn(rij, (double)a.cd.rc_coul)),
-                                       (double)a.cd.dsf1),
-                             __ddiv_rn(erfc(__dmul_rn((double)a.cd.alpha_dsf, rij)), rij));
-      eij = __dmul_rn(eij, cfqq);
-      eq = __dadd_rn(eq, __dsub_rn(eij, __dmul_rn(__dsub_rn(1.0, qs), __ddiv_rn(cfqq, rij))));
-    } else if (a.cd.q_style == CASS_Q_CUT || a.cd.q_style == CASS_Q_MINIMUM) {
-      eq = __dadd_rn(eq, __dmul_rn(qs, __ddiv_rn(__dmul_rn(kChargeFactor, __dmul_rn(qi, qj)), __dsqrt_rn(r2))));
-    }
-  }
-}
-
-// Compute_Atom_Nonbond_Intra_Energy (energy_routines.f90:691-737) of atom ia
-// against the atoms in the bit mask exist (bit k: atom k exists), trial t's
-// coordinates; returns overlap.
-template <int NT>
-__device__ bool atom_intra(const GrowArgs &a, const CbmcSpeciesDev &c, const GrowLds<NT> &S, int t, int ia,
-                           unsigned exist, double &ev, double &eq, double &eqi) {
-  ev = eq = eqi = 0.0;
-  double xi, yi, zi;
-  atom_xyz(S, t, ia, xi, yi, zi);
-  const int n = c.natoms;
-  for (int ja = 0; ja < n; ++ja) {
-    if (ja == ia || !((exist >> ja) & 1u)) continue;
-    const bool nzv = c.vs[ia * n + ja] > 0.0, nzq = c.qs[ia * n + ja] > 0.0;
-    if (!(nzv || nzq)) continue;
-    double xj, yj, zj;
-    atom_xyz(S, t, ja, xj, yj, zj);
-    const double rx = __dsub_rn(xj, xi), ry = __dsub_rn(yj, yi), rz = __dsub_rn(zj, zi);
-    const double r2 = __dadd_rn(__dadd_rn(__dmul_rn(rx, rx), __dmul_rn(ry, ry)), __dmul_rn(rz, rz));
-    if (r2 < (double)a.cd.rc_low2 && nzv) return true;
-    bool gv, gq;
-    pair_cutoff(a.cd, true, r2, gv, gq);
-    gv = gv && nzv;
-    gq = gq && nzq;
-    if (gv || gq) intra_pair(a, c, ja, ia, r2, gv, gq, ev, eq, eqi);
-  }
-  return false;
-}
-
-// The grown molecule's intramolecular terms (every atom existing) by wave 0:
-// every lane below 64 calls it and gets the results.  The nonbonded part of
-// Compute_Molecule_Nonbond_Intra_Energy (energy_routines.f90:980-1085) takes
-// one lane per atom pair and adds the pair terms in the reference's (ia, ja)
-// order up to the first pair that overlaps, where the reference returns; the
-// angles and dihedrals (:283-447) take one lane per term, added in order.
-// Returns the intramolecular overlap.
-template <int NT>
-__device__ bool mol_terms_wave(const GrowArgs &a, const CbmcSpeciesDev &c, const GrowLds<NT> &S, double &ev,
-                               double &eq, double &eqi, double &ea, double &ed) {
-  const int lane = threadIdx.x;
-  const int n = c.natoms, np = n * (n - 1) / 2;
-  ev = eq = eqi = 0.0;
-  bool ov = false;
-  for (int p0 = 0; p0 < np && !ov; p0 += 64) {
-    const int p = p0 + lane;
-    double pv = 0.0, pq = 0.0, pqi = 0.0;
-    bool po = false;
-    if (p < np) {
-      int ia = 0, rem = p;
-      while (rem >= n - 1 - ia) {
-        rem -= n - 1 - ia;
-        ++ia;
-      }
-      const int ja = ia + 1 + rem;
-      const double rx = __dsub_rn(S.x[ia], S.x[ja]), ry = __dsub_rn(S.y[ia], S.y[ja]),
-                   rz = __dsub_rn(S.z[ia], S.z[ja]);
-      const double r2 = __dadd_rn(__dadd_rn(__dmul_rn(rx, rx), __dmul_rn(ry, ry)), __dmul_rn(rz, rz));
-      if (r2 <= (double)a.cd.rc_low2 && !c.bonded[ia * n + ja]) {
-        po = true;
-      } else {
-        bool gv, gq;
-        pair_cutoff(a.cd, false, r2, gv, gq);
-        if (gv || gq) intra_pair(a, c, ia, ja, r2, gv, gq, pv, pq, pqi);
-      }
-    }
-    const uint64_t bo = __builtin_amdgcn_ballot_w64(po);
-    const int lim = min(bo ? (int)__builtin_ctzll(bo) : 64, np - p0);
-    for (int k = 0; k < lim; ++k) {
-      ev = __dadd_rn(ev, readlane_f64(pv, k));
-      eq = __dadd_rn(eq, readlane_f64(pq, k));
-      eqi = __dadd_rn(eqi, readlane_f64(pqi, k));
-    }
-    ov = bo != 0;
-  }
-  ea = 0.0;
-  for (int k0 = 0; k0 < c.nangles; k0 += 64) {
-    const double v = k0 + lane < c.nangles ? angle_term(c, S, k0 + lane) : 0.0;
-    const int cnt = min(64, c.nangles - k0);
-    for (int k = 0; k < cnt; ++k) ea = __dadd_rn(ea, readlane_f64(v, k));
-  }
-  ed = 0.0;
-  for (int k0 = 0; k0 < c.ndihed; k0 += 64) {
-    const double v = k0 + lane < c.ndihed ? dihedral_term(c, S, -1, k0 + lane) : 0.0;
-    const int cnt = min(64, c.ndihed - k0);
-    for (int k = 0; k < cnt; ++k) ed = __dadd_rn(ed, readlane_f64(v, k));
-  }
-  return ov;
-}
-
-// Get_COM / Compute_Max_Com_Distance (get_com.f90:45-121, 220-295) over the
-// atoms in exist[] with trial t's coordinates.
-template <int NT>
-__device__ double4 com_of(const CbmcSpeciesDev &c, const GrowLds<NT> &S, int t, const int *exist) {
-  double tm = 0.0, cx = 0.0, cy = 0.0, cz = 0.0;
-  for (int k = 0; k < c.natoms; ++k) {
-    if (!exist[k]) continue;
-    double x, y, z;
-    atom_xyz(S, t, k, x, y, z);
-    tm = __dadd_rn(tm, c.mass[k]);
-    cx = __dadd_rn(cx, __dmul_rn(c.mass[k], x));
-    cy = __dadd_rn(cy, __dmul_rn(c.mass[k], y));
-    cz = __dadd_rn(cz, __dmul_rn(c.mass[k], z));
-  }
-  cx = __ddiv_rn(cx, tm);
-  cy = __ddiv_rn(cy, tm);
-  cz = __ddiv_rn(cz, tm);
-  double dmax = 0.0;
-  for (int k = 0; k < c.natoms; ++k) {
-    if (!exist[k]) continue;
-    double x, y, z;
-    atom_xyz(S, t, k, x, y, z);
-    const double dx = __dsub_rn(x, cx), dy = __dsub_rn(y, cy), dz = __dsub_rn(z, cz);
-    const double r2 = __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz));
-    dmax = r2 > dmax ? r2 : dmax;
-  }
-  return make_double4(cx, cy, cz, __dsqrt_rn(dmax));
-}
-
-// com_of over the atoms of the bit mask exist.
-template <int NT>
-__device__ double4 com_of(const CbmcSpeciesDev &c, const GrowLds<NT> &S, int t, unsigned exist) {
-  double tm = 0.0, cx = 0.0, cy = 0.0, cz = 0.0;
-  for (int k = 0; k < c.natoms; ++k) {
-    if (!((exist >> k) & 1u)) continue;
-    double x, y, z;
-    atom_xyz(S, t, k, x, y, z);
-    tm = __dadd_rn(tm, c.mass[k]);
-    cx = __dadd_rn(cx, __dmul_rn(c.mass[k], x));
-    cy = __dadd_rn(cy, __dmul_rn(c.mass[k], y));
-    cz = __dadd_rn(cz, __dmul_rn(c.mass[k], z));
-  }
-  cx = __ddiv_rn(cx, tm);
-  cy = __ddiv_rn(cy, tm);
-  cz = __ddiv_rn(cz, tm);
-  double dmax = 0.0;
-  for (int k = 0; k < c.natoms; ++k) {
-    if (!((exist >> k) & 1u)) continue;
-    double x, y, z;
-    atom_xyz(S, t, k, x, y, z);
-    const double dx = __dsub_rn(x, cx), dy = __dsub_rn(y, cy), dz = __dsub_rn(z, cz);
-    const double r2 = __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz));
-    dmax = r2 > dmax ? r2 : dmax;
-  }
-  return make_double4(cx, cy, cz, __dsqrt_rn(dmax));
-}
-
-// Get_Aligner_Hanger (fragment_growth.f90:2135-2185)
-__device__ inline void aligner_hanger(double v1[3], double v2[3], double al[3][3], double ha[3][3]) {
-  const double n1 = __dsqrt_rn(__dadd_rn(__dadd_rn(__dmul_rn(v1[0], v1[0]), __dmul_rn(v1[1], v1[1])),
-                                         __dmul_rn(v1[2], v1[2])));
-  for (int i = 0; i < 3; ++i) v1[i] = __ddiv_rn(v1[i], n1);
-  const double n2 = __dsqrt_rn(__dadd_rn(__dadd_rn(__dmul_rn(v2[0], v2[0]), __dmul_rn(v2[1], v2[1])),
-                                         __dmul_rn(v2[2], v2[2])));
-  for (int i = 0; i < 3; ++i) v2[i] = __ddiv_rn(v2[i], n2);
-  double p1[3], p2[3];
-  p1[0] = __dsub_rn(__dmul_rn(v1[1], v2[2]), __dmul_rn(v1[2], v2[1]));
-  p1[1] = __dadd_rn(-__dmul_rn(v1[0], v2[2]), __dmul_rn(v1[2], v2[0]));
-  p1[2] = __dsub_rn(__dmul_rn(v1[0], v2[1]), __dmul_rn(v1[1], v2[0]));
-  const double np1 = __dsqrt_rn(__dadd_rn(__dadd_rn(__dmul_rn(p1[0], p1[0]), __dmul_rn(p1[1], p1[1])),
-                                          __dmul_rn(p1[2], p1[2])));
-  for (int i = 0; i < 3; ++i) p1[i] = __ddiv_rn(p1[i], np1);
-  p2[0] = __dsub_rn(__dmul_rn(v1[1], p1[2]), __dmul_rn(v1[2], p1[1]));
-  p2[1] = __dadd_rn(-__dmul_rn(v1[0], p1[2]), __dmul_rn(v1[2], p1[0]));
-  p2[2] = __dsub_rn(__dmul_rn(v1[0], p1[1]), __dmul_rn(v1[1], p1[0]));
-  const double np2 = __dsqrt_rn(__dadd_rn(__dadd_rn(__dmul_rn(p2[0], p2[0]), __dmul_rn(p2[1], p2[1])),
-                                          __dmul_rn(p2[2], p2[2])));
-  for (int i = 0; i < 3; ++i) p2[i] = __ddiv_rn(p2[i], np2);
-  for (int i = 0; i < 3; ++i) {
-    al[0][i] = v1[i];
-    al[1][i] = p2[i];
-    al[2][i] = p1[i];
-    ha[i][0] = v1[i];
-    ha[i][1] = p2[i];
-    ha[i][2] = p1[i];
-  }
-}
-
-// 3x3 matrix times vector in the reference's order (x m1 + y m2 + z m3)
-__device__ inline double mrow(const double m[3], double x, double y, double z) {
-  return __dadd_rn(__dadd_rn(__dmul_rn(x, m[0]), __dmul_rn(y, m[1])), __dmul_rn(z, m[2]));
-}
-
-// ------------------------------------------------------------ Build_Molecule
-// Fragment_Order (fragment_growth.f90:1317-1446); thread 0.
-template <int NT>
-__device__ void fragment_order(const CbmcSpeciesDev &c, GrowLds<NT> &S, int start, int *live) {
-  int hang[kCbF], nconnect = 0;
-  for (int i = 0; i < c.frag_nconnect[start]; ++i) {
-    const int id = c.frag_connect[start][i];
-    if (!live[id]) hang[nconnect++] = id;
-  }
-  while (nconnect > 0) {
-    double prob[kCbF], cum[kCbF];
-    for (int i = 0; i < nconnect; ++i) {
-      prob[i] = (double)(c.frag_natoms[hang[i]] - 2);
-      cum[i] = i == 0 ? prob[i] : __dadd_rn(cum[i - 1], (double)(c.frag_natoms[hang[i]] - 2));
-    }
-    for (int i = 0; i < nconnect; ++i) {
-      prob[i] = __ddiv_rn(prob[i], cum[nconnect - 1]);
-      cum[i] = __ddiv_rn(cum[i], cum[nconnect - 1]);
-    }
-    const double u = cb_uniform(S.rng);
-    int i = 0;
-    while (i < nconnect - 1 && !(u < cum[i])) ++i;
-    const int id = hang[i];
-    S.ln_pseq = __dadd_rn(S.ln_pseq, log(prob[i]));
-    S.order[S.ntotal++] = id;
-    live[id] = 1;
-    for (int j = i; j < nconnect - 1; ++j) hang[j] = hang[j + 1];
-    nconnect--;
-    for (int j = 0; j < c.frag_nconnect[id]; ++j) {
-      const int jd = c.frag_connect[id][j];
-      if (!live[jd]) hang[nconnect++] = jd;
-    }
-  }
-}
-
-// Rotate_Molecule_Eulerian (rotation_routines.f90:41-137) of the existing
-// atoms about the COM; thread 0.
-template <int NT>
-__device__ void rotate_euler(const CbmcSpeciesDev &c, GrowLds<NT> &S) {
-  const double theta = acos(__dsub_rn(1.0, __dmul_rn(2.0, cb_uniform(S.rng))));
-  const double phi = __dmul_rn(__dsub_rn(1.0, __dmul_rn(2.0, cb_uniform(S.rng))), kPi);
-  const double psi = __dmul_rn(__dsub_rn(1.0, __dmul_rn(2.0, cb_uniform(S.rng))), kPi);
-  const double cps = cos(psi), sps = sin(psi), cph = cos(phi), sph = sin(phi), cth = cos(theta), sth = sin(theta);
-  const double r11 = __dsub_rn(__dmul_rn(cps, cph), __dmul_rn(__dmul_rn(cth, sph), sps));
-  const double r12 = __dadd_rn(__dmul_rn(cps, sph), __dmul_rn(__dmul_rn(cth, cph), sps));
-  const double r13 = __dmul_rn(sps, sth);
-  const double r21 = __dsub_rn(__dmul_rn(-sps, cph), __dmul_rn(__dmul_rn(cth, sph), cps));
-  const double r22 = __dadd_rn(__dmul_rn(-sps, sph), __dmul_rn(__dmul_rn(cth, cph), cps));
-  const double r23 = __dmul_rn(cps, sth);
-  const double r31 = __dmul_rn(sth, sph);
-  const double r32 = __dmul_rn(-sth, cph);
-  const double r33 = cth;
-  for (int k = 0; k < c.natoms; ++k) {
-    if (!S.exist[k]) continue;
-    const double x = __dsub_rn(S.x[k], S.com.x), y = __dsub_rn(S.y[k], S.com.y), z = __dsub_rn(S.z[k], S.com.z);
-    const double xn = __dadd_rn(__dadd_rn(__dmul_rn(r11, x), __dmul_rn(r12, y)), __dmul_rn(r13, z));
-    const double yn = __dadd_rn(__dadd_rn(__dmul_rn(r21, x), __dmul_rn(r22, y)), __dmul_rn(r23, z));
-    const double zn = __dadd_rn(__dadd_rn(__dmul_rn(r31, x), __dmul_rn(r32, y)), __dmul_rn(r33, z));
-    S.x[k] = __dadd_rn(xn, S.com.x);
-    S.y[k] = __dadd_rn(yn, S.com.y);
-    S.z[k] = __dadd_rn(zn, S.com.z);
-  }
-}
-
-template <typename P, int NT>
-__device__ __attribute__((always_inline)) void fragment_placement(const GrowArgs &a, GrowLds<NT> &S, int self,
-                                                                  bool del_flag, int i0, double e_prev);
-
-// Build_Molecule with get_fragorder (fragment_growth.f90:72-707): S.x/y/z
-// hold the molecule's coordinates on entry when del_flag is set (deletion:
-// trial 1 of every stage is the molecule's own placement).  Every thread
-// calls it; S.flag = cbmc_overlap on return, S.ln_pbias / S.ln_pseq the
-// growth's log-probabilities, S.x/y/z/com the grown molecule.  widom: the
-// _Widom energy sums (vdW + q-q together).  keep_order: get_fragorder off
-// (the GEMC deletion half, fragment_growth.f90:245-253): the growth order
-// is S.order's, and S.ln_pseq stays.
-template <typename P, int NT>
-__device__ void build_molecule(const GrowArgs &a, GrowLds<NT> &S, int self, bool del_flag, bool keep_order = false) {
-  const CbmcSpeciesDev &c = S.sp;
-  const int lane = threadIdx.x;
-  const double beta = a.beta;
-  const int ki = c.kappa_ins;
-  // --- Step 1: first fragment and growth order; Step 2: its conformation;
-  // Step 3: orientation; the kappa_ins placements of the first fragment
-  if (lane == 0) {
-    S.ln_pbias = 0.0;
-    S.flag = 0;
-    int live[kCbF];
-    for (int k = 0; k < c.natoms; ++k) S.exist[k] = 0;
-    int fs = 0;
-    if (keep_order) {
-      for (int f = 0; f < c.nfrag; ++f) S.placed[f] = 0;
-      fs = S.order[0];
-      S.ntotal = c.nfrag;
-    } else {
-      for (int f = 0; f < c.nfrag; ++f) S.placed[f] = live[f] = S.order[f] = 0;
-      const double u = cb_uniform(S.rng);
-      while (fs < c.nfrag - 1 && !(u < c.cum_prob_ins[fs])) ++fs;
-      S.ln_pseq = log(c.prob_ins[fs]);
-      S.ntotal = 1;
-      S.order[0] = fs;
-      live[fs] = 1;
-      if (c.nfrag > 1) fragment_order(c, S, fs, live);
-    }
-    const int nfa = c.frag_natoms[fs];
-    if (!del_flag) {
-      // rranf can round to 1.0 (random_generators.f90:118): the index is clamped
-      const int conf = min((int)(cb_uniform(S.rng) * c.nconfig[fs]), c.nconfig[fs] - 1);
-      const double *lib = c.lib + c.lib_off[fs] + (size_t)conf * nfa * 3;
-      for (int j = 0; j < nfa; ++j) {
-        const int at = c.frag_atoms[fs][j];
-        S.x[at] = lib[3 * j];
-        S.y[at] = lib[3 * j + 1];
-        S.z[at] = lib[3 * j + 2];
-      }
-    }
-    for (int j = 0; j < nfa; ++j) S.exist[c.frag_atoms[fs][j]] = 1;
-    S.com = com_of(c, S, -1, S.exist);
-    if (!del_flag) rotate_euler(c, S);
-    // the stage's atoms: the first fragment's, in Fragment_Info order
-    for (int k = 0; k < c.natoms; ++k) S.tpos[k] = -1;
-    S.ntatom = nfa;
-    for (int j = 0; j < nfa; ++j) {
-      const int at = c.frag_atoms[fs][j];
-      S.tatom[j] = at;
-      S.tspa[j] = c.spa0 + at;
-      S.tpos[at] = j;
-    }
-    const double xo = S.com.x, yo = S.com.y, zo = S.com.z;
-    for (int t = 0; t < ki; ++t) {
-      double xa, ya, za;
-      if (del_flag && t == 0) {
-        xa = xo;
-        ya = yo;
-        za = zo;
-      } else {
-        xa = __dmul_rn(__dsub_rn(0.5, cb_uniform(S.rng)), a.b.L[0]);
-        ya = __dmul_rn(__dsub_rn(0.5, cb_uniform(S.rng)), a.b.L[1]);
-        za = __dmul_rn(__dsub_rn(0.5, cb_uniform(S.rng)), a.b.L[2]);
-      }
-      for (int j = 0; j < nfa; ++j) {
-        const int at = c.frag_atoms[fs][j];
-        S.tx[t][j] = __dadd_rn(__dsub_rn(S.x[at], xo), xa);
-        S.ty[t][j] = __dadd_rn(__dsub_rn(S.y[at], yo), ya);
-        S.tz[t][j] = __dadd_rn(__dsub_rn(S.z[at], zo), za);
-      }
-      S.tcom[t] = make_double4(xa, ya, za, 0.0);
-    }
-    // Compute_Max_COM_Distance once, at the first trial's placement
-    const double4 c0 = S.tcom[0];
-    double dmax = 0.0;
-    for (int j = 0; j < nfa; ++j) {
-      const double dx = __dsub_rn(S.tx[0][j], c0.x), dy = __dsub_rn(S.ty[0][j], c0.y),
-                   dz = __dsub_rn(S.tz[0][j], c0.z);
-      const double r2 = __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz));
-      dmax = r2 > dmax ? r2 : dmax;
-    }
-    const double md = __dsqrt_rn(dmax);
-    for (int t = 0; t < ki; ++t) S.tcom[t].w = md;
-  }
-  __syncthreads();
-  stage_inter<P, NT>(a, S, ki, self, true);
-  // weights (fragment_growth.f90:529-560), one lane per trial; selection
-  // (:583-620) by wave 0
-  double w = 0.0, e_t = 0.0;
-  int wk = 1;
-  if (lane < ki && !S.sov[lane]) {
-    e_t = __dadd_rn(S.sv[lane], S.sq[lane]);
-    const double bk = __dmul_rn(beta, e_t);
-    if (!(bk >= kMaxKBT)) {
-      w = exp(-bk);
-      wk = 0;
-    }
-  }
-  if (lane < 64) {
-    double wsum;
-    const int trial = select_trial(ki, w, wk, del_flag, S.rng, wsum);
-    const double e_sel = trial >= 0 ? readlane_f64(e_t, trial) : 0.0;
-    if (lane == 0) {
-      if (trial < 0) {
-        S.flag = 1;
-      } else {
-        S.ln_pbias = __dsub_rn(__dsub_rn(S.ln_pbias, __dmul_rn(beta, e_sel)), log(wsum));
-        for (int j = 0; j < S.ntatom; ++j) {
-          const int at = S.tatom[j];
-          S.x[at] = S.tx[trial][j];
-          S.y[at] = S.ty[trial][j];
-          S.z[at] = S.tz[trial][j];
-        }
-        S.com = S.tcom[trial];
-        S.placed[S.order[0]] = 1;
-        S.ndih[0] = dihedral_energy(c, S, -1, S.exist);  // e_total of Fragment_Placement
-      }
-    }
-  }
-  __syncthreads();
-  if (S.flag) return;
-  // --- Step 5: Fragment_Placement of the remaining fragments
-  fragment_placement<P, NT>(a, S, self, del_flag, 1, S.ndih[0]);
-  if (S.flag) return;
-  if (lane == 0) {
-    for (int k = 0; k < c.natoms; ++k) S.tpos[k] = -1;
-    if (S.ntotal > 1) S.com = com_of(c, S, -1, S.exist);
-  }
-  __syncthreads();
-}
-
-// Fragment_Placement (fragment_growth.f90:1449-2132) of S.order[i0..ntotal):
-// each fragment is attached to its first placed neighbour at kappa_dih
-// rotations about the connecting bond, scored (intramolecular, dihedral and
-// CBMC-cutoff intermolecular terms against e_prev, the dihedral energy
-// before the fragment) and one rotation drawn by its Boltzmann weight; with
-// del_flag trial 1 is the fragment's own placement.  Every thread calls it;
-// S.flag = cbmc_overlap on return, S.ln_pbias accumulates.
-template <typename P, int NT>
-__device__ __attribute__((always_inline)) void fragment_placement(const GrowArgs &a, GrowLds<NT> &S, int self,
-                                                                  bool del_flag, int i0, double e_prev) {
-  const CbmcSpeciesDev &c = S.sp;
-  const int lane = threadIdx.x;
-  const double beta = a.beta;
-  const int kd = c.kappa_dih;
-  for (int i = i0; i < S.ntotal; ++i) {
-    if (lane == 0) {
-      const int ifrag = S.order[i];
-      const int nfa = c.frag_natoms[ifrag];
-      unsigned grown = 0;
-      for (int k = 0; k < c.natoms; ++k) {
-        if (S.exist[k]) grown |= 1u << k;
-        S.cx[k] = S.cy[k] = S.cz[k] = 0.0;
-      }
-      if (del_flag) {
-        for (int j = 0; j < nfa; ++j) {
-          const int at = c.frag_atoms[ifrag][j];
-          S.exist[at] = 1;
-          S.cx[at] = S.x[at];
-          S.cy[at] = S.y[at];
-          S.cz[at] = S.z[at];
-        }
-      } else {
-        int conf = (int)(cb_uniform(S.rng) * c.nconfig[ifrag]);  // drawn twice, as written (:1578, :1584)
-        conf = min((int)(cb_uniform(S.rng) * c.nconfig[ifrag]), c.nconfig[ifrag] - 1);
-        const double *lib = c.lib + c.lib_off[ifrag] + (size_t)conf * nfa * 3;
-        for (int j = 0; j < nfa; ++j) {
-          const int at = c.frag_atoms[ifrag][j];
-          S.exist[at] = 1;
-          S.cx[at] = lib[3 * j];
-          S.cy[at] = lib[3 * j + 1];
-          S.cz[at] = lib[3 * j + 2];
-        }
-      }
-      int fconn = -1;
-      for (int j = 0; j < c.frag_nconnect[ifrag] && fconn < 0; ++j)
-        if (S.placed[c.frag_connect[ifrag][j]]) fconn = c.frag_connect[ifrag][j];
-      const int anc_i = c.frag_anchor[ifrag], anc_c = c.frag_anchor[fconn];
-      S.anc_i = anc_i;
-      S.anc_c = anc_c;
-      // the stage's atoms: those the fragment adds (neither anchor)
-      for (int k = 0; k < c.natoms; ++k) S.tpos[k] = -1;
-      S.ntatom = 0;
-      for (int j = 0; j < nfa; ++j) {
-        const int at = c.frag_atoms[ifrag][j];
-        if (at != anc_i && at != anc_c) {
-          S.tpos[at] = S.ntatom;
-          S.tatom[S.ntatom] = at;
-          S.tspa[S.ntatom] = c.spa0 + at;
-          S.ntatom++;
-        }
-      }
-      int atom_if = c.frag_atoms[ifrag][nfa - 1], atom_fc = c.frag_atoms[fconn][c.frag_natoms[fconn] - 1];
-      for (int j = nfa - 1; j >= 0; --j) {
-        const int at = c.frag_atoms[ifrag][j];
-        if (at != anc_i && at != anc_c) atom_if = at;
-      }
-      for (int j = c.frag_natoms[fconn] - 1; j >= 0; --j) {
-        const int at = c.frag_atoms[fconn][j];
-        if (at != anc_i && at != anc_c) atom_fc = at;
-      }
-      double v1[3] = {__dsub_rn(S.cx[anc_i], S.cx[anc_c]), __dsub_rn(S.cy[anc_i], S.cy[anc_c]),
-                      __dsub_rn(S.cz[anc_i], S.cz[anc_c])};
-      double v2[3] = {__dsub_rn(S.cx[atom_if], S.cx[anc_c]), __dsub_rn(S.cy[atom_if], S.cy[anc_c]),
-                      __dsub_rn(S.cz[atom_if], S.cz[anc_c])};
-      double al_i[3][3], ha_i[3][3], al_c[3][3];
-      aligner_hanger(v1, v2, al_i, ha_i);
-      if (!del_flag) {
-        double w1[3] = {__dsub_rn(S.x[anc_i], S.x[anc_c]), __dsub_rn(S.y[anc_i], S.y[anc_c]),
-                        __dsub_rn(S.z[anc_i], S.z[anc_c])};
-        double w2[3] = {__dsub_rn(S.x[atom_fc], S.x[anc_c]), __dsub_rn(S.y[atom_fc], S.y[anc_c]),
-                        __dsub_rn(S.z[atom_fc], S.z[anc_c])};
-        aligner_hanger(w1, w2, al_c, S.ha);
-      } else {
-        for (int r = 0; r < 3; ++r)
-          for (int q = 0; q < 3; ++q) S.ha[r][q] = ha_i[r][q];
-      }
-      const double tx0 = S.cx[anc_c], ty0 = S.cy[anc_c], tz0 = S.cz[anc_c];
-      for (int k = 0; k < c.natoms; ++k) {
-        S.cx[k] = __dsub_rn(S.cx[k], tx0);
-        S.cy[k] = __dsub_rn(S.cy[k], ty0);
-        S.cz[k] = __dsub_rn(S.cz[k], tz0);
-      }
-      for (int j = 0; j < nfa; ++j) {
-        const int at = c.frag_atoms[ifrag][j];
-        const double x = S.cx[at], y = S.cy[at], z = S.cz[at];
-        S.cx[at] = mrow(al_i[0], x, y, z);
-        S.cy[at] = mrow(al_i[1], x, y, z);
-        S.cz[at] = mrow(al_i[2], x, y, z);
-      }
-      double th = del_flag ? 0.0 : __dmul_rn(kTwoPi, cb_uniform(S.rng));
-      for (int ii = 0; ii < kd; ++ii) {
-        S.theta[ii] = th;
-        if (ii + 1 < kd) th = __dadd_rn(th, __ddiv_rn(kTwoPi, (double)kd));
-      }
-      // atoms added by this fragment: new_exist for the inter energy
-      unsigned added = 0, placed_before = 0;
-      for (int k = 0; k < c.natoms; ++k) {
-        if (S.exist[k] && !((grown >> k) & 1u)) added |= 1u << k;
-        else if (S.exist[k]) placed_before |= 1u << k;
-      }
-      S.mask_new = added;
-      S.mask_old = placed_before;
-    }
-    __syncthreads();
-    // trial placements of the added atoms, one lane per trial
-    if (lane < kd) {
-      const double th = S.theta[lane];
-      const double ct = cos(th), st = sin(th);
-      for (int p = 0; p < S.ntatom; ++p) {
-        const int at = S.tatom[p];
-        const double x = S.cx[at];
-        const double y = __dadd_rn(__dmul_rn(ct, S.cy[at]), __dmul_rn(st, S.cz[at]));
-        const double z = __dadd_rn(__dmul_rn(-st, S.cy[at]), __dmul_rn(ct, S.cz[at]));
-        S.tx[lane][p] = __dadd_rn(mrow(S.ha[0], x, y, z), S.x[S.anc_c]);
-        S.ty[lane][p] = __dadd_rn(mrow(S.ha[1], x, y, z), S.y[S.anc_c]);
-        S.tz[lane][p] = __dadd_rn(mrow(S.ha[2], x, y, z), S.z[S.anc_c]);
-      }
-    }
-    const unsigned newx = S.mask_new, oldx = S.mask_old;
-    __syncthreads();
-    // per trial: intramolecular energy of each added atom with the atoms
-    // placed so far (atom by atom), COM of the added atoms
-    double iv = 0.0, iq = 0.0, iqi = 0.0;
-    int intra_ov = 0;
-    if (lane < kd) {
-      unsigned ex = oldx;
-      for (int p = 0; p < S.ntatom; ++p) {
-        const int at = S.tatom[p];
-        ex |= 1u << at;
-        double ev, eq, eqi;
-        if (atom_intra(a, c, S, lane, at, ex, ev, eq, eqi)) {
-          intra_ov = 1;
-          break;
-        }
-        iv = __dadd_rn(iv, ev);
-        iq = __dadd_rn(iq, eq);
-        iqi = __dadd_rn(iqi, eqi);
-      }
-      S.tcom[lane] = com_of(c, S, lane, newx);
-    }
-    __syncthreads();
-    stage_inter<P, NT>(a, S, kd, self, true);
-    // the trial's energy and weight (fragment_growth.f90:2014-2056), one lane
-    // per trial; selection (:2074-2099) by wave 0
-    double w = 0.0, e = 0.0;
-    int wk = 1;
-    if (lane < kd) {
-      double ed = 0.0;
-      const int ov = intra_ov ? 2 : S.sov[lane];
-      if (!ov) {
-        const double qsum = __dadd_rn(iqi, S.sq[lane]);
-        ed = dihedral_energy(c, S, lane, S.exist);
-        e = __dsub_rn(__dadd_rn(__dadd_rn(__dadd_rn(__dadd_rn(ed, iv), iq), S.sv[lane]), qsum), e_prev);
-        const double bk = __dmul_rn(beta, e);
-        if (!(bk >= kMaxKBT)) {
-          w = exp(-bk);
-          wk = 0;
-        }
-      } else if (ov == 2) {
-        wk = 2;  // intramolecular overlap: the cumulative weight carries over
-      }
-      S.ndih[lane] = ed;
-    }
-    if (lane < 64) {
-      double wsum;
-      const int trial = select_trial(kd, w, wk, del_flag, S.rng, wsum);
-      const double e_sel = trial >= 0 ? readlane_f64(e, trial) : 0.0;
-      if (lane == 0) {
-        if (trial < 0) {
-          S.flag = 1;
-        } else {
-          S.ln_pbias = __dsub_rn(__dsub_rn(S.ln_pbias, __dmul_rn(beta, e_sel)), log(wsum));
-          for (int p = 0; p < S.ntatom; ++p) {
-            const int at = S.tatom[p];
-            S.x[at] = S.tx[trial][p];
-            S.y[at] = S.ty[trial][p];
-            S.z[at] = S.tz[trial][p];
-          }
-          S.trial = trial;
-          S.placed[S.order[i]] = 1;
-        }
-      }
-    }
-    __syncthreads();
-    if (S.flag) return;
-    e_prev = S.ndih[S.trial];
-  }
-}
-
-// ln_pbias of the caller after Build_Molecule (widom_insert.f90:361-370,
-// move_insert.f90:166-180, move_delete.f90:196-210)
-__device__ inline double ln_pbias_total(const CbmcSpeciesDev &c, double ln_pbias, double ln_pseq) {
-  double v = __dadd_rn(ln_pbias, ln_pseq);
-  v = __dadd_rn(v, log((double)c.kappa_ins));
-  if (c.kappa_rot != 0) v = __dadd_rn(v, log((double)c.kappa_rot));
-  if (c.kappa_dih != 0) v = __dadd_rn(v, __dmul_rn((double)(c.nfrag - 1), log((double)c.kappa_dih)));
-  return v;
-}
-
-// Fold_Molecule (minimum_image_separation.f90:162-260), cubic boxes; thread 0.
-template <int NT>
-__device__ void fold_molecule(const GrowArgs &a, GrowLds<NT> &S) {
-  if (!a.b.cubic) return;
-  const CbmcSpeciesDev &c = S.sp;
-  double *r[3] = {S.x, S.y, S.z};
-  double *cm[3] = {&S.com.x, &S.com.y, &S.com.z};
-  for (int d = 0; d < 3; ++d) {
-    const double L = a.b.L[d], h = a.b.hL[d];
-    if (*cm[d] > h) {
-      *cm[d] = __dsub_rn(*cm[d], L);
-      for (int k = 0; k < c.natoms; ++k) r[d][k] = __dsub_rn(r[d][k], L);
-    } else if (*cm[d] < -h) {
-      *cm[d] = __dadd_rn(*cm[d], L);
-      for (int k = 0; k < c.natoms; ++k) r[d][k] = __dadd_rn(r[d][k], L);
-    }
-  }
-}
-
-// The whole grown molecule as the stage (for the full-cutoff energy).
-template <int NT>
-__device__ void stage_whole(const CbmcSpeciesDev &c, GrowLds<NT> &S) {
-  S.ntatom = c.natoms;
-  for (int k = 0; k < c.natoms; ++k) {
-    S.tatom[k] = k;
-    S.tspa[k] = c.spa0 + k;
-    S.tpos[k] = -1;
-    S.tx[0][k] = S.x[k];
-    S.ty[0][k] = S.y[k];
-    S.tz[0][k] = S.z[k];
-  }
-  S.tcom[0] = S.com;
-}
-
-// ---------------------------------------------------------------- Widom
-struct WidomCbmcArgs {
-  GrowArgs g;
-  int64_t n_ins;
-  uint64_t seed;
-  int sequential;       // one workgroup, the reference's stream in rng
-  int64_t *rng;         // 5 words (sequential mode), in/out
-  double e_const;       // lrc_diff + E_self - E_recip_in
-  double *wvar;         // [n_ins]
-  uint8_t *over;        // [n_ins]
-  double *eij_max;      // [n_ins] or null: est_emax's Eij_max (0 where over)
-  double *rsq_min;      // [n_ins][rsq_rows][natoms] or null: closest r^2 per
-  int rsq_rows;         // (species site, inserted atom), 10000 if none in range
-};
-
-// The per-insertion LFSR of the parallel mode: five components from
-// (seed, insertion), each with the bits its shift masks keep non-zero.
-__device__ inline void seed_stream(int64_t *s, uint64_t seed, uint64_t i) {
-  const int64_t lo[5] = {2, 512, 4096, 131072, 8388608};
-  for (int k = 0; k < 5; ++k) {
-    const uint64_t h = mix64(mix64(seed ^ (i * 0xD1B54A32D192ED03ull)) + 0x9E37ull * (uint64_t)(k + 1));
-    s[k] = (int64_t)(h | (uint64_t)lo[k] << 1);
-  }
-}
-
-template <typename P, int NT>
-__global__ void __launch_bounds__(NT) k_widom_cbmc(WidomCbmcArgs w) {
-  __shared__ GrowLds<NT> S;
-  const CbmcSpeciesDev &c = S.sp;
-  const int lane = threadIdx.x;
-  const int64_t i0 = w.sequential ? 0 : (int64_t)blockIdx.x;
-  const int64_t i1 = w.sequential ? w.n_ins : i0 + 1;
-  load_tables(S, w.g.sp, w.g.tp);
-  if (lane == 0) {
-    if (w.sequential)
-      for (int k = 0; k < 5; ++k) S.rng[k] = vld(w.rng + k);
-    else
-      seed_stream(S.rng, w.seed, (uint64_t)i0);
-  }
-  __syncthreads();
-  for (int64_t i = i0; i < i1; ++i) {
-    build_molecule<P, NT>(w.g, S, -1, false);
-    // the full-cutoff energy of the grown molecule (widom_insert.f90:378-399)
-    int cov = S.flag;
-    if (w.rsq_min) {
-      // swi_atompair_rsqmin = 10000 for every insertion (widom_insert.f90:325)
-      double *rm = w.rsq_min + i * (int64_t)w.rsq_rows * c.natoms;
-      for (int k = lane; k < w.rsq_rows * c.natoms; k += NT) rm[k] = 10000.0;
-      if (lane == 0) S.rsq = rm;
-    } else if (lane == 0) {
-      S.rsq = nullptr;
-    }
-    if (!cov && lane == 0) {
-      for (int k = 0; k < c.natoms; ++k) S.exist[k] = 1;
-      if (c.nfrag > 1) fold_molecule(w.g, S);
-      stage_whole(c, S);
-    }
-    __syncthreads();
-    if (!cov) stage_inter<P, NT, true>(w.g, S, 1, -1, false);
-    double iv = 0.0, iq = 0.0, ip = 0.0, e_ang = 0.0, e_dih = 0.0;
-    bool intra_ov = false;
-    if (!cov && lane < 64) intra_ov = mol_terms_wave(w.g, c, S, iv, iq, ip, e_ang, e_dih);
-    if (lane == 0) {
-      double wv = 0.0;
-      int ov = 1;
-      if (!cov && !S.sov[0]) {
-        if (!intra_ov) {
-          const double e_inter = __dadd_rn(__dadd_rn(S.sv[0], S.sq[0]), ip);
-          const double ln_pbias = ln_pbias_total(c, S.ln_pbias, S.ln_pseq);
-          const double de_inter = __dadd_rn(e_inter, w.e_const);
-          double de_intra = __dadd_rn(iv, iq);
-          de_intra = __dadd_rn(__dadd_rn(__dadd_rn(__dadd_rn(de_intra, 0.0), e_ang), e_dih), 0.0);
-          const double de = __dadd_rn(de_intra, de_inter);
-          const double de_frag = __dadd_rn(e_ang, 0.0);
-          wv = exp(__dsub_rn(-__dmul_rn(w.g.beta, __dsub_rn(de, de_frag)), ln_pbias));
-          ov = 0;
-        }
-      }
-      w.wvar[i] = wv;
-      w.over[i] = (uint8_t)ov;
-      if (w.eij_max) w.eij_max[i] = ov ? 0.0 : S.sem;
-    }
-    __syncthreads();
-  }
-  if (w.sequential && lane == 0)
-    for (int k = 0; k < 5; ++k) w.rng[k] = S.rng[k];
+// The frame's live molecules, listed once for all insertions of a batch (one
+// wave).
+__global__ void __launch_bounds__(64) k_widom_live(GrowArgs g, LiveList l, int *nlive) {
+  const int n = build_live_list<64>(g, l);
+  if (threadIdx.x == 0) *nlive = n;
 }
 
 // Fixed-order sums of the insertions: widom_sum, overlaps and the
@@ -1327,760 +53,6 @@ __global__ void __launch_bounds__(256) k_widom_cbmc_sum(const double *wvar, cons
       if (k == nsub) out[nsub + 1] = (double)shn[0];
     }
     __syncthreads();
-  }
-}
-
-// ----------------------------------------------------------------- GCMC
-// Per box of the chain kernel.
-struct GcmcBoxArgs {
-  GrowArgs g;
-  double *x, *y, *z;  // the box's coordinates (the memory of g.b.x/y/z)
-  double4 *comd;      // (COM, max_dcom) per slot
-  int *live;          // per slot
-  int first_slot, max_mols;
-  double prob_insert, mu, lambda, log_volume;
-  // state, in/out
-  int64_t *rng;       // 5
-  double *energy;     // cass_energy as 14 doubles
-  int *nmols, *nres, *locate, *reservoir;
-  double *nbeads;     // per type
-  double volume, rcut3, rcut9, rcut_vdw;
-  int vdw_style, tail;
-  int commit;  // 0: a timing run that leaves the box untouched
-  // records [nsteps] per box, or null
-  uint8_t *kind, *accepted;
-  int *rec_nmols;
-  double *rec_energy;
-  int64_t *rec_rng;
-};
-
-enum { kE_total = 0, kE_intra, kE_inter, kE_bond, kE_angle, kE_dihedral, kE_improper, kE_intra_vdw, kE_intra_q,
-       kE_inter_vdw, kE_lrc, kE_inter_q, kE_reciprocal, kE_self };
-
-// Compute_LR_Correction (energy_routines.f90:2956-3023) at bead counts nb.
-__device__ double lrc_device(const GcmcBoxArgs &a, const double *nb) {
-  const TopoDev &tp = a.g.tp;
-  const int nt = tp.ntypes;
-  double el = 0.0;
-  if (a.vdw_style == CASS_VDW_LJ) {
-    for (int i = 0; i < nt; ++i) {
-      double eij = 0.0;
-      for (int j = 0; j < nt; ++j) {
-        const double eps = tp.eps[i * nt + j], sig = tp.sig[i * nt + j];
-        const double s2 = __dmul_rn(sig, sig), s6 = __dmul_rn(__dmul_rn(s2, s2), s2), s12 = __dmul_rn(s6, s6);
-        const double br = __dsub_rn(__ddiv_rn(s12, __dmul_rn(9.0, a.rcut9)), __ddiv_rn(s6, __dmul_rn(3.0, a.rcut3)));
-        eij = __dadd_rn(eij, __dmul_rn(__dmul_rn(__dmul_rn(nb[j], 4.0), eps), br));
-      }
-      el = __dadd_rn(el, __dmul_rn(nb[i], eij));
-    }
-    return __ddiv_rn(__dmul_rn(__dmul_rn(2.0, kPi), el), a.volume);
-  }
-  return 0.0;
-}
-
-template <typename P, int NT>
-__global__ void __launch_bounds__(NT) k_gcmc_chain(const GcmcBoxArgs *__restrict__ boxes, int64_t nsteps,
-                                                   int64_t step0, int64_t rec_stride) {
-  __shared__ GrowLds<NT> S;
-  __shared__ double E[14];
-  __shared__ int q_nmols, q_nres, q_lm, q_kind, q_skip;
-  __shared__ double nb[64];
-  const GcmcBoxArgs &a = boxes[blockIdx.x];
-  const CbmcSpeciesDev &c = S.sp;
-  const int lane = threadIdx.x;
-  const int nt = a.g.tp.ntypes;
-  load_tables(S, a.g.sp, a.g.tp);
-  if (lane == 0) {
-    for (int k = 0; k < 5; ++k) S.rng[k] = vld(a.rng + k);
-    for (int k = 0; k < 14; ++k) E[k] = vld(a.energy + k);
-    q_nmols = vld(a.nmols);
-    q_nres = vld(a.nres);
-    for (int k = 0; k < nt; ++k) nb[k] = vld(a.nbeads + k);
-  }
-  __syncthreads();
-  const double beta = a.g.beta;
-  for (int64_t st = 0; st < nsteps; ++st) {
-    // the move draw, the species draw and the molecule slot
-    if (lane == 0) {
-      const double u = cb_uniform(S.rng);
-      q_kind = u <= a.prob_insert ? 0 : 1;
-      (void)cb_uniform(S.rng);  // is_rand: one sorbate species (move_insert.f90:108, move_delete.f90:99)
-      q_skip = 0;
-      if (q_kind == 0) {
-        if (q_nres == 0) {
-          q_skip = 2;  // max_molecules reached: the reference aborts
-        } else {
-          q_lm = vld(a.reservoir + q_nres - 1);
-          q_nres--;
-          a.locate[q_nmols] = q_lm;
-          q_nmols++;
-          for (int k = 0; k < c.natoms; ++k) S.exist[k] = 0;
-        }
-      } else {
-        if (q_nmols == 0) {
-          q_skip = 1;
-        } else {
-          const int im = min((int)(cb_uniform(S.rng) * q_nmols), q_nmols - 1);
-          q_lm = vld(a.locate + im);
-          S.trial = im;
-          const int m = a.first_slot + q_lm, f = a.g.b.first[m];
-          for (int k = 0; k < c.natoms; ++k) {
-            S.x[k] = vld(a.x + f + k);
-            S.y[k] = vld(a.y + f + k);
-            S.z[k] = vld(a.z + f + k);
-          }
-        }
-      }
-    }
-    __syncthreads();
-    if (q_skip == 2) break;
-    int acc = 0;
-    if (!q_skip) {
-      const int m = a.first_slot + q_lm;
-      const bool del = q_kind == 1;
-      const int im_del = S.trial;
-      build_molecule<P, NT>(a.g, S, m, del);
-      const int cov = S.flag;
-      if (lane == 0 && !cov) {
-        for (int k = 0; k < c.natoms; ++k) S.exist[k] = 1;
-        if (!del) fold_molecule(a.g, S);
-        S.com = com_of(c, S, -1, S.exist);
-        stage_whole(c, S);
-      }
-      __syncthreads();
-      if (!cov) stage_inter<P, NT>(a.g, S, 1, m, false);
-      // the whole molecule's intramolecular, angle and dihedral terms
-      double iv = 0.0, iq = 0.0, ip = 0.0, e_ang = 0.0, e_dih = 0.0;
-      bool intra_ov = false;
-      if (!cov && lane < 64) intra_ov = mol_terms_wave(a.g, c, S, iv, iq, ip, e_ang, e_dih);
-      if (lane == 0) {
-        if (del && cov) {
-          q_skip = 2;  // the molecule to delete cannot be regrown: the reference aborts
-        } else if (!del) {
-          // Insertion (move_insert.f90:186-351)
-          if (cov || S.sov[0] || intra_ov) {
-            q_nmols--;
-            a.reservoir[q_nres++] = q_lm;
-          } else {
-            const double ev = S.sv[0], eq = __dadd_rn(S.sq[0], ip);
-            double de_inter = __dadd_rn(ev, eq), de_intra = __dadd_rn(iv, iq);
-            de_intra = __dadd_rn(__dadd_rn(__dadd_rn(__dadd_rn(de_intra, 0.0), e_ang), e_dih), 0.0);
-            double e_lrc = 0.0, nb2[64];
-            if (a.tail) {
-              for (int k = 0; k < nt; ++k) nb2[k] = nb[k];
-              for (int k = 0; k < c.natoms; ++k)
-                if (c.type[k] >= 0) nb2[c.type[k]] = __dadd_rn(nb2[c.type[k]], 1.0);
-              e_lrc = lrc_device(a, nb2);
-              de_inter = __dsub_rn(__dadd_rn(de_inter, e_lrc), E[kE_lrc]);
-            }
-            const double de = __dadd_rn(de_intra, de_inter);
-            const double de_frag = __dadd_rn(e_ang, 0.0);
-            const double ln_pbias = ln_pbias_total(c, S.ln_pbias, S.ln_pseq);
-            double lp = __dmul_rn(beta, __dsub_rn(de, de_frag));
-            lp = __dsub_rn(lp, __dmul_rn(a.mu, beta));
-            lp = __dadd_rn(lp, ln_pbias);
-            lp = __dadd_rn(__dadd_rn(lp, log((double)q_nmols)), __dmul_rn(3.0, log(a.lambda)));
-            lp = __dsub_rn(lp, a.log_volume);
-            // accept_or_reject (accept_or_reject.f90:22-65)
-            if (lp <= 0.0) acc = 1;
-            else if (lp < kMaxKBT && cb_uniform(S.rng) <= exp(-lp)) acc = 1;
-            if (acc) {
-              E[kE_total] = __dadd_rn(E[kE_total], de);
-              E[kE_intra] = __dadd_rn(E[kE_intra], de_intra);
-              E[kE_inter] = __dadd_rn(E[kE_inter], de_inter);
-              E[kE_angle] = __dadd_rn(E[kE_angle], e_ang);
-              E[kE_dihedral] = __dadd_rn(E[kE_dihedral], e_dih);
-              E[kE_intra_vdw] = __dadd_rn(E[kE_intra_vdw], iv);
-              E[kE_intra_q] = __dadd_rn(E[kE_intra_q], iq);
-              E[kE_inter_vdw] = __dadd_rn(E[kE_inter_vdw], ev);
-              E[kE_inter_q] = __dadd_rn(E[kE_inter_q], eq);
-              if (a.tail) {
-                E[kE_lrc] = e_lrc;
-                for (int k = 0; k < nt; ++k) nb[k] = nb2[k];
-              }
-              if (a.commit) {
-                const int f = a.g.b.first[m];
-                for (int k = 0; k < c.natoms; ++k) {
-                  a.x[f + k] = S.x[k];
-                  a.y[f + k] = S.y[k];
-                  a.z[f + k] = S.z[k];
-                }
-                a.comd[m] = S.com;
-                a.live[m] = 1;
-              }
-            } else {
-              q_nmols--;
-              a.reservoir[q_nres++] = q_lm;
-            }
-          }
-        } else {
-          // Deletion (move_delete.f90:196-330); the grown coordinates (trial 1
-          // of every stage) replace the stored ones as in the reference
-          if (a.commit) {
-            const int f = a.g.b.first[m];
-            for (int k = 0; k < c.natoms; ++k) {
-              a.x[f + k] = S.x[k];
-              a.y[f + k] = S.y[k];
-              a.z[f + k] = S.z[k];
-            }
-            a.comd[m] = S.com;
-          }
-          const double ev = S.sv[0];
-          double eq = S.sq[0];
-          double de_inter = __dsub_rn(-ev, eq);
-          double de_intra = __dsub_rn(__dsub_rn(__dsub_rn(-0.0, e_ang), e_dih), 0.0);
-          eq = __dadd_rn(eq, ip);
-          de_intra = __dsub_rn(__dsub_rn(de_intra, iv), iq);
-          de_inter = __dsub_rn(de_inter, ip);
-          double e_lrc = 0.0, nb2[64];
-          if (a.tail) {
-            for (int k = 0; k < nt; ++k) nb2[k] = nb[k];
-            for (int k = 0; k < c.natoms; ++k)
-              if (c.type[k] >= 0) nb2[c.type[k]] = __dsub_rn(nb2[c.type[k]], 1.0);
-            e_lrc = lrc_device(a, nb2);
-            de_inter = __dadd_rn(de_inter, __dsub_rn(e_lrc, E[kE_lrc]));
-          }
-          const double de = __dadd_rn(de_intra, de_inter);
-          const double de_frag = __dsub_rn(-e_ang, 0.0);
-          const double ln_pbias = ln_pbias_total(c, S.ln_pbias, S.ln_pseq);
-          double lp = __dmul_rn(beta, __dsub_rn(de, de_frag));
-          lp = __dadd_rn(lp, __dmul_rn(beta, a.mu));
-          lp = __dsub_rn(lp, ln_pbias);
-          lp = __dsub_rn(__dsub_rn(lp, log((double)q_nmols)), __dmul_rn(3.0, log(a.lambda)));
-          lp = __dadd_rn(lp, a.log_volume);
-          if (lp <= 0.0) acc = 1;
-          else if (lp < kMaxKBT && cb_uniform(S.rng) <= exp(-lp)) acc = 1;
-          if (acc) {
-            E[kE_total] = __dadd_rn(E[kE_total], de);
-            E[kE_intra] = __dadd_rn(E[kE_intra], de_intra);
-            E[kE_inter] = __dadd_rn(E[kE_inter], de_inter);
-            E[kE_angle] = __dsub_rn(E[kE_angle], e_ang);
-            E[kE_dihedral] = __dsub_rn(E[kE_dihedral], e_dih);
-            E[kE_intra_vdw] = __dsub_rn(E[kE_intra_vdw], iv);
-            E[kE_intra_q] = __dsub_rn(E[kE_intra_q], iq);
-            E[kE_inter_vdw] = __dsub_rn(E[kE_inter_vdw], ev);
-            E[kE_inter_q] = __dsub_rn(E[kE_inter_q], eq);
-            if (a.tail) {
-              E[kE_lrc] = e_lrc;
-              for (int k = 0; k < nt; ++k) nb[k] = nb2[k];
-            }
-            for (int k = im_del + 1; k < q_nmols; ++k) a.locate[k - 1] = vld(a.locate + k);
-            q_nmols--;
-            a.reservoir[q_nres++] = q_lm;
-            if (a.commit) a.live[m] = 0;
-          }
-        }
-      }
-    }
-    __syncthreads();
-    if (q_skip == 2) break;
-    if (lane == 0) {
-      const int64_t r = step0 + st;
-      if (a.kind) a.kind[r] = (uint8_t)q_kind;
-      if (a.accepted) a.accepted[r] = (uint8_t)acc;
-      if (a.rec_nmols) a.rec_nmols[r] = q_nmols;
-      if (a.rec_energy) a.rec_energy[r] = E[kE_total];
-      if (a.rec_rng)
-        for (int k = 0; k < 5; ++k) a.rec_rng[5 * r + k] = S.rng[k];
-    }
-    __syncthreads();
-  }
-  if (lane == 0) {
-    for (int k = 0; k < 5; ++k) a.rng[k] = S.rng[k];
-    for (int k = 0; k < 14; ++k) a.energy[k] = E[k];
-    *a.nmols = q_nmols;
-    *a.nres = q_skip == 2 ? -1 : q_nres;
-    for (int k = 0; k < nt; ++k) a.nbeads[k] = nb[k];
-  }
-  (void)rec_stride;
-}
-
-// ----------------------------------------------------------------- GEMC
-// GEMC_Particle_Transfer (move_mol_swap.f90:22-769) between the two boxes of
-// a pair, one workgroup per pair running the pair's whole sequence of moves
-// (gemc_driver.f90:91-195 with transfers only: one move draw each).  Per
-// move: box_out by molecule fraction, box_in the other box, the species draw
-// (one sorbate), the molecule; Build_Molecule into box_in drawing the
-// fragment order, its energies there (a core overlap of the grown molecule
-// rejects); then the reverse Build_Molecule in box_out with the same order,
-// its energies, and the acceptance with ln_pfor - ln_prev and
-// log(P_forward / P_reverse).  The box_out molecule keeps its re-placed
-// coordinates when rejected, as in the reference.  The pair's boxes are
-// boxes[2 * blockIdx.x] and the next; the generator is the first box's.
-template <typename P, int NT>
-__global__ void __launch_bounds__(NT) k_gemc_chain(const GcmcBoxArgs *__restrict__ boxes, int64_t nsteps) {
-  __shared__ GrowLds<NT> S;
-  __shared__ double E[2][14];
-  __shared__ double nb[2][64];
-  __shared__ int q_nmols[2], q_nres[2], q_bo, q_im, q_lm_out, q_lm_in, q_skip, q_go;
-  __shared__ double xo[kCbA], yo[kCbA], zo[kCbA], xn[kCbA], yn[kCbA], zn[kCbA];
-  __shared__ double4 com_new;
-  __shared__ double q_pf, q_pr, q_ln_pfor, t_in[9];
-  const GcmcBoxArgs *A = boxes + 2 * blockIdx.x;
-  const CbmcSpeciesDev &c = S.sp;
-  const int lane = threadIdx.x;
-  const int nt = A[0].g.tp.ntypes;
-  load_tables(S, A[0].g.sp, A[0].g.tp);
-  if (lane == 0) {
-    for (int k = 0; k < 5; ++k) S.rng[k] = vld(A[0].rng + k);
-    for (int b = 0; b < 2; ++b) {
-      for (int k = 0; k < 14; ++k) E[b][k] = vld(A[b].energy + k);
-      q_nmols[b] = vld(A[b].nmols);
-      q_nres[b] = vld(A[b].nres);
-      for (int k = 0; k < nt; ++k) nb[b][k] = vld(A[b].nbeads + k);
-    }
-  }
-  __syncthreads();
-  for (int64_t st = 0; st < nsteps; ++st) {
-    // Steps 1-3: the draws, box_in's free slot, the molecule's coordinates
-    if (lane == 0) {
-      (void)cb_uniform(S.rng);  // the move draw: transfers only
-      q_skip = 0;
-      const int tot = q_nmols[0] + q_nmols[1];
-      if (tot == 0) {
-        q_skip = 2;  // no swappable molecules: the reference aborts
-      } else {
-        const double x0 = __ddiv_rn((double)q_nmols[0], (double)tot);
-        const int bo = cb_uniform(S.rng) <= x0 ? 0 : 1;  // x_box(2) = 1
-        const int bi = 1 - bo;
-        q_bo = bo;
-        (void)cb_uniform(S.rng);  // box_in: the other box of two (:202-204)
-        const double no = (double)q_nmols[bo], ni1 = (double)(q_nmols[bi] + 1);
-        double pf = __ddiv_rn(__dmul_rn(1.0, no), (double)tot);
-        double pr = __ddiv_rn(__dmul_rn(1.0, ni1), (double)tot);
-        (void)cb_uniform(S.rng);  // the species: x_is(1) = 1
-        q_pf = __ddiv_rn(__dmul_rn(pf, no), no);
-        q_pr = __ddiv_rn(__dmul_rn(pr, ni1), ni1);
-        const int im = min((int)(cb_uniform(S.rng) * q_nmols[bo]), q_nmols[bo] - 1);
-        q_im = im;
-        q_lm_out = vld(A[bo].locate + im);
-        const int f = A[bo].g.b.first[A[bo].first_slot + q_lm_out];
-        for (int k = 0; k < c.natoms; ++k) {
-          xo[k] = vld(A[bo].x + f + k);
-          yo[k] = vld(A[bo].y + f + k);
-          zo[k] = vld(A[bo].z + f + k);
-        }
-        if (q_nres[bi] == 0) {
-          q_skip = 2;  // box_in has no free slot
-        } else {
-          q_lm_in = vld(A[bi].reservoir + q_nres[bi] - 1);
-          q_nres[bi]--;
-          A[bi].locate[q_nmols[bi]] = q_lm_in;
-          q_nmols[bi]++;
-        }
-      }
-    }
-    __syncthreads();
-    if (q_skip == 2) break;
-    const int bo = q_bo, bi = 1 - bo;
-    const GcmcBoxArgs &Ai = A[bi], &Ao = A[bo];
-    const int m_in = Ai.first_slot + q_lm_in, m_out = Ao.first_slot + q_lm_out;
-    int acc = 0;
-    // Step 4: the molecule grown into box_in
-    build_molecule<P, NT>(Ai.g, S, m_in, false);
-    const int cov = S.flag;
-    if (lane == 0 && !cov) {
-      for (int k = 0; k < c.natoms; ++k) S.exist[k] = 1;
-      S.com = com_of(c, S, -1, S.exist);
-      fold_molecule(Ai.g, S);
-      stage_whole(c, S);
-    }
-    __syncthreads();
-    if (!cov) stage_inter<P, NT>(Ai.g, S, 1, m_in, false);
-    double iv = 0.0, iq = 0.0, ip = 0.0, e_ang = 0.0, e_dih = 0.0;
-    if (!cov && lane < 64) (void)mol_terms_wave(Ai.g, c, S, iv, iq, ip, e_ang, e_dih);
-    // Step 5: box_in's change (intra_overlap is not acted on, :375-393)
-    if (lane == 0) {
-      q_go = 0;
-      if (cov || S.sov[0]) {
-        q_nmols[bi]--;
-        A[bi].reservoir[q_nres[bi]++] = q_lm_in;
-      } else {
-        const double ev = S.sv[0];
-        double eq = S.sq[0];
-        double de_inter = __dadd_rn(ev, eq);
-        double de_intra = __dadd_rn(__dadd_rn(__dadd_rn(0.0, e_ang), e_dih), 0.0);
-        eq = __dadd_rn(eq, ip);
-        de_intra = __dadd_rn(__dadd_rn(de_intra, iv), iq);
-        de_inter = __dadd_rn(de_inter, ip);
-        double lrc_in = 0.0;
-        if (Ai.tail) {
-          double nb2[64];
-          for (int k = 0; k < nt; ++k) nb2[k] = nb[bi][k];
-          for (int k = 0; k < c.natoms; ++k)
-            if (c.type[k] >= 0) nb2[c.type[k]] = __dadd_rn(nb2[c.type[k]], 1.0);
-          lrc_in = lrc_device(Ai, nb2);
-          de_inter = __dsub_rn(__dadd_rn(de_inter, lrc_in), E[bi][kE_lrc]);
-        }
-        t_in[0] = de_intra;
-        t_in[1] = de_inter;
-        t_in[2] = e_ang;
-        t_in[3] = e_dih;
-        t_in[4] = iv;
-        t_in[5] = iq;
-        t_in[6] = ev;
-        t_in[7] = eq;
-        t_in[8] = lrc_in;
-        q_ln_pfor = S.ln_pbias;
-        for (int k = 0; k < c.natoms; ++k) {
-          xn[k] = S.x[k];
-          yn[k] = S.y[k];
-          zn[k] = S.z[k];
-          S.x[k] = xo[k];
-          S.y[k] = yo[k];
-          S.z[k] = zo[k];
-        }
-        com_new = S.com;
-        q_go = 1;
-      }
-    }
-    __syncthreads();
-    if (q_go) {
-      // Step 6: the reverse growth in box_out with the forward order
-      build_molecule<P, NT>(Ao.g, S, m_out, true, true);
-      if (lane == 0) {
-        for (int k = 0; k < c.natoms; ++k) S.exist[k] = 1;
-        if (S.flag) {
-          q_skip = 2;  // the molecule cannot be regrown in box_out: the reference aborts
-        } else {
-          S.com = com_of(c, S, -1, S.exist);
-          stage_whole(c, S);
-        }
-      }
-      __syncthreads();
-      if (q_skip == 2) break;
-      stage_inter<P, NT>(Ao.g, S, 1, m_out, false);
-      double ivo = 0.0, iqo = 0.0, ipo = 0.0, ango = 0.0, diho = 0.0;
-      if (lane < 64) (void)mol_terms_wave(Ao.g, c, S, ivo, iqo, ipo, ango, diho);
-      if (lane == 0) {
-        const double evo = S.sv[0];
-        double eqo = S.sq[0];
-        double de_intra_o = __dsub_rn(__dsub_rn(__dsub_rn(-0.0, ango), diho), 0.0);
-        eqo = __dadd_rn(eqo, ipo);
-        de_intra_o = __dsub_rn(__dsub_rn(de_intra_o, ivo), iqo);
-        double de_inter_o = __dsub_rn(-evo, eqo);
-        double lrc_out = 0.0, nb3[64];
-        if (Ao.tail) {
-          for (int k = 0; k < nt; ++k) nb3[k] = nb[bo][k];
-          for (int k = 0; k < c.natoms; ++k)
-            if (c.type[k] >= 0) nb3[c.type[k]] = __dsub_rn(nb3[c.type[k]], 1.0);
-          lrc_out = lrc_device(Ao, nb3);
-          de_inter_o = __dadd_rn(de_inter_o, __dsub_rn(lrc_out, E[bo][kE_lrc]));
-        }
-        // Step 7 (:586-614)
-        const double de_in = __dadd_rn(t_in[0], t_in[1]);
-        const double de_out = __dadd_rn(de_intra_o, de_inter_o);
-        const double frag_in = __dadd_rn(t_in[2], 0.0), frag_out = __dsub_rn(-ango, 0.0);
-        double lp = __dadd_rn(__dmul_rn(Ai.g.beta, __dsub_rn(de_in, frag_in)),
-                              __dmul_rn(Ao.g.beta, __dsub_rn(de_out, frag_out)));
-        lp = __dadd_rn(__dsub_rn(lp, log((double)q_nmols[bo])), log((double)q_nmols[bi]));
-        lp = __dsub_rn(lp, Ai.log_volume);
-        lp = __dadd_rn(lp, Ao.log_volume);
-        lp = __dadd_rn(__dsub_rn(__dadd_rn(lp, q_ln_pfor), S.ln_pbias), log(__ddiv_rn(q_pf, q_pr)));
-        // accept_or_reject (accept_or_reject.f90:22-65)
-        if (lp <= 0.0) acc = 1;
-        else if (lp < kMaxKBT && cb_uniform(S.rng) <= exp(-lp)) acc = 1;
-        if (acc) {
-          for (int k = q_im + 1; k < q_nmols[bo]; ++k) Ao.locate[k - 1] = vld(Ao.locate + k);
-          q_nmols[bo]--;
-          Ao.reservoir[q_nres[bo]++] = q_lm_out;
-          E[bi][kE_total] = __dadd_rn(E[bi][kE_total], de_in);
-          E[bi][kE_intra] = __dadd_rn(E[bi][kE_intra], t_in[0]);
-          E[bi][kE_inter] = __dadd_rn(E[bi][kE_inter], t_in[1]);
-          E[bi][kE_angle] = __dadd_rn(E[bi][kE_angle], t_in[2]);
-          E[bi][kE_dihedral] = __dadd_rn(E[bi][kE_dihedral], t_in[3]);
-          E[bi][kE_intra_vdw] = __dadd_rn(E[bi][kE_intra_vdw], t_in[4]);
-          E[bi][kE_intra_q] = __dadd_rn(E[bi][kE_intra_q], t_in[5]);
-          E[bi][kE_inter_vdw] = __dadd_rn(E[bi][kE_inter_vdw], t_in[6]);
-          E[bi][kE_inter_q] = __dadd_rn(E[bi][kE_inter_q], t_in[7]);
-          E[bo][kE_total] = __dadd_rn(E[bo][kE_total], de_out);
-          E[bo][kE_intra] = __dadd_rn(E[bo][kE_intra], de_intra_o);
-          E[bo][kE_inter] = __dadd_rn(E[bo][kE_inter], de_inter_o);
-          E[bo][kE_angle] = __dsub_rn(E[bo][kE_angle], ango);
-          E[bo][kE_dihedral] = __dsub_rn(E[bo][kE_dihedral], diho);
-          E[bo][kE_intra_vdw] = __dsub_rn(E[bo][kE_intra_vdw], ivo);
-          E[bo][kE_intra_q] = __dsub_rn(E[bo][kE_intra_q], iqo);
-          E[bo][kE_inter_vdw] = __dsub_rn(E[bo][kE_inter_vdw], evo);
-          E[bo][kE_inter_q] = __dsub_rn(E[bo][kE_inter_q], eqo);
-          for (int k = 0; k < c.natoms; ++k)
-            if (c.type[k] >= 0) {
-              nb[bi][c.type[k]] = __dadd_rn(nb[bi][c.type[k]], 1.0);
-              nb[bo][c.type[k]] = __dsub_rn(nb[bo][c.type[k]], 1.0);
-            }
-          if (Ai.tail) E[bi][kE_lrc] = t_in[8];
-          if (Ao.tail) E[bo][kE_lrc] = lrc_out;
-          if (Ai.commit) {
-            const int fi = Ai.g.b.first[m_in];
-            for (int k = 0; k < c.natoms; ++k) {
-              Ai.x[fi + k] = xn[k];
-              Ai.y[fi + k] = yn[k];
-              Ai.z[fi + k] = zn[k];
-            }
-            Ai.comd[m_in] = com_new;
-            Ai.live[m_in] = 1;
-            Ao.live[m_out] = 0;
-          }
-        } else {
-          q_nmols[bi]--;
-          A[bi].reservoir[q_nres[bi]++] = q_lm_in;
-          if (Ao.commit) {
-            const int fo = Ao.g.b.first[m_out];
-            for (int k = 0; k < c.natoms; ++k) {
-              Ao.x[fo + k] = S.x[k];
-              Ao.y[fo + k] = S.y[k];
-              Ao.z[fo + k] = S.z[k];
-            }
-            Ao.comd[m_out] = S.com;
-          }
-        }
-      }
-    }
-    __syncthreads();
-    if (lane == 0)
-      for (int b = 0; b < 2; ++b) {
-        const GcmcBoxArgs &a = A[b];
-        if (a.kind) a.kind[st] = (uint8_t)bo;
-        if (a.accepted) a.accepted[st] = (uint8_t)acc;
-        if (a.rec_nmols) a.rec_nmols[st] = q_nmols[b];
-        if (a.rec_energy) a.rec_energy[st] = E[b][kE_total];
-        if (a.rec_rng)
-          for (int k = 0; k < 5; ++k) a.rec_rng[5 * st + k] = S.rng[k];
-      }
-    __syncthreads();
-  }
-  if (lane == 0)
-    for (int b = 0; b < 2; ++b) {
-      const GcmcBoxArgs &a = A[b];
-      for (int k = 0; k < 5; ++k) a.rng[k] = S.rng[k];
-      for (int k = 0; k < 14; ++k) a.energy[k] = E[b][k];
-      *a.nmols = q_nmols[b];
-      *a.nres = q_skip == 2 ? -1 : q_nres[b];
-      for (int k = 0; k < nt; ++k) a.nbeads[k] = nb[b][k];
-    }
-}
-
-// ------------------------------------------------------------- regrowth
-// Per box of the regrowth chain kernel.
-struct RegrowBoxArgs {
-  GrowArgs g;
-  double *x, *y, *z;  // the box's coordinates (the memory of g.b.x/y/z)
-  double4 *comd;      // (COM, max_dcom) per slot
-  int first_slot, nmols;
-  const int *locate;  // [nmols] slot offsets from first_slot
-  // state, in/out
-  int64_t *rng;       // 5
-  double *energy;     // cass_energy as 14 doubles
-  int *status;        // 1: a molecule's own configuration could not be regrown
-  // records [nsteps] per box, or null
-  uint8_t *kind, *accepted;
-  double *rec_energy, *ln_pacc;
-  int64_t *rec_rng;
-};
-
-// Cut_Regrow's set-up (fragment_growth.f90:1118-1312); thread 0.  Outside
-// del_flag: the fragment bond to cut and the side to delete
-// (fragment_bond_list%prob_del1), and the dead fragments' order
-// (Fragment_Order from frag_dead with frag_live live).  Then every atom
-// exists but those of the ordered fragments, the two anchors of the cut
-// bond excepted, and the ordered fragments are not placed.
-template <int NT>
-__device__ void cut_regrow_setup(const CbmcSpeciesDev &c, GrowLds<NT> &S, bool del_flag, int &frag_live,
-                                 int &frag_dead) {
-  S.ln_pbias = 0.0;
-  S.ln_pseq = 0.0;
-  S.flag = 0;
-  if (!del_flag) {
-    // rranf can round to 1.0 (random_generators.f90:118): the index is clamped
-    const int fb = min((int)(cb_uniform(S.rng) * c.nfbond), c.nfbond - 1);
-    if (cb_uniform(S.rng) < c.prob_del1[fb]) {
-      frag_dead = c.fbond[fb][0];
-      frag_live = c.fbond[fb][1];
-    } else {
-      frag_dead = c.fbond[fb][1];
-      frag_live = c.fbond[fb][0];
-    }
-    int live[kCbF];
-    for (int f = 0; f < c.nfrag; ++f) live[f] = S.order[f] = 0;
-    live[frag_live] = 1;
-    S.order[0] = frag_dead;
-    S.ntotal = 1;
-    live[frag_dead] = 1;
-    fragment_order(c, S, frag_dead, live);
-  }
-  for (int k = 0; k < c.natoms; ++k) S.exist[k] = 1;
-  for (int f = 0; f < c.nfrag; ++f) S.placed[f] = 1;
-  for (int i = 0; i < S.ntotal; ++i) {
-    const int f = S.order[i];
-    S.placed[f] = 0;
-    for (int j = 0; j < c.frag_natoms[f]; ++j) S.exist[c.frag_atoms[f][j]] = 0;
-  }
-  S.exist[c.frag_anchor[frag_live]] = 1;
-  S.exist[c.frag_anchor[frag_dead]] = 1;
-}
-
-// Chains of Cut_N_Grow regrowth moves (move_regrow.f90:22-510), one
-// workgroup per box, the box's whole move loop in one launch: per move the
-// NVT driver's move draw, the box, species and molecule draws, the forward
-// regrowth of the cut-off end (folded into the box), its full-cutoff
-// energies, the reverse pass over the molecule's own configuration and the
-// acceptance with ln_pfor - ln_prev.  Accepted: the regrown coordinates
-// replace the molecule's; rejected after the reverse pass: its re-placed
-// coordinates do, as in the reference.
-template <typename P, int NT>
-__global__ void __launch_bounds__(NT) k_regrow_chain(const RegrowBoxArgs *__restrict__ boxes, int64_t nsteps) {
-  __shared__ GrowLds<NT> S;
-  __shared__ double E[14];
-  __shared__ double ox[kCbA], oy[kCbA], oz[kCbA], nx[kCbA], ny[kCbA], nz[kCbA];
-  __shared__ double4 ncom;
-  __shared__ double en[6];  // new: angle, dihedral, intra vdW, intra q, inter vdW, inter q
-  __shared__ double q_eprev, q_lpfor;
-  __shared__ int q_m, q_live, q_dead, q_state;  // q_state: 0 go on, 1 rejected, 2 stop
-  const RegrowBoxArgs &a = boxes[blockIdx.x];
-  const CbmcSpeciesDev &c = S.sp;
-  const int lane = threadIdx.x;
-  load_tables(S, a.g.sp, a.g.tp);
-  if (lane == 0) {
-    for (int k = 0; k < 5; ++k) S.rng[k] = vld(a.rng + k);
-    for (int k = 0; k < 14; ++k) E[k] = vld(a.energy + k);
-    q_state = 0;
-  }
-  __syncthreads();
-  const double beta = a.g.beta;
-  for (int64_t st = 0; st < nsteps; ++st) {
-    if (lane == 0) {
-      (void)cb_uniform(S.rng);  // the move draw (nvtmc_driver.f90:109): regrowth only
-      (void)cb_uniform(S.rng);  // the box (one box: x_box(1) = 1)
-      (void)cb_uniform(S.rng);  // the species (one regrowable species)
-      const int im = min((int)(cb_uniform(S.rng) * a.nmols), a.nmols - 1);
-      q_m = a.first_slot + a.locate[im];
-      const int f = a.g.b.first[q_m];
-      for (int k = 0; k < c.natoms; ++k) {
-        S.x[k] = ox[k] = vld(a.x + f + k);
-        S.y[k] = oy[k] = vld(a.y + f + k);
-        S.z[k] = oz[k] = vld(a.z + f + k);
-      }
-      cut_regrow_setup(c, S, false, q_live, q_dead);
-      q_eprev = dihedral_energy(c, S, -1, S.exist);  // E_prev of the remaining atoms
-      q_state = 0;
-    }
-    __syncthreads();
-    const int m = q_m;
-    fragment_placement<P, NT>(a.g, S, m, false, 0, q_eprev);
-    if (lane == 0) {
-      if (S.flag) {
-        q_state = 1;  // cbmc_overlap: the old coordinates stay
-      } else {
-        for (int k = 0; k < c.natoms; ++k) S.exist[k] = 1;
-        S.com = com_of(c, S, -1, S.exist);
-        fold_molecule(a.g, S);
-        stage_whole(c, S);
-        q_lpfor = S.ln_pbias;
-      }
-    }
-    __syncthreads();
-    if (q_state == 0) {
-      stage_inter<P, NT>(a.g, S, 1, m, false);
-      double iv = 0.0, iq = 0.0, ip = 0.0, ea = 0.0, ed = 0.0;
-      if (lane < 64) (void)mol_terms_wave(a.g, c, S, iv, iq, ip, ea, ed);  // intra_overlap is not acted on
-      if (lane == 0) {
-        if (S.sov[0]) {
-          q_state = 1;
-        } else {
-          en[0] = ea;
-          en[1] = ed;
-          en[2] = iv;
-          en[3] = iq;
-          en[4] = S.sv[0];
-          en[5] = __dadd_rn(S.sq[0], ip);
-          for (int k = 0; k < c.natoms; ++k) {
-            nx[k] = S.x[k];
-            ny[k] = S.y[k];
-            nz[k] = S.z[k];
-            S.x[k] = ox[k];
-            S.y[k] = oy[k];
-            S.z[k] = oz[k];
-          }
-          ncom = S.com;
-          cut_regrow_setup(c, S, true, q_live, q_dead);
-        }
-      }
-      __syncthreads();
-    }
-    if (q_state == 0) {
-      // the reverse pass over the molecule's own configuration
-      fragment_placement<P, NT>(a.g, S, m, true, 0, q_eprev);
-      if (lane == 0) {
-        if (S.flag) {
-          q_state = 2;  // the reference aborts
-        } else {
-          for (int k = 0; k < c.natoms; ++k) S.exist[k] = 1;
-          S.com = com_of(c, S, -1, S.exist);
-          stage_whole(c, S);
-        }
-      }
-      __syncthreads();
-    }
-    int acc = 0;
-    double lp = __longlong_as_double(0x7ff8000000000000ll);
-    if (q_state == 0) {
-      stage_inter<P, NT>(a.g, S, 1, m, false);
-      double iv = 0.0, iq = 0.0, ip = 0.0, ea = 0.0, ed = 0.0;
-      if (lane < 64) (void)mol_terms_wave(a.g, c, S, iv, iq, ip, ea, ed);
-      if (lane == 0) {
-        const double ev = S.sv[0], eq = __dadd_rn(S.sq[0], ip);
-        double de_intra = __dadd_rn(__dadd_rn(__dadd_rn(__dadd_rn(__dadd_rn(0.0, en[0]), en[1]), 0.0), en[3]), en[2]);
-        double de_inter = __dadd_rn(en[5], en[4]);
-        de_intra = __dsub_rn(__dsub_rn(__dsub_rn(__dsub_rn(__dsub_rn(__dsub_rn(de_intra, 0.0), ea), ed), 0.0), iq), iv);
-        de_inter = __dsub_rn(__dsub_rn(de_inter, eq), ev);
-        const double de = __dadd_rn(de_intra, de_inter);
-        const double de_frag = __dsub_rn(__dadd_rn(__dsub_rn(en[0], ea), 0.0), 0.0);
-        lp = __dsub_rn(__dadd_rn(__dmul_rn(beta, __dsub_rn(de, de_frag)), q_lpfor), S.ln_pbias);
-        // accept_or_reject (accept_or_reject.f90:22-65)
-        if (lp <= 0.0) acc = 1;
-        else if (lp < kMaxKBT && cb_uniform(S.rng) <= exp(-lp)) acc = 1;
-        const int f = a.g.b.first[m];
-        if (acc) {
-          E[kE_total] = __dadd_rn(E[kE_total], de);
-          E[kE_intra] = __dadd_rn(E[kE_intra], de_intra);
-          E[kE_inter] = __dadd_rn(E[kE_inter], de_inter);
-          E[kE_angle] = __dsub_rn(__dadd_rn(E[kE_angle], en[0]), ea);
-          E[kE_dihedral] = __dsub_rn(__dadd_rn(E[kE_dihedral], en[1]), ed);
-          E[kE_intra_vdw] = __dsub_rn(__dadd_rn(E[kE_intra_vdw], en[2]), iv);
-          E[kE_intra_q] = __dsub_rn(__dadd_rn(E[kE_intra_q], en[3]), iq);
-          E[kE_inter_vdw] = __dsub_rn(__dadd_rn(E[kE_inter_vdw], en[4]), ev);
-          E[kE_inter_q] = __dsub_rn(__dadd_rn(E[kE_inter_q], en[5]), eq);
-          for (int k = 0; k < c.natoms; ++k) {
-            a.x[f + k] = nx[k];
-            a.y[f + k] = ny[k];
-            a.z[f + k] = nz[k];
-          }
-          a.comd[m] = ncom;
-        } else {
-          for (int k = 0; k < c.natoms; ++k) {
-            a.x[f + k] = S.x[k];
-            a.y[f + k] = S.y[k];
-            a.z[f + k] = S.z[k];
-          }
-          a.comd[m] = S.com;
-        }
-      }
-    }
-    __syncthreads();
-    if (q_state == 2) break;
-    if (lane == 0) {
-      if (a.kind) a.kind[st] = 2;
-      if (a.accepted) a.accepted[st] = (uint8_t)acc;
-      if (a.rec_energy) a.rec_energy[st] = E[kE_total];
-      if (a.ln_pacc) a.ln_pacc[st] = lp;
-      if (a.rec_rng)
-        for (int k = 0; k < 5; ++k) a.rec_rng[5 * st + k] = S.rng[k];
-    }
-    __syncthreads();
-  }
-  if (lane == 0) {
-    for (int k = 0; k < 5; ++k) a.rng[k] = S.rng[k];
-    for (int k = 0; k < 14; ++k) a.energy[k] = E[k];
-    *a.status = q_state == 2 ? 1 : 0;
   }
 }
 
@@ -2241,6 +213,22 @@ extern "C" int cass_cbmc_set_species(cass_engine *e, int32_t species, const cass
     c.qs[a] = e->q_scale[po + a];
     c.bonded[a] = e->bonded[po + a];
   }
+  for (int f = 0; f < kCbF; ++f) c.frag_mask[f] = 0;
+  for (int f = 0; f < c.nfrag; ++f)
+    for (int j = 0; j < c.frag_natoms[f]; ++j) c.frag_mask[f] |= 1u << c.frag_atoms[f][j];
+  for (int d = 0; d < c.ndihed; ++d) {
+    c.dihed_mask[d] = 0;
+    for (int q = 0; q < 4; ++q) c.dihed_mask[d] |= 1u << c.dihed[d][q];
+  }
+  for (int a = 0, p = 0; a < n; ++a) {
+    c.intra_mask[a] = 0;
+    for (int b = 0; b < n; ++b)
+      if (c.vs[a * n + b] > 0.0 || c.qs[a * n + b] > 0.0) c.intra_mask[a] |= 1u << b;
+    for (int b = a + 1; b < n; ++b, ++p) {
+      c.pair_i[p] = (uint8_t)a;
+      c.pair_j[p] = (uint8_t)b;
+    }
+  }
   HIP_TRY(e, hipSetDevice(e->device));
   if (hipMalloc(&hs.lib, sizeof(double) * std::max<long long>(lk, 1)) != hipSuccess ||
       hipMalloc(&hs.d, sizeof(CbmcSpeciesDev)) != hipSuccess)
@@ -2335,13 +323,29 @@ static GrowArgs grow_args(cass_engine *e, cass_box_state &b, const CbmcHostSpeci
   return g;
 }
 
-template <int NT>
-static int launch_widom_cbmc(cass_engine *e, const WidomCbmcArgs &w, int grid) {
-  auto kern = e->prec == CASS_PREC_MIXED  ? k_widom_cbmc<PrecMixed, NT>
-              : e->prec == CASS_PREC_FP32 ? k_widom_cbmc<PrecFP32, NT>
-                                          : k_widom_cbmc<PrecFP64, NT>;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), 0, e->stream, w);
-  return hipGetLastError() == hipSuccess ? CASS_OK : cass_fail(e, CASS_ERR_HIP, "k_widom_cbmc launch");
+// Whether a grown species' pairs in box b are plain LJ (the LJ kernels): LJ
+// cut / cut_tail / cut_shift, no CBMC energy table, no q-q terms of the
+// species, and a topology within the LDS tables.
+static bool lj_growth(const cass_engine *e, const cass_box_state &b, int species) {
+  const cass_params &p = b.p;
+  return p.vdw_style == CASS_VDW_LJ &&
+         (p.vdw_sum_style == CASS_SUM_CUT || p.vdw_sum_style == CASS_SUM_CUT_TAIL ||
+          p.vdw_sum_style == CASS_SUM_CUT_SHIFT) &&
+         !b.apt && (p.charge_style == CASS_Q_NONE || !species_has_charge(e, species)) && e->nspecies <= kCtSp &&
+         e->natoms_total <= kCtAt && e->ntypes <= kCtT;
+}
+
+static CbmcKernels growth_kernels(const cass_engine *e, bool lj) {
+  if (e->prec == CASS_PREC_MIXED) return lj ? cbmc_kernels_mixed_lj() : cbmc_kernels_mixed_any();
+  if (e->prec == CASS_PREC_FP32) return lj ? cbmc_kernels_fp32_lj() : cbmc_kernels_fp32_any();
+  return lj ? cbmc_kernels_fp64_lj() : cbmc_kernels_fp64_any();
+}
+
+// Index of a GCMC workgroup size (128 << k lanes).
+static int lanes_index(int nt) {
+  int k = 0;
+  while (128 << k < nt) ++k;
+  return k;
 }
 
 static int widom_cbmc(cass_engine *e, int32_t box, int32_t species, int64_t n_ins, cass_rng *rng, uint64_t seed,
@@ -2356,7 +360,6 @@ static int widom_cbmc(cass_engine *e, int32_t box, int32_t species, int64_t n_in
   cass_box_state &b = e->boxes[box];
   if (b.p.charge_style == CASS_Q_EWALD && species_has_charge(e, species))
     return cass_fail(e, CASS_ERR_ARG, "CBMC Widom of a charged species with Ewald sums is not supported");
-  const int kmax = std::max(hs->h.kappa_ins, hs->h.kappa_dih);
   HIP_TRY(e, hipSetDevice(e->device));
   // the insertion-independent constants (widom_insert.f90:212-240)
   double lrc_diff = 0.0, e_self = 0.0;
@@ -2382,11 +385,16 @@ static int widom_cbmc(cass_engine *e, int32_t box, int32_t species, int64_t n_in
   if (b.p.charge_style != CASS_Q_NONE && species_has_charge(e, species)) cass_mol_self_energy(e, box, species, &e_self);
   const int nsub = n_sub > 0 ? n_sub : 1;
   const int64_t rsq_stride = rsq_min ? (int64_t)e->natoms_total * e->sp_natoms[species] : 0;
+  const size_t live_bytes = (sizeof(float4) + sizeof(LiveMol)) * (size_t)b.nmols + 64;
   const size_t need = (size_t)n_ins * (2 * sizeof(double) + 1) + sizeof(double) * (nsub + 2) + 64 +
-                      5 * sizeof(int64_t) + sizeof(double) * (size_t)(n_ins * rsq_stride);
+                      5 * sizeof(int64_t) + sizeof(double) * (size_t)(n_ins * rsq_stride) + live_bytes;
   char *s = (char *)cass_scratch(e, need);
   if (!s) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
-  double *d_w = (double *)s;
+  // the frame's live molecules, then the per-insertion arrays
+  float4 *d_lcom = (float4 *)s;
+  LiveMol *d_lmol = (LiveMol *)(d_lcom + b.nmols);
+  int *d_nlive = (int *)(d_lmol + b.nmols);
+  double *d_w = (double *)(s + (live_bytes & ~(size_t)15));
   double *d_em = d_w + n_ins;
   double *d_rsq = d_em + n_ins;
   double *d_out = d_rsq + n_ins * rsq_stride;
@@ -2405,16 +413,23 @@ static int widom_cbmc(cass_engine *e, int32_t box, int32_t species, int64_t n_in
   w.eij_max = eij_max ? d_em : nullptr;
   w.rsq_min = rsq_min ? d_rsq : nullptr;
   w.rsq_rows = e->natoms_total;
+  w.live = LiveList{d_lmol, d_lcom};
+  w.nlive = d_nlive;
   if (rng) HIP_TRY(e, hipMemcpyAsync(d_rng, rng->s, sizeof(int64_t) * 5, hipMemcpyHostToDevice, e->stream));
   HIP_TRY(e, hipEventRecord(e->ev0, e->stream));
-  int rc;
   const int grid = rng ? 1 : (int)n_ins;
   if (rng ? false : (int64_t)grid != n_ins) return cass_fail(e, CASS_ERR_ARG, "too many insertions for one batch");
-  if (rng || b.nmols > 4096 || kmax > 16)
-    rc = launch_widom_cbmc<256>(e, w, grid);
-  else
-    rc = launch_widom_cbmc<64>(e, w, grid);
-  if (rc) return rc;
+  hipLaunchKernelGGL(k_widom_live, dim3(1), dim3(64), 0, e->stream, w.g, w.live, d_nlive);
+  HIP_TRY(e, hipGetLastError());
+  const bool lj = lj_growth(e, b, species);
+  // One insertion of the parallel mode per workgroup of 4 waves: the LDS
+  // holds three of them a CU, and 3001 pentane insertions (kappa 12 / 24) took
+  // 0.77, 0.50, 0.49 and 0.65 ms with 1, 2, 4 and 8 waves.  Insertions in
+  // sequence have one CU to themselves: 8 waves.
+  const int nt = rng ? 512 : 256;
+  const CbmcKernels kt = growth_kernels(e, lj);
+  hipLaunchKernelGGL(rng ? kt.widom_seq : kt.widom_par, dim3(grid), dim3(nt), 0, e->stream, w);
+  HIP_TRY(e, hipGetLastError());
   const int64_t subint = n_ins / nsub;
   hipLaunchKernelGGL(k_widom_cbmc_sum, dim3(1), dim3(256), 0, e->stream, d_w, d_ov, n_ins, n_sub > 0 ? n_sub : 0,
                      subint, d_out);
@@ -2662,26 +677,27 @@ static int pull_mirrors(cass_engine *e, const std::vector<int> &ids, bool live) 
   return CASS_OK;
 }
 
-template <int NT>
-static int launch_gemc(cass_engine *e, const GcmcBoxArgs *d_boxes, int npairs, int64_t nsteps) {
-  auto kern = e->prec == CASS_PREC_MIXED  ? k_gemc_chain<PrecMixed, NT>
-              : e->prec == CASS_PREC_FP32 ? k_gemc_chain<PrecFP32, NT>
-                                          : k_gemc_chain<PrecFP64, NT>;
-  hipLaunchKernelGGL(kern, dim3(npairs), dim3(NT), 0, e->stream, d_boxes, nsteps);
-  return hipGetLastError() == hipSuccess ? CASS_OK : cass_fail(e, CASS_ERR_HIP, "k_gemc_chain launch");
+// One launch of a chain kernel with the live lists of `per` boxes in the
+// dynamic LDS (cap molecules each; 0: in device memory).
+template <typename K, typename A>
+static int launch_chain(cass_engine *e, K kern, const A *d_boxes, int grid, int nt, int64_t nsteps, int cap, int per,
+                        const char *what) {
+  const size_t lds = (size_t)per * cap * kListBytes;
+  HIP_TRY(e, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(nt), lds, e->stream, d_boxes, nsteps, cap);
+  return hipGetLastError() == hipSuccess ? CASS_OK : cass_fail(e, CASS_ERR_HIP, what);
 }
 
-template <int NT>
-static int launch_gcmc(cass_engine *e, const GcmcBoxArgs *d_boxes, int nboxes, int64_t nsteps) {
-  auto kern = e->prec == CASS_PREC_MIXED  ? k_gcmc_chain<PrecMixed, NT>
-              : e->prec == CASS_PREC_FP32 ? k_gcmc_chain<PrecFP32, NT>
-                                          : k_gcmc_chain<PrecFP64, NT>;
-  hipLaunchKernelGGL(kern, dim3(nboxes), dim3(NT), 0, e->stream, d_boxes, nsteps, (int64_t)0, (int64_t)0);
-  return hipGetLastError() == hipSuccess ? CASS_OK : cass_fail(e, CASS_ERR_HIP, "k_gcmc_chain launch");
+// Live lists of up to this many bytes per workgroup stand in the LDS beside
+// the chain kernels' own 40 to 60 KB; longer ones in device memory.
+constexpr size_t kListLds = (size_t)64 << 10;
+static int list_cap_of(int maxm, int per) {
+  const int cap = (maxm + 3) & ~3;
+  return (size_t)per * cap * kListBytes <= kListLds ? cap : 0;
 }
 
 // workgroup size of the GCMC chain per engine: 0 until cass_gcmc_autotune
-// picks one (then 256, or 512 for boxes of more than 512 molecule slots)
+// picks one (then 512)
 static std::vector<std::pair<cass_engine *, int>> g_gcmc_block;
 static int &gcmc_block(cass_engine *e) {
   for (auto &p : g_gcmc_block)
@@ -2706,6 +722,8 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
   HIP_TRY(e, hipSetDevice(e->device));
   const int ntypes = e->ntypes;
   size_t bytes = 0;
+  int maxm = 0;
+  bool lj = true;
   auto up = [](size_t n) { return (n + 255) & ~size_t(255); };
   for (int i = 0; i < nboxes; ++i) {
     const cass_gcmc_box &g = boxes[i];
@@ -2739,6 +757,8 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
           return cass_fail(e, CASS_ERR_ARG, "locate / reservoir disagree with the live flags");
       }
     }
+    maxm = std::max(maxm, b.nmols);
+    lj = lj && lj_growth(e, b, g.species);
     // the same rounded pieces the layout below takes, one by one
     bytes += up(sizeof(int64_t) * 5) + up(sizeof(double) * 14) + up(sizeof(int) * 2) +
              2 * up(sizeof(int) * g.max_mols) + up(sizeof(double) * ntypes);
@@ -2746,9 +766,13 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
                       up(sizeof(int64_t) * 5 * nsteps);
   }
   bytes += up(sizeof(GcmcBoxArgs) * nboxes);
+  // the live lists, at the end: not copied to or from the host
+  const int list_cap = list_cap_of(maxm, gemc ? 2 : 1);
+  const size_t state_bytes = bytes;
+  if (list_cap == 0) bytes += (up(sizeof(float4) * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)nboxes;
   char *s0 = (char *)cass_scratch(e, bytes + 256);
   if (!s0) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
-  std::vector<char> host(bytes + 256, 0);
+  std::vector<char> host(state_bytes + 256, 0);
   size_t off = 0;
   auto take = [&](size_t n) {
     const size_t o = off;
@@ -2760,11 +784,9 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
     size_t rng, en, cnt, loc, res, nb, kind, acc, nm, ren, rr;
   };
   std::vector<Offs> offs(nboxes);
-  int maxm = 0;
   for (int i = 0; i < nboxes; ++i) {
     const cass_gcmc_box &g = boxes[i];
     cass_box_state &b = e->boxes[g.box];
-    maxm = std::max(maxm, b.nmols);
     const cass_gcmc_state &st = states[i];
     Offs &o = offs[i];
     o.rng = take(sizeof(int64_t) * 5);
@@ -2829,25 +851,27 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
     a.rec_nmols = rec ? (int *)(s0 + o.nm) : nullptr;
     a.rec_energy = rec ? (double *)(s0 + o.ren) : nullptr;
     a.rec_rng = rec ? (int64_t *)(s0 + o.rr) : nullptr;
+    const size_t o_list = state_bytes + (up(sizeof(float4) * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)i;
+    a.list = list_cap ? LiveList{nullptr, nullptr}
+                      : LiveList{(LiveMol *)(s0 + o_list + up(sizeof(float4) * maxm)), (float4 *)(s0 + o_list)};
   }
   const size_t o_args = take(sizeof(GcmcBoxArgs) * nboxes);
-  if (off > bytes) return cass_fail(e, CASS_ERR_STATE, "GCMC state layout exceeds its buffer");
+  if (off > state_bytes) return cass_fail(e, CASS_ERR_STATE, "GCMC state layout exceeds its buffer");
   std::memcpy(host.data() + o_args, args.data(), sizeof(GcmcBoxArgs) * nboxes);
   HIP_TRY(e, hipMemcpyAsync(s0, host.data(), off, hipMemcpyHostToDevice, e->stream));
   HIP_TRY(e, hipEventRecord(e->ev0, e->stream));
-  if (nt <= 0) nt = gcmc_block(e) > 0 ? gcmc_block(e) : (maxm > 512 ? 512 : 256);
+  // 8 waves unless the autotuner picked otherwise: 40 moves of 48 pentane
+  // boxes took 3.9, 2.6, 1.9 and 1.7 ms of kernel with 2, 4, 8 and 16 waves
+  // (16 leave 128 registers a lane, and the kernel then spills)
+  if (nt <= 0) nt = gcmc_block(e) > 0 ? gcmc_block(e) : 512;
   const GcmcBoxArgs *d_args = (const GcmcBoxArgs *)(s0 + o_args);
-  int rc;
-  if (gemc) nt = maxm > 512 ? 512 : 256;  // 512 lanes measured no faster on 24 pentane pairs
-  if (gemc) {
-    rc = nt == 512 ? launch_gemc<512>(e, d_args, nboxes / 2, nsteps) : launch_gemc<256>(e, d_args, nboxes / 2, nsteps);
-  } else switch (nt) {
-    case 128: rc = launch_gcmc<128>(e, d_args, nboxes, nsteps); break;
-    case 256: rc = launch_gcmc<256>(e, d_args, nboxes, nsteps); break;
-    case 512: rc = launch_gcmc<512>(e, d_args, nboxes, nsteps); break;
-    case 1024: rc = launch_gcmc<1024>(e, d_args, nboxes, nsteps); break;
-    default: return cass_fail(e, CASS_ERR_ARG, "workgroup size");
-  }
+  if (gemc) nt = 512;  // 30 transfers of 96 pentane pairs: 3.3 ms with 4 waves, 2.5 ms with 8
+  if (nt != 128 && nt != 256 && nt != 512 && nt != 1024) return cass_fail(e, CASS_ERR_ARG, "workgroup size");
+  const CbmcKernels kt = growth_kernels(e, lj);
+  const int rc = gemc ? launch_chain(e, kt.gemc, d_args, nboxes / 2, nt, nsteps, list_cap, 2,
+                                     "k_gemc_chain launch")
+                      : launch_chain(e, kt.gcmc[lanes_index(nt)], d_args, nboxes, nt, nsteps, list_cap, 1,
+                                     "k_gcmc_chain launch");
   if (rc) return rc;
   HIP_TRY(e, hipEventRecord(e->ev1, e->stream));
   HIP_TRY(e, hipMemcpyAsync(host.data(), s0, off, hipMemcpyDeviceToHost, e->stream));
@@ -2903,15 +927,6 @@ extern "C" int cass_gemc_run_device(cass_engine *e, int32_t npairs, const cass_g
   return gcmc_launch(e, 2 * npairs, boxes, states, nsteps, rec, 1, 0, nullptr, true);
 }
 
-template <int NT>
-static int launch_regrow(cass_engine *e, const RegrowBoxArgs *d_boxes, int nboxes, int64_t nsteps) {
-  auto kern = e->prec == CASS_PREC_MIXED  ? k_regrow_chain<PrecMixed, NT>
-              : e->prec == CASS_PREC_FP32 ? k_regrow_chain<PrecFP32, NT>
-                                          : k_regrow_chain<PrecFP64, NT>;
-  hipLaunchKernelGGL(kern, dim3(nboxes), dim3(NT), 0, e->stream, d_boxes, nsteps);
-  return hipGetLastError() == hipSuccess ? CASS_OK : cass_fail(e, CASS_ERR_HIP, "k_regrow_chain launch");
-}
-
 extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass_regrow_box *boxes, cass_rng *rngs,
                                       int64_t nsteps, cass_energy *energies, cass_nvt_record *recs) {
   if (!e || nboxes <= 0 || !boxes || !rngs || !energies || nsteps < 0) return CASS_ERR_ARG;
@@ -2920,6 +935,7 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
   auto up = [](size_t n) { return (n + 255) & ~size_t(255); };
   size_t bytes = 0;
   int maxm = 0;
+  bool lj = true;
   for (int i = 0; i < nboxes; ++i) {
     const cass_regrow_box &g = boxes[i];
     if (g.box < 0 || g.box >= (int)e->boxes.size()) return cass_fail(e, CASS_ERR_ARG, "bad box");
@@ -2939,13 +955,17 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
     if (b.p.charge_style != CASS_Q_NONE && species_has_charge(e, g.species))
       return cass_fail(e, CASS_ERR_ARG, "regrowth of a charged species is not supported on the device");
     maxm = std::max(maxm, b.nmols);
+    lj = lj && lj_growth(e, b, g.species);
     bytes += up(sizeof(int64_t) * 5) + up(sizeof(double) * 14) + up(sizeof(int)) + up(sizeof(int) * g.nmols);
     if (recs) bytes += 2 * up(nsteps) + 2 * up(sizeof(double) * nsteps) + up(sizeof(int64_t) * 5 * nsteps);
   }
   bytes += up(sizeof(RegrowBoxArgs) * nboxes);
+  const int list_cap = list_cap_of(maxm, 1);
+  const size_t state_bytes = bytes;
+  if (list_cap == 0) bytes += (up(sizeof(float4) * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)nboxes;
   char *s0 = (char *)cass_scratch(e, bytes + 256);
   if (!s0) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
-  std::vector<char> host(bytes + 256, 0);
+  std::vector<char> host(state_bytes + 256, 0);
   size_t off = 0;
   auto take = [&](size_t n) {
     const size_t o = off;
@@ -2993,14 +1013,19 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
     a.rec_energy = r ? (double *)(s0 + o.ren) : nullptr;
     a.ln_pacc = r ? (double *)(s0 + o.lp) : nullptr;
     a.rec_rng = r ? (int64_t *)(s0 + o.rr) : nullptr;
+    const size_t o_list = state_bytes + (up(sizeof(float4) * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)i;
+    a.list = list_cap ? LiveList{nullptr, nullptr}
+                      : LiveList{(LiveMol *)(s0 + o_list + up(sizeof(float4) * maxm)), (float4 *)(s0 + o_list)};
   }
   const size_t o_args = take(sizeof(RegrowBoxArgs) * nboxes);
-  if (off > bytes) return cass_fail(e, CASS_ERR_STATE, "regrowth state layout exceeds its buffer");
+  if (off > state_bytes) return cass_fail(e, CASS_ERR_STATE, "regrowth state layout exceeds its buffer");
   std::memcpy(host.data() + o_args, args.data(), sizeof(RegrowBoxArgs) * nboxes);
   HIP_TRY(e, hipMemcpyAsync(s0, host.data(), off, hipMemcpyHostToDevice, e->stream));
   HIP_TRY(e, hipEventRecord(e->ev0, e->stream));
   const RegrowBoxArgs *d_args = (const RegrowBoxArgs *)(s0 + o_args);
-  const int rc = maxm > 512 ? launch_regrow<512>(e, d_args, nboxes, nsteps) : launch_regrow<256>(e, d_args, nboxes, nsteps);
+  const int nt = 512;  // 60 moves of 48 pentane boxes: 6.6 ms with 4 waves, 4.2 ms with 8
+  const int rc = launch_chain(e, growth_kernels(e, lj).regrow, d_args, nboxes, nt, nsteps, list_cap,
+                              1, "k_regrow_chain launch");
   if (rc) return rc;
   HIP_TRY(e, hipEventRecord(e->ev1, e->stream));
   HIP_TRY(e, hipMemcpyAsync(host.data(), s0, off, hipMemcpyDeviceToHost, e->stream));

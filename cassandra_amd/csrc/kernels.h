@@ -66,6 +66,27 @@ struct WidomArgs {
 
 __host__ __device__ inline double rint_away(double x) { return round(x); }
 
+// Sum over the wave's 64 lanes, uniform, in a fixed order: row shifts within
+// 16 lanes, then the row broadcasts, all on the vector unit's data-parallel
+// moves (a step of about 20 cycles, against some 130 for a shuffle through
+// the LDS hardware).  Every lane of the wave must be active.
+template <int CTRL, int ROWS>
+__device__ inline double dpp_add(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
+  return v + __hiloint2double(hi, lo);
+}
+__device__ inline double wave_total(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr:1
+  v = dpp_add<0x112, 0xf>(v);  // row_shr:2
+  v = dpp_add<0x114, 0xf>(v);  // row_shr:4
+  v = dpp_add<0x118, 0xf>(v);  // row_shr:8: lane 15 of each row has its sum
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                          __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
+
 // ------------------------------------------------------------- geometry
 __device__ inline void min_image(const BoxDev &b, double &dx, double &dy, double &dz) {
   // minimum_image_separation.f90:35-112: cubic boxes shift by one box length
