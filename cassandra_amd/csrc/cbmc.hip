@@ -627,56 +627,6 @@ extern "C" int cass_rminsq_estimate(int32_t nsolv, int32_t nsolute, int32_t res,
   return CASS_OK;
 }
 
-// Refreshes the host mirrors of the given boxes (coordinates, centres and,
-// with live, the live flags) from the device in one batch: asynchronous
-// copies into pinned staging and one synchronisation.
-static int pull_mirrors(cass_engine *e, const std::vector<int> &ids, bool live) {
-  auto up = [](size_t n) { return (n + 255) & ~size_t(255); };
-  size_t bytes = 0;
-  for (int id : ids) {
-    const cass_box_state &b = e->boxes[id];
-    bytes += 3 * up(sizeof(double) * b.nsites) + up(sizeof(double4) * b.nmols) +
-             (live ? up(sizeof(int32_t) * b.nmols) : 0);
-  }
-  char *h = (char *)cass_pinned(e, bytes + 256);
-  if (!h) return cass_fail(e, CASS_ERR_NOMEM, "pinned staging");
-  size_t off = 0;
-  std::vector<size_t> offs;
-  for (int id : ids) {
-    const cass_box_state &b = e->boxes[id];
-    const double *src[3] = {b.x, b.y, b.z};
-    for (int d = 0; d < 3; ++d) {
-      offs.push_back(off);
-      HIP_TRY(e, hipMemcpyAsync(h + off, src[d], sizeof(double) * b.nsites, hipMemcpyDeviceToHost, e->stream));
-      off += up(sizeof(double) * b.nsites);
-    }
-    offs.push_back(off);
-    HIP_TRY(e, hipMemcpyAsync(h + off, b.comd, sizeof(double4) * b.nmols, hipMemcpyDeviceToHost, e->stream));
-    off += up(sizeof(double4) * b.nmols);
-    if (live) {
-      offs.push_back(off);
-      HIP_TRY(e, hipMemcpyAsync(h + off, b.d_live, sizeof(int32_t) * b.nmols, hipMemcpyDeviceToHost, e->stream));
-      off += up(sizeof(int32_t) * b.nmols);
-    }
-  }
-  HIP_TRY(e, hipStreamSynchronize(e->stream));
-  size_t q = 0;
-  for (int id : ids) {
-    cass_box_state &b = e->boxes[id];
-    const double *xs = (const double *)(h + offs[q]), *ys = (const double *)(h + offs[q + 1]),
-                 *zs = (const double *)(h + offs[q + 2]);
-    for (int k = 0; k < b.nsites; ++k) {
-      b.xyz_h[3 * k] = xs[k];
-      b.xyz_h[3 * k + 1] = ys[k];
-      b.xyz_h[3 * k + 2] = zs[k];
-    }
-    std::memcpy(b.comd_h.data(), h + offs[q + 3], sizeof(double4) * b.nmols);
-    if (live) std::memcpy(b.live.data(), h + offs[q + 4], sizeof(int32_t) * b.nmols);
-    q += live ? 5 : 4;
-  }
-  return CASS_OK;
-}
-
 // One launch of a chain kernel with the live lists of `per` boxes in the
 // dynamic LDS (cap molecules each; 0: in device memory).
 template <typename K, typename A>
@@ -803,14 +753,14 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
     std::memcpy(host.data() + o.res, st.reservoir, sizeof(int) * st.nres);
     // bead counts per type of the live molecules (Compute_Beads)
     std::vector<double> nb(ntypes, 0.0);
-    for (int m = 0; m < b.nmols; ++m) {
-      if (!b.live[m]) continue;
-      const int sp = b.mol_species[m];
+    std::vector<int64_t> count(e->nspecies, 0);
+    for (int m = 0; m < b.nmols; ++m)
+      if (b.live[m]) ++count[b.mol_species[m]];
+    for (int sp = 0; sp < e->nspecies; ++sp)
       for (int a = 0; a < e->sp_natoms[sp]; ++a) {
         const int ty = e->atom_type[e->sp_atom_off[sp] + a];
-        if (ty >= 0) nb[ty] += 1.0;
+        if (ty >= 0) nb[ty] += (double)count[sp];
       }
-    }
     std::memcpy(host.data() + o.nb, nb.data(), sizeof(double) * ntypes);
     if (rec) {
       o.kind = take(nsteps);
@@ -874,40 +824,41 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
                                      "k_gcmc_chain launch");
   if (rc) return rc;
   HIP_TRY(e, hipEventRecord(e->ev1, e->stream));
-  HIP_TRY(e, hipMemcpyAsync(host.data(), s0, off, hipMemcpyDeviceToHost, e->stream));
+  // the states and, unless this is a timing run, coordinates, live flags and
+  // centres of every box come back behind one synchronisation
+  MirrorPull mirrors;
+  std::vector<int> ids(commit ? nboxes : 0);
+  for (size_t i = 0; i < ids.size(); ++i) ids[i] = boxes[i].box;
+  if (int mrc = mirrors.begin(e, ids, true, off)) return mrc;
+  HIP_TRY(e, hipMemcpyAsync(mirrors.host, s0, off, hipMemcpyDeviceToHost, e->stream));
   HIP_TRY(e, hipStreamSynchronize(e->stream));
   float ms = 0.f;
   if (hipEventElapsedTime(&ms, e->ev0, e->ev1) == hipSuccess) e->last_kernel_ms = ms;
   if (ms_out) *ms_out = ms;
   if (!commit) return CASS_OK;
-  // the host mirrors of every box follow the device state
+  mirrors.end(e);
+  const char *back = mirrors.host;
   int bad = 0;
   for (int i = 0; i < nboxes; ++i) {
     const cass_gcmc_box &g = boxes[i];
     cass_gcmc_state &st = states[i];
     const Offs &o = offs[i];
-    std::memcpy(st.rng.s, host.data() + o.rng, sizeof(int64_t) * 5);
-    std::memcpy(&st.energy, host.data() + o.en, sizeof(double) * 14);
+    std::memcpy(st.rng.s, back + o.rng, sizeof(int64_t) * 5);
+    std::memcpy(&st.energy, back + o.en, sizeof(double) * 14);
     int cnt[2];
-    std::memcpy(cnt, host.data() + o.cnt, sizeof(cnt));
+    std::memcpy(cnt, back + o.cnt, sizeof(cnt));
     if (cnt[1] < 0) bad = 1;
     st.nmols = cnt[0];
     st.nres = cnt[1] < 0 ? g.max_mols - cnt[0] : cnt[1];
-    std::memcpy(st.locate, host.data() + o.loc, sizeof(int) * g.max_mols);
-    std::memcpy(st.reservoir, host.data() + o.res, sizeof(int) * g.max_mols);
+    std::memcpy(st.locate, back + o.loc, sizeof(int) * g.max_mols);
+    std::memcpy(st.reservoir, back + o.res, sizeof(int) * g.max_mols);
     if (rec) {
-      std::memcpy(rec->kind + (size_t)i * nsteps, host.data() + o.kind, nsteps);
-      std::memcpy(rec->accepted + (size_t)i * nsteps, host.data() + o.acc, nsteps);
-      std::memcpy(rec->nmols + (size_t)i * nsteps, host.data() + o.nm, sizeof(int) * nsteps);
-      std::memcpy(rec->energy + (size_t)i * nsteps, host.data() + o.ren, sizeof(double) * nsteps);
-      std::memcpy(rec->rng_state + (size_t)i * nsteps * 5, host.data() + o.rr, sizeof(int64_t) * 5 * nsteps);
+      std::memcpy(rec->kind + (size_t)i * nsteps, back + o.kind, nsteps);
+      std::memcpy(rec->accepted + (size_t)i * nsteps, back + o.acc, nsteps);
+      std::memcpy(rec->nmols + (size_t)i * nsteps, back + o.nm, sizeof(int) * nsteps);
+      std::memcpy(rec->energy + (size_t)i * nsteps, back + o.ren, sizeof(double) * nsteps);
+      std::memcpy(rec->rng_state + (size_t)i * nsteps * 5, back + o.rr, sizeof(int64_t) * 5 * nsteps);
     }
-  }
-  // coordinates, live flags and centres of every box
-  {
-    std::vector<int> ids(nboxes);
-    for (int i = 0; i < nboxes; ++i) ids[i] = boxes[i].box;
-    if (int rc = pull_mirrors(e, ids, true)) return rc;
   }
   ++e->gen;
   if (bad)
@@ -1028,31 +979,32 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
                               1, "k_regrow_chain launch");
   if (rc) return rc;
   HIP_TRY(e, hipEventRecord(e->ev1, e->stream));
-  HIP_TRY(e, hipMemcpyAsync(host.data(), s0, off, hipMemcpyDeviceToHost, e->stream));
+  MirrorPull mirrors;
+  std::vector<int> ids(nboxes);
+  for (int i = 0; i < nboxes; ++i) ids[i] = boxes[i].box;
+  if (int mrc = mirrors.begin(e, ids, false, off)) return mrc;
+  HIP_TRY(e, hipMemcpyAsync(mirrors.host, s0, off, hipMemcpyDeviceToHost, e->stream));
   HIP_TRY(e, hipStreamSynchronize(e->stream));
+  mirrors.end(e);
+  const char *back = mirrors.host;
   float ms = 0.f;
   if (hipEventElapsedTime(&ms, e->ev0, e->ev1) == hipSuccess) e->last_kernel_ms = ms;
   int bad = 0;
   for (int i = 0; i < nboxes; ++i) {
     const Offs &o = offs[i];
-    std::memcpy(rngs[i].s, host.data() + o.rng, sizeof(int64_t) * 5);
-    std::memcpy(&energies[i], host.data() + o.en, sizeof(double) * 14);
+    std::memcpy(rngs[i].s, back + o.rng, sizeof(int64_t) * 5);
+    std::memcpy(&energies[i], back + o.en, sizeof(double) * 14);
     int st;
-    std::memcpy(&st, host.data() + o.st, sizeof(int));
+    std::memcpy(&st, back + o.st, sizeof(int));
     bad |= st;
     if (recs) {
       cass_nvt_record &r = recs[i];
-      if (r.kind) std::memcpy(r.kind, host.data() + o.kind, nsteps);
-      if (r.accepted) std::memcpy(r.accepted, host.data() + o.acc, nsteps);
-      if (r.energy) std::memcpy(r.energy, host.data() + o.ren, sizeof(double) * nsteps);
-      if (r.ln_pacc) std::memcpy(r.ln_pacc, host.data() + o.lp, sizeof(double) * nsteps);
-      if (r.rng_state) std::memcpy(r.rng_state, host.data() + o.rr, sizeof(int64_t) * 5 * nsteps);
+      if (r.kind) std::memcpy(r.kind, back + o.kind, nsteps);
+      if (r.accepted) std::memcpy(r.accepted, back + o.acc, nsteps);
+      if (r.energy) std::memcpy(r.energy, back + o.ren, sizeof(double) * nsteps);
+      if (r.ln_pacc) std::memcpy(r.ln_pacc, back + o.lp, sizeof(double) * nsteps);
+      if (r.rng_state) std::memcpy(r.rng_state, back + o.rr, sizeof(int64_t) * 5 * nsteps);
     }
-  }
-  {
-    std::vector<int> ids(nboxes);
-    for (int i = 0; i < nboxes; ++i) ids[i] = boxes[i].box;
-    if (int rc = pull_mirrors(e, ids, false)) return rc;
   }
   ++e->gen;
   if (bad) return cass_fail(e, CASS_ERR_STATE, "a molecule's own configuration could not be regrown (the reference aborts)");

@@ -140,5 +140,23 @@ void *cass_scratch(cass_engine *e, size_t bytes);
 void *cass_pinned(cass_engine *e, size_t bytes);
 void *cass_io(cass_engine *e, size_t bytes);
 void cass_cbmc_release(cass_engine *e);
+// Host mirrors of boxes that a chain kernel moved.  begin() queues the packing
+// of every box's coordinates (x, y, z together), centres and, with live, live
+// flags into one buffer and its copy to pinned staging; the first `extra`
+// bytes of that staging are the caller's.  end(), after the caller has
+// synchronised the stream, takes them into the mirrors.
+struct MirrorPull {
+  char *host = nullptr;  // the pinned staging
+  int begin(cass_engine *e, const std::vector<int> &ids, bool live, size_t extra);
+  void end(cass_engine *e);
+
+ private:
+  struct Part {
+    int box;
+    size_t xyz, com, live;
+  };
+  std::vector<Part> parts;
+  bool with_live = false;
+};
 bool cass_cbmc_bonded_host(const cass_engine *e, int s, const double *xyz, double *angle, double *dihedral);
 double4 cass_host_com(const cass_engine *e, int s, const double *xyz);  // Get_COM and max_dcom of one molecule  // device copies of the CBMC growth descriptions

@@ -661,25 +661,21 @@ EwaldDev cass_ewald_view(const cass_box_state &b);
 namespace {
 
 // One chain's launch state: its arguments, LDS size and kernel selection,
-// the device buffers of its generator, energies, mobile list and records,
-// and where the results go on the host.
+// and where its generator, energies, mobile list and records stand in the
+// batch's buffers.
 struct NvtLaunch {
   NvtChainArgs a;
   size_t lds = 0;
   int pm = 0, nse = 0;
   bool host_loop = false;  // the box's copy exceeds the LDS: the host-driven loop runs it
   int box = -1;
-  int64_t nsteps = 0;
   cass_rng *rng = nullptr;
   const cass_nvt_options *opt = nullptr;
   cass_energy *en = nullptr;
   cass_nvt_record *rec = nullptr;
-  int64_t *d_rng = nullptr;
-  uint8_t *d_kind = nullptr, *d_acc = nullptr;
-  double *d_energy = nullptr, *d_lnp = nullptr;
-  int64_t *d_rs = nullptr;
   bool charged = false;
-  int nsite = 0;
+  std::vector<int> mols;  // locate order of the mobile species
+  size_t o_state = 0, o_kind = 0, o_acc = 0, o_energy = 0, o_lnp = 0, o_rs = 0, o_mols = 0;
 };
 
 typedef void (*nvt_kernel_t)(NvtChainArgs);
@@ -704,15 +700,14 @@ nvt_multi_kernel_t nvt_multi_kernel(int pm, int nse) {
   return kt[pm][nse];
 }
 
-// Checks, the LDS layout of the box copy, the kernel choice and the device
-// state of one chain (everything before its launches).  nsteps == 0 or a
-// box beyond the LDS leaves L.a unset (host_loop / nothing to launch).
+// Checks, the LDS layout of the box copy, the kernel choice and the arguments
+// of one chain but for its buffers (nvt_buffers).  nsteps == 0 or a box
+// beyond the LDS leaves L.a unset (host_loop / nothing to launch).
 int nvt_prepare(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_options *opt, int64_t nsteps,
                 cass_energy *en, cass_nvt_record *rec, NvtLaunch &L) {
   if (!e || !rng || !opt || !en || nsteps < 0 || box < 0 || box >= (int)e->boxes.size()) return CASS_ERR_ARG;
   cass_box_state &b = e->boxes[box];
   L.box = box;
-  L.nsteps = nsteps;
   L.rng = rng;
   L.opt = opt;
   L.en = en;
@@ -726,7 +721,7 @@ int nvt_prepare(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_optio
   const bool charged = b.p.charge_style == CASS_Q_EWALD && has_q;
   L.charged = charged;
   if (charged && !b.ewald_ready) return cass_fail(e, CASS_ERR_STATE, "Ewald sums not set up");
-  std::vector<int> mols;  // locate order of the mobile species
+  std::vector<int> &mols = L.mols;
   for (int m = 0; m < b.nmols; ++m)
     if (b.mol_species[m] == sp && b.live[m]) mols.push_back(m);
   const int nm = (int)mols.size();
@@ -735,7 +730,6 @@ int nvt_prepare(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_optio
   HIP_TRY(e, hipSetDevice(e->device));
   // LDS layout of the box copy
   const int nsite = (int)(b.xyz_h.size() / 3), nt = std::max(e->ntypes, 1);
-  L.nsite = nsite;
   size_t lds = 0;
   auto take = [&](size_t bytes) {
     const size_t o = lds;
@@ -780,29 +774,6 @@ int nvt_prepare(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_optio
   // the mixed and FP32 modes take the mixed pair arithmetic for the common
   // styles (FP64 accumulation, reciprocal space and acceptance in every mode)
   L.pm = common ? (e->prec == CASS_PREC_FP64 ? 1 : 2) : 0;
-  // device state of the chain: RNG words, energies, status, mobile list, records
-  const size_t ns = (size_t)nsteps;
-  const size_t ktrav = charged ? (size_t)b.nvecs : 0;
-  HIP_TRY(e, hipMallocAsync((void **)&L.d_rng,
-                            sizeof(int64_t) * 5 + sizeof(double) * (5 + 2 * ktrav) + sizeof(int) * (2 + nm),
-                            e->stream));
-  double *d_en = (double *)(L.d_rng + 5);
-  double *d_trav = d_en + 5;
-  int *d_status = (int *)(d_trav + 2 * ktrav);
-  int *d_mols = d_status + 2;
-  if (rec && rec->kind) HIP_TRY(e, hipMallocAsync((void **)&L.d_kind, ns, e->stream));
-  if (rec && rec->accepted) HIP_TRY(e, hipMallocAsync((void **)&L.d_acc, ns, e->stream));
-  if (rec && rec->energy) HIP_TRY(e, hipMallocAsync((void **)&L.d_energy, sizeof(double) * ns, e->stream));
-  if (rec && rec->ln_pacc) HIP_TRY(e, hipMallocAsync((void **)&L.d_lnp, sizeof(double) * ns, e->stream));
-  if (rec && rec->rng_state) HIP_TRY(e, hipMallocAsync((void **)&L.d_rs, sizeof(int64_t) * 5 * ns, e->stream));
-  const double en_in[5] = {en->total, en->inter, en->inter_vdw, en->inter_q, en->reciprocal};
-  const int zero[2] = {0, 0};
-  HIP_TRY(e, hipMemcpyAsync(L.d_rng, rng->s, sizeof(int64_t) * 5, hipMemcpyHostToDevice, e->stream));
-  HIP_TRY(e, hipMemcpyAsync(d_en, en_in, sizeof(double) * 5, hipMemcpyHostToDevice, e->stream));
-  HIP_TRY(e, hipMemcpyAsync(d_status, zero, sizeof(int) * 2, hipMemcpyHostToDevice, e->stream));
-  HIP_TRY(e, hipMemcpyAsync(d_mols, mols.data(), sizeof(int) * nm, hipMemcpyHostToDevice, e->stream));
-  HIP_TRY(e, hipStreamSynchronize(e->stream));  // mols and the staged values go out of scope
-
   a.b = cass_box_view(e, b);
   a.tp = cass_topo_view(e);
   a.cd = make_pair_const<double>(b.p, e->ntypes);
@@ -813,7 +784,6 @@ int nvt_prepare(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_optio
   a.y = b.y;
   a.z = b.z;
   a.comd = b.comd;
-  a.mols = d_mols;
   a.nm = nm;
   a.species = sp;
   a.n = n;
@@ -825,16 +795,6 @@ int nvt_prepare(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_optio
   a.max_disp = opt->max_disp;
   a.max_rot = opt->max_rot;
   a.beta = b.p.beta;
-  a.rng = L.d_rng;
-  a.en = d_en;
-  a.kind = L.d_kind;
-  a.accepted = L.d_acc;
-  a.energy = L.d_energy;
-  a.ln_pacc = L.d_lnp;
-  a.rng_state = L.d_rs;
-  a.status = d_status;
-  a.ctrav = d_trav;
-  a.strav = d_trav + ktrav;
   a.nsite = nsite;
   a.nj_uniform = b.nmols > 0 ? e->sp_natoms[b.mol_species[0]] : 0;
   for (int mm = 0; mm < b.nmols; ++mm)
@@ -845,60 +805,117 @@ int nvt_prepare(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_optio
   return CASS_OK;
 }
 
-// Results of one chain back to the host: generator state, energies,
-// records, the moved coordinates and centres; releases its device state.
-int nvt_finish(cass_engine *e, NvtLaunch &L) {
-  if (!L.d_rng) return CASS_OK;  // nothing was launched for this chain
-  cass_box_state &b = e->boxes[L.box];
-  const size_t ns = (size_t)L.nsteps;
-  const int nsite = L.nsite;
-  cass_nvt_record *rec = L.rec;
-  int64_t rs_out[5];
-  double en_out[5];
+// The state of one chain in the batch's buffer.
+struct NvtState {
+  int64_t rng[5];
+  double en[5];
   int status[2];
-  const double *d_en = L.a.en;
-  HIP_TRY(e, hipMemcpyAsync(rs_out, L.d_rng, sizeof(int64_t) * 5, hipMemcpyDeviceToHost, e->stream));
-  HIP_TRY(e, hipMemcpyAsync(en_out, d_en, sizeof(double) * 5, hipMemcpyDeviceToHost, e->stream));
-  HIP_TRY(e, hipMemcpyAsync(status, L.a.status, sizeof(int) * 2, hipMemcpyDeviceToHost, e->stream));
-  if (L.d_kind) HIP_TRY(e, hipMemcpyAsync(rec->kind, L.d_kind, ns, hipMemcpyDeviceToHost, e->stream));
-  if (L.d_acc) HIP_TRY(e, hipMemcpyAsync(rec->accepted, L.d_acc, ns, hipMemcpyDeviceToHost, e->stream));
-  if (L.d_energy)
-    HIP_TRY(e, hipMemcpyAsync(rec->energy, L.d_energy, sizeof(double) * ns, hipMemcpyDeviceToHost, e->stream));
-  if (L.d_lnp) HIP_TRY(e, hipMemcpyAsync(rec->ln_pacc, L.d_lnp, sizeof(double) * ns, hipMemcpyDeviceToHost, e->stream));
-  if (L.d_rs)
-    HIP_TRY(e, hipMemcpyAsync(rec->rng_state, L.d_rs, sizeof(int64_t) * 5 * ns, hipMemcpyDeviceToHost, e->stream));
-  // host mirrors of the moved molecules
-  std::vector<double> hx(nsite), hy(nsite), hz(nsite);
-  if (nsite) {
-    HIP_TRY(e, hipMemcpyAsync(hx.data(), b.x, sizeof(double) * nsite, hipMemcpyDeviceToHost, e->stream));
-    HIP_TRY(e, hipMemcpyAsync(hy.data(), b.y, sizeof(double) * nsite, hipMemcpyDeviceToHost, e->stream));
-    HIP_TRY(e, hipMemcpyAsync(hz.data(), b.z, sizeof(double) * nsite, hipMemcpyDeviceToHost, e->stream));
+};
+
+// The buffers of a batch, laid out over all its chains: first what comes back
+// (states and records), then the mobile lists and argument tables, then the
+// molecule sums.  One copy in, one copy out: with a set of copies per chain
+// the calls themselves outlasted the chains.
+struct NvtBuffers {
+  char *dev = nullptr;
+  size_t back = 0, in = 0;  // bytes copied back; bytes of back + lists + arguments
+  size_t o_args = 0;
+  std::vector<char> host;   // the first `in` bytes
+};
+
+int nvt_buffers(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, NvtBuffers &B) {
+  size_t off = 0;
+  auto take = [&](size_t bytes) {
+    const size_t o = off;
+    off = (off + bytes + 255) & ~(size_t)255;
+    return o;
+  };
+  const size_t ns = (size_t)nsteps;
+  for (NvtLaunch &L : Ls) {
+    if (L.host_loop) continue;
+    const cass_nvt_record *rec = L.rec;
+    L.o_state = take(sizeof(NvtState));
+    if (rec && rec->kind) L.o_kind = take(ns);
+    if (rec && rec->accepted) L.o_acc = take(ns);
+    if (rec && rec->energy) L.o_energy = take(sizeof(double) * ns);
+    if (rec && rec->ln_pacc) L.o_lnp = take(sizeof(double) * ns);
+    if (rec && rec->rng_state) L.o_rs = take(sizeof(int64_t) * 5 * ns);
   }
-  if (b.nmols)
-    HIP_TRY(e, hipMemcpyAsync(b.comd_h.data(), b.comd, sizeof(double4) * b.nmols, hipMemcpyDeviceToHost, e->stream));
-  for (void *p : {(void *)L.d_kind, (void *)L.d_acc, (void *)L.d_energy, (void *)L.d_lnp, (void *)L.d_rs})
-    if (p) HIP_TRY(e, hipFreeAsync(p, e->stream));
-  HIP_TRY(e, hipFreeAsync(L.d_rng, e->stream));
+  B.back = off;
+  for (NvtLaunch &L : Ls)
+    if (!L.host_loop) L.o_mols = take(sizeof(int) * L.mols.size());
+  B.o_args = take(sizeof(NvtChainArgs) * std::max<size_t>(1, Ls.size()));
+  B.in = off;
+  std::vector<size_t> trav(Ls.size());
+  for (size_t k = 0; k < Ls.size(); ++k)
+    if (!Ls[k].host_loop) trav[k] = take(sizeof(double) * 2 * (size_t)Ls[k].a.ew.nvecs);
+  B.dev = (char *)cass_scratch(e, off + 256);
+  if (!B.dev) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
+  B.host.assign(B.in, 0);
+  for (size_t k = 0; k < Ls.size(); ++k) {
+    NvtLaunch &L = Ls[k];
+    if (L.host_loop) continue;
+    NvtState st{};
+    std::memcpy(st.rng, L.rng->s, sizeof(st.rng));
+    const double en_in[5] = {L.en->total, L.en->inter, L.en->inter_vdw, L.en->inter_q, L.en->reciprocal};
+    std::memcpy(st.en, en_in, sizeof(st.en));
+    std::memcpy(B.host.data() + L.o_state, &st, sizeof(st));
+    std::memcpy(B.host.data() + L.o_mols, L.mols.data(), sizeof(int) * L.mols.size());
+    NvtState *d = (NvtState *)(B.dev + L.o_state);
+    const cass_nvt_record *rec = L.rec;
+    NvtChainArgs &a = L.a;
+    a.rng = d->rng;
+    a.en = d->en;
+    a.status = d->status;
+    a.kind = rec && rec->kind ? (uint8_t *)(B.dev + L.o_kind) : nullptr;
+    a.accepted = rec && rec->accepted ? (uint8_t *)(B.dev + L.o_acc) : nullptr;
+    a.energy = rec && rec->energy ? (double *)(B.dev + L.o_energy) : nullptr;
+    a.ln_pacc = rec && rec->ln_pacc ? (double *)(B.dev + L.o_lnp) : nullptr;
+    a.rng_state = rec && rec->rng_state ? (int64_t *)(B.dev + L.o_rs) : nullptr;
+    a.mols = (const int *)(B.dev + L.o_mols);
+    a.ctrav = (double *)(B.dev + trav[k]);
+    a.strav = a.ctrav + a.ew.nvecs;
+  }
+  return CASS_OK;
+}
+
+// Results of the batch back to the host: generator states, energies,
+// records, the moved coordinates and centres.
+int nvt_finish(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, const NvtBuffers &B) {
+  std::vector<int> ids;
+  for (const NvtLaunch &L : Ls)
+    if (!L.host_loop) ids.push_back(L.box);
+  MirrorPull mirrors;
+  if (int rc = mirrors.begin(e, ids, false, B.back)) return rc;
+  if (B.back) HIP_TRY(e, hipMemcpyAsync(mirrors.host, B.dev, B.back, hipMemcpyDeviceToHost, e->stream));
   HIP_TRY(e, hipStreamSynchronize(e->stream));
-  L.d_rng = nullptr;
-  L.d_kind = L.d_acc = nullptr;
-  L.d_energy = L.d_lnp = nullptr;
-  L.d_rs = nullptr;
-  for (int i = 0; i < nsite; ++i) {
-    b.xyz_h[3 * i] = hx[i];
-    b.xyz_h[3 * i + 1] = hy[i];
-    b.xyz_h[3 * i + 2] = hz[i];
-  }
+  mirrors.end(e);
   ++e->gen;
-  std::memcpy(L.rng->s, rs_out, sizeof(rs_out));
-  L.en->total = en_out[0];
-  L.en->inter = en_out[1];
-  L.en->inter_vdw = en_out[2];
-  L.en->inter_q = en_out[3];
-  L.en->reciprocal = en_out[4];
-  if (L.charged) b.e_recip = en_out[4];
-  b.staged_mol = -1;
-  if (status[0]) return cass_fail(e, CASS_ERR_STATE, "molecule energy too high before the move");
+  const size_t ns = (size_t)nsteps;
+  bool bad = false;
+  for (NvtLaunch &L : Ls) {
+    if (L.host_loop) continue;
+    cass_box_state &b = e->boxes[L.box];
+    const char *h = mirrors.host;
+    NvtState st;
+    std::memcpy(&st, h + L.o_state, sizeof(st));
+    const cass_nvt_record *rec = L.rec;
+    if (L.a.kind) std::memcpy(rec->kind, h + L.o_kind, ns);
+    if (L.a.accepted) std::memcpy(rec->accepted, h + L.o_acc, ns);
+    if (L.a.energy) std::memcpy(rec->energy, h + L.o_energy, sizeof(double) * ns);
+    if (L.a.ln_pacc) std::memcpy(rec->ln_pacc, h + L.o_lnp, sizeof(double) * ns);
+    if (L.a.rng_state) std::memcpy(rec->rng_state, h + L.o_rs, sizeof(int64_t) * 5 * ns);
+    std::memcpy(L.rng->s, st.rng, sizeof(st.rng));
+    L.en->total = st.en[0];
+    L.en->inter = st.en[1];
+    L.en->inter_vdw = st.en[2];
+    L.en->inter_q = st.en[3];
+    L.en->reciprocal = st.en[4];
+    if (L.charged) b.e_recip = st.en[4];
+    b.staged_mol = -1;
+    bad = bad || st.status[0];
+  }
+  if (bad) return cass_fail(e, CASS_ERR_STATE, "molecule energy too high before the move");
   return CASS_OK;
 }
 
@@ -909,10 +926,14 @@ constexpr int64_t kNvtChunk = 4096;
 
 extern "C" int cass_nvt_run_device(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_options *opt,
                                    int64_t nsteps, cass_energy *en, cass_nvt_record *rec) {
-  NvtLaunch L;
+  std::vector<NvtLaunch> Ls(1);
+  NvtLaunch &L = Ls[0];
   int rc = nvt_prepare(e, box, rng, opt, nsteps, en, rec, L);
   if (rc || nsteps == 0) return rc;
   if (L.host_loop) return cass_nvt_run(e, box, rng, opt, nsteps, en, rec);
+  NvtBuffers B;
+  if ((rc = nvt_buffers(e, Ls, nsteps, B))) return rc;
+  HIP_TRY(e, hipMemcpyAsync(B.dev, B.host.data(), B.in, hipMemcpyHostToDevice, e->stream));
   nvt_kernel_t kern = nvt_kernel(L.pm, L.nse);
   HIP_TRY(e, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)L.lds));
   for (int64_t s0 = 0; s0 < nsteps; s0 += kNvtChunk) {
@@ -921,7 +942,7 @@ extern "C" int cass_nvt_run_device(cass_engine *e, int32_t box, cass_rng *rng, c
     hipLaunchKernelGGL(kern, dim3(1), dim3(kNvtBlock), L.lds, e->stream, L.a);
     HIP_TRY(e, hipGetLastError());
   }
-  return nvt_finish(e, L);
+  return nvt_finish(e, Ls, nsteps, B);
 }
 
 extern "C" int cass_nvt_run_device_batch(cass_engine *e, int32_t nboxes, const int32_t *boxes, cass_rng *rngs,
@@ -933,64 +954,59 @@ extern "C" int cass_nvt_run_device_batch(cass_engine *e, int32_t nboxes, const i
       if (boxes[k] == boxes[i]) return cass_fail(e, CASS_ERR_ARG, "a box appears twice in the batch");
   std::vector<NvtLaunch> Ls(nboxes);
   int rc = CASS_OK;
-  int i = 0;
-  for (; i < nboxes; ++i)
+  for (int i = 0; i < nboxes; ++i)
     if ((rc = nvt_prepare(e, boxes[i], rngs + i, opts + i, nsteps, ens + i, recs ? recs + i : nullptr, Ls[i])))
-      break;
-  if (rc) {
-    for (int k = 0; k < i; ++k) (void)nvt_finish(e, Ls[k]);  // releases the device state
-    return rc;
-  }
-  if (nsteps == 0) return CASS_OK;
+      return rc;
+  if (nsteps == 0 || nboxes == 0) return CASS_OK;
+  NvtBuffers B;
+  if ((rc = nvt_buffers(e, Ls, nsteps, B))) return rc;
   // the chains grouped by kernel (pair arithmetic, reciprocal site count);
-  // every group is one launch per chunk of moves, one workgroup per box
+  // every group is one launch per chunk of moves, one workgroup per box.  The
+  // argument table holds the groups one after another.
+  struct Group {
+    nvt_multi_kernel_t kern;
+    size_t lds, first, count;
+  };
+  std::vector<Group> groups;
+  std::vector<NvtChainArgs> args;
   std::vector<int> done(nboxes, 0);
-  NvtChainArgs *d_args = nullptr;
-  HIP_TRY(e, hipMallocAsync((void **)&d_args, sizeof(NvtChainArgs) * std::max(1, nboxes), e->stream));
-  std::vector<NvtChainArgs> args(std::max(1, nboxes));
   for (int g = 0; g < nboxes; ++g) {
     if (done[g] || Ls[g].host_loop) continue;
-    std::vector<int> members;
-    size_t lds = 0;
+    Group grp{nvt_multi_kernel(Ls[g].pm, Ls[g].nse), 0, args.size(), 0};
     for (int k = g; k < nboxes; ++k)
       if (!done[k] && !Ls[k].host_loop && Ls[k].pm == Ls[g].pm && Ls[k].nse == Ls[g].nse) {
-        members.push_back(k);
-        lds = std::max(lds, Ls[k].lds);
+        args.push_back(Ls[k].a);
+        grp.lds = std::max(grp.lds, Ls[k].lds);
+        ++grp.count;
         done[k] = 1;
       }
-    nvt_multi_kernel_t kern = nvt_multi_kernel(Ls[g].pm, Ls[g].nse);
-    rc = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess
-             ? CASS_OK
-             : cass_fail(e, CASS_ERR_HIP, "hipFuncSetAttribute");
-    for (int64_t s0 = 0; !rc && s0 < nsteps; s0 += kNvtChunk) {
-      for (size_t m = 0; m < members.size(); ++m) {
-        args[m] = Ls[members[m]].a;
-        args[m].step0 = s0;
-        args[m].nsteps = std::min(kNvtChunk, nsteps - s0);
-      }
-      if (hipMemcpyAsync(d_args, args.data(), sizeof(NvtChainArgs) * members.size(), hipMemcpyHostToDevice,
-                         e->stream) != hipSuccess) {
-        rc = cass_fail(e, CASS_ERR_HIP, "nvt batch arguments");
-        break;
-      }
-      hipLaunchKernelGGL(kern, dim3((unsigned)members.size()), dim3(kNvtBlock), lds, e->stream,
-                         (const NvtChainArgs *)d_args);
-      if (hipGetLastError() != hipSuccess) rc = cass_fail(e, CASS_ERR_HIP, "k_nvt_chain_multi launch");
-      // the argument buffer is rewritten for the next chunk: wait for this one
-      if (!rc && hipStreamSynchronize(e->stream) != hipSuccess) rc = cass_fail(e, CASS_ERR_HIP, "nvt batch");
-    }
-    if (rc) break;
+    groups.push_back(grp);
   }
-  (void)hipFreeAsync(d_args, e->stream);
-  int rc2 = CASS_OK;
-  for (int k = 0; k < nboxes; ++k) {
-    if (Ls[k].host_loop) {
-      if (!rc && !rc2)
-        rc2 = cass_nvt_run(e, boxes[k], rngs + k, opts + k, nsteps, ens + k, recs ? recs + k : nullptr);
-      continue;
+  NvtChainArgs *d_args = (NvtChainArgs *)(B.dev + B.o_args);
+  for (int64_t s0 = 0; s0 < nsteps; s0 += kNvtChunk) {
+    for (NvtChainArgs &a : args) {
+      a.step0 = s0;
+      a.nsteps = std::min(kNvtChunk, nsteps - s0);
     }
-    const int r = nvt_finish(e, Ls[k]);
-    if (!rc2) rc2 = r;
+    if (!args.empty()) std::memcpy(B.host.data() + B.o_args, args.data(), sizeof(NvtChainArgs) * args.size());
+    if (s0 == 0) {
+      HIP_TRY(e, hipMemcpyAsync(B.dev, B.host.data(), B.in, hipMemcpyHostToDevice, e->stream));
+    } else {
+      // the argument table is rewritten: wait for the launches that read it
+      HIP_TRY(e, hipStreamSynchronize(e->stream));
+      HIP_TRY(e, hipMemcpyAsync(d_args, B.host.data() + B.o_args, sizeof(NvtChainArgs) * args.size(),
+                                hipMemcpyHostToDevice, e->stream));
+    }
+    for (const Group &g : groups) {
+      HIP_TRY(e, hipFuncSetAttribute((const void *)g.kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)g.lds));
+      hipLaunchKernelGGL(g.kern, dim3((unsigned)g.count), dim3(kNvtBlock), g.lds, e->stream,
+                         (const NvtChainArgs *)(d_args + g.first));
+      HIP_TRY(e, hipGetLastError());
+    }
   }
-  return rc ? rc : rc2;
+  rc = nvt_finish(e, Ls, nsteps, B);
+  for (int k = 0; !rc && k < nboxes; ++k)
+    if (Ls[k].host_loop)
+      rc = cass_nvt_run(e, boxes[k], rngs + k, opts + k, nsteps, ens + k, recs ? recs + k : nullptr);
+  return rc;
 }

@@ -152,6 +152,42 @@ def _p(a, t=C.c_double):
     return None if a is None else a.ctypes.data_as(C.POINTER(t))
 
 
+def _energies_in(energies):
+    """A CassEnergy array of energy dicts."""
+    ens = (abi.CassEnergy * len(energies))()
+    if energies:
+        _energy_rows(ens)[:] = [[en.get(f, 0.0) for f in abi.ENERGY_FIELDS] for en in energies]
+    return ens
+
+
+def _energy_rows(ens):
+    return np.frombuffer(ens, dtype=np.float64).reshape(len(ens), len(abi.ENERGY_FIELDS))
+
+
+def _energies_out(ens):
+    return [dict(zip(abi.ENERGY_FIELDS, row)) for row in _energy_rows(ens).tolist()] if len(ens) else []
+
+
+class _NvtRecords:
+    """The per-move records of n chains in one array per field, and the
+    CassNvtRecord table that points into them."""
+
+    def __init__(self, n, nsteps):
+        self.kind, self.acc = np.zeros((n, nsteps), dtype=np.uint8), np.zeros((n, nsteps), dtype=np.uint8)
+        self.et, self.lp = np.zeros((n, nsteps)), np.zeros((n, nsteps))
+        self.rs = np.zeros((n, nsteps, 5), dtype=np.int64)
+        self.table = (abi.CassNvtRecord * n)()
+        if n and nsteps:
+            fields = (self.kind, self.acc, self.et, self.rs, self.lp)    # the struct's order
+            at = np.frombuffer(self.table, dtype=np.uint64).reshape(n, len(fields))
+            for f, a in enumerate(fields):
+                at[:, f] = a.ctypes.data + np.arange(n, dtype=np.uint64) * np.uint64(a.strides[0])
+
+    def result(self, k, final):
+        return dict(kind=self.kind[k], accepted=self.acc[k].astype(bool), energy=self.et[k], ln_pacc=self.lp[k],
+                    rng=self.rs[k], final=final)
+
+
 class Engine:
     """One engine (one GPU, one topology) holding one or more boxes."""
 
@@ -244,21 +280,27 @@ class Engine:
         nb = len(specs)
         bx = (abi.CassGcmcBox * nb)()
         st = (abi.CassGcmcState * nb)()
+        ens = _energies_in([s["energy"] for s in states])
+        # one array for all boxes' locate and reservoir lists
+        at = np.concatenate([[0], np.cumsum([2 * g["max_mols"] for g in specs])])
+        slots = np.zeros(max(1, int(at[-1])), dtype=np.int32)
         keep = []
+        i32p = C.POINTER(C.c_int32)
         for i, (g, s) in enumerate(zip(specs, states)):
             bx[i] = abi.CassGcmcBox(g["box"], g["species"], g["first_slot"], g["max_mols"], g["prob_insert"],
                                     g["mu"], g["de_broglie"])
-            loc = np.zeros(g["max_mols"], dtype=np.int32)
+            o, m = int(at[i]), g["max_mols"]
+            loc, res = slots[o:o + m], slots[o + m:o + 2 * m]
             loc[:len(s["locate"])] = s["locate"]
-            res = np.zeros(g["max_mols"], dtype=np.int32)
             res[:len(s["reservoir"])] = s["reservoir"]
             keep += [loc, res]
-            st[i].rng = s["rng"]
-            st[i].energy = abi.CassEnergy(**{k: s["energy"].get(k, 0.0) for k in abi.ENERGY_FIELDS})
-            st[i].nmols = len(s["locate"])
-            st[i].nres = len(s["reservoir"])
-            st[i].locate = _p(loc, C.c_int32)
-            st[i].reservoir = _p(res, C.c_int32)
+            x = st[i]
+            x.rng = s["rng"]
+            x.energy = ens[i]
+            x.nmols = len(s["locate"])
+            x.nres = len(s["reservoir"])
+            x.locate = C.cast(slots.ctypes.data + 4 * o, i32p)
+            x.reservoir = C.cast(slots.ctypes.data + 4 * (o + m), i32p)
         rec = None
         if record:
             kind = np.zeros((nb, nsteps), dtype=np.uint8)
@@ -287,30 +329,23 @@ class Engine:
         n = len(boxes)
         ids = np.ascontiguousarray([b.id for b in boxes], dtype=np.int32)
         opts = (abi.CassNvtOptions * n)()
-        ens = (abi.CassEnergy * n)()
         rng_arr = (abi.CassRng * n)()
-        recs = (abi.CassNvtRecord * n)()
-        keep = []
-        for k, (b, r, en) in enumerate(zip(boxes, rngs, energies)):
+        ens = _energies_in(energies)
+        recs = _NvtRecords(n, nsteps)
+        linear = {}     # per species object: boxes of one system share theirs
+        for k, (b, r) in enumerate(zip(boxes, rngs)):
             sp = b.system.species[species]
+            if id(sp) not in linear:
+                linear[id(sp)] = int(sp.linear)
             opts[k] = abi.CassNvtOptions(b.params_prob_translate(), b.system.max_disp, b.system.max_rot_radians(),
-                                         int(sp.linear), species)
-            ens[k] = abi.CassEnergy(**{f: en.get(f, 0.0) for f in abi.ENERGY_FIELDS})
+                                         linear[id(sp)], species)
             rng_arr[k] = r
-            arrs = dict(kind=np.zeros(nsteps, dtype=np.uint8), acc=np.zeros(nsteps, dtype=np.uint8),
-                        et=np.zeros(nsteps), lp=np.zeros(nsteps), rs=np.zeros(5 * nsteps, dtype=np.int64))
-            keep.append(arrs)
-            recs[k] = abi.CassNvtRecord(_p(arrs["kind"], C.c_uint8), _p(arrs["acc"], C.c_uint8), _p(arrs["et"]),
-                                        _p(arrs["rs"], C.c_int64), _p(arrs["lp"]))
         self._chk(self.lib.cass_nvt_run_device_batch(self.h, n, _p(ids, C.c_int32), rng_arr, opts, nsteps, ens,
-                                                     recs if record else None), "cass_nvt_run_device_batch")
-        out = []
+                                                     recs.table if record else None), "cass_nvt_run_device_batch")
+        finals = _energies_out(ens)
         for k in range(n):
             C.memmove(C.addressof(rngs[k]), C.addressof(rng_arr[k]), C.sizeof(abi.CassRng))
-            a = keep[k]
-            out.append(dict(kind=a["kind"], accepted=a["acc"].astype(bool), energy=a["et"], ln_pacc=a["lp"],
-                            rng=a["rs"].reshape(-1, 5), final=ens[k].as_dict()))
-        return out
+        return [recs.result(k, finals[k]) for k in range(n)]
 
     def regrow_run(self, boxes, species, locates, rngs, nsteps, energies, first_slot=0, record=True):
         """cass_regrow_run_device: nsteps Cut_N_Grow regrowth moves of
@@ -320,29 +355,21 @@ class Engine:
         record dict per box as nvt_run_batch does."""
         n = len(boxes)
         bx = (abi.CassRegrowBox * n)()
-        ens = (abi.CassEnergy * n)()
         rng_arr = (abi.CassRng * n)()
-        recs = (abi.CassNvtRecord * n)()
+        ens = _energies_in(energies)
+        recs = _NvtRecords(n, nsteps)
         keep = []
-        for k, (b, loc, r, en) in enumerate(zip(boxes, locates, rngs, energies)):
+        for k, (b, loc, r) in enumerate(zip(boxes, locates, rngs)):
             loc = np.ascontiguousarray(loc, dtype=np.int32)
-            arrs = dict(loc=loc, kind=np.zeros(nsteps, dtype=np.uint8), acc=np.zeros(nsteps, dtype=np.uint8),
-                        et=np.zeros(nsteps), lp=np.zeros(nsteps), rs=np.zeros(5 * nsteps, dtype=np.int64))
-            keep.append(arrs)
+            keep.append(loc)
             bx[k] = abi.CassRegrowBox(b.id, species, first_slot, len(loc), _p(loc, C.c_int32))
-            ens[k] = abi.CassEnergy(**{f: en.get(f, 0.0) for f in abi.ENERGY_FIELDS})
             rng_arr[k] = r
-            recs[k] = abi.CassNvtRecord(_p(arrs["kind"], C.c_uint8), _p(arrs["acc"], C.c_uint8), _p(arrs["et"]),
-                                        _p(arrs["rs"], C.c_int64), _p(arrs["lp"]))
-        self._chk(self.lib.cass_regrow_run_device(self.h, n, bx, rng_arr, nsteps, ens, recs if record else None),
+        self._chk(self.lib.cass_regrow_run_device(self.h, n, bx, rng_arr, nsteps, ens, recs.table if record else None),
                   "cass_regrow_run_device")
-        out = []
+        finals = _energies_out(ens)
         for k in range(n):
             C.memmove(C.addressof(rngs[k]), C.addressof(rng_arr[k]), C.sizeof(abi.CassRng))
-            a = keep[k]
-            out.append(dict(kind=a["kind"], accepted=a["acc"].astype(bool), energy=a["et"], ln_pacc=a["lp"],
-                            rng=a["rs"].reshape(-1, 5), final=ens[k].as_dict()))
-        return out
+        return [recs.result(k, finals[k]) for k in range(n)]
 
     def total_energy_batch(self, boxes, intra=True):
         """cass_total_energy_batch: total energies of several boxes in one set
