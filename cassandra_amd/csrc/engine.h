@@ -30,8 +30,10 @@ struct cass_box_state {
   double *cmol = nullptr, *smol = nullptr;        // [cap_mols][nvecs]
   double *cs_new = nullptr, *sn_new = nullptr;    // staged box sums of a move
   double *cm_new = nullptr, *sm_new = nullptr;    // staged molecule sums of a move
-  int4 *rows = nullptr;
-  int32_t nrows = 0;
+  int4 *rows = nullptr;             // traversal rows, then the k segments, then the rows' positions and kperm
+  int32_t nrows = 0, nsegs = 0;
+  const int4 *segs() const { return rows + nrows; }  // runs of up to kKSeg vectors along nx: (k0 | len << 20, nx, ny, nz)
+  int32_t kmax[3] = {0, 0, 0};      // largest |nx|, |ny|, |nz|
   int32_t staged_mol = -1, staged_flag = -1;
   bool ewald_ready = false;
   double e_recip = 0.0;             // last full / committed total reciprocal energy

@@ -149,11 +149,11 @@ static EwaldDev ewald_view(const cass_box_state &b, const int *row_k0) {
 }
 
 // traversal position of each k row's first vector, stored after the rows
-static const int *row_k0_of(const cass_box_state &b) { return (const int *)(b.rows + b.nrows); }
+static const int *row_k0_of(const cass_box_state &b) { return (const int *)(b.rows + b.nrows + b.nsegs); }
 BoxDev cass_box_view(const cass_engine *e, const cass_box_state &b) { return box_view(e, b); }
 TopoDev cass_topo_view(const cass_engine *e) { return topo_view(e); }
 EwaldDev cass_ewald_view(const cass_box_state &b) {
-  return ewald_view(b, b.rows ? (const int *)(b.rows + b.nrows) : nullptr);
+  return ewald_view(b, b.rows ? row_k0_of(b) : nullptr);
 }
 
 static bool species_charged(const cass_engine *e, int s) {
@@ -1333,6 +1333,19 @@ extern "C" int cass_ewald_setup(cass_engine *e, int32_t box, int32_t *nvecs) {
       g = h;
     }
   }
+  // the segments of consecutive vectors along nx, in k order
+  std::vector<int4> tables = rows;
+  int kmax[3] = {0, 0, 0};
+  for (int k = 0; k < K; ++k) {
+    const int *c = &kn[3 * k];
+    for (int d = 0; d < 3; ++d) kmax[d] = std::max(kmax[d], std::abs(c[d]));
+    const bool follows = k > 0 && c[0] == c[-3] + 1 && c[1] == c[-2] && c[2] == c[-1];
+    if (follows && (tables.back().x >> 20) < kKSeg)
+      tables.back().x += 1 << 20;
+    else
+      tables.push_back(make_int4(k | 1 << 20, c[0], c[1], c[2]));
+  }
+  const size_t nsegs = tables.size() - rows.size();
   // (re)allocate the k-space arrays of this box
   void *old[] = {b->hx, b->hy, b->hz, b->cn, b->cs, b->sn, b->cmol, b->smol, b->cs_new, b->sn_new,
                  b->cm_new, b->sm_new, b->rows};
@@ -1351,20 +1364,25 @@ extern "C" int cass_ewald_setup(cass_engine *e, int32_t box, int32_t *nvecs) {
   HIP_TRY(e, dalloc(&b->sm_new, K));
   HIP_TRY(e, dalloc(&b->cmol, (size_t)K * b->cap_mols));
   HIP_TRY(e, dalloc(&b->smol, (size_t)K * b->cap_mols));
-  // rows, their first positions and the k permutation share one allocation
-  HIP_TRY(e, dalloc(&b->rows, rows.size() + (k0.size() + kperm.size() + 3) / 4 + 1));
+  // rows, segments, the rows' first positions and the k permutation share one
+  // allocation and one copy
+  const size_t head = tables.size();
+  tables.resize(head + (k0.size() + kperm.size() + 3) / 4 + 1);
+  std::memcpy((void *)(tables.data() + head), k0.data(), sizeof(int32_t) * k0.size());
+  std::memcpy((int32_t *)(tables.data() + head) + k0.size(), kperm.data(), sizeof(int32_t) * kperm.size());
+  HIP_TRY(e, dalloc(&b->rows, tables.size()));
   HIP_TRY(e, upload(e, b->hx, hx.data(), K));
   HIP_TRY(e, upload(e, b->hy, hy.data(), K));
   HIP_TRY(e, upload(e, b->hz, hz.data(), K));
   HIP_TRY(e, upload(e, b->cn, cn.data(), K));
-  HIP_TRY(e, upload(e, b->rows, rows.data(), rows.size()));
-  HIP_TRY(e, upload(e, (int32_t *)(b->rows + rows.size()), k0.data(), k0.size()));
-  HIP_TRY(e, upload(e, (int32_t *)(b->rows + rows.size()) + k0.size(), kperm.data(), kperm.size()));
+  HIP_TRY(e, upload(e, b->rows, tables.data(), tables.size()));
   HIP_TRY(e, hipMemsetAsync(b->cs, 0, sizeof(double) * std::max(K, 1), e->stream));
   HIP_TRY(e, hipMemsetAsync(b->sn, 0, sizeof(double) * std::max(K, 1), e->stream));
   HIP_TRY(e, hipStreamSynchronize(e->stream));
   b->nvecs = K;
   b->nrows = (int)rows.size();
+  b->nsegs = (int)nsegs;
+  std::copy(kmax, kmax + 3, b->kmax);
   b->hx_h = hx;
   b->hy_h = hy;
   b->hz_h = hz;

@@ -4,12 +4,11 @@
 // and Rotate (move_rotate.f90:23-520), with the same random-number draws
 // (random_generators.f90:51-122), energy bookkeeping and accept_or_reject
 // (accept_or_reject.f90:22-65) as the host-driven loop in nvt.cpp.  One
-// workgroup of 512 threads runs the moves in sequence: thread 0 draws the
-// move and builds the trial coordinates, all threads share the molecule-pair
-// energies (old and new placements side by side) and the k vectors of the
-// reciprocal update, and an accepted move is committed in device memory.  No
-// host round trip per move: the host launches chunks of moves and reads the
-// RNG state, energies and records back at the end.
+// workgroup per box runs the moves in sequence on a copy of the box in LDS:
+// one wave prepares the next move while the others evaluate the current one,
+// sharing the molecule-pair energies and the k vectors of the reciprocal
+// update.  No host round trip per move: the host launches chunks of moves and
+// reads the RNG state, energies and records back at the end.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -24,43 +23,56 @@
 
 namespace cass {
 
-// 512 threads: two waves per SIMD leave 256 VGPRs per lane (1024 threads cap
-// them at 128, and the move's state then spills to scratch)
-constexpr int kNvtBlock = 512;
-constexpr int kNvtWaves = kNvtBlock / 64;
+// Waves per workgroup: the last wave prepares moves, the others share the
+// molecules and the k segments.  12 waves are three per SIMD at up to 168
+// VGPRs: a move of 512 waters takes 11.9 us on 12, 17.8 on 8 (the k segments
+// no longer fit one per lane) and 13.7 on 16 (128 VGPRs, which spill).  A box
+// whose copy leaves no room for their buffers runs on fewer (nvt_prepare).
+constexpr int kNvtWaves = 12;
+constexpr int kNvtMinWaves = 2;
+constexpr int kNvtSeg = kKSeg;   // k vectors per segment
+constexpr int kNvtRing = 32;     // generator states kept around the current move
+constexpr int kNvtAhead = 10;    // draws of one move (6 at most, its acceptance, the other start) and some
+constexpr int kNvtList = 128;    // entries of a wave's molecule list and of its pair list
 
 struct NvtChainArgs {
   BoxDev b;
   TopoDev tp;
   PairConst<double> cd;
-  PairConst<float> cf;
   EwaldDev ew;
+  const int4 *segs;   // k segments: (first k | length << 20, nx, ny, nz), nx rising by one per k
+  int nsegs;
+  int tx, ty, tz, nt_site;  // powers of the unit phases kept per axis; their sum
+  int tabled;               // the phases' powers fit in LDS
   double *x, *y, *z;  // the box's site coordinates (the memory of b.x, b.y, b.z)
   double4 *comd;      // the box's (COM, max_dcom) (the memory of b.comd)
   const int *mols;    // mobile molecules in locate order
-  int nm, species, n, spa0, charged, linear, coul_cbmc;
-  int nj_uniform;  // the common site count of every molecule of the box, or 0
+  int nm, n, spa0, charged, linear;
+  int nj_max;  // the largest site count of the box's molecules
   double prob_translate, max_disp, max_rot, beta;
-  int64_t nsteps, step0;  // moves of this launch; index of its first move
   int64_t *rng;           // 5 words, in/out
   double *en;             // total, inter, inter_vdw, inter_q, reciprocal; in/out
-  uint8_t *kind, *accepted;  // records per move (index step0 + s), or null
+  uint8_t *kind, *accepted;  // records per move or null
   double *energy, *ln_pacc;
   int64_t *rng_state;
   int *status;  // set to 1 when a molecule overlaps before its move
-  double *ctrav, *strav;  // molecule sums in k-traversal order (nvecs each)
   // the box held in LDS for the whole chain (offsets in bytes)
   int nsite, natoms_total, nspecies, ntypes;
-  int o_x, o_y, o_z, o_comd, o_first, o_spec, o_live, o_atype, o_acharge, o_spn, o_spo, o_pt, o_pq, o_prow,
-      o_mols, o_ent, o_eoff;
+  int o_x, o_y, o_z, o_comd, o_first, o_meta, o_atype, o_acharge, o_spn, o_spo, o_pt, o_pq, o_pm, o_prow, o_cand,
+      o_eph, o_tab, o_ent, o_pr2, o_pcode;
 };
 
-// One site pair of Compute_MoleculePair_Energy (energy_routines.f90:1589-1730):
-// site ia of the moving molecule (px/py/pz, type pt, charge pq) against site
-// (x, y, z, type tj, charge qj) of another molecule, full cutoffs, with the
-// reference's FP64 operations (the arithmetic of molpair_energy<PrecFP64>);
-// prow[ia * ntypes + tj] holds (eps, sigma, n, m) of the pair's types.
-// Returns true on overlap r^2 < rcut_low^2, else adds the pair's terms.
+// Orders this wave's LDS traffic for the compiler; a wave's LDS operations
+// execute in order.
+__device__ __forceinline__ void nvt_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The energies of one site pair of Compute_MoleculePair_Energy
+// (energy_routines.f90:1589-1730) at squared distance r2d, full cutoffs, with
+// the reference's FP64 operations (the arithmetic of molpair_energy<PrecFP64>).
 // PM: 0 any style with the reference's FP64 operations (vdw_inter,
 // qq_inter); 1 the common styles (LJ cut / cut_tail / cut_shift or none with
 // Ewald, cut or no Coulomb), whose cutoff tests and pair terms are
@@ -68,38 +80,54 @@ struct NvtChainArgs {
 // vdw_inter and qq_inter take for them), FP64 operations; 2 the common
 // styles in the mixed mode (hardware rcp/rsq seeds refined by Newton steps).
 template <int PM>
-__device__ inline bool nvt_pair(const BoxDev &b, const PairConst<double> &cd, double px, double py, double pz,
-                                int ti, double qi, const double4 *prow_i, double x, double y, double z, int tj,
-                                double qj, double &ev, double &eq) {
-  double dx = px - x, dy = py - y, dz = pz - z;
-  min_image(b, dx, dy, dz);
-  const double r2d = dx * dx + dy * dy + dz * dz;
-  if (r2d < cd.rc_low2) return true;
-  bool gv, gq;
-  constexpr bool COMMON = PM > 0;
-  using M = typename std::conditional<PM == 2, MathFast, MathRef>::type;
-  if (COMMON) {
+__device__ __forceinline__ void nvt_cutoff(const PairConst<double> &cd, double r2d, bool &gv, bool &gq) {
+  if (PM > 0) {
     gv = cd.vdw_style == CASS_VDW_LJ && r2d <= cd.rc_vdw2;
     gq = cd.q_style != CASS_Q_NONE && r2d <= cd.rc_coul2;
   } else {
     pair_cutoff(cd, false, r2d, gv, gq);
   }
-  if (!(gv || gq)) return false;
-  double e_v = 0.0, e_q = 0.0;
-  if (ti >= 0 && tj >= 0 && gv) {
-    const double4 p = prow_i[tj];
-    e_v = COMMON ? lj_cut<double, M>(cd, r2d, p.x, p.y) : vdw_inter<double, MathRef>(cd, r2d, p.x, p.y, p.z, p.w);
+}
+
+template <int PM>
+__device__ __forceinline__ void nvt_pair(const PairConst<double> &cd, double r2d, int ti, double qi,
+                                         const double4 *prow_i, int tj, double qj, double &ev, double &eq) {
+  bool gv, gq;
+  nvt_cutoff<PM>(cd, r2d, gv, gq);
+  using M = typename std::conditional<PM == 2, MathFast, MathRef>::type;
+  gv = gv && ti >= 0 && tj >= 0;
+  gq = gq && cd.q_style != CASS_Q_NONE && qi != 0.0 && qj != 0.0;
+  if (PM > 0) {
+    // both terms side by side and selected: their serial chains overlap
+    const double4 p = prow_i[tj < 0 ? 0 : tj];
+    double e_v = 0.0, e_q = 0.0;
+    if (cd.vdw_style == CASS_VDW_LJ) e_v = lj_cut<double, M>(cd, r2d, p.x, p.y);
+    if (cd.q_style == CASS_Q_EWALD)
+      e_q = ewald_real<double, M>(cd, r2d, qi * qj);
+    else if (cd.q_style != CASS_Q_NONE)
+      e_q = coul_cut<double, M>(r2d, qi * qj);
+    ev += gv ? e_v : 0.0;
+    eq += gq ? e_q : 0.0;
+  } else {
+    if (gv) {
+      const double4 p = prow_i[tj];
+      ev += vdw_inter<double, MathRef>(cd, r2d, p.x, p.y, p.z, p.w);
+    }
+    if (gq) eq += qq_inter<double, MathRef>(cd, r2d, qi * qj);
   }
-  const bool any_q = cd.q_style != CASS_Q_NONE && qi != 0.0 && qj != 0.0;
-  if (any_q && gq) {
-    if (COMMON)
-      e_q = cd.q_style == CASS_Q_EWALD ? ewald_real<double, M>(cd, r2d, qi * qj) : coul_cut<double, M>(r2d, qi * qj);
-    else
-      e_q = qq_inter<double, MathRef>(cd, r2d, qi * qj);
+}
+
+// min_image with the box kind known at compile time: the other kind's
+// matrices would hold 36 scalar registers through the pair loop.
+template <bool CUBIC>
+__device__ __forceinline__ void nvt_image(const BoxDev &b, double &dx, double &dy, double &dz) {
+  if (CUBIC) {
+    if (dx > b.hL[0]) dx -= b.L[0]; else if (dx < -b.hL[0]) dx += b.L[0];
+    if (dy > b.hL[1]) dy -= b.L[1]; else if (dy < -b.hL[1]) dy += b.L[1];
+    if (dz > b.hL[2]) dz -= b.L[2]; else if (dz < -b.hL[2]) dz += b.L[2];
+  } else {
+    min_image(b, dx, dy, dz);
   }
-  if (gv) ev += e_v;
-  if (gq) eq += e_q;
-  return false;
 }
 
 // The centre prefilter of Check_MoleculePair_Cutoff (energy_routines.f90:
@@ -107,545 +135,753 @@ __device__ inline bool nvt_pair(const BoxDev &b, const PairConst<double> &cd, do
 // the two can differ only at the prefilter distance itself, where every site
 // pair lies beyond the cutoff and beyond rcut_low, so the energies and the
 // overlap test do not depend on the choice.
-__device__ inline bool nvt_in_range(const BoxDev &b, double4 ci, double4 cj) {
+template <bool CUBIC>
+__device__ __forceinline__ bool nvt_in_range(const BoxDev &b, double4 ci, double4 cj) {
   if (b.vdw_minimum) return true;
   double dx = ci.x - cj.x, dy = ci.y - cj.y, dz = ci.z - cj.z;
-  min_image(b, dx, dy, dz);
+  nvt_image<CUBIC>(b, dx, dy, dz);
   const double rint = b.rcut_max + ci.w + cj.w;
   return dx * dx + dy * dy + dz * dz <= rint * rint;
 }
 
-// Exclusive workgroup scan of two counts (fixed order); also returns the
-// totals.  sc/st: LDS scratch of kNvtWaves ints each.
-__device__ inline void nvt_scan2(int c, int t, int &cpre, int &tpre, int &ctot, int &ttot, int *sc, int *st) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  int ci = c, ti = t;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int cu = __shfl_up(ci, o, 64), tu = __shfl_up(ti, o, 64);
-    if (lane >= o) {
-      ci += cu;
-      ti += tu;
+__device__ __forceinline__ double nvt_readlane(double v, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                          __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+
+// Set bits of a ballot below this lane.
+__device__ __forceinline__ int nvt_rank(uint64_t bal) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0));
+}
+
+// Sums over the 16 lanes of each row, in the row's last lane.
+__device__ __forceinline__ double nvt_row_sum(double v) {
+  v = dpp_add<0x111, 0xf>(v);
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  return dpp_add<0x118, 0xf>(v);
+}
+
+// A move ahead of its evaluation.  Two are prepared per step, since the move
+// before it consumes one draw more when its acceptance is drawn.
+struct NvtCand {
+  double4 com_old, com_new;  // Get_COM of the old and of the trial sites
+  double cx, cy, cz;         // the folded centre of a translation
+  int m, rot, draws;         // molecule, rotation, draws before the acceptance
+};
+
+// The generator's states: ring[i % kNvtRing] after i draws, u[i % kNvtRing]
+// the i-th draw of rranf (random_generators.f90:51-122): five-component LFSR,
+// u in (0, 1).  The components step side by side on five lanes; `st` is the
+// lane's component after `filled` draws.
+struct NvtRng {
+  int64_t st;
+  int64_t filled;
+};
+
+__device__ __forceinline__ void nvt_fill(NvtRng &g, int64_t upto, int64_t (*ring)[5], double *u) {
+  const int lane = threadIdx.x & 63;
+  const int c = lane < 5 ? lane : 4;
+  const int s1 = c == 0 ? 1 : c == 1 ? 24 : c == 3 ? 5 : 3;
+  const int s2 = c == 0 ? 53 : c == 1 ? 50 : c == 2 ? 23 : c == 3 ? 24 : 33;
+  const int s3 = c == 0 ? 10 : c == 1 ? 5 : c == 2 ? 29 : c == 3 ? 23 : 8;
+  const uint64_t mask = c == 0 ? (uint64_t)-2 : c == 1 ? (uint64_t)-512 : c == 2 ? (uint64_t)-4096
+                                                  : c == 3 ? (uint64_t)-131072 : (uint64_t)-8388608;
+  const int64_t from = g.filled;
+  while (g.filled < upto) {
+    const uint64_t v = (uint64_t)g.st;
+    const uint64_t b = ((v << s1) ^ v) >> s2;
+    g.st = (int64_t)(((v & mask) << s3) ^ b);
+    ++g.filled;
+    if (lane < 5) ring[g.filled & (kNvtRing - 1)][lane] = g.st;
+  }
+  nvt_wave_sync();
+  if (lane < (int)(g.filled - from)) {
+    const int64_t *r = ring[(from + lane + 1) & (kNvtRing - 1)];
+    u[(from + lane) & (kNvtRing - 1)] = (double)(r[0] ^ r[1] ^ r[2] ^ r[3] ^ r[4]) * 5.4210108624275221E-20 + 0.5;
+  }
+  nvt_wave_sync();
+}
+
+// One axis of Fold_Molecule for a cubic box: the shift of the centre c and of
+// its sites by one box length when c leaves [-h, h].
+__device__ __forceinline__ int nvt_fold(double c, double h) { return c > h ? -1 : c < -h ? 1 : 0; }
+__device__ __forceinline__ double nvt_shift(double v, int f, double L) { return f < 0 ? v - L : f > 0 ? v + L : v; }
+
+// The LDS of a chain.
+struct NvtLds {
+  double *lx, *ly, *lz;
+  double4 *lcomd;
+  int *lfirst, *lmeta, *atype;
+  double *acharge;
+  int *spn, *spo, *pt;
+  double *pq, *pm;
+  double4 *prow;
+  double *cand;  // [3][2][6 n]: old x, y, z, trial x, y, z
+  cplx *eph;     // [2][3 n]
+  cplx *tab;     // [2][2][n][nt_site]
+};
+
+// Both candidates of the move `step` by one wave, a half wave each: variant v
+// starts at draw pos + v.  The draws and the operations are those of
+// nvtmc_driver.f90:94-152 and Translate / Rotate.  A molecule whose accepted
+// move the owning wave may still be writing (fm) is read from that move's
+// candidate (fc, its sites at fq).
+__device__ __forceinline__ void nvt_prepare_move(const NvtChainArgs &a, const NvtLds &S, const double *u,
+                                                 int64_t pos, int step, NvtCand (*cand)[2], int fm,
+                                                 const NvtCand *fc, const double *fq) {
+  const int lane = threadIdx.x & 63, v = lane >> 5, l = lane & 31;
+  const int n = a.n;
+  auto draw = [&](int i) { return u[(pos + v + i) & (kNvtRing - 1)]; };
+  const int rot = !(draw(0) <= a.prob_translate);
+  // draw 1: the species pick (one mobile species)
+  const int m = a.mols[(int)(draw(2) * a.nm)];
+  const int f = S.lfirst[m];
+  const bool fwd = m == fm;
+  double4 co = S.lcomd[m];
+  if (fwd) {
+    co.x = fc->rot ? fc->com_new.x : fc->cx;
+    co.y = fc->rot ? fc->com_new.y : fc->cy;
+    co.z = fc->rot ? fc->com_new.z : fc->cz;
+  }
+  const int slot = step % 3;
+  double *o = S.cand + (size_t)(slot * 2 + v) * 6 * n, *q = o + 3 * n;
+  double cx = co.x, cy = co.y, cz = co.z;
+  double r[9] = {};
+  double dx = 0.0, dy = 0.0, dz = 0.0;
+  int fx = 0, fy = 0, fz = 0, draws = 6;
+  if (!rot) {
+    dx = (2.0 * draw(3) - 1.0) * a.max_disp;
+    dy = (2.0 * draw(4) - 1.0) * a.max_disp;
+    dz = (2.0 * draw(5) - 1.0) * a.max_disp;
+    cx = co.x + dx;
+    cy = co.y + dy;
+    cz = co.z + dz;
+    // Fold_Molecule (minimum_image_separation.f90:162-240), cubic boxes
+    if (a.b.cubic) {
+      fx = nvt_fold(cx, a.b.hL[0]);
+      fy = nvt_fold(cy, a.b.hL[1]);
+      fz = nvt_fold(cz, a.b.hL[2]);
+      cx = nvt_shift(cx, fx, a.b.L[0]);
+      cy = nvt_shift(cy, fy, a.b.L[1]);
+      cz = nvt_shift(cz, fz, a.b.L[2]);
+    }
+  } else if (a.linear) {
+    // Rotate_Molecule_Eulerian (move_rotate.f90:468-520)
+    const double th = acos(1.0 - 2.0 * draw(3));
+    const double ph = (1.0 - 2.0 * draw(4)) * kPi;
+    const double ps = (1.0 - 2.0 * draw(5)) * kPi;
+    double sth, cth, sph, cph, sps, cps;
+    sincos(th, &sth, &cth);
+    sincos(ph, &sph, &cph);
+    sincos(ps, &sps, &cps);
+    r[0] = cps * cph - cth * sph * sps;
+    r[1] = cps * sph + cth * cph * sps;
+    r[2] = sps * sth;
+    r[3] = -sps * cph - cth * sph * cps;
+    r[4] = -sps * sph + cth * cph * cps;
+    r[5] = cps * sth;
+    r[6] = sth * sph;
+    r[7] = -sth * cph;
+    r[8] = cth;
+  } else {
+    // Rotate_Molecule_Axis (move_rotate.f90:362-463)
+    const int axis = (int)(3.0 * draw(3)) + 1;
+    const double ang = (2.0 * draw(4) - 1.0) * a.max_rot;
+    draws = 5;
+    // cos(0) = 1 and sin(0) = 0 exactly: only the drawn axis needs them
+    double sa, ca;
+    sincos(ang, &sa, &ca);
+    const double c1 = axis == 1 ? ca : 1.0, c2 = axis == 2 ? ca : 1.0, c3 = axis == 3 ? ca : 1.0;
+    const double s1 = axis == 1 ? sa : 0.0, s2 = axis == 2 ? sa : 0.0, s3 = axis == 3 ? sa : 0.0;
+    r[0] = c1 * c3 - s1 * c2 * s3;
+    r[1] = s1 * c3 + c1 * c2 * s3;
+    r[2] = s2 * s3;
+    r[3] = -c1 * s3 - s1 * c2 * c3;
+    r[4] = -s1 * s3 + c1 * c2 * c3;
+    r[5] = s2 * c3;
+    r[6] = s1 * s2;
+    r[7] = -c1 * s2;
+    r[8] = c2;
+  }
+  for (int i = l; i < n; i += 32) {
+    const double x = fwd ? fq[i] : S.lx[f + i], y = fwd ? fq[n + i] : S.ly[f + i], z = fwd ? fq[2 * n + i] : S.lz[f + i];
+    o[i] = x;
+    o[n + i] = y;
+    o[2 * n + i] = z;
+    if (!rot) {
+      q[i] = nvt_shift(x + dx, fx, a.b.L[0]);
+      q[n + i] = nvt_shift(y + dy, fy, a.b.L[1]);
+      q[2 * n + i] = nvt_shift(z + dz, fz, a.b.L[2]);
+    } else {
+      const double px = x - co.x, py = y - co.y, pz = z - co.z;
+      q[i] = (r[0] * px + r[1] * py + r[2] * pz) + co.x;
+      q[n + i] = (r[3] * px + r[4] * py + r[5] * pz) + co.y;
+      q[2 * n + i] = (r[6] * px + r[7] * py + r[8] * pz) + co.z;
     }
   }
-  if (lane == 63) {
-    sc[wid] = ci;
-    st[wid] = ti;
+  nvt_wave_sync();
+  // the trial kernel's prefilter centres: Get_COM of each placement
+  TopoDev tp = a.tp;
+  tp.atom_mass = S.pm;
+  const double *pp = (l & 1) ? q : o;
+  const double4 com = molecule_com(tp, 0, n, pp, pp + n, pp + 2 * n);
+  NvtCand &C = cand[slot][v];
+  if (l == 0) {
+    C.com_old = com;
+    C.cx = cx;
+    C.cy = cy;
+    C.cz = cz;
+    C.m = m;
+    C.rot = rot;
+    C.draws = draws;
   }
-  __syncthreads();
-  int cw = 0, tw = 0, ca = 0, ta = 0;
-  for (int w = 0; w < kNvtWaves; ++w) {
-    if (w < wid) {
-      cw += sc[w];
-      tw += st[w];
+  if (l == 1) C.com_new = com;
+  if (a.tabled) {
+    // (2 pi as the reference truncates it) the unit phases exp(2 pi i s) of the trial sites' fractional
+    // coordinates, then their powers
+    cplx *eph = S.eph + v * 3 * n;
+    for (int t = l; t < 3 * n; t += 32) {
+      const int i = t / 3, d = t - 3 * i;
+      const double sd = a.b.Li[d] * q[i] + a.b.Li[3 + d] * q[n + i] + a.b.Li[6 + d] * q[2 * n + i];
+      double sv, cv;
+      sincos(kTwoPi * sd, &sv, &cv);
+      eph[t] = cplx{cv, sv};
     }
-    ca += sc[w];
-    ta += st[w];
-  }
-  cpre = cw + ci - c;
-  tpre = tw + ti - t;
-  ctot = ca;
-  ttot = ta;
-  __syncthreads();
-}
-
-__device__ inline int64_t nvt_lsl(int64_t v, int k) { return (int64_t)((uint64_t)v << k); }
-__device__ inline int64_t nvt_lsr(int64_t v, int k) { return (int64_t)((uint64_t)v >> k); }
-
-// rranf (random_generators.f90:51-122): five-component LFSR, u in (0, 1)
-__device__ inline double nvt_uniform(int64_t *s) {
-  int64_t b;
-  b = nvt_lsr(nvt_lsl(s[0], 1) ^ s[0], 53);
-  s[0] = nvt_lsl(s[0] & -2, 10) ^ b;
-  b = nvt_lsr(nvt_lsl(s[1], 24) ^ s[1], 50);
-  s[1] = nvt_lsl(s[1] & -512, 5) ^ b;
-  b = nvt_lsr(nvt_lsl(s[2], 3) ^ s[2], 23);
-  s[2] = nvt_lsl(s[2] & -4096, 29) ^ b;
-  b = nvt_lsr(nvt_lsl(s[3], 5) ^ s[3], 24);
-  s[3] = nvt_lsl(s[3] & -131072, 23) ^ b;
-  b = nvt_lsr(nvt_lsl(s[4], 3) ^ s[4], 33);
-  s[4] = nvt_lsl(s[4] & -8388608, 8) ^ b;
-  return (double)(s[0] ^ s[1] ^ s[2] ^ s[3] ^ s[4]) * 5.4210108624275221E-20 + 0.5;
-}
-
-__device__ inline double nvt_wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  return v;
-}
-
-__device__ inline int nvt_wave_or(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v |= __shfl_down(v, o, 64);
-  return v;
-}
-
-// Workgroup sum of NV doubles and an OR of flags in a fixed order (waves,
-// then the waves in index order); every thread receives the result.
-template <int NV>
-__device__ inline void nvt_reduce(double (&v)[NV], int &flag, double (*sh)[kNvtWaves], int *shf, double *res,
-                                  int *resf) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-  for (int k = 0; k < NV; ++k) v[k] = nvt_wave_sum(v[k]);
-  flag = nvt_wave_or(flag);
-  if (lane == 0) {
-#pragma unroll
-    for (int k = 0; k < NV; ++k) sh[k][wid] = v[k];
-    shf[wid] = flag;
-  }
-  __syncthreads();
-  if (wid == 0) {
-    // the wave partials on the first kNvtWaves lanes, summed by a fixed
-    // shuffle tree
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      double s = lane < kNvtWaves ? sh[k][lane] : 0.0;
-#pragma unroll
-      for (int o = kNvtWaves / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-      if (lane == 0) res[k] = s;
+    nvt_wave_sync();
+    cplx *tab = S.tab + (size_t)((step & 1) * 2 + v) * n * a.nt_site;
+    for (int t = l; t < n * a.nt_site; t += 32) {
+      const int i = t / a.nt_site;
+      int p = t - i * a.nt_site, d = 0;
+      if (p >= a.tx + a.ty) {
+        p -= a.tx + a.ty;
+        d = 2;
+      } else if (p >= a.tx) {
+        p -= a.tx;
+        d = 1;
+      }
+      tab[t] = cpow_int(eph[3 * i + d], p);
     }
-    int f = lane < kNvtWaves ? shf[lane] : 0;
-#pragma unroll
-    for (int o = kNvtWaves / 2; o > 0; o >>= 1) f |= __shfl_xor(f, o, 64);
-    if (lane == 0) *resf = f;
   }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < NV; ++k) v[k] = res[k];
-  flag = *resf;
+  nvt_wave_sync();
 }
 
-// One axis of Fold_Molecule for a cubic box: the centre c and the sites q
-// move by one box length when c leaves [-h, h].
-__device__ inline void nvt_fold(double &c, double *q, int n, double L, double h) {
-  if (c > h) {
-    c = c - L;
-    for (int i = 0; i < n; ++i) q[i] = q[i] - L;
-  } else if (c < -h) {
-    c = c + L;
-    for (int i = 0; i < n; ++i) q[i] = q[i] + L;
+// Molecule sums of one k segment from the powers of its sites' unit phases:
+// exp(i k.r) at the segment's first vector is a product of three, then one
+// factor exp(2 pi i s_x) per vector.
+__device__ __forceinline__ void nvt_segment(const NvtChainArgs &a, const NvtLds &S, const cplx *tab, int4 sg,
+                                            double (&c)[kNvtSeg], double (&s)[kNvtSeg]) {
+  const int ny = sg.z < 0 ? -sg.z : sg.z, nz = sg.w < 0 ? -sg.w : sg.w;
+#pragma unroll
+  for (int t = 0; t < kNvtSeg; ++t) c[t] = s[t] = 0.0;
+  for (int i = 0; i < a.n; ++i) {
+    const cplx *ti = tab + i * a.nt_site;
+    const cplx X = ti[sg.y], E = ti[1];
+    cplx Y = ti[a.tx + ny], Z = ti[a.tx + a.ty + nz];
+    Y.im = sg.z < 0 ? -Y.im : Y.im;
+    Z.im = sg.w < 0 ? -Z.im : Z.im;
+    cplx p = cmul(cmul(X, Z), Y);
+    const double q = S.pq[i];
+    p.re = q * p.re;
+    p.im = q * p.im;
+#pragma unroll
+    for (int t = 0; t < kNvtSeg; ++t) {
+      c[t] = c[t] + p.re;
+      s[t] = s[t] + p.im;
+      if (t + 1 < kNvtSeg) p = cmul(p, E);
+    }
   }
 }
 
-template <int PM, int NSE>
-__device__ __forceinline__ void nvt_chain_run(const NvtChainArgs &a) {
-  __shared__ double ox[kMaxSites], oy[kMaxSites], oz[kMaxSites];
-  __shared__ double qx[kMaxSites], qy[kMaxSites], qz[kMaxSites];
-  __shared__ int pspa[kMaxSites];
-  __shared__ double4 com_old, com_new, cn_fold;
-  __shared__ int s_m, s_rot, s_acc;
-  __shared__ double sh[4][kNvtWaves];
-  __shared__ int shf[kNvtWaves];
-  __shared__ int scan_c[kNvtWaves], scan_t[kNvtWaves];
-  __shared__ double eph[6 * kMaxSites];  // (cos, sin) of 2 pi s_x, s_y, s_z per new site
-  __shared__ double res[4];
-  __shared__ int resf;
+// The same for one vector without tables: a sine and cosine per site.
+__device__ __forceinline__ void nvt_vector(const NvtChainArgs &a, const NvtLds &S, const double *q, int k, double &c,
+                                           double &s) {
+  const double hx = a.ew.hx[k], hy = a.ew.hy[k], hz = a.ew.hz[k];
+  c = s = 0.0;
+  for (int i = 0; i < a.n; ++i) {
+    double sn, cs;
+    sincos(hx * q[i] + hy * q[a.n + i] + hz * q[2 * a.n + i], &sn, &cs);
+    c = c + S.pq[i] * cs;
+    s = s + S.pq[i] * sn;
+  }
+}
+
+// The staged sums of one vector in device memory (Update_System_Ewald_
+// Reciprocal_Energy) and its energy term.
+__device__ __forceinline__ double nvt_stage(const EwaldDev &ew, size_t mk, int k, double c, double s) {
+  const double cb = ew.cs[k] + (c - ew.cmol[mk + k]), sb = ew.sn[k] + (s - ew.smol[mk + k]);
+  ew.cs_new[k] = cb;
+  ew.sn_new[k] = sb;
+  ew.cm_new[k] = c;
+  ew.sm_new[k] = s;
+  return ew.cn[k] * (cb * cb + sb * sb);
+}
+
+// The acceptance of a move from the waves' partial sums (accept_or_reject.f90:
+// 22-65), taken by every wave for itself; en: the running energies.
+struct NvtOutcome {
+  int stop, acc, drawn;  // overlap before the move; accepted; acceptance drawn
+  double lnp;
+};
+
+__device__ __forceinline__ NvtOutcome nvt_decide(const NvtChainArgs &a, const double (*red)[16], const int *redf,
+                                                 int nc, int rot, double u, double (&en)[5]) {
+  const int lane = threadIdx.x & 63, rw = lane & 15;
+  const double part = nvt_row_sum(rw < nc ? red[lane >> 4][rw] : 0.0);
+  const double pk = nvt_row_sum(rw < nc ? red[4][rw] : 0.0);
+  const int f = rw < nc ? redf[rw] : 0;
+  const double v0 = nvt_readlane(part, 15), v1 = nvt_readlane(part, 31), v2 = nvt_readlane(part, 47),
+               v3 = nvt_readlane(part, 63);
+  const double erm = nvt_readlane(pk, 15) * kChargeFactor;
+  NvtOutcome r{__any(f & 1), 0, 0, std::numeric_limits<double>::quiet_NaN()};
+  if (r.stop || __any(f & 2)) return r;
+  double dE = 0.0;
+  if (a.charged) dE = erm - en[4];
+  if (!rot)
+    dE = dE + (v2 - v0) + (v3 - v1);
+  else
+    dE = dE + v2 - v0 + v3 - v1;
+  r.lnp = a.beta * dE;
+  int acc = 0, drawn = 0;
+  if (r.lnp <= 0.0) {
+    acc = 1;
+  } else if (r.lnp < kMaxKBT) {
+    drawn = 1;
+    if (u <= exp(-r.lnp)) acc = 1;
+  }
+  r.acc = __builtin_amdgcn_readfirstlane(acc);
+  r.drawn = __builtin_amdgcn_readfirstlane(drawn);
+  if (r.acc) {
+    en[0] = en[0] + dE;
+    en[1] = en[1] + dE;
+    en[2] = en[2] + v2 - v0;
+    en[3] = en[3] + v3 - v1;
+    if (a.charged) en[4] = erm;
+  }
+  return r;
+}
+
+// The chain is one workgroup's serial work, so a move costs one compute unit's
+// latency and, now, its issue rate: 28.6 us per move for 512 waters (2354 k
+// vectors) when thread 0 drew and built the move, a workgroup-wide list was
+// scanned together and the reciprocal sums went through global scratch, over
+// a dozen barriers; 11.9 us here (6.2 to 8 the pairs, 1 the k vectors, 1.5 the
+// sums and the decision), bound by the pair terms' instructions.  One barrier
+// ends each move:
+// - The last wave prepares the next move while the others evaluate this one:
+//   both possible starts in the random stream (nvt_prepare_move).
+// - Each other wave owns the molecules j = w, w + NC, ...: it alone reads and
+//   commits their LDS copy.  Its lanes list the molecules in range of either
+//   placement, walk their site pairs for both r^2, and compact the pairs
+//   within the cutoff, so that the pair terms run on full waves (4 in 10 pairs
+//   of listed molecules lie outside the cutoff).
+// - Each lane owns a k segment whose box sums stay in registers; the moving
+//   molecule's old sums are loaded before the pairs and used after them.
+// - Every wave adds up the partial sums and takes the decision itself.
+template <int PM, bool CUBIC>
+__device__ __forceinline__ void nvt_chain_run(const NvtChainArgs &a, int64_t step0, int64_t nsteps) {
+  __shared__ NvtCand cand[3][2];
+  __shared__ int64_t ring[kNvtRing][5];
+  __shared__ double uring[kNvtRing];
+  __shared__ double red[2][5][16];
+  __shared__ int redf[2][16];
   extern __shared__ char lds[];
-  double *lx = (double *)(lds + a.o_x), *ly = (double *)(lds + a.o_y), *lz = (double *)(lds + a.o_z);
-  double4 *lcomd = (double4 *)(lds + a.o_comd);
-  int *lfirst = (int *)(lds + a.o_first), *lspec = (int *)(lds + a.o_spec), *llive = (int *)(lds + a.o_live);
-  int *atype = (int *)(lds + a.o_atype);
-  double *acharge = (double *)(lds + a.o_acharge);
-  int *spn = (int *)(lds + a.o_spn), *spo = (int *)(lds + a.o_spo);
-  int *pt = (int *)(lds + a.o_pt);
-  double *pq = (double *)(lds + a.o_pq);
-  double4 *prow = (double4 *)(lds + a.o_prow);
-  int *lmols = (int *)(lds + a.o_mols);
-  int *ent_j = (int *)(lds + a.o_ent), *ent_off = (int *)(lds + a.o_eoff);
-  const int tid = threadIdx.x;
+  NvtLds S;
+  S.lx = (double *)(lds + a.o_x);
+  S.ly = (double *)(lds + a.o_y);
+  S.lz = (double *)(lds + a.o_z);
+  S.lcomd = (double4 *)(lds + a.o_comd);
+  S.lfirst = (int *)(lds + a.o_first);
+  S.lmeta = (int *)(lds + a.o_meta);
+  S.atype = (int *)(lds + a.o_atype);
+  S.acharge = (double *)(lds + a.o_acharge);
+  S.spn = (int *)(lds + a.o_spn);
+  S.spo = (int *)(lds + a.o_spo);
+  S.pt = (int *)(lds + a.o_pt);
+  S.pq = (double *)(lds + a.o_pq);
+  S.pm = (double *)(lds + a.o_pm);
+  S.prow = (double4 *)(lds + a.o_prow);
+  S.cand = (double *)(lds + a.o_cand);
+  S.eph = (cplx *)(lds + a.o_eph);
+  S.tab = (cplx *)(lds + a.o_tab);
+  const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), nc = (nthr >> 6) - 1;
+  const bool ahead = w == nc;  // the preparing wave
   const int n = a.n, K = a.ew.nvecs, nmols = a.b.nmols;
-  for (int i = tid; i < a.nsite; i += kNvtBlock) {
-    lx[i] = a.x[i];
-    ly[i] = a.y[i];
-    lz[i] = a.z[i];
+  for (int i = tid; i < a.nsite; i += nthr) {
+    S.lx[i] = a.x[i];
+    S.ly[i] = a.y[i];
+    S.lz[i] = a.z[i];
   }
-  for (int i = tid; i < nmols; i += kNvtBlock) {
-    lcomd[i] = a.comd[i];
-    lfirst[i] = a.b.first[i];
-    lspec[i] = a.b.species[i];
-    llive[i] = a.b.live[i];
+  for (int i = tid; i < nmols; i += nthr) {
+    S.lcomd[i] = a.comd[i];
+    S.lfirst[i] = a.b.first[i];
+    S.lmeta[i] = (a.b.species[i] << 1) | (a.b.live[i] ? 1 : 0);
   }
-  for (int i = tid; i < a.natoms_total; i += kNvtBlock) {
-    atype[i] = a.tp.atom_type[i];
-    acharge[i] = a.tp.atom_charge[i];
+  for (int i = tid; i < a.natoms_total; i += nthr) {
+    S.atype[i] = a.tp.atom_type[i];
+    S.acharge[i] = a.tp.atom_charge[i];
   }
-  for (int i = tid; i < a.nspecies; i += kNvtBlock) {
-    spn[i] = a.tp.sp_natoms[i];
-    spo[i] = a.tp.sp_atom_off[i];
+  for (int i = tid; i < a.nspecies; i += nthr) {
+    S.spn[i] = a.tp.sp_natoms[i];
+    S.spo[i] = a.tp.sp_atom_off[i];
   }
-  for (int i = tid; i < a.nm; i += kNvtBlock) lmols[i] = a.mols[i];
-  for (int i = tid; i < n * a.ntypes; i += kNvtBlock) {
+  for (int i = tid; i < n * a.ntypes; i += nthr) {
     const int ia = i / a.ntypes, tj = i - ia * a.ntypes;
     const int ti = a.tp.atom_type[a.spa0 + ia];
     const int k = (ti < 0 ? 0 : ti) * a.ntypes + tj;
-    prow[i] = make_double4(a.tp.eps[k], a.tp.sig[k], a.tp.mn[k], a.tp.mm[k]);
+    S.prow[i] = make_double4(a.tp.eps[k], a.tp.sig[k], a.tp.mn[k], a.tp.mm[k]);
   }
   if (tid < n) {
-    pspa[tid] = a.spa0 + tid;
-    pt[tid] = a.tp.atom_type[a.spa0 + tid];
-    pq[tid] = a.tp.atom_charge[a.spa0 + tid];
+    S.pt[tid] = a.tp.atom_type[a.spa0 + tid];
+    S.pq[tid] = a.tp.atom_charge[a.spa0 + tid];
+    S.pm[tid] = a.tp.atom_mass[a.spa0 + tid];
   }
-  // RNG words and energies: used by thread 0 only, kept in LDS
-  __shared__ int64_t rs[5];
-  __shared__ double en[5];
-  if (tid == 0) {
-    for (int k = 0; k < 5; ++k) rs[k] = a.rng[k];
-    for (int k = 0; k < 5; ++k) en[k] = a.en[k];
+  double en[5];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) en[k] = a.en[k];
+  // this lane's first k segment and its box sums
+  int4 sg = make_int4(0, 0, 0, 0);
+  double rcs[kNvtSeg], rsn[kNvtSeg], kn[kNvtSeg];
+  const int ct = w * 64 + lane, nct = nc * 64;  // evaluating lanes
+  const bool has = a.charged && a.tabled && !ahead && ct < a.nsegs;
+  const int more = a.tabled ? ct + nct : ct;  // the segments whose sums stay in device memory
+#pragma unroll
+  for (int t = 0; t < kNvtSeg; ++t) rcs[t] = rsn[t] = kn[t] = 0.0;
+  if (has) {
+    sg = a.segs[ct];
+    const int k0 = sg.x & 0xfffff, len = sg.x >> 20;
+#pragma unroll
+    for (int t = 0; t < kNvtSeg; ++t) {
+      const int k = k0 + (t < len ? t : len - 1);
+      rcs[t] = a.ew.cs[k];
+      rsn[t] = a.ew.sn[k];
+      kn[t] = t < len ? a.ew.cn[k] : 0.0;
+    }
   }
+  const int sk0 = sg.x & 0xfffff, slen = sg.x >> 20;
+  // this lane's place in a round of site pairs: E molecules of P pairs each
+  const int P = n * a.nj_max, E = P <= 64 ? 64 / P : 1;
+  const int pe = P <= 64 ? lane / P : 0, pp0 = P <= 64 ? lane - pe * P : lane;
+  const int pia = pp0 / a.nj_max, pja = pp0 - pia * a.nj_max;
+  int2 *ent = (int2 *)(lds + a.o_ent) + (ahead ? 0 : w) * kNvtList;
+  double *pr2 = (double *)(lds + a.o_pr2) + (ahead ? 0 : w) * kNvtList;
+  int *pcode = (int *)(lds + a.o_pcode) + (ahead ? 0 : w) * kNvtList;
   __syncthreads();
-  for (int64_t st = 0; st < a.nsteps; ++st) {
-    // --- the move (thread 0): draws in the order of nvtmc_driver / Translate / Rotate
-    if (tid == 0) {
-      const double rno = nvt_uniform(rs);
-      const int rot = !(rno <= a.prob_translate);
-      (void)nvt_uniform(rs);  // species pick (one mobile species)
-      const int im = (int)(nvt_uniform(rs) * a.nm);
-      const int m = lmols[im];
-      const int f = lfirst[m];
-      const double4 co = lcomd[m];
-      double4 cn = co;
-      for (int i = 0; i < n; ++i) {
-        ox[i] = lx[f + i];
-        oy[i] = ly[f + i];
-        oz[i] = lz[f + i];
+  int64_t pos = 0;  // draws consumed
+  int var = 0;      // which candidate of the move holds
+  int64_t st = 0;
+  if (ahead) {
+    NvtRng g;
+    g.filled = 0;
+    g.st = a.rng[lane < 5 ? lane : 4];
+    if (lane < 5) ring[0][lane] = g.st;
+    // the first move, then during move `st` the one after it; `to`: the move
+    // to prepare, fm and pvar: the molecule moved last and its variant
+    int fm = -1, pvar = 0;
+    int64_t to = 0, next = 0;
+    for (;;) {
+      if (to < nsteps) {
+        nvt_fill(g, next + kNvtAhead, ring, uring);
+        const int ps = (int)((to + 1) % 3);  // the slot of the move before the current one
+        nvt_prepare_move(a, S, uring, next, (int)(to % 6), cand, fm, &cand[ps][pvar],
+                         S.cand + (size_t)(ps * 2 + pvar) * 6 * n + 3 * n);
       }
-      if (!rot) {
-        const double dx = (2.0 * nvt_uniform(rs) - 1.0) * a.max_disp;
-        const double dy = (2.0 * nvt_uniform(rs) - 1.0) * a.max_disp;
-        const double dz = (2.0 * nvt_uniform(rs) - 1.0) * a.max_disp;
-        for (int i = 0; i < n; ++i) {
-          qx[i] = ox[i] + dx;
-          qy[i] = oy[i] + dy;
-          qz[i] = oz[i] + dz;
-        }
-        cn.x = co.x + dx;
-        cn.y = co.y + dy;
-        cn.z = co.z + dz;
-        // Fold_Molecule (minimum_image_separation.f90:162-240), cubic boxes
-        if (a.b.cubic) {
-          nvt_fold(cn.x, qx, n, a.b.L[0], a.b.hL[0]);
-          nvt_fold(cn.y, qy, n, a.b.L[1], a.b.hL[1]);
-          nvt_fold(cn.z, qz, n, a.b.L[2], a.b.hL[2]);
-        }
-      } else {
-        double r[9];
-        if (a.linear) {
-          // Rotate_Molecule_Eulerian (move_rotate.f90:468-520)
-          const double th = acos(1.0 - 2.0 * nvt_uniform(rs));
-          const double ph = (1.0 - 2.0 * nvt_uniform(rs)) * kPi;
-          const double ps = (1.0 - 2.0 * nvt_uniform(rs)) * kPi;
-          r[0] = cos(ps) * cos(ph) - cos(th) * sin(ph) * sin(ps);
-          r[1] = cos(ps) * sin(ph) + cos(th) * cos(ph) * sin(ps);
-          r[2] = sin(ps) * sin(th);
-          r[3] = -sin(ps) * cos(ph) - cos(th) * sin(ph) * cos(ps);
-          r[4] = -sin(ps) * sin(ph) + cos(th) * cos(ph) * cos(ps);
-          r[5] = cos(ps) * sin(th);
-          r[6] = sin(th) * sin(ph);
-          r[7] = -sin(th) * cos(ph);
-          r[8] = cos(th);
-        } else {
-          // Rotate_Molecule_Axis (move_rotate.f90:362-463)
-          double p1 = 0.0, p2 = 0.0, p3 = 0.0;
-          const int axis = (int)(3.0 * nvt_uniform(rs)) + 1;
-          const double ang = (2.0 * nvt_uniform(rs) - 1.0) * a.max_rot;
-          if (axis == 1)
-            p1 = ang;
-          else if (axis == 2)
-            p2 = ang;
-          else
-            p3 = ang;
-          // cos(0) = 1 and sin(0) = 0 exactly: only the drawn axis needs them
-          const double ca = cos(ang), sa = sin(ang);
-          const double c1 = axis == 1 ? ca : 1.0, c2 = axis == 2 ? ca : 1.0, c3 = axis == 3 ? ca : 1.0;
-          const double s1 = axis == 1 ? sa : 0.0, s2 = axis == 2 ? sa : 0.0, s3 = axis == 3 ? sa : 0.0;
-          (void)p1;
-          (void)p2;
-          (void)p3;
-          r[0] = c1 * c3 - s1 * c2 * s3;
-          r[1] = s1 * c3 + c1 * c2 * s3;
-          r[2] = s2 * s3;
-          r[3] = -c1 * s3 - s1 * c2 * c3;
-          r[4] = -s1 * s3 + c1 * c2 * c3;
-          r[5] = s2 * c3;
-          r[6] = s1 * s2;
-          r[7] = -c1 * s2;
-          r[8] = c2;
-        }
-        for (int i = 0; i < n; ++i) {
-          const double px = ox[i] - co.x, py = oy[i] - co.y, pz = oz[i] - co.z;
-          qx[i] = (r[0] * px + r[1] * py + r[2] * pz) + co.x;
-          qy[i] = (r[3] * px + r[4] * py + r[5] * pz) + co.y;
-          qz[i] = (r[6] * px + r[7] * py + r[8] * pz) + co.z;
-        }
-      }
-      s_m = m;
-      s_rot = rot;
-      cn_fold = cn;
-    }
-    __syncthreads();
-    // the trial kernel's prefilter centres: Get_COM of each placement; and,
-    // on a third wave, the unit phases exp(2 pi i s) of the new sites'
-    // fractional coordinates for the reciprocal sums
-    if (tid == 0) com_old = molecule_com(a.tp, a.spa0, n, ox, oy, oz);
-    if (tid == 64) com_new = molecule_com(a.tp, a.spa0, n, qx, qy, qz);
-    if (NSE > 0 && a.charged && tid >= 128 && tid < 128 + 3 * n) {
-      const int t = tid - 128, i = t / 3, d = t - 3 * i;
-      const double sd = a.b.Li[d] * qx[i] + a.b.Li[3 + d] * qy[i] + a.b.Li[6 + d] * qz[i];
-      double sv, cv;
-      sincos(kTwoPi * sd, &sv, &cv);
-      eph[2 * t] = cv;
-      eph[2 * t + 1] = sv;
-    }
-    __syncthreads();
-    const int m = s_m;
-    // --- inter energies of the old and the new placement (Compute_Molecule_Nonbond_Inter_Energy):
-    // the molecules that pass the COM prefilter (Check_MoleculePair_Cutoff)
-    // are listed in LDS, then every site pair of the list is one task
-    int nent = 0, ntask = 0;
-    for (int base = 0; base < 2 * nmols; base += kNvtBlock) {
-      const int t = base + tid;
-      int take = 0, tasks = 0, j = 0, which = 0;
-      if (t < 2 * nmols) {
-        which = t >= nmols ? 1 : 0;
-        j = t - which * nmols;
-        if (j != m && llive[j] && nvt_in_range(a.b, which ? com_new : com_old, lcomd[j])) {
-          take = 1;
-          tasks = n * spn[lspec[j]];
-        }
-      }
-      int cpre, tpre, ctot, ttot;
-      nvt_scan2(take, tasks, cpre, tpre, ctot, ttot, scan_c, scan_t);
-      if (take) {
-        ent_j[nent + cpre] = (j << 1) | which;
-        ent_off[nent + cpre] = ntask + tpre;
-      }
-      nent += ctot;
-      ntask += ttot;
-    }
-    if (tid == 0) ent_off[nent] = ntask;
-    __syncthreads();
-    double ev0 = 0.0, eq0 = 0.0, ev1 = 0.0, eq1 = 0.0;  // old / new placement
-    int ov = 0;
-    const int tpe = n * a.nj_uniform;  // tasks per listed molecule when all have nj_uniform sites
-    for (int task = tid; task < ntask; task += kNvtBlock) {
-      int lo;
-      if (tpe > 0) {
-        lo = task / tpe;
-      } else {
-        lo = 0;
-        int hi = nent - 1;
-        while (lo < hi) {
-          const int mid = (lo + hi + 1) >> 1;
-          if (ent_off[mid] <= task)
-            lo = mid;
-          else
-            hi = mid - 1;
-        }
-      }
-      const int code = ent_j[lo], which = code & 1, j = code >> 1;
-      const int sj = lspec[j], nj = spn[sj], oj = spo[sj], fj = lfirst[j];
-      const int local = task - ent_off[lo], ia = local / nj, ja = local - ia * nj;
-      const double *px = which ? qx : ox, *py = which ? qy : oy, *pz = which ? qz : oz;
-      double ev = 0.0, eq = 0.0;
-      if (nvt_pair<PM>(a.b, a.cd, px[ia], py[ia], pz[ia], pt[ia], pq[ia], prow + ia * a.ntypes, lx[fj + ja], ly[fj + ja],
-                   lz[fj + ja], atype[oj + ja], acharge[oj + ja], ev, eq)) {
-        ov |= which ? 2 : 1;
-      } else if (which) {
-        ev1 += ev;
-        eq1 += eq;
-      } else {
-        ev0 += ev;
-        eq0 += eq;
-      }
-    }
-    double v[4] = {ev0, eq0, ev1, eq1};
-    nvt_reduce<4>(v, ov, sh, shf, res, &resf);
-    if (ov & 1) {
-      if (tid == 0) *a.status = 1;
       __syncthreads();
-      break;
+      if (to > st) {
+        // the current move has been evaluated
+        const NvtCand &C = cand[st % 3][var];
+        const int m = __builtin_amdgcn_readfirstlane(C.m), rot = __builtin_amdgcn_readfirstlane(C.rot);
+        pos += __builtin_amdgcn_readfirstlane(C.draws);
+        const NvtOutcome r = nvt_decide(a, red[st & 1], redf[st & 1], nc, rot, uring[pos & (kNvtRing - 1)], en);
+        if (r.stop) {
+          if (lane == 0) *a.status = 1;
+          break;
+        }
+        pos += r.drawn;
+        const int64_t gi = step0 + st;
+        if (lane == 0) {
+          if (a.kind) a.kind[gi] = (uint8_t)rot;
+          if (a.accepted) a.accepted[gi] = (uint8_t)r.acc;
+          if (a.energy) a.energy[gi] = en[0];
+          if (a.ln_pacc) a.ln_pacc[gi] = r.lnp;
+        }
+        if (a.rng_state && lane < 5) a.rng_state[5 * gi + lane] = ring[pos & (kNvtRing - 1)][lane];
+        fm = r.acc ? m : -1;
+        pvar = var;
+        var = r.drawn;
+        if (++st >= nsteps) break;
+        if (r.acc && __builtin_amdgcn_readfirstlane(cand[st % 3][var].m) == m) {
+          // the next move takes the molecule that has just moved: once more,
+          // from the committed coordinates
+          fm = -1;
+          next = pos - var;
+          to = st;
+          __syncthreads();
+          continue;
+        }
+      }
+      // (the same start in the stream for both variants of the move after)
+      next = pos + __builtin_amdgcn_readfirstlane(cand[st % 3][var].draws);
+      to = st + 1;
+    }
+  }
+  if (!ahead) __syncthreads();
+  for (; !ahead && st < nsteps;) {
+    const int slot = (int)(st % 3), buf = (int)(st & 1);
+    const NvtCand &C = cand[slot][var];
+    const int m = __builtin_amdgcn_readfirstlane(C.m), rot = __builtin_amdgcn_readfirstlane(C.rot);
+    const double *o = S.cand + (size_t)(slot * 2 + var) * 6 * n, *q = o + 3 * n;
+    const size_t mk = (size_t)m * K;
+    double kc[kNvtSeg], ks[kNvtSeg], dc[kNvtSeg], ds[kNvtSeg];
+    if (has) {
+      // the old sums of the molecule, on their way during the pairs
+#pragma unroll
+      for (int t = 0; t < kNvtSeg; ++t) {
+        const int k = sk0 + (t < slen ? t : slen - 1);
+        dc[t] = a.ew.cmol[mk + k];
+        ds[t] = a.ew.smol[mk + k];
+      }
+    }
+    // --- inter energies of the old and the new placement (Compute_Molecule_Nonbond_Inter_Energy)
+    double ev0 = 0.0, eq0 = 0.0, ev1 = 0.0, eq1 = 0.0;
+    int ov = 0;
+    // lists: molecules in range of either placement (ent, cnt from head on),
+    // then site pairs within the cutoff (pr2, pcode, pcnt from phead on).  A
+    // molecule beyond the prefilter of one placement has no site pair within
+    // its cutoff there.
+    int head = 0, cnt = 0, phead = 0, pcnt = 0;
+    const double4 c0 = C.com_old, c1 = C.com_new;
+    int jbase = w, pb = 0;
+    for (;;) {
+      if (cnt < E && jbase < nmols) {
+        const int j = jbase + nc * lane;
+        jbase += nct;
+        bool take = false;
+        int2 entry = make_int2(0, 0);
+        if (j < nmols && j != m) {
+          const int meta = S.lmeta[j], first = S.lfirst[j];
+          const double4 cj = S.lcomd[j];
+          const bool in0 = nvt_in_range<CUBIC>(a.b, c0, cj), in1 = nvt_in_range<CUBIC>(a.b, c1, cj);
+          take = (meta & 1) && (in0 || in1);
+          entry = make_int2(first, (S.spo[meta >> 1] << 8) | S.spn[meta >> 1]);
+        }
+        const uint64_t bal = __ballot(take);
+        if (take) ent[(head + cnt + nvt_rank(bal)) & (kNvtList - 1)] = entry;
+        cnt += __builtin_popcountll(bal);
+        nvt_wave_sync();
+        continue;
+      }
+      double r2o = 0.0, r2n = 0.0;
+      bool co = false, cn = false;
+      int code = 0;
+      if (cnt > 0) {
+        const int take = cnt < E ? cnt : E;
+        int e = pe, ia = pia, ja = pja;
+        bool in = pe < take;
+        if (P > 64) {
+          const int p = pb + lane;
+          e = 0;
+          ia = p / a.nj_max;
+          ja = p - ia * a.nj_max;
+          in = p < P;
+        }
+        if (in) {
+          const int2 en2 = ent[(head + e) & (kNvtList - 1)];
+          if (ja < (en2.y & 255)) {
+            const double x = S.lx[en2.x + ja], y = S.ly[en2.x + ja], z = S.lz[en2.x + ja];
+            double dx = o[ia] - x, dy = o[n + ia] - y, dz = o[2 * n + ia] - z;
+            nvt_image<CUBIC>(a.b, dx, dy, dz);
+            r2o = dx * dx + dy * dy + dz * dz;
+            dx = q[ia] - x;
+            dy = q[n + ia] - y;
+            dz = q[2 * n + ia] - z;
+            nvt_image<CUBIC>(a.b, dx, dy, dz);
+            r2n = dx * dx + dy * dy + dz * dz;
+            bool gv, gq;
+            nvt_cutoff<PM>(a.cd, r2o, gv, gq);
+            co = gv || gq;
+            nvt_cutoff<PM>(a.cd, r2n, gv, gq);
+            cn = gv || gq;
+            code = (((en2.y >> 8) + ja) << 7) | (ia << 1);
+            if (r2o < a.cd.rc_low2) {
+              ov |= 1;
+              co = false;
+            }
+            if (r2n < a.cd.rc_low2) {
+              ov |= 2;
+              cn = false;
+            }
+          }
+        }
+        pb += 64;
+        if (pb >= P) {
+          head += take;
+          cnt -= take;
+          pb = 0;
+        }
+      }
+      // the old placement's pairs, the new one's, at the end the remainder
+      const bool last = cnt == 0 && jbase >= nmols;
+#pragma unroll 1
+      for (int h = 0; h < (last ? 3 : 2); ++h) {
+        const bool close = h == 0 ? co : h == 1 ? cn : false;
+        const uint64_t bal = __ballot(close);
+        if (close) {
+          const int at = (phead + pcnt + nvt_rank(bal)) & (kNvtList - 1);
+          pr2[at] = h ? r2n : r2o;
+          pcode[at] = code | h;
+        }
+        pcnt += __builtin_popcountll(bal);
+        nvt_wave_sync();
+        if (pcnt >= 64 || (h == 2 && pcnt > 0)) {
+          const int take = pcnt < 64 ? pcnt : 64;
+          if (lane < take) {
+            const int at = (phead + lane) & (kNvtList - 1), cd = pcode[at], ia = (cd >> 1) & 63, ja = cd >> 7;
+            double ev = 0.0, eq = 0.0;
+            nvt_pair<PM>(a.cd, pr2[at], S.pt[ia], S.pq[ia], S.prow + ia * a.ntypes, S.atype[ja], S.acharge[ja], ev,
+                         eq);
+            ev0 += (cd & 1) ? 0.0 : ev;
+            eq0 += (cd & 1) ? 0.0 : eq;
+            ev1 += (cd & 1) ? ev : 0.0;
+            eq1 += (cd & 1) ? eq : 0.0;
+          }
+          phead += take;
+          pcnt -= take;
+          nvt_wave_sync();
+        }
+      }
+      if (last) break;
     }
     // --- reciprocal space: Update_System_Ewald_Reciprocal_Energy (staged)
-    double erm = 0.0;
-    const bool reach = !(ov & 2);
-    if (reach && a.charged) {
-      // from the unit phases computed beside the centres, each lane walks
-      // k runs of the traversal (ny runs at fixed (nz, nx)) with the cosine
-      // recurrence and stores the molecule sums at the run's k indices
-      double e1[1] = {0.0};
-      int f0 = 0;
-      double *__restrict__ ctrav = a.ctrav, *__restrict__ strav = a.strav;
-      const int *__restrict__ kperm = a.ew.kperm;
-      const double *__restrict__ ecn = a.ew.cn;
-      const double *__restrict__ ecs = a.ew.cs, *__restrict__ esn = a.ew.sn;
-      const double *__restrict__ ecm = a.ew.cmol, *__restrict__ esm = a.ew.smol;
-      double *__restrict__ cs_new = a.ew.cs_new, *__restrict__ sn_new = a.ew.sn_new;
-      double *__restrict__ cm_new = a.ew.cm_new, *__restrict__ sm_new = a.ew.sm_new;
-      if (NSE > 0) {
-        // molecule sums along the runs, in traversal order
-        const int4 *__restrict__ rows = a.ew.rows;
-        const int *__restrict__ row_k0 = a.ew.row_k0;
-        for (int r = tid; r < a.ew.nrows; r += kNvtBlock) {
-          const int4 row = rows[r];
-          const int nx = row.x, nz = row.y, ny0 = row.z, cnt = row.w;
-          const int dir = cnt > 0 ? 1 : -1, len = cnt > 0 ? cnt : -cnt;
-          const int j0 = row_k0[r];
-          cplx t[NSE > 0 ? NSE : 1], u[NSE > 0 ? NSE : 1];
-          double c2[NSE > 0 ? NSE : 1];
+    double er = 0.0;
+    if (a.charged) {
+      const cplx *tab = S.tab + (size_t)(buf * 2 + var) * n * a.nt_site;
+      if (has) {
+        nvt_segment(a, S, tab, sg, kc, ks);
 #pragma unroll
-          for (int i = 0; i < NSE; ++i) {
-            const cplx ea = {eph[6 * i], eph[6 * i + 1]}, eb = {eph[6 * i + 2], eph[6 * i + 3]};
-            const cplx ec = {eph[6 * i + 4], eph[6 * i + 5]};
-            const cplx p = cmul(cmul(cpow_int(ea, nx), cpow_int(ec, nz)), cpow_int(eb, ny0));
-            t[i] = {pq[i] * p.re, pq[i] * p.im};
-            u[i] = cmul(t[i], {eb.re, -dir * eb.im});
-            c2[i] = 2.0 * eb.re;
-          }
-          for (int kk = 0; kk < len; ++kk) {
-            double c = t[0].re, sv = t[0].im;
-#pragma unroll
-            for (int i = 1; i < NSE; ++i) {
-              c = c + t[i].re;
-              sv = sv + t[i].im;
-            }
-#pragma unroll
-            for (int i = 0; i < NSE; ++i) {
-              const cplx tn = {fma(c2[i], t[i].re, -u[i].re), fma(c2[i], t[i].im, -u[i].im)};
-              u[i] = t[i];
-              t[i] = tn;
-            }
-            ctrav[j0 + kk] = c;
-            strav[j0 + kk] = sv;
-          }
-        }
-        __threadfence_block();
-        __syncthreads();
-        // the staged box sums and the energy, one k per lane
-        for (int jt = tid; jt < K; jt += kNvtBlock) {
-          const int k = kperm[jt];
-          const size_t mk = (size_t)m * K + k;
-          const double c = ctrav[jt], sv = strav[jt];
-          const double c1 = ecs[k] + (c - ecm[mk]), s1 = esn[k] + (sv - esm[mk]);
-          cs_new[k] = c1;
-          sn_new[k] = s1;
-          cm_new[k] = c;
-          sm_new[k] = sv;
-          e1[0] += ecn[k] * (c1 * c1 + s1 * s1);
-        }
-      } else {
-        for (int k = tid; k < K; k += kNvtBlock) {
-          const size_t mk = (size_t)m * K + k;
-          const double hx = a.ew.hx[k], hy = a.ew.hy[k], hz = a.ew.hz[k];
-          double c = 0.0, sv = 0.0;
-          for (int i = 0; i < n; ++i) {
-            const double hr = hx * qx[i] + hy * qy[i] + hz * qz[i];
-            double sn, cs;
-            sincos(hr, &sn, &cs);
-            c = c + pq[i] * cs;
-            sv = sv + pq[i] * sn;
-          }
-          const double c1 = a.ew.cs[k] + (c - a.ew.cmol[mk]), s1 = a.ew.sn[k] + (sv - a.ew.smol[mk]);
-          a.ew.cs_new[k] = c1;
-          a.ew.sn_new[k] = s1;
-          a.ew.cm_new[k] = c;
-          a.ew.sm_new[k] = sv;
-          e1[0] += a.ew.cn[k] * (c1 * c1 + s1 * s1);
+        for (int t = 0; t < kNvtSeg; ++t) {
+          dc[t] = kc[t] - dc[t];
+          ds[t] = ks[t] - ds[t];
+          const double cb = rcs[t] + dc[t], sb = rsn[t] + ds[t];
+          er += kn[t] * (cb * cb + sb * sb);
         }
       }
-      nvt_reduce<1>(e1, f0, sh, shf, res, &resf);
-      erm = e1[0] * kChargeFactor;
+      // further segments, their staged sums in device memory
+      for (int i = more; i < a.nsegs; i += nct) {
+        const int4 s2 = a.segs[i];
+        const int k0 = s2.x & 0xfffff, len = s2.x >> 20;
+        double c[kNvtSeg], s[kNvtSeg];
+        if (a.tabled) {
+          nvt_segment(a, S, tab, s2, c, s);
+#pragma unroll
+          for (int t = 0; t < kNvtSeg; ++t)
+            if (t < len) er += nvt_stage(a.ew, mk, k0 + t, c[t], s[t]);
+        } else {
+#pragma unroll 1
+          for (int t = 0; t < len; ++t) {
+            nvt_vector(a, S, q, k0 + t, c[0], s[0]);
+            er += nvt_stage(a.ew, mk, k0 + t, c[0], s[0]);
+          }
+        }
+      }
     }
-    // --- acceptance (thread 0)
-    if (tid == 0) {
-      double lnp = std::numeric_limits<double>::quiet_NaN();
-      int acc = 0;
-      if (reach) {
-        double dE = 0.0;
-        if (a.charged) dE = erm - en[4];
-        if (!s_rot)
-          dE = dE + (v[2] - v[0]) + (v[3] - v[1]);
-        else
-          dE = dE + v[2] - v[0] + v[3] - v[1];
-        lnp = a.beta * dE;
-        if (lnp <= 0.0) {
-          acc = 1;
-        } else if (lnp < kMaxKBT) {
-          const double pacc = exp(-lnp);
-          if (nvt_uniform(rs) <= pacc) acc = 1;
-        }
-        if (acc) {
-          en[0] = en[0] + dE;
-          en[1] = en[1] + dE;
-          en[2] = en[2] + v[2] - v[0];
-          en[3] = en[3] + v[3] - v[1];
-          if (a.charged) en[4] = erm;
-          // the stored centre: the folded one after a translation, Get_COM
-          // after a rotation (move_rotate.f90:287); max_dcom unchanged
-          double4 c = lcomd[m];
-          if (!s_rot) {
-            c.x = cn_fold.x;
-            c.y = cn_fold.y;
-            c.z = cn_fold.z;
-          } else {
-            // Get_COM of the rotated sites: the new placement's centre
-            c.x = com_new.x;
-            c.y = com_new.y;
-            c.z = com_new.z;
-          }
-          lcomd[m] = c;
-          a.comd[m] = c;
-        }
-      }
-      s_acc = acc;
-      const int64_t g = a.step0 + st;
-      if (a.kind) a.kind[g] = (uint8_t)s_rot;
-      if (a.accepted) a.accepted[g] = (uint8_t)acc;
-      if (a.energy) a.energy[g] = en[0];
-      if (a.ln_pacc) a.ln_pacc[g] = lnp;
-      if (a.rng_state)
-        for (int k = 0; k < 5; ++k) a.rng_state[5 * g + k] = rs[k];
+    const double p0 = wave_total(ev0), p1 = wave_total(eq0), p2 = wave_total(ev1), p3 = wave_total(eq1);
+    const double p4 = wave_total(er);
+    const int f = (__any(ov & 1) ? 1 : 0) | (__any(ov & 2) ? 2 : 0);
+    if (lane == 0) {
+      red[buf][0][w] = p0;
+      red[buf][1][w] = p1;
+      red[buf][2][w] = p2;
+      red[buf][3][w] = p3;
+      red[buf][4][w] = p4;
+      redf[buf][w] = f;
     }
     __syncthreads();
-    if (s_acc) {
-      const int f = lfirst[m];
-      if (tid < n) {
-        lx[f + tid] = qx[tid];
-        ly[f + tid] = qy[tid];
-        lz[f + tid] = qz[tid];
-        a.x[f + tid] = qx[tid];
-        a.y[f + tid] = qy[tid];
-        a.z[f + tid] = qz[tid];
+    pos += __builtin_amdgcn_readfirstlane(C.draws);
+    const NvtOutcome r = nvt_decide(a, red[buf], redf[buf], nc, rot, uring[pos & (kNvtRing - 1)], en);
+    if (r.stop) break;
+    pos += r.drawn;
+    var = r.drawn;
+    ++st;
+    if (r.acc) {
+      if (w == m % nc) {
+        // the owning wave commits the molecule; the stored centre is the
+        // folded one after a translation, Get_COM after a rotation
+        // (move_rotate.f90:287), max_dcom unchanged
+        const int f0 = S.lfirst[m];
+        for (int i = lane; i < n; i += 64) {
+          S.lx[f0 + i] = q[i];
+          S.ly[f0 + i] = q[n + i];
+          S.lz[f0 + i] = q[2 * n + i];
+        }
+        if (lane == 0) {
+          S.lcomd[m].x = rot ? C.com_new.x : C.cx;
+          S.lcomd[m].y = rot ? C.com_new.y : C.cy;
+          S.lcomd[m].z = rot ? C.com_new.z : C.cz;
+        }
+        nvt_wave_sync();
+      }
+      if (has) {
+#pragma unroll
+        for (int t = 0; t < kNvtSeg; ++t) {
+          rcs[t] = rcs[t] + dc[t];
+          rsn[t] = rsn[t] + ds[t];
+          if (t < slen) {
+            a.ew.cmol[mk + sk0 + t] = kc[t];
+            a.ew.smol[mk + sk0 + t] = ks[t];
+          }
+        }
       }
       if (a.charged)
-        for (int k = tid; k < K; k += kNvtBlock) {
-          const size_t mk = (size_t)m * K + k;
-          a.ew.cs[k] = a.ew.cs_new[k];
-          a.ew.sn[k] = a.ew.sn_new[k];
-          a.ew.cmol[mk] = a.ew.cm_new[k];
-          a.ew.smol[mk] = a.ew.sm_new[k];
+        for (int i = more; i < a.nsegs; i += nct) {
+          const int4 s2 = a.segs[i];
+          const int k0 = s2.x & 0xfffff, len = s2.x >> 20;
+          for (int t = 0; t < len; ++t) {
+            const int k = k0 + t;
+            a.ew.cs[k] = a.ew.cs_new[k];
+            a.ew.sn[k] = a.ew.sn_new[k];
+            a.ew.cmol[mk + k] = a.ew.cm_new[k];
+            a.ew.smol[mk + k] = a.ew.sm_new[k];
+          }
         }
+      if (st < nsteps && __builtin_amdgcn_readfirstlane(cand[st % 3][var].m) == m) {
+        // the next move takes the same molecule: it is prepared anew
+        __syncthreads();
+        __syncthreads();
+      }
     }
-    __threadfence_block();
-    __syncthreads();
   }
-  if (tid == 0) {
-    for (int k = 0; k < 5; ++k) a.rng[k] = rs[k];
+  __syncthreads();
+  for (int i = tid; i < a.nsite; i += nthr) {
+    a.x[i] = S.lx[i];
+    a.y[i] = S.ly[i];
+    a.z[i] = S.lz[i];
+  }
+  for (int i = tid; i < nmols; i += nthr) a.comd[i] = S.lcomd[i];
+  if (has) {
+#pragma unroll
+    for (int t = 0; t < kNvtSeg; ++t)
+      if (t < slen) {
+        a.ew.cs[sk0 + t] = rcs[t];
+        a.ew.sn[sk0 + t] = rsn[t];
+      }
+  }
+  if (tid < 5) a.rng[tid] = ring[pos & (kNvtRing - 1)][tid];
+  if (tid == 0)
     for (int k = 0; k < 5; ++k) a.en[k] = en[k];
-  }
-}
-
-// One chain per launch (the arguments in the kernel's argument segment).
-template <int PM, int NSE>
-__global__ void __launch_bounds__(kNvtBlock) k_nvt_chain(NvtChainArgs a) {
-  nvt_chain_run<PM, NSE>(a);
 }
 
 // Independent chains of several boxes, one workgroup per box: replicas of a
-// system, or boxes of different state points, each on its own generator.
-template <int PM, int NSE>
-__global__ void __launch_bounds__(kNvtBlock) k_nvt_chain_multi(const NvtChainArgs *__restrict__ args) {
-  nvt_chain_run<PM, NSE>(args[blockIdx.x]);
+// system, or boxes of different state points, each on its own generator.  The
+// table is constant while the kernel runs, which its address space tells the
+// compiler: through a plain pointer every field would be loaded again after
+// each store.
+template <int PM, bool CUBIC>
+__global__ void __launch_bounds__(64 * kNvtWaves)
+    k_nvt_chain(const NvtChainArgs *__restrict__ args, int64_t step0, int64_t nsteps) {
+  typedef const __attribute__((address_space(4))) NvtChainArgs *ConstArgs;
+  nvt_chain_run<PM, CUBIC>(*(const NvtChainArgs *)((ConstArgs)args + blockIdx.x), step0, nsteps);
 }
 
 }  // namespace cass
@@ -666,7 +902,7 @@ namespace {
 struct NvtLaunch {
   NvtChainArgs a;
   size_t lds = 0;
-  int pm = 0, nse = 0;
+  int pm = 0, waves = kNvtWaves;
   bool host_loop = false;  // the box's copy exceeds the LDS: the host-driven loop runs it
   int box = -1;
   cass_rng *rng = nullptr;
@@ -678,26 +914,13 @@ struct NvtLaunch {
   size_t o_state = 0, o_kind = 0, o_acc = 0, o_energy = 0, o_lnp = 0, o_rs = 0, o_mols = 0;
 };
 
-typedef void (*nvt_kernel_t)(NvtChainArgs);
-typedef void (*nvt_multi_kernel_t)(const NvtChainArgs *);
+typedef void (*nvt_kernel_t)(const NvtChainArgs *, int64_t, int64_t);
 
-nvt_kernel_t nvt_kernel(int pm, int nse) {
-  static nvt_kernel_t const kt[3][5] = {
-      {k_nvt_chain<0, 0>, k_nvt_chain<0, 1>, k_nvt_chain<0, 2>, k_nvt_chain<0, 3>, k_nvt_chain<0, 4>},
-      {k_nvt_chain<1, 0>, k_nvt_chain<1, 1>, k_nvt_chain<1, 2>, k_nvt_chain<1, 3>, k_nvt_chain<1, 4>},
-      {k_nvt_chain<2, 0>, k_nvt_chain<2, 1>, k_nvt_chain<2, 2>, k_nvt_chain<2, 3>, k_nvt_chain<2, 4>}};
-  return kt[pm][nse];
-}
-
-nvt_multi_kernel_t nvt_multi_kernel(int pm, int nse) {
-  static nvt_multi_kernel_t const kt[3][5] = {
-      {k_nvt_chain_multi<0, 0>, k_nvt_chain_multi<0, 1>, k_nvt_chain_multi<0, 2>, k_nvt_chain_multi<0, 3>,
-       k_nvt_chain_multi<0, 4>},
-      {k_nvt_chain_multi<1, 0>, k_nvt_chain_multi<1, 1>, k_nvt_chain_multi<1, 2>, k_nvt_chain_multi<1, 3>,
-       k_nvt_chain_multi<1, 4>},
-      {k_nvt_chain_multi<2, 0>, k_nvt_chain_multi<2, 1>, k_nvt_chain_multi<2, 2>, k_nvt_chain_multi<2, 3>,
-       k_nvt_chain_multi<2, 4>}};
-  return kt[pm][nse];
+nvt_kernel_t nvt_kernel(int pm, bool cubic) {
+  static nvt_kernel_t const kt[3][2] = {{k_nvt_chain<0, false>, k_nvt_chain<0, true>},
+                                        {k_nvt_chain<1, false>, k_nvt_chain<1, true>},
+                                        {k_nvt_chain<2, false>, k_nvt_chain<2, true>}};
+  return kt[pm][cubic ? 1 : 0];
 }
 
 // Checks, the LDS layout of the box copy, the kernel choice and the arguments
@@ -728,77 +951,89 @@ int nvt_prepare(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_optio
   if (nm == 0) return cass_fail(e, CASS_ERR_STATE, "no molecules to move");
   if (nsteps == 0) return CASS_OK;
   HIP_TRY(e, hipSetDevice(e->device));
-  // LDS layout of the box copy
+  // LDS layout of the box copy and the waves' buffers.  Twelve waves hold 28
+  // KB of buffers; a box that leaves less takes fewer of them (the cost of
+  // that stands at kNvtWaves), then goes without the phase powers.
   const int nsite = (int)(b.xyz_h.size() / 3), nt = std::max(e->ntypes, 1);
-  size_t lds = 0;
-  auto take = [&](size_t bytes) {
-    const size_t o = lds;
-    lds = (lds + bytes + 15) & ~(size_t)15;
-    return (int)o;
-  };
+  int lds_max = 0;
+  HIP_TRY(e, hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, e->device));
   NvtChainArgs &a = L.a;
   std::memset(&a, 0, sizeof(a));
-  a.o_x = take(sizeof(double) * nsite);
-  a.o_y = take(sizeof(double) * nsite);
-  a.o_z = take(sizeof(double) * nsite);
-  a.o_comd = take(sizeof(double4) * b.nmols);
-  a.o_first = take(sizeof(int) * b.nmols);
-  a.o_spec = take(sizeof(int) * b.nmols);
-  a.o_live = take(sizeof(int) * b.nmols);
-  a.o_atype = take(sizeof(int) * e->natoms_total);
-  a.o_acharge = take(sizeof(double) * e->natoms_total);
-  a.o_spn = take(sizeof(int) * e->nspecies);
-  a.o_spo = take(sizeof(int) * e->nspecies);
-  a.o_pt = take(sizeof(int) * n);
-  a.o_pq = take(sizeof(double) * n);
-  a.o_prow = take(sizeof(double4) * n * nt);
-  a.o_mols = take(sizeof(int) * nm);
-  a.o_ent = take(sizeof(int) * (2 * b.nmols + 1));
-  a.o_eoff = take(sizeof(int) * (2 * b.nmols + 1));
-  L.lds = lds;
+  a.tx = std::max(2, b.kmax[0] + 1);
+  a.ty = b.kmax[1] + 1;
+  a.tz = b.kmax[2] + 1;
+  a.nt_site = a.tx + a.ty + a.tz;
+  auto layout = [&](int waves, bool tabled) {
+    size_t lds = 0;
+    auto take = [&](size_t bytes) {
+      const size_t o = lds;
+      lds = (lds + bytes + 15) & ~(size_t)15;
+      return (int)o;
+    };
+    a.o_x = take(sizeof(double) * nsite);
+    a.o_y = take(sizeof(double) * nsite);
+    a.o_z = take(sizeof(double) * nsite);
+    a.o_comd = take(sizeof(double4) * b.nmols);
+    a.o_first = take(sizeof(int) * b.nmols);
+    a.o_meta = take(sizeof(int) * b.nmols);
+    a.o_atype = take(sizeof(int) * e->natoms_total);
+    a.o_acharge = take(sizeof(double) * e->natoms_total);
+    a.o_spn = take(sizeof(int) * e->nspecies);
+    a.o_spo = take(sizeof(int) * e->nspecies);
+    a.o_pt = take(sizeof(int) * n);
+    a.o_pq = take(sizeof(double) * n);
+    a.o_pm = take(sizeof(double) * n);
+    a.o_prow = take(sizeof(double4) * n * nt);
+    a.o_cand = take(sizeof(double) * 36 * n);
+    a.o_eph = take(tabled ? sizeof(cplx) * 6 * n : 0);
+    a.o_tab = take(tabled ? sizeof(cplx) * 4 * n * a.nt_site : 0);
+    a.o_ent = take(sizeof(int2) * kNvtList * (waves - 1));
+    a.o_pr2 = take(sizeof(double) * kNvtList * (waves - 1));
+    a.o_pcode = take(sizeof(int) * kNvtList * (waves - 1));
+    L.lds = lds;
+    L.waves = waves;
+    a.tabled = tabled ? 1 : 0;
+    return lds + 4096 <= (size_t)lds_max;  // beside the kernel's own
+  };
+  bool fits = false;
+  for (int waves = kNvtWaves; !fits && waves >= kNvtMinWaves; waves -= 2) fits = layout(waves, charged);
+  for (int waves = kNvtWaves; !fits && charged && waves >= kNvtMinWaves; waves -= 2) fits = layout(waves, false);
+  if (!fits) {
+    L.host_loop = true;
+    return CASS_OK;
+  }
   const bool common = (b.p.vdw_style == CASS_VDW_NONE ||
                        (b.p.vdw_style == CASS_VDW_LJ &&
                         (b.p.vdw_sum_style == CASS_SUM_CUT || b.p.vdw_sum_style == CASS_SUM_CUT_TAIL ||
                          b.p.vdw_sum_style == CASS_SUM_CUT_SHIFT))) &&
                       (b.p.charge_style == CASS_Q_NONE || b.p.charge_style == CASS_Q_EWALD ||
                        b.p.charge_style == CASS_Q_CUT);
-  int lds_max = 0;
-  HIP_TRY(e, hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, e->device));
-  if (lds > (size_t)lds_max - 8192) {
-    L.host_loop = true;
-    return CASS_OK;
-  }
-  // the reciprocal sums of molecules up to 4 sites by phase recurrences
-  // along the k runs, larger ones by sincos per k
-  L.nse = (charged && n <= 4 && b.nrows > 0) ? n : 0;
   // the mixed and FP32 modes take the mixed pair arithmetic for the common
   // styles (FP64 accumulation, reciprocal space and acceptance in every mode)
   L.pm = common ? (e->prec == CASS_PREC_FP64 ? 1 : 2) : 0;
   a.b = cass_box_view(e, b);
   a.tp = cass_topo_view(e);
   a.cd = make_pair_const<double>(b.p, e->ntypes);
-  a.cf = make_pair_const<float>(b.p, e->ntypes);
   a.ew = cass_ewald_view(b);
+  a.segs = b.segs();
+  a.nsegs = charged ? b.nsegs : 0;
   if (!charged) a.ew.nvecs = 0;
   a.x = b.x;
   a.y = b.y;
   a.z = b.z;
   a.comd = b.comd;
   a.nm = nm;
-  a.species = sp;
   a.n = n;
   a.spa0 = e->sp_atom_off[sp];
   a.charged = charged ? 1 : 0;
   a.linear = opt->linear;
-  a.coul_cbmc = e->sp_coul_cbmc[sp];
   a.prob_translate = opt->prob_translate;
   a.max_disp = opt->max_disp;
   a.max_rot = opt->max_rot;
   a.beta = b.p.beta;
   a.nsite = nsite;
-  a.nj_uniform = b.nmols > 0 ? e->sp_natoms[b.mol_species[0]] : 0;
-  for (int mm = 0; mm < b.nmols; ++mm)
-    if (e->sp_natoms[b.mol_species[mm]] != a.nj_uniform) a.nj_uniform = 0;
+  a.nj_max = 1;
+  for (int mm = 0; mm < b.nmols; ++mm) a.nj_max = std::max(a.nj_max, e->sp_natoms[b.mol_species[mm]]);
   a.natoms_total = e->natoms_total;
   a.nspecies = e->nspecies;
   a.ntypes = nt;
@@ -813,8 +1048,7 @@ struct NvtState {
 };
 
 // The buffers of a batch, laid out over all its chains: first what comes back
-// (states and records), then the mobile lists and argument tables, then the
-// molecule sums.  One copy in, one copy out: with a set of copies per chain
+// (states and records), then the mobile lists and argument tables.  One copy in, one copy out: with a set of copies per chain
 // the calls themselves outlasted the chains.
 struct NvtBuffers {
   char *dev = nullptr;
@@ -846,9 +1080,6 @@ int nvt_buffers(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, NvtB
     if (!L.host_loop) L.o_mols = take(sizeof(int) * L.mols.size());
   B.o_args = take(sizeof(NvtChainArgs) * std::max<size_t>(1, Ls.size()));
   B.in = off;
-  std::vector<size_t> trav(Ls.size());
-  for (size_t k = 0; k < Ls.size(); ++k)
-    if (!Ls[k].host_loop) trav[k] = take(sizeof(double) * 2 * (size_t)Ls[k].a.ew.nvecs);
   B.dev = (char *)cass_scratch(e, off + 256);
   if (!B.dev) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
   B.host.assign(B.in, 0);
@@ -873,8 +1104,6 @@ int nvt_buffers(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, NvtB
     a.ln_pacc = rec && rec->ln_pacc ? (double *)(B.dev + L.o_lnp) : nullptr;
     a.rng_state = rec && rec->rng_state ? (int64_t *)(B.dev + L.o_rs) : nullptr;
     a.mols = (const int *)(B.dev + L.o_mols);
-    a.ctrav = (double *)(B.dev + trav[k]);
-    a.strav = a.ctrav + a.ew.nvecs;
   }
   return CASS_OK;
 }
@@ -924,27 +1153,6 @@ constexpr int64_t kNvtChunk = 4096;
 
 }  // namespace
 
-extern "C" int cass_nvt_run_device(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_options *opt,
-                                   int64_t nsteps, cass_energy *en, cass_nvt_record *rec) {
-  std::vector<NvtLaunch> Ls(1);
-  NvtLaunch &L = Ls[0];
-  int rc = nvt_prepare(e, box, rng, opt, nsteps, en, rec, L);
-  if (rc || nsteps == 0) return rc;
-  if (L.host_loop) return cass_nvt_run(e, box, rng, opt, nsteps, en, rec);
-  NvtBuffers B;
-  if ((rc = nvt_buffers(e, Ls, nsteps, B))) return rc;
-  HIP_TRY(e, hipMemcpyAsync(B.dev, B.host.data(), B.in, hipMemcpyHostToDevice, e->stream));
-  nvt_kernel_t kern = nvt_kernel(L.pm, L.nse);
-  HIP_TRY(e, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)L.lds));
-  for (int64_t s0 = 0; s0 < nsteps; s0 += kNvtChunk) {
-    L.a.step0 = s0;
-    L.a.nsteps = std::min(kNvtChunk, nsteps - s0);
-    hipLaunchKernelGGL(kern, dim3(1), dim3(kNvtBlock), L.lds, e->stream, L.a);
-    HIP_TRY(e, hipGetLastError());
-  }
-  return nvt_finish(e, Ls, nsteps, B);
-}
-
 extern "C" int cass_nvt_run_device_batch(cass_engine *e, int32_t nboxes, const int32_t *boxes, cass_rng *rngs,
                                          const cass_nvt_options *opts, int64_t nsteps, cass_energy *ens,
                                          cass_nvt_record *recs) {
@@ -960,21 +1168,22 @@ extern "C" int cass_nvt_run_device_batch(cass_engine *e, int32_t nboxes, const i
   if (nsteps == 0 || nboxes == 0) return CASS_OK;
   NvtBuffers B;
   if ((rc = nvt_buffers(e, Ls, nsteps, B))) return rc;
-  // the chains grouped by kernel (pair arithmetic, reciprocal site count);
-  // every group is one launch per chunk of moves, one workgroup per box.  The
-  // argument table holds the groups one after another.
+  // the chains grouped by kernel and workgroup size; every group is one launch
+  // per chunk of moves, one workgroup per box.  The argument table holds the
+  // groups one after another.
   struct Group {
-    nvt_multi_kernel_t kern;
+    nvt_kernel_t kern;
     size_t lds, first, count;
+    int waves;
   };
   std::vector<Group> groups;
   std::vector<NvtChainArgs> args;
   std::vector<int> done(nboxes, 0);
   for (int g = 0; g < nboxes; ++g) {
     if (done[g] || Ls[g].host_loop) continue;
-    Group grp{nvt_multi_kernel(Ls[g].pm, Ls[g].nse), 0, args.size(), 0};
+    Group grp{nvt_kernel(Ls[g].pm, Ls[g].a.b.cubic), 0, args.size(), 0, Ls[g].waves};
     for (int k = g; k < nboxes; ++k)
-      if (!done[k] && !Ls[k].host_loop && Ls[k].pm == Ls[g].pm && Ls[k].nse == Ls[g].nse) {
+      if (!done[k] && !Ls[k].host_loop && nvt_kernel(Ls[k].pm, Ls[k].a.b.cubic) == grp.kern && Ls[k].waves == grp.waves) {
         args.push_back(Ls[k].a);
         grp.lds = std::max(grp.lds, Ls[k].lds);
         ++grp.count;
@@ -982,25 +1191,14 @@ extern "C" int cass_nvt_run_device_batch(cass_engine *e, int32_t nboxes, const i
       }
     groups.push_back(grp);
   }
-  NvtChainArgs *d_args = (NvtChainArgs *)(B.dev + B.o_args);
-  for (int64_t s0 = 0; s0 < nsteps; s0 += kNvtChunk) {
-    for (NvtChainArgs &a : args) {
-      a.step0 = s0;
-      a.nsteps = std::min(kNvtChunk, nsteps - s0);
-    }
-    if (!args.empty()) std::memcpy(B.host.data() + B.o_args, args.data(), sizeof(NvtChainArgs) * args.size());
-    if (s0 == 0) {
-      HIP_TRY(e, hipMemcpyAsync(B.dev, B.host.data(), B.in, hipMemcpyHostToDevice, e->stream));
-    } else {
-      // the argument table is rewritten: wait for the launches that read it
-      HIP_TRY(e, hipStreamSynchronize(e->stream));
-      HIP_TRY(e, hipMemcpyAsync(d_args, B.host.data() + B.o_args, sizeof(NvtChainArgs) * args.size(),
-                                hipMemcpyHostToDevice, e->stream));
-    }
-    for (const Group &g : groups) {
-      HIP_TRY(e, hipFuncSetAttribute((const void *)g.kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)g.lds));
-      hipLaunchKernelGGL(g.kern, dim3((unsigned)g.count), dim3(kNvtBlock), g.lds, e->stream,
-                         (const NvtChainArgs *)(d_args + g.first));
+  if (!args.empty()) std::memcpy(B.host.data() + B.o_args, args.data(), sizeof(NvtChainArgs) * args.size());
+  const NvtChainArgs *d_args = (const NvtChainArgs *)(B.dev + B.o_args);
+  HIP_TRY(e, hipMemcpyAsync(B.dev, B.host.data(), B.in, hipMemcpyHostToDevice, e->stream));
+  for (const Group &g : groups) {
+    HIP_TRY(e, hipFuncSetAttribute((const void *)g.kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)g.lds));
+    for (int64_t s0 = 0; s0 < nsteps; s0 += kNvtChunk) {
+      hipLaunchKernelGGL(g.kern, dim3((unsigned)g.count), dim3(64 * g.waves), g.lds, e->stream, d_args + g.first, s0,
+                         std::min(kNvtChunk, nsteps - s0));
       HIP_TRY(e, hipGetLastError());
     }
   }
@@ -1009,4 +1207,10 @@ extern "C" int cass_nvt_run_device_batch(cass_engine *e, int32_t nboxes, const i
     if (Ls[k].host_loop)
       rc = cass_nvt_run(e, boxes[k], rngs + k, opts + k, nsteps, ens + k, recs ? recs + k : nullptr);
   return rc;
+}
+
+extern "C" int cass_nvt_run_device(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_options *opt,
+                                   int64_t nsteps, cass_energy *en, cass_nvt_record *rec) {
+  if (!rng || !opt || !en) return CASS_ERR_ARG;
+  return cass_nvt_run_device_batch(e, 1, &box, rng, opt, nsteps, en, rec);
 }

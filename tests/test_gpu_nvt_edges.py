@@ -1,0 +1,71 @@
+"""The device NVT chain against the host-driven loop where its parts change:
+one and two molecules (the next move takes the molecule just moved), molecule
+pairs of more than 64 site pairs, species of unlike site counts, k vectors
+beyond the lanes' registers, phases without tables, orthogonal boxes, a style
+without its own pair arithmetic, a box on fewer waves."""
+import numpy as np
+import pytest
+
+from cassandra_amd import engine as E
+from cassandra_amd import systems as S
+
+REL = 1e-10   # the energies' tolerance against the reference
+
+
+def _chain(n, q):
+    """n sites on a zigzag, charges alternating (the first of an odd count 0)"""
+    xyz = np.array([[1.1 * i, 0.3 * (i % 2), 0.0] for i in range(n)])
+    charge = [0.0] * (n % 2) + [q if i % 2 else -q for i in range(n - n % 2)]
+    atoms = [S.Atom(f"A{i % 3}", "C", 12.0 + i % 3, charge[i], 40.0 + 10.0 * (i % 3), 2.6 + 0.1 * (i % 3))
+             for i in range(n)]
+    return S.Species("chain", atoms, xyz)
+
+
+def _system(case):
+    w = S.species_spce()
+    if case == "lj2000":
+        return S.config_lj2000().parsed()
+    species, counts, box, rc, style = {
+        "one": ([w], [1], [20.0] * 3, 9.0, "cut"),   # (Ewald: its energy changes are rounding alone)
+        "two": ([w], [2], [20.0] * 3, 9.0, "ewald"),
+        "dsf": ([w], [40], [20.0] * 3, 9.0, "dsf"),
+        "orthogonal": ([w], [70], [19.0, 24.0, 21.5], 9.0, "ewald"),
+        "many_k": ([w], [30], [44.0] * 3, 9.0, "ewald"),
+        "mixture": ([w, S.species_methane(), _chain(11, 0.2)], [33, 20, 4], [24.0] * 3, 9.0, "ewald"),
+        "sites9": ([_chain(9, 0.15)], [25], [30.0] * 3, 10.0, "ewald"),
+        "sites64": ([_chain(64, 0.1)], [2], [76.0] * 3, 9.0, "ewald"),
+    }[case]
+    coords = S.place_random(list(zip(species, counts)), box, 5, 1.2, 2.6)
+    return S.System(species, counts, coords, np.array(box), 350.0, "lj", "cut_tail", rc, charge_style=style,
+                    rcut_coul=rc, alpha_dsf=0.2 if style == "dsf" else None, rcut_low=0.85,
+                    box_shape="orthogonal" if case == "orthogonal" else "cubic", prob_translate=0.5, max_disp=0.4,
+                    max_rot=25.0, seed=(101, 203), name=case).parsed()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", [E.FP64, E.MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("case", ["one", "two", "dsf", "orthogonal", "many_k", "mixture", "sites9", "sites64", "lj2000"])
+def test_nvt_chain_equals_host_loop(case, prec):
+    print(f"[gpu] nvt chain edges {case} {prec}", flush=True)
+    system, steps = _system(case), 120
+    got = []
+    for device in (True, False):
+        eng = E.Engine(system, precision=E.FP64 if not device else prec)
+        box = eng.add_box(system)
+        if system.charge_style == "ewald":
+            box.ewald_setup()
+        e0 = box.compute_system_total_energy()
+        rng = E.rng(*system.seed)
+        out = box.nvt_run(rng, steps, e0, device=device)
+        got.append((out, list(rng.s), box.download(), box.compute_system_total_energy()))
+        eng.close()
+    (a, ra, xa, ta), (b, rb, xb, _) = got
+    tol = REL if prec == E.FP64 else 1e-8   # the mixed chain's tolerance in the replay of the reference
+    for k in ("kind", "accepted", "rng"):
+        assert np.array_equal(a[k], b[k]), k
+    assert ra == rb
+    assert np.max(np.abs(a["energy"] - b["energy"]) / np.maximum(np.abs(b["energy"]), 1.0)) < tol
+    assert np.array_equal(np.isnan(a["ln_pacc"]), np.isnan(b["ln_pacc"]))
+    assert np.max(np.abs(xa - xb)) < 1e-9
+    # the running sums of the chain against a fresh evaluation of its end state
+    assert abs(a["final"]["total"] - ta["total"]) <= tol * max(1.0, abs(ta["total"]))
