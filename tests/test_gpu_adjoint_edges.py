@@ -1,0 +1,68 @@
+"""The adjoint's reciprocal and pair kernels at their edges: n_y ranges of two,
+three and four register steps and beyond, boxes of unlike edges, molecules of
+one to eight sites (site groups of three), site counts around a tile, one and
+many frames.  Against the total energy and its central differences."""
+import numpy as np
+import pytest
+
+from cassandra_amd import engine as E
+from cassandra_amd import systems as S
+
+
+def _species(n):
+    xyz = np.array([[1.0 * i, 0.4 * (i % 2), 0.2 * (i % 3)] for i in range(n)])
+    q = [0.0] if n == 1 else [(-0.3 if i % 2 else 0.3) if i < n - n % 2 else 0.0 for i in range(n)]
+    return S.Species(f"s{n}", [S.Atom(f"T{i % 2}", "C", 12.0 + i % 2, q[i], 50.0 + 20.0 * (i % 2), 2.7 + 0.2 * (i % 2))
+                               for i in range(n)], xyz)
+
+
+CASES = {
+    # name: (sites, molecules, box, cutoff) -- n_y up to 4, 9, 13, 17
+    "two_steps": (3, 21, [16.0] * 3, 7.5),
+    "three_steps": (4, 16, [27.0] * 3, 11.0),
+    "four_steps": (8, 8, [28.0] * 3, 8.0),
+    "beyond": (2, 33, [30.0] * 3, 6.5),
+    "unlike_edges": (5, 13, [18.0, 31.0, 23.0], 8.5),
+    "tile": (1, 64, [24.0] * 3, 8.0),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", list(CASES))
+def test_adjoint_edges(case):
+    print(f"[gpu] adjoint edges {case}", flush=True)
+    n, count, box, rc = CASES[case]
+    sp = _species(n)
+    coords = S.place_random([(sp, count)], box, 9, 1.2, 2.6)
+    system = S.System([sp], [count], coords, np.array(box), 300.0, "lj", "cut_tail", rc, charge_style="ewald",
+                      rcut_coul=rc, rcut_low=0.85, box_shape="cubic" if len(set(box)) == 1 else "orthogonal",
+                      name=case).parsed()
+    eng = E.Engine(system, precision=E.FP64)
+    b = eng.add_box(system)
+    b.ewald_setup()
+    e0 = b.compute_system_total_energy()["total"]
+    energy, _, _, dq, forces = b.adjoint()
+    assert abs(energy - e0) <= 1e-10 * max(1.0, abs(e0))
+    # frames: the box's own coordinates and shifted ones; each equal to one alone
+    xyz = b.download().reshape(-1, 3)
+    rng = np.random.default_rng(3)
+    h = 1e-4
+    site = int(rng.integers(n * count))
+    frames = [xyz]
+    for d in range(3):
+        for sgn in (1.0, -1.0):
+            f = xyz.copy()
+            f[site, d] += sgn * h
+            frames.append(f)
+    b.adjoint_set_frames(np.array(frames))
+    ef, _, _, dqf, ff = b.adjoint_frames(0, len(frames), forces=True)
+    assert ef[0] == pytest.approx(energy, rel=1e-12, abs=1e-9)
+    fmax = np.max(np.abs(forces))
+    assert np.max(np.abs(ff[0] - forces)) <= 1e-11 * max(1.0, fmax)
+    assert np.max(np.abs(dqf[0] - dq)) <= 1e-11 * max(1.0, np.max(np.abs(dq)))
+    # central differences of step h: truncation h^2 |U'''| / 6 (two powers of a
+    # site distance below the force) and rounding eps |U| / h
+    fd = [-(ef[1 + 2 * d] - ef[2 + 2 * d]) / (2 * h) for d in range(3)]
+    tol = 50.0 * h * h * max(1.0, fmax) + 1e-15 * max(1.0, abs(e0)) * count / h
+    assert np.max(np.abs(np.array(fd) - forces.reshape(-1, 3)[site])) <= tol
+    eng.close()
