@@ -145,6 +145,11 @@ static EwaldDev ewald_view(const cass_box_state &b, const int *row_k0) {
   w.rows = b.rows;
   w.row_k0 = row_k0;
   w.kperm = row_k0 ? row_k0 + b.nrows : nullptr;
+  w.segs = b.segs();
+  w.nsegs = b.nsegs;
+  w.tx = std::max(2, b.kmax[0] + 1);
+  w.ty = b.kmax[1] + 1;
+  w.tz = b.kmax[2] + 1;
   return w;
 }
 
@@ -999,11 +1004,18 @@ static bool total_intra(const cass_engine *e, const cass_box_state *b, cass_ener
 // their overlap flags into out; false: an overlap.
 static bool total_pair_sums(const double *hp, const int *ho, size_t np, cass_energy *out) {
   bool ov = false;
+  double sum[2] = {0.0, 0.0}, low[2] = {0.0, 0.0};
   for (size_t i = 0; i < np; ++i) {
-    out->inter_vdw += hp[2 * i];
-    out->inter_q += hp[2 * i + 1];
+    for (int k = 0; k < 2; ++k) {
+      // each addition's rounding error is kept (Knuth's two-sum)
+      const double v = hp[2 * i + k], t = sum[k] + v, w = t - sum[k];
+      if (std::isfinite(t)) low[k] += (sum[k] - (t - w)) + (v - w);
+      sum[k] = t;
+    }
     if (ho[i]) ov = true;
   }
+  out->inter_vdw += sum[0] + low[0];
+  out->inter_q += sum[1] + low[1];
   return !ov;
 }
 
@@ -1060,9 +1072,7 @@ extern "C" int cass_total_energy(cass_engine *e, int32_t box, int32_t intra_flag
     return CASS_OK;
   }
   // intermolecular pairs on the device
-  const int blk = kMaxBlock;
-  const int nblk = std::max(1, (b->nmols + blk - 1) / blk);
-  const size_t np = (size_t)nblk * std::max(1, b->nmols);
+  const size_t np = (size_t)std::max(1, b->nmols);
   char *s = (char *)cass_scratch(e, np * (2 * sizeof(double) + sizeof(int)) + 256);
   if (!s) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
   double *part = (double *)s;
@@ -1071,12 +1081,12 @@ extern "C" int cass_total_energy(cass_engine *e, int32_t box, int32_t intra_flag
     BoxDev bv = box_view(e, *b);
     TopoDev tv = topo_view(e);
     PairConst<double> cd = make_pair_const<double>(b->p, e->ntypes);
-    dim3 grid(nblk, b->nmols);
     PairConst<float> cf = make_pair_const<float>(b->p, e->ntypes);
     auto kern = e->prec == CASS_PREC_MIXED  ? k_total_pairs<PrecMixed>
                 : e->prec == CASS_PREC_FP32 ? k_total_pairs<PrecFP32>
                                             : k_total_pairs<PrecFP64>;
-    hipLaunchKernelGGL(kern, grid, dim3(blk), 0, e->stream, bv, tv, cd, cf, part, part_ov);
+    hipLaunchKernelGGL(kern, dim3((b->nmols + kPairMols - 1) / kPairMols), dim3(64 * kPairMols), 0, e->stream, bv, tv,
+                       cd, cf, part, part_ov);
     HIP_TRY(e, hipGetLastError());
     std::vector<double> hp(2 * np);
     std::vector<int> ho(np);
@@ -1125,9 +1135,7 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
     }
   const int blk = kMaxBlock;
   std::vector<RecomputeBox> rb(nboxes);
-  std::vector<int4> items;
-  std::vector<int4> kitems_mol;
-  std::vector<int2> kitems_box;
+  std::vector<int2> items, kitems_mol, kitems_box;
   int64_t np = 0, nk = 0;
   for (int i = 0; i < nboxes; ++i) {
     const cass_box_state &b = *bs[i];
@@ -1135,18 +1143,16 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
     r.b = box_view(e, b);
     r.cd = make_pair_const<double>(b.p, e->ntypes);
     r.cf = make_pair_const<float>(b.p, e->ntypes);
-    r.nblk = std::max(1, (b.nmols + blk - 1) / blk);
     r.part_off = np;
-    for (int m = 0; m < b.nmols; ++m)
-      for (int bx = 0; bx < r.nblk; ++bx) items.push_back(make_int4(i, m, bx, 0));
-    np += (int64_t)r.nblk * std::max(1, b.nmols);
+    for (int m = 0; m < b.nmols; m += kPairMols) items.push_back(make_int2(i, m));
+    np += std::max(1, b.nmols);
     const bool ewald = b.p.charge_style == CASS_Q_EWALD;
     r.ew = ewald ? ewald_view(b, row_k0_of(b)) : EwaldDev{};
-    r.kblk = ewald ? std::max(1, (b.nvecs + blk - 1) / blk) : 0;
+    r.kblk = ewald ? std::max(1, (b.nvecs + kBoxVecs - 1) / kBoxVecs) : 0;
     r.kpart_off = nk;
     if (ewald) {
-      for (int m = 0; m < b.nmols; ++m)
-        for (int kb = 0; kb < (b.nvecs + blk - 1) / blk; ++kb) kitems_mol.push_back(make_int4(i, m, kb, 0));
+      if (b.nvecs > 0)
+        for (int m = 0; m < b.nmols; ++m) kitems_mol.push_back(make_int2(i, m));
       for (int kb = 0; kb < r.kblk; ++kb) kitems_box.push_back(make_int2(i, kb));
       nk += r.kblk;
     }
@@ -1159,8 +1165,8 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
     return o;
   };
   const size_t o_rb = take(sizeof(RecomputeBox) * std::max(1, nboxes)),
-               o_it = take(sizeof(int4) * std::max<size_t>(1, items.size())),
-               o_km = take(sizeof(int4) * std::max<size_t>(1, kitems_mol.size())),
+               o_it = take(sizeof(int2) * std::max<size_t>(1, items.size())),
+               o_km = take(sizeof(int2) * std::max<size_t>(1, kitems_mol.size())),
                o_kb = take(sizeof(int2) * std::max<size_t>(1, kitems_box.size())),
                o_part = take(2 * sizeof(double) * std::max<int64_t>(1, np)),
                o_pov = take(sizeof(int) * std::max<int64_t>(1, np)),
@@ -1170,9 +1176,9 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
   if (!s) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
   HIP_TRY(e, hipMemcpyAsync(s + o_rb, rb.data(), sizeof(RecomputeBox) * nboxes, hipMemcpyHostToDevice, e->stream));
   if (!items.empty())
-    HIP_TRY(e, hipMemcpyAsync(s + o_it, items.data(), sizeof(int4) * items.size(), hipMemcpyHostToDevice, e->stream));
+    HIP_TRY(e, hipMemcpyAsync(s + o_it, items.data(), sizeof(int2) * items.size(), hipMemcpyHostToDevice, e->stream));
   if (!kitems_mol.empty())
-    HIP_TRY(e, hipMemcpyAsync(s + o_km, kitems_mol.data(), sizeof(int4) * kitems_mol.size(), hipMemcpyHostToDevice,
+    HIP_TRY(e, hipMemcpyAsync(s + o_km, kitems_mol.data(), sizeof(int2) * kitems_mol.size(), hipMemcpyHostToDevice,
                               e->stream));
   if (!kitems_box.empty())
     HIP_TRY(e, hipMemcpyAsync(s + o_kb, kitems_box.data(), sizeof(int2) * kitems_box.size(), hipMemcpyHostToDevice,
@@ -1186,13 +1192,13 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
     auto kern = e->prec == CASS_PREC_MIXED  ? k_total_pairs_multi<PrecMixed>
                 : e->prec == CASS_PREC_FP32 ? k_total_pairs_multi<PrecFP32>
                                             : k_total_pairs_multi<PrecFP64>;
-    hipLaunchKernelGGL(kern, dim3((unsigned)items.size()), dim3(blk), 0, e->stream, d_rb, tv,
-                       (const int4 *)(s + o_it), d_part, d_pov);
+    hipLaunchKernelGGL(kern, dim3((unsigned)items.size()), dim3(64 * kPairMols), 0, e->stream, d_rb, tv,
+                       (const int2 *)(s + o_it), d_part, d_pov);
     HIP_TRY(e, hipGetLastError());
   }
   if (!kitems_mol.empty()) {
     hipLaunchKernelGGL(k_ewald_mol_multi, dim3((unsigned)kitems_mol.size()), dim3(blk), 0, e->stream, d_rb, tv,
-                       (const int4 *)(s + o_km));
+                       (const int2 *)(s + o_km));
     HIP_TRY(e, hipGetLastError());
   }
   if (!kitems_box.empty()) {
@@ -1227,8 +1233,7 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
       continue;
     }
     if (b->nmols > 0 &&
-        !total_pair_sums(hp.data() + 2 * rb[i].part_off, ho.data() + rb[i].part_off,
-                         (size_t)rb[i].nblk * b->nmols, o)) {
+        !total_pair_sums(hp.data() + 2 * rb[i].part_off, ho.data() + rb[i].part_off, (size_t)b->nmols, o)) {
       overlap[i] = 1;
       continue;
     }
@@ -1406,13 +1411,13 @@ extern "C" int cass_ewald_full(cass_engine *e, int32_t box, double *e_recip) {
   TopoDev tv = topo_view(e);
   EwaldDev ew = ewald_view(*b, row_k0_of(*b));
   if (b->nmols > 0 && K > 0) {
-    hipLaunchKernelGGL(k_ewald_mol, dim3((K + 255) / 256, b->nmols), dim3(256), 0, e->stream, bv, tv, ew);
+    hipLaunchKernelGGL(k_ewald_mol, dim3(b->nmols), dim3(kMaxBlock), 0, e->stream, bv, tv, ew);
     HIP_TRY(e, hipGetLastError());
   }
-  const int nb = std::max(1, (K + 255) / 256);
+  const int nb = std::max(1, (K + kBoxVecs - 1) / kBoxVecs);
   double *part = (double *)cass_scratch(e, sizeof(double) * (nb + 1));
   if (!part) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
-  hipLaunchKernelGGL(k_ewald_box, dim3(nb), dim3(256), 0, e->stream, bv, ew, part);
+  hipLaunchKernelGGL(k_ewald_box, dim3(nb), dim3(kMaxBlock), 0, e->stream, bv, ew, part);
   HIP_TRY(e, hipGetLastError());
   hipLaunchKernelGGL(k_sum, dim3(1), dim3(256), 0, e->stream, part, (size_t)nb, 1, 0, part + nb);
   HIP_TRY(e, hipGetLastError());

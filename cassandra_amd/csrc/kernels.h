@@ -52,6 +52,9 @@ struct EwaldDev {
   const int4 *rows;      // (nx, nz, ny0, +-count): a run of consecutive ny from ny0
   const int *row_k0;     // first traversal position of each row
   const int *kperm;      // k index of each traversal position
+  const int4 *segs;      // runs of up to kKSeg vectors along nx: (k0 | len << 20, nx, ny, nz)
+  int nsegs;
+  int tx, ty, tz;        // powers of a site's unit phases per axis
 };
 
 struct WidomArgs {
@@ -329,7 +332,7 @@ struct RecomputeBox {
   PairConst<double> cd;
   PairConst<float> cf;
   EwaldDev ew;
-  int nblk, kblk;
+  int kblk;
   int64_t part_off, kpart_off;
 };
 
@@ -351,6 +354,10 @@ __host__ __device__ inline cplx cpow_int(cplx e, int n) {
   return r;
 }
 
+constexpr int kPairMols = 4;   // molecules per workgroup of the total pair sums, one wave each
+constexpr int kBoxVecs = 64;   // k vectors per workgroup of the box sums
+constexpr int kEwTab = 1024;   // phase powers held per molecule
+
 // kernels (kernels.hip)
 template <typename P>
 __global__ void k_trials(BoxDev b, TopoDev tp, PairConst<double> cd, PairConst<float> cf, int species, int ni,
@@ -364,9 +371,9 @@ __global__ void k_total_pairs(BoxDev b, TopoDev tp, PairConst<double> cd, PairCo
 __global__ void k_ewald_mol(BoxDev b, TopoDev tp, EwaldDev ew);
 __global__ void k_ewald_box(BoxDev b, EwaldDev ew, double *part);
 template <typename P>
-__global__ void k_total_pairs_multi(const RecomputeBox *boxes, TopoDev tp, const int4 *items, double *part,
+__global__ void k_total_pairs_multi(const RecomputeBox *boxes, TopoDev tp, const int2 *items, double *part,
                                     int *part_ov);
-__global__ void k_ewald_mol_multi(const RecomputeBox *boxes, TopoDev tp, const int4 *items);
+__global__ void k_ewald_mol_multi(const RecomputeBox *boxes, TopoDev tp, const int2 *items);
 __global__ void k_ewald_box_multi(const RecomputeBox *boxes, const int2 *items, double *kpart);
 __global__ void k_sum_multi(const RecomputeBox *boxes, const double *kpart, double *out);
 __global__ void k_ewald_move(TopoDev tp, EwaldDev ew, int m, int species, int flag, int n, const double *nxyz,

@@ -118,101 +118,263 @@ __global__ void k_sum(const double *in, size_t n, int stride, int comp, double *
 }
 
 // ---------------------------------------------------- total pair energy
-// Compute_System_Total_Energy inter part (energy_routines.f90:2775-2917):
-// block (bx, i) covers pairs (i, j) with j > i, j in [bx*blockDim, +blockDim);
-// partial o = i * nblk + bx of part / part_ov.
+// Compute_System_Total_Energy inter part (energy_routines.f90:2775-2917): one
+// wave per molecule i and the pairs (i, j) with j > i.  The sites of the
+// molecules in range are compacted in LDS and scored 64 at a time against
+// every site of i.  A workgroup of one j per lane left five lanes in six idle
+// (j <= i, or out of range) and dominated the sum: 24 boxes of 512 waters took
+// 0.60 ms, 0.27 here.  part[i], part_ov[i]: i's sums.
 template <typename P>
-__device__ inline void total_pairs_block(const BoxDev &b, const TopoDev &tp, const PairConst<double> &cd,
-                                         const PairConst<float> &cf, int i, int bx, int nblk, double *part,
-                                         int *part_ov) {
-  __shared__ double px[kMaxSites], py[kMaxSites], pz[kMaxSites];
-  __shared__ int pspa[kMaxSites];
+__device__ inline void total_pairs_wave(const BoxDev &b, const TopoDev &tp, const PairConst<double> &cd,
+                                        const PairConst<float> &cf, int i, double *part, int *part_ov) {
+  using TV = typename P::V;
+  using TQ = typename P::Q;
+  const PairConst<TV> &cv = pconst<TV>(cd, cf);
+  const PairConst<TQ> &cq = pconst<TQ>(cd, cf);
+  __shared__ int2 ring[kPairMols][128];  // (site, species atom) of partners in range
+  const int lane = threadIdx.x & 63;
+  int2 *ent = ring[threadIdx.x >> 6];
   const int si = b.species[i], fi = b.first[i];
   const int ni = tp.sp_natoms[si], oi = tp.sp_atom_off[si];
-  if (threadIdx.x < ni) {
-    px[threadIdx.x] = b.x[fi + threadIdx.x];
-    py[threadIdx.x] = b.y[fi + threadIdx.x];
-    pz[threadIdx.x] = b.z[fi + threadIdx.x];
-    pspa[threadIdx.x] = oi + threadIdx.x;
+  const double4 ci = b.comd[i];
+  double ev = 0.0, eq = 0.0;
+  bool ov = false;
+  int head = 0, cnt = 0;
+  auto sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  int base = b.live[i] ? i + 1 : b.nmols, ja = 0, nj = 0, fj = 0, oj = 0;
+  bool take = false;
+  for (;;) {
+    // the ja-th sites of 64 molecules, then the next 64
+    if (__any(take && ja < nj)) {
+      const bool push = take && ja < nj;
+      const uint64_t bal = __ballot(push);
+      const int before =
+          __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0));
+      if (push) ent[(head + cnt + before) & 127] = make_int2(fj + ja, oj + ja);
+      cnt += __popcll(bal);
+      ++ja;
+      sync();
+    } else if (base < b.nmols) {
+      const int j = base + lane;
+      base += 64;
+      take = j < b.nmols && b.live[j] && molpair_in_range(b, false, ci, b.comd[j]);
+      if (take) {
+        const int sj = b.species[j];
+        fj = b.first[j];
+        oj = tp.sp_atom_off[sj];
+        nj = tp.sp_natoms[sj];
+      }
+      ja = 0;
+      continue;
+    } else if (cnt == 0) {
+      break;
+    }
+    const bool last = base >= b.nmols && !__any(take && ja < nj);
+    if (cnt >= 64 || last) {
+      const int n = cnt < 64 ? cnt : 64;
+      if (lane < n) {
+        const int2 e = ent[(head + lane) & 127];
+        const double x = b.x[e.x], y = b.y[e.x], z = b.z[e.x], qj = tp.atom_charge[e.y];
+        const int tj = tp.atom_type[e.y];
+        for (int ia = 0; ia < ni; ++ia) {
+          double dx = b.x[fi + ia] - x, dy = b.y[fi + ia] - y, dz = b.z[fi + ia] - z;
+          min_image(b, dx, dy, dz);
+          const double r2 = dx * dx + dy * dy + dz * dz;
+          if (r2 < cd.rc_low2) {
+            ov = true;
+            continue;
+          }
+          bool gv, gq;
+          pair_cutoff(cd, false, r2, gv, gq);
+          const int ti = tp.atom_type[oi + ia];
+          if (gv && ti >= 0 && tj >= 0) {
+            const int k = ti * tp.ntypes + tj;
+            ev += (double)vdw_inter<TV, typename P::M>(cv, (TV)r2, (TV)tp.eps[k], (TV)tp.sig[k], (TV)tp.mn[k],
+                                                       (TV)tp.mm[k]);
+          }
+          const double qi = tp.atom_charge[oi + ia];
+          if (gq && cd.q_style != CASS_Q_NONE && qi != 0.0 && qj != 0.0)
+            eq += (double)qq_inter<TQ, typename P::M>(cq, (TQ)r2, (TQ)(qi * qj));
+        }
+      }
+      head += n;
+      cnt -= n;
+      sync();
+    }
   }
-  __syncthreads();
-  double v[2] = {0.0, 0.0};
-  int ov = 0;
-  const int j = bx * blockDim.x + threadIdx.x;
-  if (b.live[i] && j > i && j < b.nmols && b.live[j]) {
-    if (molpair_in_range(b, false, b.comd[i], b.comd[j]))
-      ov = molpair_energy<P>(b, tp, cd, cf, false, true, ni, px, py, pz, pspa, j, v[0], v[1], nullptr);
-  }
-  block_reduce<2>(v, ov);
-  if (threadIdx.x == 0) {
-    const size_t o = (size_t)i * nblk + bx;
-    part[2 * o] = v[0];
-    part[2 * o + 1] = v[1];
-    part_ov[o] = ov;
+  ev = wave_total(ev);
+  eq = wave_total(eq);
+  const int any = __any(ov);
+  if (lane == 0) {
+    part[2 * (size_t)i] = ev;
+    part[2 * (size_t)i + 1] = eq;
+    part_ov[i] = any;
   }
 }
 
-// grid (nblk, nmols)
+// grid ceil(nmols / kPairMols)
 template <typename P>
-__global__ void __launch_bounds__(kMaxBlock) k_total_pairs(BoxDev b, TopoDev tp, PairConst<double> cd,
-                                                           PairConst<float> cf, double *part, int *part_ov) {
-  total_pairs_block<P>(b, tp, cd, cf, blockIdx.y, blockIdx.x, gridDim.x, part, part_ov);
+__global__ void __launch_bounds__(64 * kPairMols) k_total_pairs(BoxDev b, TopoDev tp, PairConst<double> cd,
+                                                                PairConst<float> cf, double *part, int *part_ov) {
+  const int i = blockIdx.x * kPairMols + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (i < b.nmols) total_pairs_wave<P>(b, tp, cd, cf, i, part, part_ov);
 }
 
-// The same over many boxes: one workgroup per item (box, i, bx); the box's
-// partials start at part_off (pairs) in part / part_ov.
+// The same over many boxes: one workgroup per item (box, first molecule); the
+// box's partials start at part_off in part / part_ov.
 template <typename P>
-__global__ void __launch_bounds__(kMaxBlock) k_total_pairs_multi(const RecomputeBox *__restrict__ boxes, TopoDev tp,
-                                                                 const int4 *__restrict__ items, double *part,
-                                                                 int *part_ov) {
-  const int4 it = items[blockIdx.x];
+__global__ void __launch_bounds__(64 * kPairMols)
+    k_total_pairs_multi(const RecomputeBox *__restrict__ boxes, TopoDev tp, const int2 *__restrict__ items,
+                        double *part, int *part_ov) {
+  const int2 it = items[blockIdx.x];
   const RecomputeBox &r = boxes[it.x];
-  total_pairs_block<P>(r.b, tp, r.cd, r.cf, it.y, it.z, r.nblk, part + 2 * r.part_off, part_ov + r.part_off);
+  const int i = it.y + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (i < r.b.nmols) total_pairs_wave<P>(r.b, tp, r.cd, r.cf, i, part + 2 * r.part_off, part_ov + r.part_off);
 }
 
 // ----------------------------------------------------------------- Ewald
 // Compute_System_Ewald_Reciprocal_Energy (energy_routines.f90:4111-4231),
-// stage 1: per-molecule sums of k vectors [kb*blockDim, +blockDim).
-__device__ inline void ewald_mol_block(const BoxDev &b, const TopoDev &tp, const EwaldDev &ew, int m, int kb) {
-  const int k = kb * blockDim.x + threadIdx.x;
-  if (k >= ew.nvecs) return;
-  double c = 0.0, s = 0.0;
-  if (b.live[m]) {
-    const int sp = b.species[m], f = b.first[m];
-    const int n = tp.sp_natoms[sp], o = tp.sp_atom_off[sp];
-    const double hx = ew.hx[k], hy = ew.hy[k], hz = ew.hz[k];
+// stage 1: the sums of one molecule over all k vectors, one workgroup.  The
+// powers of the sites' unit phases stand in LDS (2 pi as the reference
+// truncates it), a lane takes a segment of consecutive n_x, and each wave
+// passes its segments' sums through LDS to store them in k order: 24 boxes of
+// 512 waters took 0.32 ms with a sine and cosine per site and vector, 0.13
+// here, for 0.46 GB of stores.  Molecules whose powers exceed the table keep
+// the sine and cosine.
+__device__ inline void ewald_mol_block(const BoxDev &b, const TopoDev &tp, const EwaldDev &ew, int m) {
+  __shared__ cplx tab[kEwTab];
+  __shared__ cplx eph[3 * kMaxSites];
+  __shared__ double out[kMaxBlock / 64][64 * kKSeg];
+  const int tid = threadIdx.x, lane = tid & 63, K = ew.nvecs;
+  double *cm = ew.cmol + (size_t)m * K, *sm = ew.smol + (size_t)m * K;
+  if (!b.live[m]) {
+    for (int k = tid; k < K; k += blockDim.x) cm[k] = sm[k] = 0.0;
+    return;
+  }
+  const int sp = b.species[m], f = b.first[m];
+  const int n = tp.sp_natoms[sp], o = tp.sp_atom_off[sp], nt = ew.tx + ew.ty + ew.tz;
+  if (n > kMaxSites || n * nt > kEwTab) {
+    for (int k = tid; k < K; k += blockDim.x) {
+      const double hx = ew.hx[k], hy = ew.hy[k], hz = ew.hz[k];
+      double c = 0.0, s = 0.0;
+      for (int a = 0; a < n; ++a) {
+        const double q = tp.atom_charge[o + a];
+        double sv, cv;
+        sincos(hx * b.x[f + a] + hy * b.y[f + a] + hz * b.z[f + a], &sv, &cv);
+        c = c + q * cv;
+        s = s + q * sv;
+      }
+      cm[k] = c;
+      sm[k] = s;
+    }
+    return;
+  }
+  for (int t = tid; t < 3 * n; t += blockDim.x) {
+    const int a = t / 3, d = t - 3 * a;
+    const double sd = b.Li[d] * b.x[f + a] + b.Li[3 + d] * b.y[f + a] + b.Li[6 + d] * b.z[f + a];
+    sincos(kTwoPi * sd, &eph[t].im, &eph[t].re);
+  }
+  __syncthreads();
+  for (int t = tid; t < n * nt; t += blockDim.x) {
+    const int a = t / nt, r = t - a * nt;
+    const int d = r < ew.tx ? 0 : r < ew.tx + ew.ty ? 1 : 2;
+    tab[t] = cpow_int(eph[3 * a + d], r - (d == 0 ? 0 : d == 1 ? ew.tx : ew.tx + ew.ty));
+  }
+  __syncthreads();
+  double *buf = out[tid >> 6];
+  for (int s0 = tid - lane; s0 < ew.nsegs; s0 += blockDim.x) {  // wave-uniform
+    const int4 sg = ew.segs[min(s0 + lane, ew.nsegs - 1)];
+    const int k0 = sg.x & 0xfffff, len = sg.x >> 20;
+    const int ny = sg.z < 0 ? -sg.z : sg.z, nz = sg.w < 0 ? -sg.w : sg.w;
+    double c[kKSeg], s[kKSeg];
+#pragma unroll
+    for (int t = 0; t < kKSeg; ++t) c[t] = s[t] = 0.0;
     for (int a = 0; a < n; ++a) {
-      const double hr = hx * b.x[f + a] + hy * b.y[f + a] + hz * b.z[f + a];
+      const cplx *ta = tab + a * nt;
+      const cplx X = ta[sg.y], E = ta[1];
+      cplx Y = ta[ew.tx + ny], Z = ta[ew.tx + ew.ty + nz];
+      Y.im = sg.z < 0 ? -Y.im : Y.im;
+      Z.im = sg.w < 0 ? -Z.im : Z.im;
+      cplx p = cmul(cmul(X, Z), Y);
       const double q = tp.atom_charge[o + a];
-      double sv, cv;
-      sincos(hr, &sv, &cv);
-      c = c + q * cv;
-      s = s + q * sv;
+      p.re = q * p.re;
+      p.im = q * p.im;
+#pragma unroll
+      for (int t = 0; t < kKSeg; ++t) {
+        c[t] = c[t] + p.re;
+        s[t] = s[t] + p.im;
+        if (t + 1 < kKSeg) p = cmul(p, E);
+      }
+    }
+    // the wave's segments cover consecutive vectors
+    const int last = min(s0 + 63, ew.nsegs - 1) - s0;
+    const int kb = __builtin_amdgcn_readfirstlane(k0);
+    const int kn = __builtin_amdgcn_readlane(k0 + len, last) - kb;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (lane <= last) {
+#pragma unroll
+        for (int t = 0; t < kKSeg; ++t)
+          if (t < len) buf[k0 - kb + t] = h ? s[t] : c[t];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      for (int t = lane; t < kn; t += 64) (h ? sm : cm)[kb + t] = buf[t];
     }
   }
-  ew.cmol[(size_t)m * ew.nvecs + k] = c;
-  ew.smol[(size_t)m * ew.nvecs + k] = s;
 }
 
-// grid (ceil(K/blk), nmols)
-__global__ void k_ewald_mol(BoxDev b, TopoDev tp, EwaldDev ew) { ewald_mol_block(b, tp, ew, blockIdx.y, blockIdx.x); }
+// grid nmols
+__global__ void __launch_bounds__(kMaxBlock) k_ewald_mol(BoxDev b, TopoDev tp, EwaldDev ew) {
+  ewald_mol_block(b, tp, ew, blockIdx.x);
+}
 
-// stage 2: box sums over molecules (molecule order) and the energy term of
-// k block kb, written to part[kb].
+// stage 2: the box sums over molecules (zero for dead ones) and the energy
+// term of kBoxVecs k vectors, written to part[kb].  The molecules are shared
+// by the workgroup's waves and read several at a time: one lane per vector
+// over all molecules was a chain of 512 loads on a tenth of the chip (24 boxes
+// of 512 waters: 0.60 ms, 0.13 here).
 __device__ inline void ewald_box_block(const BoxDev &b, const EwaldDev &ew, int kb, double *part) {
-  const int k = kb * blockDim.x + threadIdx.x;
+  __shared__ double sh[2][kMaxBlock / 64][kBoxVecs];
+  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6, G = blockDim.x >> 6;
+  const int k = kb * kBoxVecs + lane;
   double v[1] = {0.0};
   int f = 0;
+  double c[4] = {0.0, 0.0, 0.0, 0.0}, s[4] = {0.0, 0.0, 0.0, 0.0};
   if (k < ew.nvecs) {
-    double c = 0.0, s = 0.0;
-    for (int m = 0; m < b.nmols; ++m) {
-      if (!b.live[m]) continue;
-      c = c + ew.cmol[(size_t)m * ew.nvecs + k];
-      s = s + ew.smol[(size_t)m * ew.nvecs + k];
+    int m = g;
+    for (; m + 3 * G < b.nmols; m += 4 * G) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const size_t o = (size_t)(m + u * G) * ew.nvecs + k;
+        c[u] = c[u] + ew.cmol[o];
+        s[u] = s[u] + ew.smol[o];
+      }
     }
-    ew.cs[k] = c;
-    ew.sn[k] = s;
-    v[0] = ew.cn[k] * (c * c + s * s);
+    for (; m < b.nmols; m += G) {
+      const size_t o = (size_t)m * ew.nvecs + k;
+      c[0] = c[0] + ew.cmol[o];
+      s[0] = s[0] + ew.smol[o];
+    }
+  }
+  sh[0][g][lane] = (c[0] + c[1]) + (c[2] + c[3]);
+  sh[1][g][lane] = (s[0] + s[1]) + (s[2] + s[3]);
+  __syncthreads();
+  if (g == 0 && k < ew.nvecs) {
+    double ct = 0.0, st = 0.0;
+    for (int u = 0; u < G; ++u) {
+      ct = ct + sh[0][u][lane];
+      st = st + sh[1][u][lane];
+    }
+    ew.cs[k] = ct;
+    ew.sn[k] = st;
+    v[0] = ew.cn[k] * (ct * ct + st * st);
   }
   block_reduce<1>(v, f);
   if (threadIdx.x == 0) part[kb] = v[0];
@@ -220,12 +382,13 @@ __device__ inline void ewald_box_block(const BoxDev &b, const EwaldDev &ew, int 
 
 __global__ void k_ewald_box(BoxDev b, EwaldDev ew, double *part) { ewald_box_block(b, ew, blockIdx.x, part); }
 
-// The two stages over many boxes: items (box, molecule, k block) and
-// (box, k block); a box's k-block terms start at kpart_off in kpart.
-__global__ void k_ewald_mol_multi(const RecomputeBox *__restrict__ boxes, TopoDev tp, const int4 *__restrict__ items) {
-  const int4 it = items[blockIdx.x];
+// The two stages over many boxes: items (box, molecule) and (box, k block); a
+// box's k-block terms start at kpart_off in kpart.
+__global__ void __launch_bounds__(kMaxBlock)
+    k_ewald_mol_multi(const RecomputeBox *__restrict__ boxes, TopoDev tp, const int2 *__restrict__ items) {
+  const int2 it = items[blockIdx.x];
   const RecomputeBox &r = boxes[it.x];
-  ewald_mol_block(r.b, tp, r.ew, it.y, it.z);
+  ewald_mol_block(r.b, tp, r.ew, it.y);
 }
 
 __global__ void k_ewald_box_multi(const RecomputeBox *__restrict__ boxes, const int2 *__restrict__ items,
@@ -369,7 +532,7 @@ __global__ void k_sum_widom(const double *part, const int64_t *part_ov, int n, d
                                        const double *, int, int, double *, int *);                        \
   template __global__ void k_total_pairs<P>(BoxDev, TopoDev, PairConst<double>, PairConst<float>,         \
                                             double *, int *);                                             \
-  template __global__ void k_total_pairs_multi<P>(const RecomputeBox *, TopoDev, const int4 *, double *, int *);
+  template __global__ void k_total_pairs_multi<P>(const RecomputeBox *, TopoDev, const int2 *, double *, int *);
 CASS_INSTANTIATE(PrecFP64)
 CASS_INSTANTIATE(PrecMixed)
 CASS_INSTANTIATE(PrecFP32)

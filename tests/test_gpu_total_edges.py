@@ -1,0 +1,83 @@
+"""The pair and structure-factor kernels of the total energy at their edges:
+molecule counts around a workgroup's four and a wave's 64, one site to 40 (the
+phase table is exceeded), unlike species, unlike edges, dead molecules.  Pair
+terms against half the sum of the molecules' own energies, the reciprocal term
+against numpy's direct sum, one box and a batch."""
+import numpy as np
+import pytest
+
+from cassandra_amd import engine as E
+from cassandra_amd import systems as S
+
+REL = 1e-10
+
+
+def _species(n, q):
+    xyz = np.array([[1.0 * i, 0.4 * (i % 2), 0.0] for i in range(n)])
+    atoms = [S.Atom(f"T{n}_{i % 2}", "C", 12.0, 0.0 if i == n - 1 and n % 2 else (-q if i % 2 else q), 45.0, 2.7)
+             for i in range(n)]
+    return S.Species(f"s{n}", atoms, xyz)
+
+
+CASES = {
+    "one": ([1], [1], [18.0] * 3), "five": ([3], [5], [18.0] * 3), "wave": ([2], [65], [22.0] * 3),
+    "mixture": ([4, 1, 7], [12, 31, 6], [19.0, 26.0, 23.0]), "long": ([40, 2], [3, 6], [46.0] * 3),
+}
+
+
+def _reciprocal(system, xyz, charges):
+    """Compute_System_Ewald_Reciprocal_Energy by direct sums"""
+    L, rc = system.box, system.rcut_coul
+    alpha = np.sqrt(-np.log(system.ewald_tol)) / rc
+    hc = 2.0 * (-np.log(system.ewald_tol)) / rc
+    top = [int(hc * l / S.TWO_PI) + 1 for l in L]
+    nz, ny, nx = np.meshgrid(*[np.arange(-top[2], top[2] + 1), np.arange(-top[1], top[1] + 1),
+                               np.arange(0, top[0] + 1)], indexing="ij")
+    n = np.stack([nx.ravel(), ny.ravel(), nz.ravel()], axis=1)
+    h = S.TWO_PI * n / L
+    h2 = np.sum(h * h, axis=1)
+    keep = (h2 < hc * hc) & (h2 > 0.0)
+    h, h2, n = h[keep], h2[keep], n[keep]
+    cn = np.where(n[:, 0] == 0, 1.0, 2.0) * S.TWO_PI / np.prod(L) * np.exp(-h2 / (4.0 * alpha * alpha)) / h2
+    s = np.exp(1j * (h @ xyz.T)) @ charges
+    return float(np.sum(cn * np.abs(s) ** 2) * S.CHARGE_FACTOR)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", [E.FP64, E.MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("case", list(CASES))
+def test_total_energy_edges(case, prec):
+    print(f"[gpu] total energy edges {case} {prec}", flush=True)
+    sites, counts, box = CASES[case]
+    species = [_species(n, 0.25) for n in sites]
+    coords = S.place_random(list(zip(species, counts)), box, 21, 1.2, 2.6)
+    system = S.System(species, counts, coords, np.array(box), 300.0, "lj", "cut", 8.5, charge_style="ewald",
+                      rcut_coul=8.5, rcut_low=0.85, box_shape="cubic" if len(set(box)) == 1 else "orthogonal",
+                      name=case).parsed()
+    eng = E.Engine(system, max_boxes=2, precision=prec)
+    boxes = [eng.add_box(system), eng.add_box(system)]
+    for b in boxes:
+        b.ewald_setup()
+    # the second box with its last molecule dead
+    xyz = boxes[0].download()
+    live = np.array(boxes[1].live).copy()
+    live[-1] = 0
+    boxes[1].upload(boxes[1].spec, live, xyz)
+    batch = eng.total_energy_batch(boxes)
+    batch = batch[0] if isinstance(batch, tuple) else batch
+    nat = [sp.natoms for sp, n in zip(species, counts) for _ in range(n)]
+    charges = np.concatenate([[a.charge for a in sp.atoms] for sp, n in zip(species, counts) for _ in range(n)])
+    tol = REL if prec == E.FP64 else 1e-8
+    for b, lv, got in zip(boxes, (np.ones(len(nat), dtype=int), live), batch):
+        one = b.compute_system_total_energy()
+        assert all(one[k] == got[k] for k in ("total", "inter_vdw", "reciprocal"))
+        half = np.zeros(2)
+        for m in np.flatnonzero(lv):
+            ev, eq, ov = b.compute_molecule_nonbond_inter_energy(int(m))
+            assert not ov
+            half += 0.5 * np.array([ev, eq])
+        assert abs(one["inter_vdw"] - half[0]) <= tol * max(1.0, abs(half[0]))
+        weight = np.repeat(lv, nat) * charges
+        ref = _reciprocal(system, xyz.reshape(-1, 3), weight)
+        assert abs(one["reciprocal"] - ref) <= tol * max(1.0, abs(ref))
+    eng.close()
