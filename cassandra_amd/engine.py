@@ -152,6 +152,13 @@ def _p(a, t=C.c_double):
     return None if a is None else a.ctypes.data_as(C.POINTER(t))
 
 
+def _at_least(n, **lists):
+    """The native call reads and writes n entries of each list: fewer raise."""
+    for name, entries in lists.items():
+        if len(entries) < n:
+            raise ValueError(f"{name}: {len(entries)} entries for {n} boxes")
+
+
 def _energies_in(energies):
     """A CassEnergy array of energy dicts."""
     ens = (abi.CassEnergy * len(energies))()
@@ -327,6 +334,8 @@ class Engine:
         in place) from its energy dict energies[i]; returns one record dict
         per box as Box.nvt_run does."""
         n = len(boxes)
+        energies = list(energies)
+        _at_least(n, rngs=rngs, energies=energies)
         ids = np.ascontiguousarray([b.id for b in boxes], dtype=np.int32)
         opts = (abi.CassNvtOptions * n)()
         rng_arr = (abi.CassRng * n)()
@@ -354,6 +363,8 @@ class Engine:
         updated in place) from its energy dict energies[i]; returns one
         record dict per box as nvt_run_batch does."""
         n = len(boxes)
+        locates, energies = list(locates), list(energies)
+        _at_least(n, locates=locates, rngs=rngs, energies=energies)
         bx = (abi.CassRegrowBox * n)()
         rng_arr = (abi.CassRng * n)()
         ens = _energies_in(energies)
