@@ -4,7 +4,8 @@
 // and Rotate (move_rotate.f90:23-520), with the same random-number draws
 // (random_generators.f90:51-122), energy bookkeeping and accept_or_reject
 // (accept_or_reject.f90:22-65) as the host-driven loop in nvt.cpp.  One
-// workgroup per box runs the moves in sequence on a copy of the box in LDS:
+// workgroup per box runs the moves in sequence on a copy of the box in LDS, or
+// on the box itself where a copy does not fit (nvt_prepare):
 // one wave prepares the next move while the others evaluate the current one,
 // sharing the molecule-pair energies and the k vectors of the reciprocal
 // update.  No host round trip per move: the host launches chunks of moves and
@@ -26,10 +27,8 @@ namespace cass {
 // Waves per workgroup: the last wave prepares moves, the others share the
 // molecules and the k segments.  12 waves are three per SIMD at up to 168
 // VGPRs: a move of 512 waters takes 11.9 us on 12, 17.8 on 8 (the k segments
-// no longer fit one per lane) and 13.7 on 16 (128 VGPRs, which spill).  A box
-// whose copy leaves no room for their buffers runs on fewer (nvt_prepare).
+// no longer fit one per lane) and 13.7 on 16 (128 VGPRs, which spill).
 constexpr int kNvtWaves = 12;
-constexpr int kNvtMinWaves = 2;
 constexpr int kNvtSeg = kKSeg;   // k vectors per segment
 constexpr int kNvtRing = 32;     // generator states kept around the current move
 constexpr int kNvtAhead = 10;    // draws of one move (6 at most, its acceptance, the other start) and some
@@ -46,6 +45,7 @@ struct NvtChainArgs {
   int tabled;               // the phases' powers fit in LDS
   double *x, *y, *z;  // the box's site coordinates (the memory of b.x, b.y, b.z)
   double4 *comd;      // the box's (COM, max_dcom) (the memory of b.comd)
+  int *meta;          // species and live flag per molecule where the box stays in device memory
   const int *mols;    // mobile molecules in locate order
   int nm, n, spa0, charged, linear;
   int nj_max;  // the largest site count of the box's molecules
@@ -56,7 +56,7 @@ struct NvtChainArgs {
   double *energy, *ln_pacc;
   int64_t *rng_state;
   int *status;  // set to 1 when a molecule overlaps before its move
-  // the box held in LDS for the whole chain (offsets in bytes)
+  // the box held in LDS for the whole chain, and the waves' buffers (offsets in bytes)
   int nsite, natoms_total, nspecies, ntypes;
   int o_x, o_y, o_z, o_comd, o_first, o_meta, o_atype, o_acharge, o_spn, o_spo, o_pt, o_pq, o_pm, o_prow, o_cand,
       o_eph, o_tab, o_ent, o_pr2, o_pcode;
@@ -208,7 +208,11 @@ __device__ __forceinline__ void nvt_fill(NvtRng &g, int64_t upto, int64_t (*ring
 __device__ __forceinline__ int nvt_fold(double c, double h) { return c > h ? -1 : c < -h ? 1 : 0; }
 __device__ __forceinline__ double nvt_shift(double v, int f, double L) { return f < 0 ? v - L : f > 0 ? v + L : v; }
 
-// The LDS of a chain.
+template <typename T>
+using NvtGlobal = __attribute__((address_space(1))) T;
+
+// The LDS of a chain; lx to lmeta stand in device memory where the box is not
+// copied.
 struct NvtLds {
   double *lx, *ly, *lz;
   double4 *lcomd;
@@ -471,14 +475,15 @@ __device__ __forceinline__ NvtOutcome nvt_decide(const NvtChainArgs &a, const do
 // - The last wave prepares the next move while the others evaluate this one:
 //   both possible starts in the random stream (nvt_prepare_move).
 // - Each other wave owns the molecules j = w, w + NC, ...: it alone reads and
-//   commits their LDS copy.  Its lanes list the molecules in range of either
+//   commits their sites.  Its lanes list the molecules in range of either
 //   placement, walk their site pairs for both r^2, and compact the pairs
 //   within the cutoff, so that the pair terms run on full waves (4 in 10 pairs
 //   of listed molecules lie outside the cutoff).
 // - Each lane owns a k segment whose box sums stay in registers; the moving
 //   molecule's old sums are loaded before the pairs and used after them.
 // - Every wave adds up the partial sums and takes the decision itself.
-template <int PM, bool CUBIC>
+// LOCAL: the box is copied to LDS; else it stays in device memory.
+template <int PM, bool CUBIC, bool LOCAL>
 __device__ __forceinline__ void nvt_chain_run(const NvtChainArgs &a, int64_t step0, int64_t nsteps) {
   __shared__ NvtCand cand[3][2];
   __shared__ int64_t ring[kNvtRing][5];
@@ -487,12 +492,22 @@ __device__ __forceinline__ void nvt_chain_run(const NvtChainArgs &a, int64_t ste
   __shared__ int redf[2][16];
   extern __shared__ char lds[];
   NvtLds S;
-  S.lx = (double *)(lds + a.o_x);
-  S.ly = (double *)(lds + a.o_y);
-  S.lz = (double *)(lds + a.o_z);
-  S.lcomd = (double4 *)(lds + a.o_comd);
-  S.lfirst = (int *)(lds + a.o_first);
-  S.lmeta = (int *)(lds + a.o_meta);
+  if (LOCAL) {
+    S.lx = (double *)(lds + a.o_x);
+    S.ly = (double *)(lds + a.o_y);
+    S.lz = (double *)(lds + a.o_z);
+    S.lcomd = (double4 *)(lds + a.o_comd);
+    S.lfirst = (int *)(lds + a.o_first);
+    S.lmeta = (int *)(lds + a.o_meta);
+  } else {
+    // (through the global address space, for global loads and not flat ones)
+    S.lx = (double *)(NvtGlobal<double> *)a.x;
+    S.ly = (double *)(NvtGlobal<double> *)a.y;
+    S.lz = (double *)(NvtGlobal<double> *)a.z;
+    S.lcomd = (double4 *)(NvtGlobal<double4> *)a.comd;
+    S.lfirst = (int *)(NvtGlobal<int> *)a.b.first;
+    S.lmeta = (int *)(NvtGlobal<int> *)a.meta;
+  }
   S.atype = (int *)(lds + a.o_atype);
   S.acharge = (double *)(lds + a.o_acharge);
   S.spn = (int *)(lds + a.o_spn);
@@ -508,14 +523,17 @@ __device__ __forceinline__ void nvt_chain_run(const NvtChainArgs &a, int64_t ste
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), nc = (nthr >> 6) - 1;
   const bool ahead = w == nc;  // the preparing wave
   const int n = a.n, K = a.ew.nvecs, nmols = a.b.nmols;
-  for (int i = tid; i < a.nsite; i += nthr) {
-    S.lx[i] = a.x[i];
-    S.ly[i] = a.y[i];
-    S.lz[i] = a.z[i];
-  }
+  if (LOCAL)
+    for (int i = tid; i < a.nsite; i += nthr) {
+      S.lx[i] = a.x[i];
+      S.ly[i] = a.y[i];
+      S.lz[i] = a.z[i];
+    }
   for (int i = tid; i < nmols; i += nthr) {
-    S.lcomd[i] = a.comd[i];
-    S.lfirst[i] = a.b.first[i];
+    if (LOCAL) {
+      S.lcomd[i] = a.comd[i];
+      S.lfirst[i] = a.b.first[i];
+    }
     S.lmeta[i] = (a.b.species[i] << 1) | (a.b.live[i] ? 1 : 0);
   }
   for (int i = tid; i < a.natoms_total; i += nthr) {
@@ -853,12 +871,14 @@ __device__ __forceinline__ void nvt_chain_run(const NvtChainArgs &a, int64_t ste
     }
   }
   __syncthreads();
-  for (int i = tid; i < a.nsite; i += nthr) {
-    a.x[i] = S.lx[i];
-    a.y[i] = S.ly[i];
-    a.z[i] = S.lz[i];
+  if (LOCAL) {
+    for (int i = tid; i < a.nsite; i += nthr) {
+      a.x[i] = S.lx[i];
+      a.y[i] = S.ly[i];
+      a.z[i] = S.lz[i];
+    }
+    for (int i = tid; i < nmols; i += nthr) a.comd[i] = S.lcomd[i];
   }
-  for (int i = tid; i < nmols; i += nthr) a.comd[i] = S.lcomd[i];
   if (has) {
 #pragma unroll
     for (int t = 0; t < kNvtSeg; ++t)
@@ -877,11 +897,11 @@ __device__ __forceinline__ void nvt_chain_run(const NvtChainArgs &a, int64_t ste
 // table is constant while the kernel runs, which its address space tells the
 // compiler: through a plain pointer every field would be loaded again after
 // each store.
-template <int PM, bool CUBIC>
+template <int PM, bool CUBIC, bool LOCAL>
 __global__ void __launch_bounds__(64 * kNvtWaves)
     k_nvt_chain(const NvtChainArgs *__restrict__ args, int64_t step0, int64_t nsteps) {
   typedef const __attribute__((address_space(4))) NvtChainArgs *ConstArgs;
-  nvt_chain_run<PM, CUBIC>(*(const NvtChainArgs *)((ConstArgs)args + blockIdx.x), step0, nsteps);
+  nvt_chain_run<PM, CUBIC, LOCAL>(*(const NvtChainArgs *)((ConstArgs)args + blockIdx.x), step0, nsteps);
 }
 
 }  // namespace cass
@@ -902,8 +922,9 @@ namespace {
 struct NvtLaunch {
   NvtChainArgs a;
   size_t lds = 0;
-  int pm = 0, waves = kNvtWaves;
-  bool host_loop = false;  // the box's copy exceeds the LDS: the host-driven loop runs it
+  int pm = 0;
+  bool local = true;       // the box in LDS, else in device memory
+  bool host_loop = false;  // the host-driven loop runs it
   int box = -1;
   cass_rng *rng = nullptr;
   const cass_nvt_options *opt = nullptr;
@@ -911,21 +932,26 @@ struct NvtLaunch {
   cass_nvt_record *rec = nullptr;
   bool charged = false;
   std::vector<int> mols;  // locate order of the mobile species
-  size_t o_state = 0, o_kind = 0, o_acc = 0, o_energy = 0, o_lnp = 0, o_rs = 0, o_mols = 0;
+  size_t o_state = 0, o_kind = 0, o_acc = 0, o_energy = 0, o_lnp = 0, o_rs = 0, o_mols = 0, o_meta = 0;
 };
 
 typedef void (*nvt_kernel_t)(const NvtChainArgs *, int64_t, int64_t);
 
-nvt_kernel_t nvt_kernel(int pm, bool cubic) {
-  static nvt_kernel_t const kt[3][2] = {{k_nvt_chain<0, false>, k_nvt_chain<0, true>},
-                                        {k_nvt_chain<1, false>, k_nvt_chain<1, true>},
-                                        {k_nvt_chain<2, false>, k_nvt_chain<2, true>}};
-  return kt[pm][cubic ? 1 : 0];
+template <int PM>
+nvt_kernel_t nvt_kernel(bool cubic, bool local) {
+  return cubic ? (local ? k_nvt_chain<PM, true, true> : k_nvt_chain<PM, true, false>)
+               : (local ? k_nvt_chain<PM, false, true> : k_nvt_chain<PM, false, false>);
+}
+
+nvt_kernel_t nvt_kernel(const NvtLaunch &L) {
+  const bool cubic = L.a.b.cubic;
+  return L.pm == 0 ? nvt_kernel<0>(cubic, L.local) : L.pm == 1 ? nvt_kernel<1>(cubic, L.local)
+                                                               : nvt_kernel<2>(cubic, L.local);
 }
 
 // Checks, the LDS layout of the box copy, the kernel choice and the arguments
-// of one chain but for its buffers (nvt_buffers).  nsteps == 0 or a box
-// beyond the LDS leaves L.a unset (host_loop / nothing to launch).
+// of one chain but for its buffers (nvt_buffers).  With nsteps == 0 or
+// host_loop there is nothing to launch.
 int nvt_prepare(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_options *opt, int64_t nsteps,
                 cass_energy *en, cass_nvt_record *rec, NvtLaunch &L) {
   if (!e || !rng || !opt || !en || nsteps < 0 || box < 0 || box >= (int)e->boxes.size()) return CASS_ERR_ARG;
@@ -951,31 +977,34 @@ int nvt_prepare(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_optio
   if (nm == 0) return cass_fail(e, CASS_ERR_STATE, "no molecules to move");
   if (nsteps == 0) return CASS_OK;
   HIP_TRY(e, hipSetDevice(e->device));
-  // LDS layout of the box copy and the waves' buffers.  Twelve waves hold 28
-  // KB of buffers; a box that leaves less takes fewer of them (the cost of
-  // that stands at kNvtWaves), then goes without the phase powers.
+  // LDS layout of the box copy and the waves' buffers, with the phase powers
+  // where they fit
   const int nsite = (int)(b.xyz_h.size() / 3), nt = std::max(e->ntypes, 1);
   int lds_max = 0;
   HIP_TRY(e, hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, e->device));
   NvtChainArgs &a = L.a;
   std::memset(&a, 0, sizeof(a));
+  a.nj_max = 1;
+  for (int m = 0; m < b.nmols; ++m) a.nj_max = std::max(a.nj_max, e->sp_natoms[b.mol_species[m]]);
   a.tx = std::max(2, b.kmax[0] + 1);
   a.ty = b.kmax[1] + 1;
   a.tz = b.kmax[2] + 1;
   a.nt_site = a.tx + a.ty + a.tz;
-  auto layout = [&](int waves, bool tabled) {
+  auto layout = [&](bool tabled, bool local) {
     size_t lds = 0;
     auto take = [&](size_t bytes) {
       const size_t o = lds;
       lds = (lds + bytes + 15) & ~(size_t)15;
       return (int)o;
     };
-    a.o_x = take(sizeof(double) * nsite);
-    a.o_y = take(sizeof(double) * nsite);
-    a.o_z = take(sizeof(double) * nsite);
-    a.o_comd = take(sizeof(double4) * b.nmols);
-    a.o_first = take(sizeof(int) * b.nmols);
-    a.o_meta = take(sizeof(int) * b.nmols);
+    if (local) {
+      a.o_x = take(sizeof(double) * nsite);
+      a.o_y = take(sizeof(double) * nsite);
+      a.o_z = take(sizeof(double) * nsite);
+      a.o_comd = take(sizeof(double4) * b.nmols);
+      a.o_first = take(sizeof(int) * b.nmols);
+      a.o_meta = take(sizeof(int) * b.nmols);
+    }
     a.o_atype = take(sizeof(int) * e->natoms_total);
     a.o_acharge = take(sizeof(double) * e->natoms_total);
     a.o_spn = take(sizeof(int) * e->nspecies);
@@ -987,20 +1016,39 @@ int nvt_prepare(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_optio
     a.o_cand = take(sizeof(double) * 36 * n);
     a.o_eph = take(tabled ? sizeof(cplx) * 6 * n : 0);
     a.o_tab = take(tabled ? sizeof(cplx) * 4 * n * a.nt_site : 0);
-    a.o_ent = take(sizeof(int2) * kNvtList * (waves - 1));
-    a.o_pr2 = take(sizeof(double) * kNvtList * (waves - 1));
-    a.o_pcode = take(sizeof(int) * kNvtList * (waves - 1));
+    a.o_ent = take(sizeof(int2) * kNvtList * (kNvtWaves - 1));
+    a.o_pr2 = take(sizeof(double) * kNvtList * (kNvtWaves - 1));
+    a.o_pcode = take(sizeof(int) * kNvtList * (kNvtWaves - 1));
     L.lds = lds;
-    L.waves = waves;
+    L.local = local;
     a.tabled = tabled ? 1 : 0;
     return lds + 4096 <= (size_t)lds_max;  // beside the kernel's own
   };
-  bool fits = false;
-  for (int waves = kNvtWaves; !fits && waves >= kNvtMinWaves; waves -= 2) fits = layout(waves, charged);
-  for (int waves = kNvtWaves; !fits && charged && waves >= kNvtMinWaves; waves -= 2) fits = layout(waves, false);
-  if (!fits) {
+  // A copy with the phase powers, the box in device memory with them, then
+  // both without.  In device memory a move of 512 waters takes 12.4 us for
+  // 12.0, one of 1080 (the largest copy) 24.3 for 23.2; fewer waves beside a
+  // copy are the slower choice (1130 waters: 29.0 on eight, 24.9 here; 1300
+  // without Coulomb sums: 16.9 on six, 14.9 here), so is a sine and cosine per
+  // site and vector on twelve (1.3 ms for molecules of 64 sites and 16700
+  // vectors, of which the vectors take 0.8).
+  if (!layout(charged, true) && !layout(charged, false) && !layout(false, true) && !layout(false, false)) {
     L.host_loop = true;
     return CASS_OK;
+  }
+  // One workgroup passes over all molecules and k vectors for every move; from
+  // some size on the host loop's launches over the whole chip are faster.  Both
+  // sides in us a move, from runs of 2500 to 160000 one-site molecules (9 to
+  // 245 here; 47 to 123 there), 1360 to 20000 waters without Coulomb sums (13
+  // to 38; 38 to 45) and with 6000 to 55000 vectors (27 to 256; 80 to 92), and
+  // molecules of 20 and 64 sites (104 and 690; 391 and 2500).
+  if (!L.local) {
+    const double pairs = (double)n * a.nj_max, K = charged ? b.nvecs : 0.0;
+    const double here = 8.0 + 1.35e-3 * b.nmols + 0.17 * pairs + (a.tabled ? 3.5e-3 * K : 0.75e-3 * K * n);
+    const double there = 40.0 + 0.6 * pairs + (charged ? 40.0 + 0.5e-3 * K : 0.0);
+    if (here > there) {
+      L.host_loop = true;
+      return CASS_OK;
+    }
   }
   const bool common = (b.p.vdw_style == CASS_VDW_NONE ||
                        (b.p.vdw_style == CASS_VDW_LJ &&
@@ -1032,8 +1080,6 @@ int nvt_prepare(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_optio
   a.max_rot = opt->max_rot;
   a.beta = b.p.beta;
   a.nsite = nsite;
-  a.nj_max = 1;
-  for (int mm = 0; mm < b.nmols; ++mm) a.nj_max = std::max(a.nj_max, e->sp_natoms[b.mol_species[mm]]);
   a.natoms_total = e->natoms_total;
   a.nspecies = e->nspecies;
   a.ntypes = nt;
@@ -1077,7 +1123,10 @@ int nvt_buffers(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, NvtB
   }
   B.back = off;
   for (NvtLaunch &L : Ls)
-    if (!L.host_loop) L.o_mols = take(sizeof(int) * L.mols.size());
+    if (!L.host_loop) {
+      L.o_mols = take(sizeof(int) * L.mols.size());
+      if (!L.local) L.o_meta = take(sizeof(int) * e->boxes[L.box].nmols);
+    }
   B.o_args = take(sizeof(NvtChainArgs) * std::max<size_t>(1, Ls.size()));
   B.in = off;
   B.dev = (char *)cass_scratch(e, off + 256);
@@ -1104,6 +1153,7 @@ int nvt_buffers(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, NvtB
     a.ln_pacc = rec && rec->ln_pacc ? (double *)(B.dev + L.o_lnp) : nullptr;
     a.rng_state = rec && rec->rng_state ? (int64_t *)(B.dev + L.o_rs) : nullptr;
     a.mols = (const int *)(B.dev + L.o_mols);
+    a.meta = L.local ? nullptr : (int *)(B.dev + L.o_meta);
   }
   return CASS_OK;
 }
@@ -1168,22 +1218,21 @@ extern "C" int cass_nvt_run_device_batch(cass_engine *e, int32_t nboxes, const i
   if (nsteps == 0 || nboxes == 0) return CASS_OK;
   NvtBuffers B;
   if ((rc = nvt_buffers(e, Ls, nsteps, B))) return rc;
-  // the chains grouped by kernel and workgroup size; every group is one launch
-  // per chunk of moves, one workgroup per box.  The argument table holds the
-  // groups one after another.
+  // the chains grouped by kernel; every group is one launch per chunk of
+  // moves, one workgroup per box.  The argument table holds the groups one
+  // after another.
   struct Group {
     nvt_kernel_t kern;
     size_t lds, first, count;
-    int waves;
   };
   std::vector<Group> groups;
   std::vector<NvtChainArgs> args;
   std::vector<int> done(nboxes, 0);
   for (int g = 0; g < nboxes; ++g) {
     if (done[g] || Ls[g].host_loop) continue;
-    Group grp{nvt_kernel(Ls[g].pm, Ls[g].a.b.cubic), 0, args.size(), 0, Ls[g].waves};
+    Group grp{nvt_kernel(Ls[g]), 0, args.size(), 0};
     for (int k = g; k < nboxes; ++k)
-      if (!done[k] && !Ls[k].host_loop && nvt_kernel(Ls[k].pm, Ls[k].a.b.cubic) == grp.kern && Ls[k].waves == grp.waves) {
+      if (!done[k] && !Ls[k].host_loop && nvt_kernel(Ls[k]) == grp.kern) {
         args.push_back(Ls[k].a);
         grp.lds = std::max(grp.lds, Ls[k].lds);
         ++grp.count;
@@ -1197,7 +1246,7 @@ extern "C" int cass_nvt_run_device_batch(cass_engine *e, int32_t nboxes, const i
   for (const Group &g : groups) {
     HIP_TRY(e, hipFuncSetAttribute((const void *)g.kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)g.lds));
     for (int64_t s0 = 0; s0 < nsteps; s0 += kNvtChunk) {
-      hipLaunchKernelGGL(g.kern, dim3((unsigned)g.count), dim3(64 * g.waves), g.lds, e->stream, d_args + g.first, s0,
+      hipLaunchKernelGGL(g.kern, dim3((unsigned)g.count), dim3(64 * kNvtWaves), g.lds, e->stream, d_args + g.first, s0,
                          std::min(kNvtChunk, nsteps - s0));
       HIP_TRY(e, hipGetLastError());
     }

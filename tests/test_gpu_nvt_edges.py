@@ -2,7 +2,7 @@
 one and two molecules (the next move takes the molecule just moved), molecule
 pairs of more than 64 site pairs, species of unlike site counts, k vectors
 beyond the lanes' registers, phases without tables, orthogonal boxes, a style
-without its own pair arithmetic, a box on fewer waves."""
+without its own pair arithmetic, boxes beyond the LDS copy."""
 import numpy as np
 import pytest
 
@@ -21,6 +21,16 @@ def _chain(n, q):
     return S.Species("chain", atoms, xyz)
 
 
+def _lattice(sp, n, box):
+    """n molecules, each along x, in cells as long as a molecule and 2.6 A"""
+    x = sp.ref_coords - sp.ref_coords.mean(0)
+    nx = max(1, min(int(np.ceil(n ** (1 / 3))), int(box[0] // (np.ptp(x[:, 0]) + 2.6))))
+    m = int(np.ceil(np.sqrt(n / nx)))
+    cell = np.stack(np.meshgrid(np.arange(nx), np.arange(m), np.arange(m), indexing="ij"), -1).reshape(-1, 3)[:n]
+    box = np.array(box)
+    return ((cell + 0.5) / [nx, m, m] * box - 0.5 * box)[:, None, :] + x
+
+
 def _system(case):
     w = S.species_spce()
     if case == "lj2000":
@@ -34,17 +44,31 @@ def _system(case):
         "mixture": ([w, S.species_methane(), _chain(11, 0.2)], [33, 20, 4], [24.0] * 3, 9.0, "ewald"),
         "sites9": ([_chain(9, 0.15)], [25], [30.0] * 3, 10.0, "ewald"),
         "sites64": ([_chain(64, 0.1)], [2], [76.0] * 3, 9.0, "ewald"),
+        # the copy and the waves' buffers take 156.6 kB of the 159.7 for 2000
+        # one-site molecules and 161.7 for 2080; 164.9 for 1130 waters with the
+        # phase powers, 156.0 without; 180.9 for 80 of 64 sites; the phase
+        # powers alone 140 for 40 sites
+        "memory": ([S.species_lj()], [2080], [46.0] * 3, 9.0, "none"),
+        "memory_k": ([w], [1130], [32.3] * 3, 9.0, "ewald"),
+        "memory_dsf": ([w], [1400], [36.0] * 3, 9.0, "dsf"),
+        "memory_orthogonal": ([w], [1130], [30.0, 34.0, 33.0], 9.0, "ewald"),
+        "memory_sites64": ([_chain(64, 0.1)], [80], [110.0] * 3, 10.0, "cut"),
+        "memory_sites40": ([_chain(40, 0.1)], [150], [90.0] * 3, 20.0, "ewald"),
     }[case]
-    coords = S.place_random(list(zip(species, counts)), box, 5, 1.2, 2.6)
+    coords = ([_lattice(species[0], counts[0], box)] if case.startswith("memory") else
+              S.place_random(list(zip(species, counts)), box, 5, 1.2, 2.6))
     return S.System(species, counts, coords, np.array(box), 350.0, "lj", "cut_tail", rc, charge_style=style,
                     rcut_coul=rc, alpha_dsf=0.2 if style == "dsf" else None, rcut_low=0.85,
-                    box_shape="orthogonal" if case == "orthogonal" else "cubic", prob_translate=0.5, max_disp=0.4,
-                    max_rot=25.0, seed=(101, 203), name=case).parsed()
+                    box_shape="orthogonal" if case.endswith("orthogonal") else "cubic", max_disp=0.4,
+                    # (a site's own rotation changes its energy by rounding alone)
+                    prob_translate=1.0 if species[0].natoms == 1 else 0.5, max_rot=25.0, seed=(101, 203), name=case).parsed()
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("prec", [E.FP64, E.MIXED], ids=["fp64", "mixed"])
-@pytest.mark.parametrize("case", ["one", "two", "dsf", "orthogonal", "many_k", "mixture", "sites9", "sites64", "lj2000"])
+@pytest.mark.parametrize("case", ["one", "two", "dsf", "orthogonal", "many_k", "mixture", "sites9", "sites64", "lj2000",
+                                  "memory", "memory_k", "memory_dsf", "memory_orthogonal", "memory_sites64",
+                                  "memory_sites40"])
 def test_nvt_chain_equals_host_loop(case, prec):
     print(f"[gpu] nvt chain edges {case} {prec}", flush=True)
     system, steps = _system(case), 120
@@ -69,3 +93,33 @@ def test_nvt_chain_equals_host_loop(case, prec):
     assert np.max(np.abs(xa - xb)) < 1e-9
     # the running sums of the chain against a fresh evaluation of its end state
     assert abs(a["final"]["total"] - ta["total"]) <= tol * max(1.0, abs(ta["total"]))
+
+
+@pytest.mark.gpu
+def test_nvt_batch_over_all_paths():
+    """a box copied to LDS, one in device memory and one for the host loop in
+    one batch, each as in a run of its own"""
+    print("[gpu] nvt batch over all paths", flush=True)
+    sp, steps = S.species_lj(), 40
+    systems = [S.System([sp], [n], [_lattice(sp, n, [L] * 3)], np.array([L] * 3), 150.0, "lj", "cut_tail", 9.0,
+                        rcut_low=0.85, prob_translate=1.0, max_disp=0.4, seed=(7, 9 + n), name="lj").parsed()
+               for n, L in ((100, 22.0), (40000, 130.0), (2400, 50.0))]
+
+    def run(batch):
+        eng = E.Engine(systems[0], max_boxes=3, precision=E.FP64)
+        boxes = [eng.add_box(s) for s in systems]
+        e0 = eng.total_energy_batch(boxes)
+        rngs = [E.rng(*s.seed) for s in systems]
+        if batch:
+            out = eng.nvt_run_batch(boxes, rngs, steps, e0)
+        else:
+            out = [b.nvt_run(r, steps, e, device=True) for b, r, e in zip(boxes, rngs, e0)]
+        got = [(o, b.download(), list(r.s)) for o, b, r in zip(out, boxes, rngs)]
+        eng.close()
+        return got
+
+    for (a, xa, ra), (b, xb, rb) in zip(run(True), run(False)):
+        for k in ("kind", "accepted", "energy", "rng"):
+            assert np.array_equal(a[k], b[k]), k
+        assert np.array_equal(xa, xb) and ra == rb and a["final"] == b["final"]
+        assert 0 < a["accepted"].sum()
