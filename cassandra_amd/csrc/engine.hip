@@ -167,6 +167,22 @@ static bool species_charged(const cass_engine *e, int s) {
   return false;
 }
 
+// Workgroups that share one molecule's structure-factor sums in
+// ewald_mol_block: one where the molecules of the call alone fill the chip, else
+// as many as bring them to 512, and at most one per 256 segments.  With one
+// each, 4 waters and 56000 vectors took 100 us a call (31 shared), 128 took 130
+// (81); 512 waters take the same 53 us either way.
+static int ewald_parts(const cass_box_state &b, int call_mols) {
+  return std::max(1, std::min((b.nsegs + kMaxBlock - 1) / kMaxBlock, 512 / std::max(1, call_mols)));
+}
+
+// Whether a box has molecules of the two ways to take those sums.
+static void ewald_ways(const cass_engine *e, const cass_box_state &b, const EwaldDev &ew, bool &tabled, bool &direct) {
+  tabled = direct = false;
+  for (int m = 0; m < b.nmols; ++m)
+    (ewald_direct(ew, b.nmols, e->sp_natoms[b.mol_species[m]]) ? direct : tabled) = true;
+}
+
 // ------------------------------------------------------------------ setup
 static int noalloc_init(cass_engine *e);
 
@@ -1135,8 +1151,12 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
     }
   const int blk = kMaxBlock;
   std::vector<RecomputeBox> rb(nboxes);
-  std::vector<int2> items, kitems_mol, kitems_box;
+  std::vector<int2> items, kitems_box;
+  std::vector<int4> kitems_mol, kitems_direct;
   int64_t np = 0, nk = 0;
+  int kmols = 0;  // molecules of the Ewald boxes
+  for (int i = 0; i < nboxes; ++i)
+    if (bs[i]->p.charge_style == CASS_Q_EWALD) kmols += bs[i]->nmols;
   for (int i = 0; i < nboxes; ++i) {
     const cass_box_state &b = *bs[i];
     RecomputeBox &r = rb[i];
@@ -1148,11 +1168,16 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
     np += std::max(1, b.nmols);
     const bool ewald = b.p.charge_style == CASS_Q_EWALD;
     r.ew = ewald ? ewald_view(b, row_k0_of(b)) : EwaldDev{};
-    r.kblk = ewald ? std::max(1, (b.nvecs + kBoxVecs - 1) / kBoxVecs) : 0;
+    r.kblk = ewald ? box_blocks(b.nvecs, b.nmols) : 0;
+    r.kparts = ewald ? ewald_parts(b, kmols) : 1;
     r.kpart_off = nk;
     if (ewald) {
       if (b.nvecs > 0)
-        for (int m = 0; m < b.nmols; ++m) kitems_mol.push_back(make_int2(i, m));
+        for (int m = 0; m < b.nmols; ++m) {
+          const bool direct = ewald_direct(r.ew, b.nmols, e->sp_natoms[b.mol_species[m]]);
+          const int parts = direct ? (b.nvecs + blk - 1) / blk : r.kparts;
+          for (int k = 0; k < parts; ++k) (direct ? kitems_direct : kitems_mol).push_back(make_int4(i, m, k, 0));
+        }
       for (int kb = 0; kb < r.kblk; ++kb) kitems_box.push_back(make_int2(i, kb));
       nk += r.kblk;
     }
@@ -1166,7 +1191,8 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
   };
   const size_t o_rb = take(sizeof(RecomputeBox) * std::max(1, nboxes)),
                o_it = take(sizeof(int2) * std::max<size_t>(1, items.size())),
-               o_km = take(sizeof(int2) * std::max<size_t>(1, kitems_mol.size())),
+               o_km = take(sizeof(int4) * std::max<size_t>(1, kitems_mol.size())),
+               o_kd = take(sizeof(int4) * std::max<size_t>(1, kitems_direct.size())),
                o_kb = take(sizeof(int2) * std::max<size_t>(1, kitems_box.size())),
                o_part = take(2 * sizeof(double) * std::max<int64_t>(1, np)),
                o_pov = take(sizeof(int) * std::max<int64_t>(1, np)),
@@ -1178,8 +1204,11 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
   if (!items.empty())
     HIP_TRY(e, hipMemcpyAsync(s + o_it, items.data(), sizeof(int2) * items.size(), hipMemcpyHostToDevice, e->stream));
   if (!kitems_mol.empty())
-    HIP_TRY(e, hipMemcpyAsync(s + o_km, kitems_mol.data(), sizeof(int2) * kitems_mol.size(), hipMemcpyHostToDevice,
+    HIP_TRY(e, hipMemcpyAsync(s + o_km, kitems_mol.data(), sizeof(int4) * kitems_mol.size(), hipMemcpyHostToDevice,
                               e->stream));
+  if (!kitems_direct.empty())
+    HIP_TRY(e, hipMemcpyAsync(s + o_kd, kitems_direct.data(), sizeof(int4) * kitems_direct.size(),
+                              hipMemcpyHostToDevice, e->stream));
   if (!kitems_box.empty())
     HIP_TRY(e, hipMemcpyAsync(s + o_kb, kitems_box.data(), sizeof(int2) * kitems_box.size(), hipMemcpyHostToDevice,
                               e->stream));
@@ -1198,7 +1227,12 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
   }
   if (!kitems_mol.empty()) {
     hipLaunchKernelGGL(k_ewald_mol_multi, dim3((unsigned)kitems_mol.size()), dim3(blk), 0, e->stream, d_rb, tv,
-                       (const int2 *)(s + o_km));
+                       (const int4 *)(s + o_km));
+    HIP_TRY(e, hipGetLastError());
+  }
+  if (!kitems_direct.empty()) {
+    hipLaunchKernelGGL(k_ewald_direct_multi, dim3((unsigned)kitems_direct.size()), dim3(blk), 0, e->stream, d_rb, tv,
+                       (const int4 *)(s + o_kd));
     HIP_TRY(e, hipGetLastError());
   }
   if (!kitems_box.empty()) {
@@ -1411,10 +1445,17 @@ extern "C" int cass_ewald_full(cass_engine *e, int32_t box, double *e_recip) {
   TopoDev tv = topo_view(e);
   EwaldDev ew = ewald_view(*b, row_k0_of(*b));
   if (b->nmols > 0 && K > 0) {
-    hipLaunchKernelGGL(k_ewald_mol, dim3(b->nmols), dim3(kMaxBlock), 0, e->stream, bv, tv, ew);
+    bool tabled, direct;
+    ewald_ways(e, *b, ew, tabled, direct);
+    if (tabled)
+      hipLaunchKernelGGL(k_ewald_mol, dim3(b->nmols, ewald_parts(*b, b->nmols)), dim3(kMaxBlock), 0, e->stream, bv,
+                         tv, ew);
+    if (direct)
+      hipLaunchKernelGGL(k_ewald_direct, dim3((K + kMaxBlock - 1) / kMaxBlock, b->nmols), dim3(kMaxBlock), 0,
+                         e->stream, bv, tv, ew);
     HIP_TRY(e, hipGetLastError());
   }
-  const int nb = std::max(1, (K + kBoxVecs - 1) / kBoxVecs);
+  const int nb = box_blocks(K, b->nmols);
   double *part = (double *)cass_scratch(e, sizeof(double) * (nb + 1));
   if (!part) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
   hipLaunchKernelGGL(k_ewald_box, dim3(nb), dim3(kMaxBlock), 0, e->stream, bv, ew, part);

@@ -332,7 +332,7 @@ struct RecomputeBox {
   PairConst<double> cd;
   PairConst<float> cf;
   EwaldDev ew;
-  int kblk;
+  int kblk, kparts;
   int64_t part_off, kpart_off;
 };
 
@@ -355,8 +355,21 @@ __host__ __device__ inline cplx cpow_int(cplx e, int n) {
 }
 
 constexpr int kPairMols = 4;   // molecules per workgroup of the total pair sums, one wave each
-constexpr int kBoxVecs = 64;   // k vectors per workgroup of the box sums
+constexpr int kBoxVecs = 64;   // k vectors per workgroup of the box sums,
+constexpr int kBoxShare = 16;  // where a box has at least this many molecules, else kMaxBlock
+inline int box_blocks(int nvecs, int nmols) {
+  const int vecs = nmols >= kBoxShare ? kBoxVecs : kMaxBlock;
+  return nvecs > vecs ? (nvecs + vecs - 1) / vecs : 1;
+}
 constexpr int kEwTab = 1024;   // phase powers held per molecule
+// Whether a molecule of n sites takes a sine and cosine per site and k vector
+// in the total energy's structure factors: its powers exceed the table, or the
+// box has so few molecules that building the tables is what a call waits for
+// (one water and 56000 vectors: the call takes 30.3 us by the table, 28.3
+// without; four: 31.3 and 32.1).
+__host__ __device__ inline bool ewald_direct(const EwaldDev &ew, int nmols, int n) {
+  return nmols <= 2 || n * (ew.tx + ew.ty + ew.tz) > kEwTab;
+}
 
 // kernels (kernels.hip)
 template <typename P>
@@ -369,11 +382,13 @@ template <typename P>
 __global__ void k_total_pairs(BoxDev b, TopoDev tp, PairConst<double> cd, PairConst<float> cf, double *part,
                               int *part_ov);
 __global__ void k_ewald_mol(BoxDev b, TopoDev tp, EwaldDev ew);
+__global__ void k_ewald_direct(BoxDev b, TopoDev tp, EwaldDev ew);
 __global__ void k_ewald_box(BoxDev b, EwaldDev ew, double *part);
 template <typename P>
 __global__ void k_total_pairs_multi(const RecomputeBox *boxes, TopoDev tp, const int2 *items, double *part,
                                     int *part_ov);
-__global__ void k_ewald_mol_multi(const RecomputeBox *boxes, TopoDev tp, const int2 *items);
+__global__ void k_ewald_mol_multi(const RecomputeBox *boxes, TopoDev tp, const int4 *items);
+__global__ void k_ewald_direct_multi(const RecomputeBox *boxes, TopoDev tp, const int4 *items);
 __global__ void k_ewald_box_multi(const RecomputeBox *boxes, const int2 *items, double *kpart);
 __global__ void k_sum_multi(const RecomputeBox *boxes, const double *kpart, double *out);
 __global__ void k_ewald_move(TopoDev tp, EwaldDev ew, int m, int species, int flag, int n, const double *nxyz,

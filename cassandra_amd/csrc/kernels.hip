@@ -238,39 +238,24 @@ __global__ void __launch_bounds__(64 * kPairMols)
 
 // ----------------------------------------------------------------- Ewald
 // Compute_System_Ewald_Reciprocal_Energy (energy_routines.f90:4111-4231),
-// stage 1: the sums of one molecule over all k vectors, one workgroup.  The
-// powers of the sites' unit phases stand in LDS (2 pi as the reference
-// truncates it), a lane takes a segment of consecutive n_x, and each wave
-// passes its segments' sums through LDS to store them in k order: 24 boxes of
-// 512 waters took 0.32 ms with a sine and cosine per site and vector, 0.13
-// here, for 0.46 GB of stores.  Molecules whose powers exceed the table keep
-// the sine and cosine.
-__device__ inline void ewald_mol_block(const BoxDev &b, const TopoDev &tp, const EwaldDev &ew, int m) {
+// stage 1: the sums of one molecule over the k vectors, `parts` workgroups
+// sharing them.  The powers of the sites' unit phases stand in LDS (2 pi as the
+// reference truncates it), a lane takes a segment of consecutive n_x, and each
+// wave passes its segments' sums through LDS to store them in k order: 24 boxes
+// of 512 waters took 0.32 ms with a sine and cosine per site and vector, 0.13
+// here, for 0.46 GB of stores.
+__device__ inline void ewald_mol_block(const BoxDev &b, const TopoDev &tp, const EwaldDev &ew, int m, int part,
+                                       int parts) {
   __shared__ cplx tab[kEwTab];
   __shared__ cplx eph[3 * kMaxSites];
   __shared__ double out[kMaxBlock / 64][64 * kKSeg];
-  const int tid = threadIdx.x, lane = tid & 63, K = ew.nvecs;
-  double *cm = ew.cmol + (size_t)m * K, *sm = ew.smol + (size_t)m * K;
-  if (!b.live[m]) {
-    for (int k = tid; k < K; k += blockDim.x) cm[k] = sm[k] = 0.0;
-    return;
-  }
+  const int tid = threadIdx.x, lane = tid & 63;
   const int sp = b.species[m], f = b.first[m];
   const int n = tp.sp_natoms[sp], o = tp.sp_atom_off[sp], nt = ew.tx + ew.ty + ew.tz;
-  if (n > kMaxSites || n * nt > kEwTab) {
-    for (int k = tid; k < K; k += blockDim.x) {
-      const double hx = ew.hx[k], hy = ew.hy[k], hz = ew.hz[k];
-      double c = 0.0, s = 0.0;
-      for (int a = 0; a < n; ++a) {
-        const double q = tp.atom_charge[o + a];
-        double sv, cv;
-        sincos(hx * b.x[f + a] + hy * b.y[f + a] + hz * b.z[f + a], &sv, &cv);
-        c = c + q * cv;
-        s = s + q * sv;
-      }
-      cm[k] = c;
-      sm[k] = s;
-    }
+  if (ewald_direct(ew, b.nmols, n)) return;  // ewald_direct_block takes it
+  double *cm = ew.cmol + (size_t)m * ew.nvecs, *sm = ew.smol + (size_t)m * ew.nvecs;
+  if (!b.live[m]) {
+    for (int k = part * blockDim.x + tid; k < ew.nvecs; k += parts * blockDim.x) cm[k] = sm[k] = 0.0;
     return;
   }
   for (int t = tid; t < 3 * n; t += blockDim.x) {
@@ -286,7 +271,7 @@ __device__ inline void ewald_mol_block(const BoxDev &b, const TopoDev &tp, const
   }
   __syncthreads();
   double *buf = out[tid >> 6];
-  for (int s0 = tid - lane; s0 < ew.nsegs; s0 += blockDim.x) {  // wave-uniform
+  for (int s0 = part * blockDim.x + tid - lane; s0 < ew.nsegs; s0 += parts * blockDim.x) {  // wave-uniform
     const int4 sg = ew.segs[min(s0 + lane, ew.nsegs - 1)];
     const int k0 = sg.x & 0xfffff, len = sg.x >> 20;
     const int ny = sg.z < 0 ? -sg.z : sg.z, nz = sg.w < 0 ? -sg.w : sg.w;
@@ -330,20 +315,53 @@ __device__ inline void ewald_mol_block(const BoxDev &b, const TopoDev &tp, const
   }
 }
 
-// grid nmols
+// The same by a sine and cosine per site and vector (ewald_direct), a vector
+// per lane.
+__device__ inline void ewald_direct_block(const BoxDev &b, const TopoDev &tp, const EwaldDev &ew, int m, int kb) {
+  const int k = kb * blockDim.x + threadIdx.x;
+  const int sp = b.species[m], f = b.first[m];
+  const int n = tp.sp_natoms[sp], o = tp.sp_atom_off[sp];
+  if (k >= ew.nvecs || !ewald_direct(ew, b.nmols, n)) return;
+  double c = 0.0, s = 0.0;
+  if (b.live[m]) {
+    const double hx = ew.hx[k], hy = ew.hy[k], hz = ew.hz[k];
+    for (int a = 0; a < n; ++a) {
+      const double hr = hx * b.x[f + a] + hy * b.y[f + a] + hz * b.z[f + a];
+      const double q = tp.atom_charge[o + a];
+      double sv, cv;
+      sincos(hr, &sv, &cv);
+      c = c + q * cv;
+      s = s + q * sv;
+    }
+  }
+  ew.cmol[(size_t)m * ew.nvecs + k] = c;
+  ew.smol[(size_t)m * ew.nvecs + k] = s;
+}
+
+// grid (nmols, parts)
 __global__ void __launch_bounds__(kMaxBlock) k_ewald_mol(BoxDev b, TopoDev tp, EwaldDev ew) {
-  ewald_mol_block(b, tp, ew, blockIdx.x);
+  ewald_mol_block(b, tp, ew, blockIdx.x, blockIdx.y, gridDim.y);
+}
+
+// grid (ceil(K / block), nmols)
+__global__ void k_ewald_direct(BoxDev b, TopoDev tp, EwaldDev ew) {
+  ewald_direct_block(b, tp, ew, blockIdx.y, blockIdx.x);
 }
 
 // stage 2: the box sums over molecules (zero for dead ones) and the energy
-// term of kBoxVecs k vectors, written to part[kb].  The molecules are shared
-// by the workgroup's waves and read several at a time: one lane per vector
-// over all molecules was a chain of 512 loads on a tenth of the chip (24 boxes
-// of 512 waters: 0.60 ms, 0.13 here).
+// term of a block of k vectors (box_vecs), written to part[kb].  The molecules
+// are shared by the workgroup's waves and read several at a time: one lane per
+// vector over all molecules was a chain of 512 loads on a tenth of the chip (24
+// boxes of 512 waters: 0.60 ms, 0.13 here).  Few molecules are not shared: a
+// block of 64 vectors leaves four times the partials to add up (one water and
+// 56000 vectors: the call 31.3 us shared, 30.3 not; 15 waters not shared 43.0,
+// 16 shared 41.4).
 __device__ inline void ewald_box_block(const BoxDev &b, const EwaldDev &ew, int kb, double *part) {
   __shared__ double sh[2][kMaxBlock / 64][kBoxVecs];
-  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6, G = blockDim.x >> 6;
-  const int k = kb * kBoxVecs + lane;
+  const bool shared = b.nmols >= kBoxShare;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = shared ? wave : 0, G = shared ? blockDim.x >> 6 : 1;
+  const int k = shared ? kb * kBoxVecs + lane : kb * (int)blockDim.x + (int)threadIdx.x;
   double v[1] = {0.0};
   int f = 0;
   double c[4] = {0.0, 0.0, 0.0, 0.0}, s[4] = {0.0, 0.0, 0.0, 0.0};
@@ -363,15 +381,18 @@ __device__ inline void ewald_box_block(const BoxDev &b, const EwaldDev &ew, int 
       s[0] = s[0] + ew.smol[o];
     }
   }
-  sh[0][g][lane] = (c[0] + c[1]) + (c[2] + c[3]);
-  sh[1][g][lane] = (s[0] + s[1]) + (s[2] + s[3]);
-  __syncthreads();
-  if (g == 0 && k < ew.nvecs) {
-    double ct = 0.0, st = 0.0;
+  double ct = (c[0] + c[1]) + (c[2] + c[3]), st = (s[0] + s[1]) + (s[2] + s[3]);
+  if (shared) {
+    sh[0][wave][lane] = ct;
+    sh[1][wave][lane] = st;
+    __syncthreads();
+    ct = st = 0.0;
     for (int u = 0; u < G; ++u) {
       ct = ct + sh[0][u][lane];
       st = st + sh[1][u][lane];
     }
+  }
+  if (g == 0 && k < ew.nvecs) {
     ew.cs[k] = ct;
     ew.sn[k] = st;
     v[0] = ew.cn[k] * (ct * ct + st * st);
@@ -382,13 +403,21 @@ __device__ inline void ewald_box_block(const BoxDev &b, const EwaldDev &ew, int 
 
 __global__ void k_ewald_box(BoxDev b, EwaldDev ew, double *part) { ewald_box_block(b, ew, blockIdx.x, part); }
 
-// The two stages over many boxes: items (box, molecule) and (box, k block); a
-// box's k-block terms start at kpart_off in kpart.
+// The two stages over many boxes: items (box, molecule, part), (box, molecule,
+// k block) and (box, k block); a box's k-block terms start at kpart_off in
+// kpart.
 __global__ void __launch_bounds__(kMaxBlock)
-    k_ewald_mol_multi(const RecomputeBox *__restrict__ boxes, TopoDev tp, const int2 *__restrict__ items) {
-  const int2 it = items[blockIdx.x];
+    k_ewald_mol_multi(const RecomputeBox *__restrict__ boxes, TopoDev tp, const int4 *__restrict__ items) {
+  const int4 it = items[blockIdx.x];
   const RecomputeBox &r = boxes[it.x];
-  ewald_mol_block(r.b, tp, r.ew, it.y);
+  ewald_mol_block(r.b, tp, r.ew, it.y, it.z, r.kparts);
+}
+
+__global__ void k_ewald_direct_multi(const RecomputeBox *__restrict__ boxes, TopoDev tp,
+                                     const int4 *__restrict__ items) {
+  const int4 it = items[blockIdx.x];
+  const RecomputeBox &r = boxes[it.x];
+  ewald_direct_block(r.b, tp, r.ew, it.y, it.z);
 }
 
 __global__ void k_ewald_box_multi(const RecomputeBox *__restrict__ boxes, const int2 *__restrict__ items,

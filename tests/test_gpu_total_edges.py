@@ -1,6 +1,7 @@
 """The pair and structure-factor kernels of the total energy at their edges:
 molecule counts around a workgroup's four and a wave's 64, one site to 40 (the
-phase table is exceeded), unlike species, unlike edges, dead molecules.  Pair
+phase table is exceeded), few molecules whose k vectors several workgroups
+share, unlike species, unlike edges, dead molecules.  Pair
 terms against half the sum of the molecules' own energies, the reciprocal term
 against numpy's direct sum, one box and a batch."""
 import numpy as np
@@ -21,6 +22,7 @@ def _species(n, q):
 
 CASES = {
     "one": ([1], [1], [18.0] * 3), "five": ([3], [5], [18.0] * 3), "wave": ([2], [65], [22.0] * 3),
+    "shared_k": ([3], [2], [44.0] * 3),
     "mixture": ([4, 1, 7], [12, 31, 6], [19.0, 26.0, 23.0]), "long": ([40, 2], [3, 6], [46.0] * 3),
 }
 
