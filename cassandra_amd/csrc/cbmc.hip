@@ -807,6 +807,10 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
   }
   const size_t o_args = take(sizeof(GcmcBoxArgs) * nboxes);
   if (off > state_bytes) return cass_fail(e, CASS_ERR_STATE, "GCMC state layout exceeds its buffer");
+  MirrorPull mirrors;
+  std::vector<int> ids(commit ? nboxes : 0);
+  for (size_t i = 0; i < ids.size(); ++i) ids[i] = boxes[i].box;
+  if (int mrc = mirrors.reserve(e, ids, true, off)) return mrc;
   std::memcpy(host.data() + o_args, args.data(), sizeof(GcmcBoxArgs) * nboxes);
   HIP_TRY(e, hipMemcpyAsync(s0, host.data(), off, hipMemcpyHostToDevice, e->stream));
   HIP_TRY(e, hipEventRecord(e->ev0, e->stream));
@@ -826,10 +830,7 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
   HIP_TRY(e, hipEventRecord(e->ev1, e->stream));
   // the states and, unless this is a timing run, coordinates, live flags and
   // centres of every box come back behind one synchronisation
-  MirrorPull mirrors;
-  std::vector<int> ids(commit ? nboxes : 0);
-  for (size_t i = 0; i < ids.size(); ++i) ids[i] = boxes[i].box;
-  if (int mrc = mirrors.begin(e, ids, true, off)) return mrc;
+  if (int mrc = mirrors.queue(e)) return mrc;
   HIP_TRY(e, hipMemcpyAsync(mirrors.host, s0, off, hipMemcpyDeviceToHost, e->stream));
   HIP_TRY(e, hipStreamSynchronize(e->stream));
   float ms = 0.f;
@@ -970,6 +971,10 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
   }
   const size_t o_args = take(sizeof(RegrowBoxArgs) * nboxes);
   if (off > state_bytes) return cass_fail(e, CASS_ERR_STATE, "regrowth state layout exceeds its buffer");
+  MirrorPull mirrors;
+  std::vector<int> ids(nboxes);
+  for (int i = 0; i < nboxes; ++i) ids[i] = boxes[i].box;
+  if (int mrc = mirrors.reserve(e, ids, false, off)) return mrc;
   std::memcpy(host.data() + o_args, args.data(), sizeof(RegrowBoxArgs) * nboxes);
   HIP_TRY(e, hipMemcpyAsync(s0, host.data(), off, hipMemcpyHostToDevice, e->stream));
   HIP_TRY(e, hipEventRecord(e->ev0, e->stream));
@@ -979,10 +984,7 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
                               1, "k_regrow_chain launch");
   if (rc) return rc;
   HIP_TRY(e, hipEventRecord(e->ev1, e->stream));
-  MirrorPull mirrors;
-  std::vector<int> ids(nboxes);
-  for (int i = 0; i < nboxes; ++i) ids[i] = boxes[i].box;
-  if (int mrc = mirrors.begin(e, ids, false, off)) return mrc;
+  if (int mrc = mirrors.queue(e)) return mrc;
   HIP_TRY(e, hipMemcpyAsync(mirrors.host, s0, off, hipMemcpyDeviceToHost, e->stream));
   HIP_TRY(e, hipStreamSynchronize(e->stream));
   mirrors.end(e);

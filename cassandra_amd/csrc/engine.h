@@ -120,6 +120,7 @@ struct cass_engine {
   size_t scratch_bytes = 0;
   void *pinned = nullptr;
   size_t pinned_bytes = 0;
+  size_t pinned_limit = ~(size_t)0;  // a request beyond it fails (cass_test_pinned_limit)
   void *io = nullptr;               // device input/output staging of the small calls
   hipEvent_t ev0 = nullptr, ev1 = nullptr;  // brackets the last batched kernel
   double last_kernel_ms = 0.0;
@@ -142,14 +143,16 @@ void *cass_scratch(cass_engine *e, size_t bytes);
 void *cass_pinned(cass_engine *e, size_t bytes);
 void *cass_io(cass_engine *e, size_t bytes);
 void cass_cbmc_release(cass_engine *e);
-// Host mirrors of boxes that a chain kernel moved.  begin() queues the packing
-// of every box's coordinates (x, y, z together), centres and, with live, live
-// flags into one buffer and its copy to pinned staging; the first `extra`
-// bytes of that staging are the caller's.  end(), after the caller has
-// synchronised the stream, takes them into the mirrors.
+// Host mirrors of boxes that a chain kernel moves.  reserve(), before anything
+// is launched, obtains the staging, so that a lack of memory leaves the boxes
+// untouched; the first `extra` bytes of it are the caller's.  queue(), after
+// the launches, packs every box's coordinates (x, y, z together), centres and,
+// with live, live flags into one buffer and copies that to the staging; end(),
+// after the caller has synchronised the stream, takes them into the mirrors.
 struct MirrorPull {
   char *host = nullptr;  // the pinned staging
-  int begin(cass_engine *e, const std::vector<int> &ids, bool live, size_t extra);
+  int reserve(cass_engine *e, const std::vector<int> &ids, bool live, size_t extra);
+  int queue(cass_engine *e);
   void end(cass_engine *e);
 
  private:
@@ -159,6 +162,8 @@ struct MirrorPull {
   };
   std::vector<Part> parts;
   bool with_live = false;
+  size_t base = 0, bytes = 0;  // the caller's bytes; the packed ones
+  char *dev = nullptr;
 };
 bool cass_cbmc_bonded_host(const cass_engine *e, int s, const double *xyz, double *angle, double *dihedral);
 double4 cass_host_com(const cass_engine *e, int s, const double *xyz);  // Get_COM and max_dcom of one molecule  // device copies of the CBMC growth descriptions

@@ -38,7 +38,11 @@ void *cass_scratch(cass_engine *e, size_t bytes) {
   return e->scratch;
 }
 
+// For tests of a failed allocation: pinned staging beyond `bytes` is refused.
+extern "C" void cass_test_pinned_limit(cass_engine *e, size_t bytes) { e->pinned_limit = bytes; }
+
 void *cass_pinned(cass_engine *e, size_t bytes) {
+  if (bytes > e->pinned_limit) return nullptr;
   if (bytes <= e->pinned_bytes) return e->pinned;
   if (e->pinned) {
     (void)hipStreamSynchronize(e->stream);
@@ -747,50 +751,56 @@ static __global__ void __launch_bounds__(256) k_pack_mirrors(const MirrorBox *__
   }
 }
 
-int MirrorPull::begin(cass_engine *e, const std::vector<int> &ids, bool live, size_t extra) {
+int MirrorPull::reserve(cass_engine *e, const std::vector<int> &ids, bool live, size_t extra) {
   auto up = [](size_t n) { return (n + 255) & ~size_t(255); };
-  const size_t base = up(extra);
-  std::vector<MirrorBox> mb;
-  size_t off = 0;
+  base = up(extra);
+  bytes = 0;
   parts.clear();
   with_live = live;
-  int most = 1;
   for (int id : ids) {
     const cass_box_state &b = e->boxes[id];
-    MirrorBox m{b.x, b.y, b.z, b.comd, live ? b.d_live : nullptr, b.nsites, b.nmols, 0, 0, 0};
-    m.xyz = off;
-    off += up(sizeof(double) * 3 * b.nsites);
-    m.com = off;
-    off += up(sizeof(double4) * b.nmols);
-    m.flags = off;
-    if (live) off += up(sizeof(int32_t) * b.nmols);
-    mb.push_back(m);
-    parts.push_back(Part{id, base + m.xyz, base + m.com, base + m.flags});
+    Part p{id, bytes, 0, 0};
+    bytes += up(sizeof(double) * 3 * b.nsites);
+    p.com = bytes;
+    bytes += up(sizeof(double4) * b.nmols);
+    p.live = bytes;
+    if (live) bytes += up(sizeof(int32_t) * b.nmols);
+    parts.push_back(p);
+  }
+  const size_t table = up(sizeof(MirrorBox) * std::max<size_t>(1, parts.size()));
+  host = (char *)cass_pinned(e, base + bytes + table);
+  dev = (char *)cass_io(e, bytes + table);
+  return host && dev ? CASS_OK : cass_fail(e, CASS_ERR_NOMEM, "mirror staging");
+}
+
+int MirrorPull::queue(cass_engine *e) {
+  if (parts.empty()) return CASS_OK;
+  // the box table goes through the tail of the staging
+  MirrorBox *table = (MirrorBox *)(host + base + bytes);
+  int most = 1;
+  for (size_t i = 0; i < parts.size(); ++i) {
+    const Part &p = parts[i];
+    const cass_box_state &b = e->boxes[p.box];
+    table[i] = MirrorBox{b.x,   b.y,   b.z,   b.comd, with_live ? b.d_live : nullptr, b.nsites,
+                         b.nmols, p.xyz, p.com, p.live};
     most = std::max(most, 3 * b.nsites);
   }
-  const size_t args = up(sizeof(MirrorBox) * std::max<size_t>(1, mb.size()));
-  host = (char *)cass_pinned(e, base + off + args);
-  char *dev = (char *)cass_io(e, off + args);
-  if (!host || !dev) return cass_fail(e, CASS_ERR_NOMEM, "mirror staging");
-  if (mb.empty()) return CASS_OK;
-  // the box table goes through the tail of the staging
-  std::memcpy(host + base + off, mb.data(), sizeof(MirrorBox) * mb.size());
-  HIP_TRY(e, hipMemcpyAsync(dev + off, host + base + off, sizeof(MirrorBox) * mb.size(), hipMemcpyHostToDevice,
-                            e->stream));
+  HIP_TRY(e, hipMemcpyAsync(dev + bytes, table, sizeof(MirrorBox) * parts.size(), hipMemcpyHostToDevice, e->stream));
   const unsigned ny = (unsigned)std::min(64, (most + 1023) / 1024);
-  hipLaunchKernelGGL(k_pack_mirrors, dim3((unsigned)mb.size(), ny), dim3(256), 0, e->stream,
-                     (const MirrorBox *)(dev + off), dev);
+  hipLaunchKernelGGL(k_pack_mirrors, dim3((unsigned)parts.size(), ny), dim3(256), 0, e->stream,
+                     (const MirrorBox *)(dev + bytes), dev);
   HIP_TRY(e, hipGetLastError());
-  if (off) HIP_TRY(e, hipMemcpyAsync(host + base, dev, off, hipMemcpyDeviceToHost, e->stream));
+  if (bytes) HIP_TRY(e, hipMemcpyAsync(host + base, dev, bytes, hipMemcpyDeviceToHost, e->stream));
   return CASS_OK;
 }
 
 void MirrorPull::end(cass_engine *e) {
   for (const Part &p : parts) {
     cass_box_state &b = e->boxes[p.box];
-    std::memcpy(b.xyz_h.data(), host + p.xyz, sizeof(double) * 3 * b.nsites);
-    std::memcpy(b.comd_h.data(), host + p.com, sizeof(double4) * b.nmols);
-    if (with_live) std::memcpy(b.live.data(), host + p.live, sizeof(int32_t) * b.nmols);
+    const char *h = host + base;
+    std::memcpy(b.xyz_h.data(), h + p.xyz, sizeof(double) * 3 * b.nsites);
+    std::memcpy(b.comd_h.data(), h + p.com, sizeof(double4) * b.nmols);
+    if (with_live) std::memcpy(b.live.data(), h + p.live, sizeof(int32_t) * b.nmols);
   }
 }
 

@@ -1160,12 +1160,8 @@ int nvt_buffers(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, NvtB
 
 // Results of the batch back to the host: generator states, energies,
 // records, the moved coordinates and centres.
-int nvt_finish(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, const NvtBuffers &B) {
-  std::vector<int> ids;
-  for (const NvtLaunch &L : Ls)
-    if (!L.host_loop) ids.push_back(L.box);
-  MirrorPull mirrors;
-  if (int rc = mirrors.begin(e, ids, false, B.back)) return rc;
+int nvt_finish(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, const NvtBuffers &B, MirrorPull &mirrors) {
+  if (int rc = mirrors.queue(e)) return rc;
   if (B.back) HIP_TRY(e, hipMemcpyAsync(mirrors.host, B.dev, B.back, hipMemcpyDeviceToHost, e->stream));
   HIP_TRY(e, hipStreamSynchronize(e->stream));
   mirrors.end(e);
@@ -1218,6 +1214,11 @@ extern "C" int cass_nvt_run_device_batch(cass_engine *e, int32_t nboxes, const i
   if (nsteps == 0 || nboxes == 0) return CASS_OK;
   NvtBuffers B;
   if ((rc = nvt_buffers(e, Ls, nsteps, B))) return rc;
+  std::vector<int> ids;
+  for (const NvtLaunch &L : Ls)
+    if (!L.host_loop) ids.push_back(L.box);
+  MirrorPull mirrors;
+  if ((rc = mirrors.reserve(e, ids, false, B.back))) return rc;
   // the chains grouped by kernel; every group is one launch per chunk of
   // moves, one workgroup per box.  The argument table holds the groups one
   // after another.
@@ -1251,7 +1252,7 @@ extern "C" int cass_nvt_run_device_batch(cass_engine *e, int32_t nboxes, const i
       HIP_TRY(e, hipGetLastError());
     }
   }
-  rc = nvt_finish(e, Ls, nsteps, B);
+  rc = nvt_finish(e, Ls, nsteps, B, mirrors);
   for (int k = 0; !rc && k < nboxes; ++k)
     if (Ls[k].host_loop)
       rc = cass_nvt_run(e, boxes[k], rngs + k, opts + k, nsteps, ens + k, recs ? recs + k : nullptr);

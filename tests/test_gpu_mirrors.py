@@ -1,9 +1,13 @@
 """A batch of NVT chains over boxes of different sizes, styles and species:
 each box equal bit for bit to its own run, its host mirrors equal to the
-device's coordinates, one launch and several."""
+device's coordinates, one launch and several.  A batch whose staging cannot be
+had leaves its boxes as they were."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
+from cassandra_amd import cbmc
 from cassandra_amd import engine as E
 from cassandra_amd import systems as S
 
@@ -53,3 +57,62 @@ def test_nvt_batch_of_unlike_boxes(steps):
     eng = E.Engine(systems[0])
     assert eng.nvt_run_batch([], [], 5, []) == []
     eng.close()
+
+
+def _pentanes(n, cap):
+    sp = cbmc.pentane_frag_species(S.species_pentane())
+    coords = np.zeros((cap, sp.natoms, 3))
+    coords[:n] = S.place_random_grid([(sp, n)], [30.0] * 3, 5, 2.2, 3.0)[0]
+    system = S.System([sp], [cap], [coords], np.array([30.0] * 3), 420.0, "lj", "cut_tail", 13.0, rcut_low=1.0,
+                      rcut_cbmc=6.5, seed=(3, 8), name="staging")
+    return sp, system, (np.arange(cap) < n).astype(np.int32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("entry", ["nvt", "gcmc", "regrow"])
+def test_no_staging_leaves_boxes_untouched(entry):
+    print(f"[gpu] no staging, {entry}", flush=True)
+    n, cap, steps = 20, 30, 25
+    sp, system, live = _pentanes(n, cap)
+    if entry == "nvt":
+        system, live = _systems()[0], None
+    lim = E.load_library().cass_test_pinned_limit
+    lim.argtypes, lim.restype = [C.c_void_p, C.c_size_t], None
+
+    def run(fail):
+        eng = E.Engine(system, precision=E.FP64)
+        box = eng.add_box(system, live=live)
+        if entry != "nvt":
+            eng.set_cbmc_species(0, cbmc.pentane_growth(420.0, 12, 24, seed=1)[1])
+        elif system.charge_style == "ewald":
+            box.ewald_setup()
+        e0 = box.compute_system_total_energy()
+        rng = E.startup_rng(3, 8, [sp]) if entry != "nvt" else E.rng(*system.seed)
+        state = dict(rng=rng, energy=e0, locate=np.arange(n), reservoir=np.arange(cap - 1, n - 1, -1))
+
+        def call():
+            if entry == "nvt":
+                return eng.nvt_run_batch([box], [rng], steps, [e0])[0]
+            if entry == "regrow":
+                return eng.regrow_run([box], 0, [np.arange(n)], [rng], steps, [e0])[0]
+            lam = cbmc.de_broglie(sp, 420.0)
+            return eng.gcmc_run([dict(box=box.id, species=0, first_slot=0, max_mols=cap, prob_insert=0.5, mu=-6000.0,
+                                      de_broglie=lam)], [state], steps)
+
+        if fail:
+            before, words = box.download(), list(rng.s)
+            lim(eng.h, 1)
+            with pytest.raises(E.CassError) as ex:
+                call()
+            assert ex.value.code == 3
+            lim(eng.h, 1 << 40)
+            assert np.array_equal(box.download(), before) and list(rng.s) == words
+            assert box.compute_system_total_energy() == e0
+        out = call()
+        got = out["energy"], box.download(), box.compute_system_total_energy()
+        eng.close()
+        return got
+
+    (ea, xa, ta), (eb, xb, tb) = run(True), run(False)
+    assert np.array_equal(ea, eb) and np.array_equal(xa, xb) and ta == tb
+    assert len(np.unique(ea)) > 1   # moves were accepted
