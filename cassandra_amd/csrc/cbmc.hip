@@ -674,6 +674,11 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
   size_t bytes = 0;
   int maxm = 0;
   bool lj = true;
+  ChainRecords recs;
+  struct Offs {
+    size_t rng, en, cnt, loc, res, nb, kind, acc, nm, ren, rr;
+  };
+  std::vector<Offs> offs(nboxes);
   auto up = [](size_t n) { return (n + 255) & ~size_t(255); };
   for (int i = 0; i < nboxes; ++i) {
     const cass_gcmc_box &g = boxes[i];
@@ -712,16 +717,24 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
     // the same rounded pieces the layout below takes, one by one
     bytes += up(sizeof(int64_t) * 5) + up(sizeof(double) * 14) + up(sizeof(int) * 2) +
              2 * up(sizeof(int) * g.max_mols) + up(sizeof(double) * ntypes);
-    if (rec) bytes += 2 * up(nsteps) + up(sizeof(int) * nsteps) + up(sizeof(double) * nsteps) +
-                      up(sizeof(int64_t) * 5 * nsteps);
+    Offs &o = offs[i];
+    if (rec) {
+      const size_t at = (size_t)i * nsteps;
+      o.kind = recs.add(rec->kind + at, nsteps);
+      o.acc = recs.add(rec->accepted + at, nsteps);
+      o.nm = recs.add(rec->nmols + at, sizeof(int) * nsteps);
+      o.ren = recs.add(rec->energy + at, sizeof(double) * nsteps);
+      o.rr = recs.add(rec->rng_state + 5 * at, sizeof(int64_t) * 5 * nsteps);
+    }
   }
   bytes += up(sizeof(GcmcBoxArgs) * nboxes);
   // the live lists, at the end: not copied to or from the host
   const int list_cap = list_cap_of(maxm, gemc ? 2 : 1);
   const size_t state_bytes = bytes;
   if (list_cap == 0) bytes += (up(sizeof(float4) * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)nboxes;
-  char *s0 = (char *)cass_scratch(e, bytes + 256);
+  char *s0 = (char *)cass_scratch(e, bytes + recs.staged() + 256);
   if (!s0) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
+  if (int rrc = recs.place(e, s0 + bytes)) return rrc;
   std::vector<char> host(state_bytes + 256, 0);
   size_t off = 0;
   auto take = [&](size_t n) {
@@ -730,10 +743,6 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
     return o;
   };
   std::vector<GcmcBoxArgs> args(nboxes);
-  struct Offs {
-    size_t rng, en, cnt, loc, res, nb, kind, acc, nm, ren, rr;
-  };
-  std::vector<Offs> offs(nboxes);
   for (int i = 0; i < nboxes; ++i) {
     const cass_gcmc_box &g = boxes[i];
     cass_box_state &b = e->boxes[g.box];
@@ -762,13 +771,6 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
         if (ty >= 0) nb[ty] += (double)count[sp];
       }
     std::memcpy(host.data() + o.nb, nb.data(), sizeof(double) * ntypes);
-    if (rec) {
-      o.kind = take(nsteps);
-      o.acc = take(nsteps);
-      o.nm = take(sizeof(int) * nsteps);
-      o.ren = take(sizeof(double) * nsteps);
-      o.rr = take(sizeof(int64_t) * 5 * nsteps);
-    }
     GcmcBoxArgs &a = args[i];
     a.g = grow_args(e, b, cbmc_of(e, g.species));
     a.x = b.x;
@@ -796,11 +798,11 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
     a.vdw_style = b.p.vdw_style;
     a.tail = b.p.vdw_sum_style == CASS_SUM_CUT_TAIL;
     a.commit = commit;
-    a.kind = rec ? (uint8_t *)(s0 + o.kind) : nullptr;
-    a.accepted = rec ? (uint8_t *)(s0 + o.acc) : nullptr;
-    a.rec_nmols = rec ? (int *)(s0 + o.nm) : nullptr;
-    a.rec_energy = rec ? (double *)(s0 + o.ren) : nullptr;
-    a.rec_rng = rec ? (int64_t *)(s0 + o.rr) : nullptr;
+    a.kind = rec ? recs.at<uint8_t>(o.kind) : nullptr;
+    a.accepted = rec ? recs.at<uint8_t>(o.acc) : nullptr;
+    a.rec_nmols = rec ? recs.at<int>(o.nm) : nullptr;
+    a.rec_energy = rec ? recs.at<double>(o.ren) : nullptr;
+    a.rec_rng = rec ? recs.at<int64_t>(o.rr) : nullptr;
     const size_t o_list = state_bytes + (up(sizeof(float4) * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)i;
     a.list = list_cap ? LiveList{nullptr, nullptr}
                       : LiveList{(LiveMol *)(s0 + o_list + up(sizeof(float4) * maxm)), (float4 *)(s0 + o_list)};
@@ -810,7 +812,7 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
   MirrorPull mirrors;
   std::vector<int> ids(commit ? nboxes : 0);
   for (size_t i = 0; i < ids.size(); ++i) ids[i] = boxes[i].box;
-  if (int mrc = mirrors.reserve(e, ids, true, off)) return mrc;
+  if (int mrc = mirrors.reserve(e, ids, true, off + recs.staged())) return mrc;
   std::memcpy(host.data() + o_args, args.data(), sizeof(GcmcBoxArgs) * nboxes);
   HIP_TRY(e, hipMemcpyAsync(s0, host.data(), off, hipMemcpyHostToDevice, e->stream));
   HIP_TRY(e, hipEventRecord(e->ev0, e->stream));
@@ -832,12 +834,14 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
   // centres of every box come back behind one synchronisation
   if (int mrc = mirrors.queue(e)) return mrc;
   HIP_TRY(e, hipMemcpyAsync(mirrors.host, s0, off, hipMemcpyDeviceToHost, e->stream));
+  if (int mrc = recs.queue(e, mirrors.host + off)) return mrc;
   HIP_TRY(e, hipStreamSynchronize(e->stream));
   float ms = 0.f;
   if (hipEventElapsedTime(&ms, e->ev0, e->ev1) == hipSuccess) e->last_kernel_ms = ms;
   if (ms_out) *ms_out = ms;
   if (!commit) return CASS_OK;
   mirrors.end(e);
+  recs.end(mirrors.host + off);
   const char *back = mirrors.host;
   int bad = 0;
   for (int i = 0; i < nboxes; ++i) {
@@ -853,13 +857,6 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
     st.nres = cnt[1] < 0 ? g.max_mols - cnt[0] : cnt[1];
     std::memcpy(st.locate, back + o.loc, sizeof(int) * g.max_mols);
     std::memcpy(st.reservoir, back + o.res, sizeof(int) * g.max_mols);
-    if (rec) {
-      std::memcpy(rec->kind + (size_t)i * nsteps, back + o.kind, nsteps);
-      std::memcpy(rec->accepted + (size_t)i * nsteps, back + o.acc, nsteps);
-      std::memcpy(rec->nmols + (size_t)i * nsteps, back + o.nm, sizeof(int) * nsteps);
-      std::memcpy(rec->energy + (size_t)i * nsteps, back + o.ren, sizeof(double) * nsteps);
-      std::memcpy(rec->rng_state + (size_t)i * nsteps * 5, back + o.rr, sizeof(int64_t) * 5 * nsteps);
-    }
   }
   ++e->gen;
   if (bad)
@@ -888,6 +885,11 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
   size_t bytes = 0;
   int maxm = 0;
   bool lj = true;
+  ChainRecords pull;
+  struct Offs {
+    size_t rng, en, st, loc, kind, acc, ren, lp, rr;
+  };
+  std::vector<Offs> offs(nboxes);
   for (int i = 0; i < nboxes; ++i) {
     const cass_regrow_box &g = boxes[i];
     if (g.box < 0 || g.box >= (int)e->boxes.size()) return cass_fail(e, CASS_ERR_ARG, "bad box");
@@ -909,14 +911,23 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
     maxm = std::max(maxm, b.nmols);
     lj = lj && lj_growth(e, b, g.species);
     bytes += up(sizeof(int64_t) * 5) + up(sizeof(double) * 14) + up(sizeof(int)) + up(sizeof(int) * g.nmols);
-    if (recs) bytes += 2 * up(nsteps) + 2 * up(sizeof(double) * nsteps) + up(sizeof(int64_t) * 5 * nsteps);
+    if (recs) {
+      const cass_nvt_record &r = recs[i];
+      Offs &o = offs[i];
+      if (r.kind) o.kind = pull.add(r.kind, nsteps);
+      if (r.accepted) o.acc = pull.add(r.accepted, nsteps);
+      if (r.energy) o.ren = pull.add(r.energy, sizeof(double) * nsteps);
+      if (r.ln_pacc) o.lp = pull.add(r.ln_pacc, sizeof(double) * nsteps);
+      if (r.rng_state) o.rr = pull.add(r.rng_state, sizeof(int64_t) * 5 * nsteps);
+    }
   }
   bytes += up(sizeof(RegrowBoxArgs) * nboxes);
   const int list_cap = list_cap_of(maxm, 1);
   const size_t state_bytes = bytes;
   if (list_cap == 0) bytes += (up(sizeof(float4) * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)nboxes;
-  char *s0 = (char *)cass_scratch(e, bytes + 256);
+  char *s0 = (char *)cass_scratch(e, bytes + pull.staged() + 256);
   if (!s0) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
+  if (int prc = pull.place(e, s0 + bytes)) return prc;
   std::vector<char> host(state_bytes + 256, 0);
   size_t off = 0;
   auto take = [&](size_t n) {
@@ -924,10 +935,6 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
     off += up(n);
     return o;
   };
-  struct Offs {
-    size_t rng, en, st, loc, kind, acc, ren, lp, rr;
-  };
-  std::vector<Offs> offs(nboxes);
   std::vector<RegrowBoxArgs> args(nboxes);
   for (int i = 0; i < nboxes; ++i) {
     const cass_regrow_box &g = boxes[i];
@@ -940,14 +947,6 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
     std::memcpy(host.data() + o.rng, rngs[i].s, sizeof(int64_t) * 5);
     std::memcpy(host.data() + o.en, &energies[i], sizeof(double) * 14);
     std::memcpy(host.data() + o.loc, g.locate, sizeof(int) * g.nmols);
-    const bool r = recs != nullptr;
-    if (r) {
-      o.kind = take(nsteps);
-      o.acc = take(nsteps);
-      o.ren = take(sizeof(double) * nsteps);
-      o.lp = take(sizeof(double) * nsteps);
-      o.rr = take(sizeof(int64_t) * 5 * nsteps);
-    }
     RegrowBoxArgs &a = args[i];
     a.g = grow_args(e, b, cbmc_of(e, g.species));
     a.x = b.x;
@@ -960,11 +959,12 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
     a.rng = (int64_t *)(s0 + o.rng);
     a.energy = (double *)(s0 + o.en);
     a.status = (int *)(s0 + o.st);
-    a.kind = r ? (uint8_t *)(s0 + o.kind) : nullptr;
-    a.accepted = r ? (uint8_t *)(s0 + o.acc) : nullptr;
-    a.rec_energy = r ? (double *)(s0 + o.ren) : nullptr;
-    a.ln_pacc = r ? (double *)(s0 + o.lp) : nullptr;
-    a.rec_rng = r ? (int64_t *)(s0 + o.rr) : nullptr;
+    const cass_nvt_record *r = recs ? recs + i : nullptr;
+    a.kind = r && r->kind ? pull.at<uint8_t>(o.kind) : nullptr;
+    a.accepted = r && r->accepted ? pull.at<uint8_t>(o.acc) : nullptr;
+    a.rec_energy = r && r->energy ? pull.at<double>(o.ren) : nullptr;
+    a.ln_pacc = r && r->ln_pacc ? pull.at<double>(o.lp) : nullptr;
+    a.rec_rng = r && r->rng_state ? pull.at<int64_t>(o.rr) : nullptr;
     const size_t o_list = state_bytes + (up(sizeof(float4) * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)i;
     a.list = list_cap ? LiveList{nullptr, nullptr}
                       : LiveList{(LiveMol *)(s0 + o_list + up(sizeof(float4) * maxm)), (float4 *)(s0 + o_list)};
@@ -974,7 +974,7 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
   MirrorPull mirrors;
   std::vector<int> ids(nboxes);
   for (int i = 0; i < nboxes; ++i) ids[i] = boxes[i].box;
-  if (int mrc = mirrors.reserve(e, ids, false, off)) return mrc;
+  if (int mrc = mirrors.reserve(e, ids, false, off + pull.staged())) return mrc;
   std::memcpy(host.data() + o_args, args.data(), sizeof(RegrowBoxArgs) * nboxes);
   HIP_TRY(e, hipMemcpyAsync(s0, host.data(), off, hipMemcpyHostToDevice, e->stream));
   HIP_TRY(e, hipEventRecord(e->ev0, e->stream));
@@ -986,8 +986,10 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
   HIP_TRY(e, hipEventRecord(e->ev1, e->stream));
   if (int mrc = mirrors.queue(e)) return mrc;
   HIP_TRY(e, hipMemcpyAsync(mirrors.host, s0, off, hipMemcpyDeviceToHost, e->stream));
+  if (int prc = pull.queue(e, mirrors.host + off)) return prc;
   HIP_TRY(e, hipStreamSynchronize(e->stream));
   mirrors.end(e);
+  pull.end(mirrors.host + off);
   const char *back = mirrors.host;
   float ms = 0.f;
   if (hipEventElapsedTime(&ms, e->ev0, e->ev1) == hipSuccess) e->last_kernel_ms = ms;
@@ -999,14 +1001,6 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
     int st;
     std::memcpy(&st, back + o.st, sizeof(int));
     bad |= st;
-    if (recs) {
-      cass_nvt_record &r = recs[i];
-      if (r.kind) std::memcpy(r.kind, back + o.kind, nsteps);
-      if (r.accepted) std::memcpy(r.accepted, back + o.acc, nsteps);
-      if (r.energy) std::memcpy(r.energy, back + o.ren, sizeof(double) * nsteps);
-      if (r.ln_pacc) std::memcpy(r.ln_pacc, back + o.lp, sizeof(double) * nsteps);
-      if (r.rng_state) std::memcpy(r.rng_state, back + o.rr, sizeof(int64_t) * 5 * nsteps);
-    }
   }
   ++e->gen;
   if (bad) return cass_fail(e, CASS_ERR_STATE, "a molecule's own configuration could not be regrown (the reference aborts)");

@@ -165,5 +165,37 @@ struct MirrorPull {
   size_t base = 0, bytes = 0;  // the caller's bytes; the packed ones
   char *dev = nullptr;
 };
+// Per-move records of a chain batch, on their way from the device to the
+// caller's arrays.  Up to kRecordStage bytes of them go through the batch's
+// scratch and pinned staging in one copy; more, from a stream allocation that
+// is given back, are copied straight into the caller's arrays, so that the
+// engine keeps no memory that grows with the moves of a call.
+constexpr size_t kRecordStage = (size_t)16 << 20;
+struct ChainRecords {
+  ~ChainRecords();
+  // one array of `bytes` for dst; returns its place for at()
+  size_t add(void *dst, size_t bytes);
+  size_t staged() const { return total <= kRecordStage ? total : 0; }
+  // zeroed device memory: `room`, with staged() bytes of it, or its own
+  int place(cass_engine *e, char *room);
+  template <typename T>
+  T *at(size_t off) const {
+    return (T *)(dev + off);
+  }
+  // queues the copies, through `pinned` where staged; end() after the
+  // synchronisation
+  int queue(cass_engine *e, char *pinned);
+  void end(const char *pinned);
+
+ private:
+  struct Part {
+    size_t off, bytes;
+    void *dst;
+  };
+  std::vector<Part> parts;
+  size_t total = 0;
+  char *dev = nullptr;
+  cass_engine *owner = nullptr;  // of a stream allocation
+};
 bool cass_cbmc_bonded_host(const cass_engine *e, int s, const double *xyz, double *angle, double *dihedral);
 double4 cass_host_com(const cass_engine *e, int s, const double *xyz);  // Get_COM and max_dcom of one molecule  // device copies of the CBMC growth descriptions

@@ -804,6 +804,48 @@ void MirrorPull::end(cass_engine *e) {
   }
 }
 
+// -------------------------------------------------------------- records
+ChainRecords::~ChainRecords() {
+  if (owner) (void)hipFreeAsync(dev, owner->stream);
+}
+
+size_t ChainRecords::add(void *dst, size_t bytes) {
+  const size_t off = total;
+  parts.push_back(Part{off, bytes, dst});
+  total += (bytes + 255) & ~size_t(255);
+  return off;
+}
+
+int ChainRecords::place(cass_engine *e, char *room) {
+  if (total == 0) return CASS_OK;
+  dev = room;
+  if (!staged()) {
+    if (hipMallocAsync((void **)&dev, total, e->stream) != hipSuccess) {
+      (void)hipGetLastError();
+      return cass_fail(e, CASS_ERR_NOMEM, "per-move records");
+    }
+    owner = e;
+  }
+  HIP_TRY(e, hipMemsetAsync(dev, 0, total, e->stream));
+  return CASS_OK;
+}
+
+int ChainRecords::queue(cass_engine *e, char *pinned) {
+  if (total == 0) return CASS_OK;
+  if (staged()) {
+    HIP_TRY(e, hipMemcpyAsync(pinned, dev, total, hipMemcpyDeviceToHost, e->stream));
+    return CASS_OK;
+  }
+  for (const Part &p : parts)
+    if (p.bytes) HIP_TRY(e, hipMemcpyAsync(p.dst, dev + p.off, p.bytes, hipMemcpyDeviceToHost, e->stream));
+  return CASS_OK;
+}
+
+void ChainRecords::end(const char *pinned) {
+  if (staged())
+    for (const Part &p : parts) std::memcpy(p.dst, pinned + p.off, p.bytes);
+}
+
 // ------------------------------------------------------- trial energies
 // Launches k_trials + k_finalize_trials; results (E_vdw, E_qq, overlap)
 // land in dev_out[2*t], dev_ov[t] (device) -- the caller copies back.

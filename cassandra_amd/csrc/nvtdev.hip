@@ -1093,14 +1093,16 @@ struct NvtState {
   int status[2];
 };
 
-// The buffers of a batch, laid out over all its chains: first what comes back
-// (states and records), then the mobile lists and argument tables.  One copy in, one copy out: with a set of copies per chain
-// the calls themselves outlasted the chains.
+// The buffers of a batch, laid out over all its chains: first the states, which
+// come back, then the mobile lists and argument tables, then the records.  One
+// copy in, one or two out: with a set of copies per chain the calls themselves
+// outlasted the chains.
 struct NvtBuffers {
   char *dev = nullptr;
-  size_t back = 0, in = 0;  // bytes copied back; bytes of back + lists + arguments
+  size_t back = 0, in = 0;  // bytes of the states; with the lists and arguments
   size_t o_args = 0;
   std::vector<char> host;   // the first `in` bytes
+  ChainRecords rec;
 };
 
 int nvt_buffers(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, NvtBuffers &B) {
@@ -1115,11 +1117,11 @@ int nvt_buffers(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, NvtB
     if (L.host_loop) continue;
     const cass_nvt_record *rec = L.rec;
     L.o_state = take(sizeof(NvtState));
-    if (rec && rec->kind) L.o_kind = take(ns);
-    if (rec && rec->accepted) L.o_acc = take(ns);
-    if (rec && rec->energy) L.o_energy = take(sizeof(double) * ns);
-    if (rec && rec->ln_pacc) L.o_lnp = take(sizeof(double) * ns);
-    if (rec && rec->rng_state) L.o_rs = take(sizeof(int64_t) * 5 * ns);
+    if (rec && rec->kind) L.o_kind = B.rec.add(rec->kind, ns);
+    if (rec && rec->accepted) L.o_acc = B.rec.add(rec->accepted, ns);
+    if (rec && rec->energy) L.o_energy = B.rec.add(rec->energy, sizeof(double) * ns);
+    if (rec && rec->ln_pacc) L.o_lnp = B.rec.add(rec->ln_pacc, sizeof(double) * ns);
+    if (rec && rec->rng_state) L.o_rs = B.rec.add(rec->rng_state, sizeof(int64_t) * 5 * ns);
   }
   B.back = off;
   for (NvtLaunch &L : Ls)
@@ -1129,8 +1131,9 @@ int nvt_buffers(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, NvtB
     }
   B.o_args = take(sizeof(NvtChainArgs) * std::max<size_t>(1, Ls.size()));
   B.in = off;
-  B.dev = (char *)cass_scratch(e, off + 256);
+  B.dev = (char *)cass_scratch(e, off + B.rec.staged() + 256);
   if (!B.dev) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
+  if (int rc = B.rec.place(e, B.dev + off)) return rc;
   B.host.assign(B.in, 0);
   for (size_t k = 0; k < Ls.size(); ++k) {
     NvtLaunch &L = Ls[k];
@@ -1147,11 +1150,11 @@ int nvt_buffers(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, NvtB
     a.rng = d->rng;
     a.en = d->en;
     a.status = d->status;
-    a.kind = rec && rec->kind ? (uint8_t *)(B.dev + L.o_kind) : nullptr;
-    a.accepted = rec && rec->accepted ? (uint8_t *)(B.dev + L.o_acc) : nullptr;
-    a.energy = rec && rec->energy ? (double *)(B.dev + L.o_energy) : nullptr;
-    a.ln_pacc = rec && rec->ln_pacc ? (double *)(B.dev + L.o_lnp) : nullptr;
-    a.rng_state = rec && rec->rng_state ? (int64_t *)(B.dev + L.o_rs) : nullptr;
+    a.kind = rec && rec->kind ? B.rec.at<uint8_t>(L.o_kind) : nullptr;
+    a.accepted = rec && rec->accepted ? B.rec.at<uint8_t>(L.o_acc) : nullptr;
+    a.energy = rec && rec->energy ? B.rec.at<double>(L.o_energy) : nullptr;
+    a.ln_pacc = rec && rec->ln_pacc ? B.rec.at<double>(L.o_lnp) : nullptr;
+    a.rng_state = rec && rec->rng_state ? B.rec.at<int64_t>(L.o_rs) : nullptr;
     a.mols = (const int *)(B.dev + L.o_mols);
     a.meta = L.local ? nullptr : (int *)(B.dev + L.o_meta);
   }
@@ -1160,13 +1163,14 @@ int nvt_buffers(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, NvtB
 
 // Results of the batch back to the host: generator states, energies,
 // records, the moved coordinates and centres.
-int nvt_finish(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, const NvtBuffers &B, MirrorPull &mirrors) {
+int nvt_finish(cass_engine *e, std::vector<NvtLaunch> &Ls, NvtBuffers &B, MirrorPull &mirrors) {
   if (int rc = mirrors.queue(e)) return rc;
   if (B.back) HIP_TRY(e, hipMemcpyAsync(mirrors.host, B.dev, B.back, hipMemcpyDeviceToHost, e->stream));
+  if (int rc = B.rec.queue(e, mirrors.host + B.back)) return rc;
   HIP_TRY(e, hipStreamSynchronize(e->stream));
   mirrors.end(e);
+  B.rec.end(mirrors.host + B.back);
   ++e->gen;
-  const size_t ns = (size_t)nsteps;
   bool bad = false;
   for (NvtLaunch &L : Ls) {
     if (L.host_loop) continue;
@@ -1174,12 +1178,6 @@ int nvt_finish(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, const
     const char *h = mirrors.host;
     NvtState st;
     std::memcpy(&st, h + L.o_state, sizeof(st));
-    const cass_nvt_record *rec = L.rec;
-    if (L.a.kind) std::memcpy(rec->kind, h + L.o_kind, ns);
-    if (L.a.accepted) std::memcpy(rec->accepted, h + L.o_acc, ns);
-    if (L.a.energy) std::memcpy(rec->energy, h + L.o_energy, sizeof(double) * ns);
-    if (L.a.ln_pacc) std::memcpy(rec->ln_pacc, h + L.o_lnp, sizeof(double) * ns);
-    if (L.a.rng_state) std::memcpy(rec->rng_state, h + L.o_rs, sizeof(int64_t) * 5 * ns);
     std::memcpy(L.rng->s, st.rng, sizeof(st.rng));
     L.en->total = st.en[0];
     L.en->inter = st.en[1];
@@ -1218,7 +1216,7 @@ extern "C" int cass_nvt_run_device_batch(cass_engine *e, int32_t nboxes, const i
   for (const NvtLaunch &L : Ls)
     if (!L.host_loop) ids.push_back(L.box);
   MirrorPull mirrors;
-  if ((rc = mirrors.reserve(e, ids, false, B.back))) return rc;
+  if ((rc = mirrors.reserve(e, ids, false, B.back + B.rec.staged()))) return rc;
   // the chains grouped by kernel; every group is one launch per chunk of
   // moves, one workgroup per box.  The argument table holds the groups one
   // after another.
@@ -1252,7 +1250,7 @@ extern "C" int cass_nvt_run_device_batch(cass_engine *e, int32_t nboxes, const i
       HIP_TRY(e, hipGetLastError());
     }
   }
-  rc = nvt_finish(e, Ls, nsteps, B, mirrors);
+  rc = nvt_finish(e, Ls, B, mirrors);
   for (int k = 0; !rc && k < nboxes; ++k)
     if (Ls[k].host_loop)
       rc = cass_nvt_run(e, boxes[k], rngs + k, opts + k, nsteps, ens + k, recs ? recs + k : nullptr);

@@ -1,7 +1,8 @@
 """A batch of NVT chains over boxes of different sizes, styles and species:
 each box equal bit for bit to its own run, its host mirrors equal to the
 device's coordinates, one launch and several.  A batch whose staging cannot be
-had leaves its boxes as they were."""
+had leaves its boxes as they were; records of any length need no more than the
+bounded staging."""
 import ctypes as C
 
 import numpy as np
@@ -59,6 +60,12 @@ def test_nvt_batch_of_unlike_boxes(steps):
     eng.close()
 
 
+def _pinned_limit():
+    lim = E.load_library().cass_test_pinned_limit
+    lim.argtypes, lim.restype = [C.c_void_p, C.c_size_t], None
+    return lim
+
+
 def _pentanes(n, cap):
     sp = cbmc.pentane_frag_species(S.species_pentane())
     coords = np.zeros((cap, sp.natoms, 3))
@@ -76,8 +83,7 @@ def test_no_staging_leaves_boxes_untouched(entry):
     sp, system, live = _pentanes(n, cap)
     if entry == "nvt":
         system, live = _systems()[0], None
-    lim = E.load_library().cass_test_pinned_limit
-    lim.argtypes, lim.restype = [C.c_void_p, C.c_size_t], None
+    lim = _pinned_limit()
 
     def run(fail):
         eng = E.Engine(system, precision=E.FP64)
@@ -116,3 +122,49 @@ def test_no_staging_leaves_boxes_untouched(entry):
     (ea, xa, ta), (eb, xb, tb) = run(True), run(False)
     assert np.array_equal(ea, eb) and np.array_equal(xa, xb) and ta == tb
     assert len(np.unique(ea)) > 1   # moves were accepted
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("entry", ["nvt", "gcmc", "regrow"])
+def test_long_records_within_bounded_staging(entry):
+    """54 to 58 bytes a move and box: 18 to 19 MB in one call, past the 16 MiB that
+    go through the staging; the same moves in two calls, which do."""
+    print(f"[gpu] long records, {entry}", flush=True)
+    nb, steps = {"nvt": (16, 20000), "gcmc": (48, 7000), "regrow": (48, 6800)}[entry]
+    n, cap = 6, 12
+    sp, system, live = _pentanes(n, cap)
+    if entry == "nvt":
+        ar = S.species_lj()
+        system, live = S.System([ar], [2], S.place_random([(ar, 2)], [20.0] * 3, 3, 1.2, 2.6), np.array([20.0] * 3),
+                                300.0, "lj", "cut", 9.0, rcut_low=0.85, max_disp=1.0, name="two").parsed(), None
+
+    def run(calls):
+        eng = E.Engine(system, max_boxes=nb, precision=E.FP64)
+        boxes = [eng.add_box(system, live=live) for _ in range(nb)]
+        if entry != "nvt":
+            eng.set_cbmc_species(0, cbmc.pentane_growth(420.0, 4, 4, seed=1)[1])
+        e0 = eng.total_energy_batch(boxes)
+        rngs = [E.startup_rng(3 + k, 8, [sp]) if entry != "nvt" else E.rng(3 + k, 8) for k in range(nb)]
+        lam = cbmc.de_broglie(sp, 420.0)
+        mu = S.KBOLTZ * 420.0 * (np.log(n / 30.0 ** 3 * lam ** 3) - 1.0)
+        specs = [dict(box=b.id, species=0, first_slot=0, max_mols=cap, prob_insert=0.45, mu=mu, de_broglie=lam)
+                 for b in boxes]
+        states = [dict(rng=r, energy=e, locate=np.arange(n), reservoir=np.arange(cap - 1, n - 1, -1))
+                  for r, e in zip(rngs, e0)]
+        _pinned_limit()(eng.h, 17 << 20)
+        out = []
+        for _ in range(calls):
+            if entry == "gcmc":
+                out.append(eng.gcmc_run(specs, states, steps // calls))
+                continue
+            r = (eng.nvt_run_batch(boxes, rngs, steps // calls, e0) if entry == "nvt" else
+                 eng.regrow_run(boxes, 0, [np.arange(n)] * nb, rngs, steps // calls, e0))
+            e0 = [x["final"] for x in r]
+            out.append({k: np.array([x[k] for x in r]) for k in ("kind", "accepted", "energy", "ln_pacc", "rng")})
+        eng.close()
+        return {k: np.concatenate([o[k] for o in out], axis=1) for k in out[0]}
+
+    one, two = run(1), run(2)
+    for k in one:
+        assert np.array_equal(one[k], two[k], equal_nan=one[k].dtype == np.float64), k
+    assert one["rng"][:, -1].all() and 0 < one["accepted"][:, -100:].sum()
