@@ -76,15 +76,14 @@ struct ChainTopo {
 
 // One live molecule of a box as the stage sums walk them: slot, and first
 // site << 4 | species (species only where the LDS tables are used, <= 8).
-// Its centre stands beside it in single precision for the distance
-// prefilter, whose reach carries a margin for the rounding.
+// Its centre stands beside it for the distance prefilter.
 struct LiveMol {
   int slot, fs;
 };
 // The live molecules of one box, in LDS or in device memory.
 struct LiveList {
   LiveMol *mol;
-  float4 *com;  // (x, y, z, max_dcom)
+  double4 *com;  // (x, y, z, max_dcom)
 };
 
 constexpr int kRing = 128;   // random draws held ready
@@ -324,7 +323,7 @@ __device__ __forceinline__ int build_live_list(const GrowArgs &a, const LiveList
       const int p = n + __popcll(m & ((1ull << wl) - 1ull));
       const double *c = (const double *)(a.b.comd + j);
       l.mol[p] = LiveMol{j, (a.b.first[j] << 4) | (a.b.species[j] & 15)};
-      l.com[p] = make_float4((float)vld(c), (float)vld(c + 1), (float)vld(c + 2), (float)vld(c + 3));
+      l.com[p] = make_double4(vld(c), vld(c + 1), vld(c + 2), vld(c + 3));
     }
     n += __popcll(m);
   }
@@ -342,46 +341,24 @@ __device__ __forceinline__ int live_find(const LiveList &l, int n, int m) {
 }
 
 // Check_MoleculePair_Cutoff (energy_routines.f90:3027-3088) for the walk of a
-// stage, on the single-precision centres: reach is the cutoff, the trial's
-// max_dcom and a margin above the rounding.  A molecule the exact test
-// rejects and this one keeps adds nothing: its site pairs all lie beyond the
-// cutoff.
+// stage, on squared distances (molpair_in_range takes the root as the
+// reference does; the two differ only at the prefilter distance itself, where
+// every site pair lies beyond the cutoff): reach is the cutoff and the trial's
+// max_dcom.
 struct Reach {
-  float x, y, z, r;
-  float L[3], Li[3];
-  int mode;  // 0 cubic, 1 general cell, 2 everything in range
+  double x, y, z, r;
 };
 
 __device__ __forceinline__ Reach make_reach(const BoxDev &b, bool cbmc, double4 ci) {
-  Reach r;
-  r.x = (float)ci.x;
-  r.y = (float)ci.y;
-  r.z = (float)ci.z;
-  r.r = (float)((cbmc ? b.rcut_cbmc : b.rcut_max) + ci.w + 1e-3 + 1e-6 * (b.L[0] + b.L[1] + b.L[2]));
-  for (int d = 0; d < 3; ++d) {
-    r.L[d] = (float)b.L[d];
-    r.Li[d] = 1.0f / (float)b.L[d];
-  }
-  r.mode = b.vdw_minimum ? 2 : (b.cubic ? 0 : 1);
-  return r;
+  return Reach{ci.x, ci.y, ci.z, (cbmc ? b.rcut_cbmc : b.rcut_max) + ci.w};
 }
 
-__device__ __forceinline__ bool in_reach(const BoxDev &b, const Reach &r, float4 c) {
-  if (r.mode == 2) return true;
-  float dx = r.x - c.x, dy = r.y - c.y, dz = r.z - c.z;
-  if (r.mode == 0) {
-    dx = fmaf(-r.L[0], rintf(dx * r.Li[0]), dx);
-    dy = fmaf(-r.L[1], rintf(dy * r.Li[1]), dy);
-    dz = fmaf(-r.L[2], rintf(dz * r.Li[2]), dz);
-  } else {
-    double ex = dx, ey = dy, ez = dz;
-    min_image(b, ex, ey, ez);
-    dx = (float)ex;
-    dy = (float)ey;
-    dz = (float)ez;
-  }
-  const float q = r.r + c.w;
-  return fmaf(dx, dx, fmaf(dy, dy, dz * dz)) <= q * q;
+__device__ __forceinline__ bool in_reach(const BoxDev &b, const Reach &r, double4 c) {
+  if (b.vdw_minimum) return true;
+  double dx = r.x - c.x, dy = r.y - c.y, dz = r.z - c.z;
+  min_image(b, dx, dy, dz);
+  const double q = r.r + c.w;
+  return dx * dx + dy * dy + dz * dz <= q * q;
 }
 
 // Atomic minimum in device memory.
@@ -1643,14 +1620,14 @@ __device__ __forceinline__ int accept_or_reject(const GrowLds<NT> &S, GrowReg &G
 
 // Where a chain kernel keeps its lists: cap > 0: in the dynamic LDS, per box
 // the centres, the entries, then (gcmc) locate and reservoir.
-constexpr size_t kListBytes = sizeof(float4) + sizeof(LiveMol) + 2 * sizeof(int);
+constexpr size_t kListBytes = sizeof(double4) + sizeof(LiveMol) + 2 * sizeof(int);
 __device__ __forceinline__ LiveList chain_list(char *dyn, int cap, int box, const LiveList &g) {
   if (cap == 0) return g;
   char *p = dyn + (size_t)box * cap * kListBytes;
-  return LiveList{(LiveMol *)(p + sizeof(float4) * cap), (float4 *)p};
+  return LiveList{(LiveMol *)(p + sizeof(double4) * cap), (double4 *)p};
 }
 __device__ __forceinline__ int *chain_slots(char *dyn, int cap, int box, int which) {
-  return (int *)(dyn + (size_t)box * cap * kListBytes + (sizeof(float4) + sizeof(LiveMol)) * cap) + which * cap;
+  return (int *)(dyn + (size_t)box * cap * kListBytes + (sizeof(double4) + sizeof(LiveMol)) * cap) + which * cap;
 }
 
 // Removes entry im of locate[0 .. n): the later ones move down (whole wave).
@@ -1669,7 +1646,7 @@ __device__ __forceinline__ void locate_remove(int *locate, int im, int n) {
 __device__ __forceinline__ void list_add(const LiveList &l, int &n, const BoxDev &b, int m, double4 com) {
   if (threadIdx.x == 0) {
     l.mol[n] = LiveMol{m, (b.first[m] << 4) | (b.species[m] & 15)};
-    l.com[n] = make_float4((float)com.x, (float)com.y, (float)com.z, (float)com.w);
+    l.com[n] = com;
   }
   ++n;
 }
@@ -1684,8 +1661,7 @@ __device__ __forceinline__ void list_drop(const LiveList &l, int &n, int m) {
 }
 __device__ __forceinline__ void list_move(const LiveList &l, int n, int m, double4 com) {
   const int p = live_find(l, n, m);
-  if (p >= 0 && threadIdx.x == 0)
-    l.com[p] = make_float4((float)com.x, (float)com.y, (float)com.z, (float)com.w);
+  if (p >= 0 && threadIdx.x == 0) l.com[p] = com;
 }
 
 // Copies a slot list between device memory and LDS (wave 0).

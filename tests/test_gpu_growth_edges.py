@@ -1,12 +1,12 @@
 """The growth kernels at the edges of their ranges, against the oracle: one
 and the most trials a stage takes, live lists about a wave's 64 lanes and
-beyond the LDS, and pair styles off the LJ kernels."""
+beyond the LDS, pair styles off the LJ kernels, and molecules many images away."""
 import dataclasses
 
 import numpy as np
 import pytest
 
-from cassandra_amd import cbmc
+from cassandra_amd import abi, cbmc
 from cassandra_amd import engine as E
 from cassandra_amd import systems as S
 
@@ -85,4 +85,33 @@ def test_growth_chains_at_edges(n, cap, ki, kd, style, oracle_mod):
     ok = ref > 0
     assert np.array_equal(wv > 0, ok)
     assert np.all(np.abs(wv[ok] - ref[ok]) <= REL * 10 * ref[ok])  # a weight is exp(-beta dE): |beta dE| to some tens
+    eng.close()
+
+
+@pytest.mark.gpu
+def test_growth_many_images_away(oracle_mod):
+    """One-site molecules whose coordinates stand 8000 box lengths off (those of a
+    non-cubic box are never folded): each pair within the cutoff counts, also
+    the last hundredth of an angstrom, which single precision cannot tell there."""
+    print("[gpu] growth many images away", flush=True)
+    ch4 = S.species_methane()
+    ch4.fragments = [[0]]
+    box, n = np.array([24.0, 27.0, 25.0]), 400
+    rng = np.random.default_rng(4)
+    cell = np.stack(np.meshgrid(*[np.arange(8)] * 3, indexing="ij"), -1).reshape(-1, 3)[rng.permutation(512)[:n]]
+    xyz = (cell + 0.5 + rng.uniform(-0.1, 0.1, (n, 3))) / 8 * box - box / 2 + box * [8000.0, -9000.0, 7000.0]
+    system = S.System([ch4], [n + 1], [np.concatenate([xyz, np.zeros((1, 3))])[:, None, :]], box, 300.0, "lj", "cut",
+                      9.0, rcut_low=1.0, rcut_cbmc=6.5, box_shape="orthogonal", seed=(3, 5), name="far")
+    live = (np.arange(n + 1) < n).astype(np.int32)
+    growth = abi.CbmcSpecies(ch4, [np.zeros((1, 1, 3))], kappa_ins=8)
+    eng = E.Engine(system, precision=E.FP64)
+    eng.set_cbmc_species(0, growth)
+    b = eng.add_box(system, live=live)
+    wv = b.widom_cbmc(0, 1500, seed=11, per_insertion=True)[3]
+    ref, _ = oracle_mod.OracleCbmc(oracle_mod.OracleBox(system, live=live), 0, growth).widom_streams(11, 1500)
+    ok = ref > 0
+    assert ok.sum() > 500 and np.array_equal(wv > 0, ok)
+    # the separations carry the rounding of coordinates of 2e5 (2e5 * 2^-53 = 2e-11),
+    # r^-12 of them 1e-10 of a term, exp(-beta dE) at |beta dE| of some tens 1e-8
+    assert np.all(np.abs(wv[ok] - ref[ok]) <= 1e-7 * ref[ok])
     eng.close()
