@@ -306,11 +306,12 @@ __global__ void __launch_bounds__(64) k_adj_pairs(BoxDev b, TopoDev tp, AdjParam
       int code = -1;
       if (j < b.nmols) {
         // (squared distances: the reference's root differs at the prefilter
-        // distance alone, where no site pair is within its cutoff)
+        // distance alone, where no site pair is within its cutoff; and its one
+        // image shift of centres, whatever their distance)
         code = mcode[j];
         const double4 cj = COM[j];
         double dx = ci.x - cj.x, dy = ci.y - cj.y, dz = ci.z - cj.z;
-        adj_image(b, dx, dy, dz);
+        min_image(b, dx, dy, dz);
         const double rint = b.rcut_max + ci.w + cj.w;
         cand = code >= 0 && j != i && (b.vdw_minimum || dx * dx + dy * dy + dz * dz <= rint * rint);
       }

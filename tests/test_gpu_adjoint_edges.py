@@ -1,7 +1,8 @@
 """The adjoint's reciprocal and pair kernels at their edges: n_y ranges of two,
 three and four register steps and beyond, boxes of unlike edges, molecules of
 one to eight sites (site groups of three), site counts around a tile, one and
-many frames.  Against the total energy and its central differences."""
+many frames, molecules more than an image away.  Against the total energy and
+its central differences."""
 import numpy as np
 import pytest
 
@@ -65,4 +66,33 @@ def test_adjoint_edges(case):
     fd = [-(ef[1 + 2 * d] - ef[2 + 2 * d]) / (2 * h) for d in range(3)]
     tol = 50.0 * h * h * max(1.0, fmax) + 1e-15 * max(1.0, abs(e0)) * count / h
     assert np.max(np.abs(np.array(fd) - forces.reshape(-1, 3)[site])) <= tol
+    eng.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 3])
+def test_adjoint_of_molecules_images_away(n):
+    """Frames are not folded: a molecule three box lengths off is beyond the one
+    image shift that the energy takes (minimum_image_separation.f90:35-112), so
+    it has no neighbours there, and none in the derivatives."""
+    print(f"[gpu] adjoint images away {n}", flush=True)
+    sp, L = _species(n), 20.0
+    coords = S.place_random([(sp, 40)], [L] * 3, 13, 1.2, 2.6)
+    system = S.System([sp], [40], coords, np.array([L] * 3), 300.0, "lj", "cut", 8.0, charge_style="cut", rcut_coul=8.0,
+                      rcut_low=0.85, name="away").parsed()
+    eng = E.Engine(system, precision=E.FP64)
+    b = eng.add_box(system)
+    xyz = b.download().reshape(-1, 3)
+    far = xyz.copy()
+    far[5 * n:6 * n] += [3 * L, 0.0, 0.0]
+    far[9 * n:10 * n] += [0.0, -3 * L, 3 * L]
+    b.adjoint_set_frames(np.array([xyz, far]))
+    energy, _, _, _, forces = b.adjoint_frames(0, 2, forces=True)
+    for k, x in enumerate((xyz, far)):
+        b.upload(b.spec, b.live, x.ravel())
+        total = b.compute_system_total_energy()["total"]
+        assert abs(energy[k] - total) <= 1e-10 * max(1.0, abs(total))
+    assert abs(energy[0] - energy[1]) > 1.0
+    intra = forces[1].reshape(40, n, 3)[[5, 9]].sum(1)   # no net force from others
+    assert np.max(np.abs(intra)) <= 1e-9 * np.max(np.abs(forces[1]))
     eng.close()
