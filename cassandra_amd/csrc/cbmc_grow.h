@@ -1359,6 +1359,9 @@ __device__ __forceinline__ void fragment_placement(const GrowArgs &a, GrowLds<NT
       int wk = 1;
       if (lane < kd) {
         const int ov = intra_ov ? 2 : S.sov[lane];
+        // an overlapping trial's dihedrals are not taken (:2030-2044): the next
+        // fragment starts from 0 where a deletion keeps one
+        if (ov) ed = 0.0;
         if (!ov) {
           const double qsum = __dadd_rn(iqi, S.sq[lane]);
           e = __dsub_rn(__dadd_rn(__dadd_rn(__dadd_rn(__dadd_rn(ed, iv), iq), S.sv[lane]), qsum), e_prev);
