@@ -627,23 +627,25 @@ extern "C" int cass_rminsq_estimate(int32_t nsolv, int32_t nsolute, int32_t res,
   return CASS_OK;
 }
 
-// One launch of a chain kernel with the live lists of `per` boxes in the
-// dynamic LDS (cap molecules each; 0: in device memory).
-template <typename K, typename A>
-static int launch_chain(cass_engine *e, K kern, const A *d_boxes, int grid, int nt, int64_t nsteps, int cap, int per,
-                        const char *what) {
-  const size_t lds = (size_t)per * cap * kListBytes;
-  HIP_TRY(e, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(nt), lds, e->stream, d_boxes, nsteps, cap);
-  return hipGetLastError() == hipSuccess ? CASS_OK : cass_fail(e, CASS_ERR_HIP, what);
-}
-
 // Live lists of up to this many bytes per workgroup stand in the LDS beside
 // the chain kernels' own 40 to 60 KB; longer ones in device memory.
 constexpr size_t kListLds = (size_t)96 << 10;
 static int list_cap_of(int maxm, int per) {
   const int cap = (maxm + 3) & ~3;
   return (size_t)per * cap * kListBytes <= kListLds ? cap : 0;
+}
+
+// One launch of a chain kernel with the live lists of `per` boxes in the
+// dynamic LDS (cap molecules each; 0: in device memory).
+template <typename K, typename A>
+static int launch_chain(cass_engine *e, K kern, const A *d_boxes, int grid, int nt, int64_t nsteps, int cap, int per,
+                        const char *what) {
+  const size_t lds = (size_t)per * cap * kListBytes;
+  // the attribute belongs to the process: always the largest, so that engines on
+  // other threads never find a smaller one than they launch with
+  HIP_TRY(e, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kListLds));
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(nt), lds, e->stream, d_boxes, nsteps, cap);
+  return hipGetLastError() == hipSuccess ? CASS_OK : cass_fail(e, CASS_ERR_HIP, what);
 }
 
 // workgroup size of the GCMC chain per engine: 0 until cass_gcmc_autotune

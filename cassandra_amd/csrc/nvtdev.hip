@@ -32,6 +32,7 @@ constexpr int kNvtWaves = 12;
 constexpr int kNvtSeg = kKSeg;   // k vectors per segment
 constexpr int kNvtRing = 32;     // generator states kept around the current move
 constexpr int kNvtAhead = 10;    // draws of one move (6 at most, its acceptance, the other start) and some
+constexpr int kNvtStatic = 4096;  // LDS bytes left for the kernel's own
 constexpr int kNvtList = 128;    // entries of a wave's molecule list and of its pair list
 
 struct NvtChainArgs {
@@ -1022,7 +1023,7 @@ int nvt_prepare(cass_engine *e, int32_t box, cass_rng *rng, const cass_nvt_optio
     L.lds = lds;
     L.local = local;
     a.tabled = tabled ? 1 : 0;
-    return lds + 4096 <= (size_t)lds_max;  // beside the kernel's own
+    return lds + kNvtStatic <= (size_t)lds_max;
   };
   // A copy with the phase powers, the box in device memory with them, then
   // both without.  In device memory a move of 512 waters takes 12.4 us for
@@ -1242,8 +1243,13 @@ extern "C" int cass_nvt_run_device_batch(cass_engine *e, int32_t nboxes, const i
   if (!args.empty()) std::memcpy(B.host.data() + B.o_args, args.data(), sizeof(NvtChainArgs) * args.size());
   const NvtChainArgs *d_args = (const NvtChainArgs *)(B.dev + B.o_args);
   HIP_TRY(e, hipMemcpyAsync(B.dev, B.host.data(), B.in, hipMemcpyHostToDevice, e->stream));
+  int lds_max = 0;
+  HIP_TRY(e, hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, e->device));
   for (const Group &g : groups) {
-    HIP_TRY(e, hipFuncSetAttribute((const void *)g.kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)g.lds));
+    // the attribute belongs to the process: always the largest, so that engines
+    // on other threads never find a smaller one than they launch with
+    HIP_TRY(e, hipFuncSetAttribute((const void *)g.kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   lds_max - kNvtStatic));
     for (int64_t s0 = 0; s0 < nsteps; s0 += kNvtChunk) {
       hipLaunchKernelGGL(g.kern, dim3((unsigned)g.count), dim3(64 * kNvtWaves), g.lds, e->stream, d_args + g.first, s0,
                          std::min(kNvtChunk, nsteps - s0));
