@@ -5,6 +5,7 @@
 // the GPU; the host keeps the canonical coordinates and the RNG.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <limits>
@@ -40,7 +41,8 @@ extern "C" int cass_nvt_run(cass_engine *e, int32_t box, cass_rng *rng, const ca
     const double rno = cass_rng_uniform(rng);
     const bool rot = !(rno <= opt->prob_translate);
     (void)cass_rng_uniform(rng);  // species pick (one mobile species)
-    const int im = (int)(cass_rng_uniform(rng) * nm);
+    // rranf can round to 1.0 (random_generators.f90:118): the index is clamped
+    const int im = std::min((int)(cass_rng_uniform(rng) * nm), nm - 1);
     const int m = mols[im];
     const double *xo = b.xyz_h.data() + 3 * (size_t)b.mol_first[m];
     const double4 co = b.comd_h[m];

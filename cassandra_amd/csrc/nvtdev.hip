@@ -240,7 +240,8 @@ __device__ __forceinline__ void nvt_prepare_move(const NvtChainArgs &a, const Nv
   auto draw = [&](int i) { return u[(pos + v + i) & (kNvtRing - 1)]; };
   const int rot = !(draw(0) <= a.prob_translate);
   // draw 1: the species pick (one mobile species)
-  const int m = a.mols[(int)(draw(2) * a.nm)];
+  // rranf can round to 1.0 (random_generators.f90:118): the index is clamped
+  const int m = a.mols[min((int)(draw(2) * a.nm), a.nm - 1)];
   const int f = S.lfirst[m];
   const bool fwd = m == fm;
   double4 co = S.lcomd[m];

@@ -1209,6 +1209,7 @@ int orc_nvt_run(orc_box *b, int64_t s[5], double prob_trans, double max_disp, do
     if (kind) kind[step] = (uint8_t)rot;
     (void)orc_rng_uniform(s);                   /* species pick (:158 / rotate :103) */
     int im = (int)(orc_rng_uniform(s) * nm);  /* molecule pick */
+    if (im > nm - 1) im = nm - 1;             /* rranf can round to 1.0 */
     int m = im;                                 /* locate = identity for a packed box */
     int f = b->mol_first[m];
     double Ev, Eq, Evn, Eqn;

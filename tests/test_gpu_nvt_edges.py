@@ -3,6 +3,8 @@ one and two molecules (the next move takes the molecule just moved), molecule
 pairs of more than 64 site pairs, species of unlike site counts, k vectors
 beyond the lanes' registers, phases without tables, orthogonal boxes, a style
 without its own pair arithmetic, boxes beyond the LDS copy."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -123,3 +125,27 @@ def test_nvt_batch_over_all_paths():
             assert np.array_equal(a[k], b[k]), k
         assert np.array_equal(xa, xb) and ra == rb and a["final"] == b["final"]
         assert 0 < a["accepted"].sum()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("device", [True, False])
+def test_nvt_draw_of_one(device):
+    """rranf rounds its largest words to 1.0 (random_generators.f90:118): a first
+    word for which the third draw, the molecule's, does takes the last molecule"""
+    print(f"[gpu] nvt draw of one, device={device}", flush=True)
+    sp, n = S.species_lj(), 5
+    system = S.System([sp], [n], [_lattice(sp, n, [22.0] * 3)], np.array([22.0] * 3), 150.0, "lj", "cut_tail", 9.0,
+                      rcut_low=0.85, prob_translate=1.0, max_disp=0.4, name="lj").parsed()
+    eng = E.Engine(system, precision=E.FP64)
+    box = eng.add_box(system)
+    rng = E.rng(101, 203)
+    rng.s[0] = 4707937272820449914
+    probe = E.rng(101, 203)
+    probe.s[0] = rng.s[0]
+    assert [eng.lib.cass_rng_uniform(C.byref(probe)) for _ in range(3)][2] == 1.0
+    before = box.download().reshape(n, 3)
+    out = box.nvt_run(rng, 1, box.compute_system_total_energy(), device=device)
+    assert out["accepted"][0]
+    moved = np.any(box.download().reshape(n, 3) != before, axis=1)
+    assert list(np.flatnonzero(moved)) == [n - 1]
+    eng.close()
