@@ -2,7 +2,8 @@
 three and four register steps and beyond, boxes of unlike edges, molecules of
 one to eight sites (site groups of three), site counts around a tile, one and
 many frames, molecules more than an image away.  Against the total energy and
-its central differences."""
+its central differences in the coordinates, the types' parameters and the
+charges."""
 import numpy as np
 import pytest
 
@@ -42,7 +43,7 @@ def test_adjoint_edges(case):
     b = eng.add_box(system)
     b.ewald_setup()
     e0 = b.compute_system_total_energy()["total"]
-    energy, _, _, dq, forces = b.adjoint()
+    energy, deps, dsig, dq, forces = b.adjoint()
     assert abs(energy - e0) <= 1e-10 * max(1.0, abs(e0))
     # frames: the box's own coordinates and shifted ones; each equal to one alone
     xyz = b.download().reshape(-1, 3)
@@ -66,6 +67,32 @@ def test_adjoint_edges(case):
     fd = [-(ef[1 + 2 * d] - ef[2 + 2 * d]) / (2 * h) for d in range(3)]
     tol = 50.0 * h * h * max(1.0, fmax) + 1e-15 * max(1.0, abs(e0)) * count / h
     assert np.max(np.abs(np.array(fd) - forces.reshape(-1, 3)[site])) <= tol
+    # the derivatives by the parameters, as the total energy has them
+    eps, sig, _, _ = system.type_tables()
+    charge = np.array([a.charge for a in sp.atoms])
+
+    def total(eps_t=None, sig_t=None, q=None):
+        e = None if eps_t is None else np.sqrt(np.outer(eps_t, eps_t))
+        g = None if sig_t is None else 0.5 * (sig_t[:, None] + sig_t[None, :])
+        eng.set_nonbond_params(eps if e is None else e, sig if g is None else g, charge if q is None else q)
+        return b.compute_system_total_energy()["total"]
+
+    # four-point differences of relative step 1e-3.  A term of order sigma^12 is off
+    # by h^4 / 30 of its fifth derivative, 12 * 11 * 10 * 9 * 8 / 30 * 1e-12 = 3e-9
+    # of itself over x, one of order sqrt(eps) or q^2 by less; rounding adds eps |U|
+    # / (x h), 1e-13 of it.  The derivative and U are differences of sums of such
+    # terms, taken to be within 30 of |grad| + |U| / x.
+    for name, grad, x in (("eps_t", deps, np.diag(eps)), ("sig_t", dsig, np.diag(sig)), ("q", dq, charge)):
+        for k in range(len(x)):
+            scale = max(abs(x[k]), 0.1)
+
+            def at(steps):
+                y = x.copy()
+                y[k] += steps * 1e-3 * scale
+                return total(**{name: y})
+
+            fd = (8 * (at(1) - at(-1)) - (at(2) - at(-2))) / (12e-3 * scale)
+            assert abs(fd - grad[k]) <= 1e-7 * (np.max(np.abs(grad)) + abs(e0) / scale), (name, k)
     eng.close()
 
 

@@ -2,8 +2,9 @@
 molecule counts around a workgroup's four and a wave's 64, one site to 40 (the
 phase table is exceeded), few molecules whose k vectors several workgroups
 share, unlike species, unlike edges, dead molecules.  Pair
-terms against half the sum of the molecules' own energies, the reciprocal term
-against numpy's direct sum, one box and a batch."""
+terms against half the sum of the molecules' own energies (and, for charges, the
+molecules' periodic part), the reciprocal term against numpy's direct sum, one
+box and a batch."""
 import numpy as np
 import pytest
 
@@ -72,13 +73,19 @@ def test_total_energy_edges(case, prec):
     tol = REL if prec == E.FP64 else 1e-8
     for b, lv, got in zip(boxes, (np.ones(len(nat), dtype=int), live), batch):
         one = b.compute_system_total_energy()
-        assert all(one[k] == got[k] for k in ("total", "inter_vdw", "reciprocal"))
-        half = np.zeros(2)
+        assert all(one[k] == got[k] for k in ("total", "inter_vdw", "inter_q", "reciprocal"))
+        half, first = np.zeros(2), np.concatenate([[0], np.cumsum(nat)])
+        periodic = 0.0
         for m in np.flatnonzero(lv):
             ev, eq, ov = b.compute_molecule_nonbond_inter_energy(int(m))
             assert not ov
             half += 0.5 * np.array([ev, eq])
+            sp = int(b.spec[m])
+            periodic += b.compute_molecule_nonbond_intra_energy(sp, xyz.reshape(-1, 3)[first[m]:first[m + 1]])[2]
         assert abs(one["inter_vdw"] - half[0]) <= tol * max(1.0, abs(half[0]))
+        # (the two parts cancel in part: the tolerance is that of the larger)
+        q_ref = half[1] + periodic
+        assert abs(one["inter_q"] - q_ref) <= tol * max(1.0, abs(half[1]), abs(periodic))
         weight = np.repeat(lv, nat) * charges
         ref = _reciprocal(system, xyz.reshape(-1, 3), weight)
         assert abs(one["reciprocal"] - ref) <= tol * max(1.0, abs(ref))
