@@ -385,14 +385,14 @@ static int widom_cbmc(cass_engine *e, int32_t box, int32_t species, int64_t n_in
   if (b.p.charge_style != CASS_Q_NONE && species_has_charge(e, species)) cass_mol_self_energy(e, box, species, &e_self);
   const int nsub = n_sub > 0 ? n_sub : 1;
   const int64_t rsq_stride = rsq_min ? (int64_t)e->natoms_total * e->sp_natoms[species] : 0;
-  const size_t live_bytes = (sizeof(double4) + sizeof(LiveMol)) * (size_t)b.nmols + 64;
+  const size_t live_bytes = (kCentre + sizeof(LiveMol)) * (size_t)b.nmols + 64;
   const size_t need = (size_t)n_ins * (2 * sizeof(double) + 1) + sizeof(double) * (nsub + 2) + 64 +
                       5 * sizeof(int64_t) + sizeof(double) * (size_t)(n_ins * rsq_stride) + live_bytes;
   char *s = (char *)cass_scratch(e, need);
   if (!s) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
   // the frame's live molecules, then the per-insertion arrays
-  double4 *d_lcom = (double4 *)s;
-  LiveMol *d_lmol = (LiveMol *)(d_lcom + b.nmols);
+  double *d_lcom = (double *)s;
+  LiveMol *d_lmol = (LiveMol *)(d_lcom + 4 * (size_t)b.nmols);
   int *d_nlive = (int *)(d_lmol + b.nmols);
   double *d_w = (double *)(s + (live_bytes & ~(size_t)15));
   double *d_em = d_w + n_ins;
@@ -413,7 +413,7 @@ static int widom_cbmc(cass_engine *e, int32_t box, int32_t species, int64_t n_in
   w.eij_max = eij_max ? d_em : nullptr;
   w.rsq_min = rsq_min ? d_rsq : nullptr;
   w.rsq_rows = e->natoms_total;
-  w.live = LiveList{d_lmol, d_lcom};
+  w.live = LiveList{d_lmol, d_lcom, b.nmols};
   w.nlive = d_nlive;
   if (rng) HIP_TRY(e, hipMemcpyAsync(d_rng, rng->s, sizeof(int64_t) * 5, hipMemcpyHostToDevice, e->stream));
   HIP_TRY(e, hipEventRecord(e->ev0, e->stream));
@@ -733,7 +733,7 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
   // the live lists, at the end: not copied to or from the host
   const int list_cap = list_cap_of(maxm, gemc ? 2 : 1);
   const size_t state_bytes = bytes;
-  if (list_cap == 0) bytes += (up(sizeof(double4) * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)nboxes;
+  if (list_cap == 0) bytes += (up(kCentre * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)nboxes;
   char *s0 = (char *)cass_scratch(e, bytes + recs.staged() + 256);
   if (!s0) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
   if (int rrc = recs.place(e, s0 + bytes)) return rrc;
@@ -805,9 +805,9 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
     a.rec_nmols = rec ? recs.at<int>(o.nm) : nullptr;
     a.rec_energy = rec ? recs.at<double>(o.ren) : nullptr;
     a.rec_rng = rec ? recs.at<int64_t>(o.rr) : nullptr;
-    const size_t o_list = state_bytes + (up(sizeof(double4) * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)i;
-    a.list = list_cap ? LiveList{nullptr, nullptr}
-                      : LiveList{(LiveMol *)(s0 + o_list + up(sizeof(double4) * maxm)), (double4 *)(s0 + o_list)};
+    const size_t o_list = state_bytes + (up(kCentre * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)i;
+    a.list = list_cap ? LiveList{nullptr, nullptr, 0}
+                      : LiveList{(LiveMol *)(s0 + o_list + up(kCentre * maxm)), (double *)(s0 + o_list), maxm};
   }
   const size_t o_args = take(sizeof(GcmcBoxArgs) * nboxes);
   if (off > state_bytes) return cass_fail(e, CASS_ERR_STATE, "GCMC state layout exceeds its buffer");
@@ -926,7 +926,7 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
   bytes += up(sizeof(RegrowBoxArgs) * nboxes);
   const int list_cap = list_cap_of(maxm, 1);
   const size_t state_bytes = bytes;
-  if (list_cap == 0) bytes += (up(sizeof(double4) * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)nboxes;
+  if (list_cap == 0) bytes += (up(kCentre * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)nboxes;
   char *s0 = (char *)cass_scratch(e, bytes + pull.staged() + 256);
   if (!s0) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
   if (int prc = pull.place(e, s0 + bytes)) return prc;
@@ -967,9 +967,9 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
     a.rec_energy = r && r->energy ? pull.at<double>(o.ren) : nullptr;
     a.ln_pacc = r && r->ln_pacc ? pull.at<double>(o.lp) : nullptr;
     a.rec_rng = r && r->rng_state ? pull.at<int64_t>(o.rr) : nullptr;
-    const size_t o_list = state_bytes + (up(sizeof(double4) * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)i;
-    a.list = list_cap ? LiveList{nullptr, nullptr}
-                      : LiveList{(LiveMol *)(s0 + o_list + up(sizeof(double4) * maxm)), (double4 *)(s0 + o_list)};
+    const size_t o_list = state_bytes + (up(kCentre * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)i;
+    a.list = list_cap ? LiveList{nullptr, nullptr, 0}
+                      : LiveList{(LiveMol *)(s0 + o_list + up(kCentre * maxm)), (double *)(s0 + o_list), maxm};
   }
   const size_t o_args = take(sizeof(RegrowBoxArgs) * nboxes);
   if (off > state_bytes) return cass_fail(e, CASS_ERR_STATE, "regrowth state layout exceeds its buffer");

@@ -83,7 +83,17 @@ struct LiveMol {
 // The live molecules of one box, in LDS or in device memory.
 struct LiveList {
   LiveMol *mol;
-  double4 *com;  // (x, y, z, max_dcom)
+  double *com;  // x[cap], y[cap], z[cap], max_dcom[cap]: lanes on neighbouring entries read without bank conflicts
+  int cap;
+  __device__ __forceinline__ double4 centre(int i) const {
+    return make_double4(com[i], com[cap + i], com[2 * cap + i], com[3 * cap + i]);
+  }
+  __device__ __forceinline__ void put(int i, double4 c) const {
+    com[i] = c.x;
+    com[cap + i] = c.y;
+    com[2 * cap + i] = c.z;
+    com[3 * cap + i] = c.w;
+  }
 };
 
 constexpr int kRing = 128;   // random draws held ready
@@ -323,7 +333,7 @@ __device__ __forceinline__ int build_live_list(const GrowArgs &a, const LiveList
       const int p = n + __popcll(m & ((1ull << wl) - 1ull));
       const double *c = (const double *)(a.b.comd + j);
       l.mol[p] = LiveMol{j, (a.b.first[j] << 4) | (a.b.species[j] & 15)};
-      l.com[p] = make_double4(vld(c), vld(c + 1), vld(c + 2), vld(c + 3));
+      l.put(p, make_double4(vld(c), vld(c + 1), vld(c + 2), vld(c + 3)));
     }
     n += __popcll(m);
   }
@@ -341,10 +351,12 @@ __device__ __forceinline__ int live_find(const LiveList &l, int n, int m) {
 }
 
 // Check_MoleculePair_Cutoff (energy_routines.f90:3027-3088) for the walk of a
-// stage, on squared distances (molpair_in_range takes the root as the
-// reference does; the two differ only at the prefilter distance itself, where
-// every site pair lies beyond the cutoff): reach is the cutoff and the trial's
-// max_dcom.
+// stage, in double precision: reach is the cutoff and the trial's max_dcom.
+// Squared distances where molpair_in_range takes the root as the reference
+// does, and in cubic boxes the nearest image where the reference shifts by one
+// box length: the two differ at the prefilter distance itself and for centres
+// more than 1.5 lengths apart, where every site pair that the walk then meets
+// (with the one shift) lies beyond the cutoff.
 struct Reach {
   double x, y, z, r;
 };
@@ -356,7 +368,13 @@ __device__ __forceinline__ Reach make_reach(const BoxDev &b, bool cbmc, double4 
 __device__ __forceinline__ bool in_reach(const BoxDev &b, const Reach &r, double4 c) {
   if (b.vdw_minimum) return true;
   double dx = r.x - c.x, dy = r.y - c.y, dz = r.z - c.z;
-  min_image(b, dx, dy, dz);
+  if (b.cubic) {
+    dx = fma(-rint(dx * b.Li[0]), b.L[0], dx);
+    dy = fma(-rint(dy * b.Li[4]), b.L[1], dy);
+    dz = fma(-rint(dz * b.Li[8]), b.L[2], dz);
+  } else {
+    min_image(b, dx, dy, dz);
+  }
   const double q = r.r + c.w;
   return dx * dx + dy * dy + dz * dz <= q * q;
 }
@@ -539,7 +557,7 @@ __device__ __forceinline__ void stage_trials(const GrowArgs &a, GrowLds<NT> &S, 
     for (int s0 = 0; s0 < nl; s0 += 64) {
       const int i = s0 + wl;
       bool in = false;
-      if (i < nl) in = in_reach(a.b, r, l.com[i]) && l.mol[i].slot != self;
+      if (i < nl) in = in_reach(a.b, r, l.centre(i)) && l.mol[i].slot != self;
       const uint64_t m = __builtin_amdgcn_ballot_w64(in);
       if (in) cl[cnt + __popcll(m & ((1ull << wl) - 1ull))] = i;
       cnt += __popcll(m);
@@ -585,7 +603,7 @@ __device__ __forceinline__ void stage_full(const GrowArgs &a, GrowLds<NT> &S, co
     // a lane takes whole molecules
     for (int i = w * 64 + wl; i < nl; i += NT) {
       const int j = l.mol[i].slot;
-      if (j == self || !in_reach(b, r, l.com[i])) continue;
+      if (j == self || !in_reach(b, r, l.centre(i))) continue;
       int spa[kCbA];
       for (int q = 0; q < na; ++q) spa[q] = S.sp.spa0 + q;
       ov = molpair_energy<P>(b, a.tp, a.cd, a.cf, false, S.sp.coul_cbmc != 0, na, S.x, S.y, S.z, spa, j, ev, eq,
@@ -599,7 +617,7 @@ __device__ __forceinline__ void stage_full(const GrowArgs &a, GrowLds<NT> &S, co
       const int c = fast_div(it, nj, rnj, big), ja = it - c * nj;
       const LiveMol m = l.mol[c];
       const int sj = m.fs & 15;
-      if (m.slot == self || ja >= S.ct.sp_natoms[sj] || !in_reach(b, r, l.com[c])) continue;
+      if (m.slot == self || ja >= S.ct.sp_natoms[sj] || !in_reach(b, r, l.centre(c))) continue;
       const int f = (m.fs >> 4) + ja, o = S.ct.sp_atom_off[sj] + ja;
       const double xj = b.x[f], yj = b.y[f], zj = b.z[f], qj = LJ ? 0.0 : S.ct.atom_charge[o];
       const int tj = S.ct.atom_type[o];
@@ -1623,14 +1641,15 @@ __device__ __forceinline__ int accept_or_reject(const GrowLds<NT> &S, GrowReg &G
 
 // Where a chain kernel keeps its lists: cap > 0: in the dynamic LDS, per box
 // the centres, the entries, then (gcmc) locate and reservoir.
-constexpr size_t kListBytes = sizeof(double4) + sizeof(LiveMol) + 2 * sizeof(int);
+constexpr size_t kCentre = 4 * sizeof(double);
+constexpr size_t kListBytes = kCentre + sizeof(LiveMol) + 2 * sizeof(int);
 __device__ __forceinline__ LiveList chain_list(char *dyn, int cap, int box, const LiveList &g) {
   if (cap == 0) return g;
   char *p = dyn + (size_t)box * cap * kListBytes;
-  return LiveList{(LiveMol *)(p + sizeof(double4) * cap), (double4 *)p};
+  return LiveList{(LiveMol *)(p + kCentre * cap), (double *)p, cap};
 }
 __device__ __forceinline__ int *chain_slots(char *dyn, int cap, int box, int which) {
-  return (int *)(dyn + (size_t)box * cap * kListBytes + (sizeof(double4) + sizeof(LiveMol)) * cap) + which * cap;
+  return (int *)(dyn + (size_t)box * cap * kListBytes + (kCentre + sizeof(LiveMol)) * cap) + which * cap;
 }
 
 // Removes entry im of locate[0 .. n): the later ones move down (whole wave).
@@ -1649,7 +1668,7 @@ __device__ __forceinline__ void locate_remove(int *locate, int im, int n) {
 __device__ __forceinline__ void list_add(const LiveList &l, int &n, const BoxDev &b, int m, double4 com) {
   if (threadIdx.x == 0) {
     l.mol[n] = LiveMol{m, (b.first[m] << 4) | (b.species[m] & 15)};
-    l.com[n] = com;
+    l.put(n, com);
   }
   ++n;
 }
@@ -1659,12 +1678,12 @@ __device__ __forceinline__ void list_drop(const LiveList &l, int &n, int m) {
   --n;
   if (threadIdx.x == 0) {
     l.mol[p] = l.mol[n];
-    l.com[p] = l.com[n];
+    l.put(p, l.centre(n));
   }
 }
 __device__ __forceinline__ void list_move(const LiveList &l, int n, int m, double4 com) {
   const int p = live_find(l, n, m);
-  if (p >= 0 && threadIdx.x == 0) l.com[p] = com;
+  if (p >= 0 && threadIdx.x == 0) l.put(p, com);
 }
 
 // Copies a slot list between device memory and LDS (wave 0).
