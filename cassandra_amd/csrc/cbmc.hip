@@ -730,14 +730,16 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
     }
   }
   bytes += up(sizeof(GcmcBoxArgs) * nboxes);
-  // the live lists, at the end: not copied to or from the host
+  // the records, then the live lists, which are not copied to or from the host
   const int list_cap = list_cap_of(maxm, gemc ? 2 : 1);
   const size_t state_bytes = bytes;
+  bytes += recs.staged();
+  const size_t list_at = bytes;
   if (list_cap == 0) bytes += (up(kCentre * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)nboxes;
-  char *s0 = (char *)cass_scratch(e, bytes + recs.staged() + 256);
+  char *s0 = (char *)cass_scratch(e, bytes + 256);
   if (!s0) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
-  if (int rrc = recs.place(e, s0 + bytes)) return rrc;
-  std::vector<char> host(state_bytes + 256, 0);
+  if (int rrc = recs.place(e, s0 + state_bytes)) return rrc;
+  std::vector<char> host(state_bytes, 0);
   size_t off = 0;
   auto take = [&](size_t n) {
     const size_t o = off;
@@ -805,12 +807,12 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
     a.rec_nmols = rec ? recs.at<int>(o.nm) : nullptr;
     a.rec_energy = rec ? recs.at<double>(o.ren) : nullptr;
     a.rec_rng = rec ? recs.at<int64_t>(o.rr) : nullptr;
-    const size_t o_list = state_bytes + (up(kCentre * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)i;
+    const size_t o_list = list_at + (up(kCentre * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)i;
     a.list = list_cap ? LiveList{nullptr, nullptr, 0}
                       : LiveList{(LiveMol *)(s0 + o_list + up(kCentre * maxm)), (double *)(s0 + o_list), maxm};
   }
   const size_t o_args = take(sizeof(GcmcBoxArgs) * nboxes);
-  if (off > state_bytes) return cass_fail(e, CASS_ERR_STATE, "GCMC state layout exceeds its buffer");
+  if (off != state_bytes) return cass_fail(e, CASS_ERR_STATE, "GCMC state layout differs from its buffer");
   MirrorPull mirrors;
   std::vector<int> ids(commit ? nboxes : 0);
   for (size_t i = 0; i < ids.size(); ++i) ids[i] = boxes[i].box;
@@ -835,8 +837,8 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
   // the states and, unless this is a timing run, coordinates, live flags and
   // centres of every box come back behind one synchronisation
   if (int mrc = mirrors.queue(e)) return mrc;
-  HIP_TRY(e, hipMemcpyAsync(mirrors.host, s0, off, hipMemcpyDeviceToHost, e->stream));
-  if (int mrc = recs.queue(e, mirrors.host + off)) return mrc;
+  HIP_TRY(e, hipMemcpyAsync(mirrors.host, s0, off + recs.staged(), hipMemcpyDeviceToHost, e->stream));
+  if (int mrc = recs.queue(e)) return mrc;
   HIP_TRY(e, hipStreamSynchronize(e->stream));
   float ms = 0.f;
   if (hipEventElapsedTime(&ms, e->ev0, e->ev1) == hipSuccess) e->last_kernel_ms = ms;
@@ -926,11 +928,13 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
   bytes += up(sizeof(RegrowBoxArgs) * nboxes);
   const int list_cap = list_cap_of(maxm, 1);
   const size_t state_bytes = bytes;
+  bytes += pull.staged();
+  const size_t list_at = bytes;
   if (list_cap == 0) bytes += (up(kCentre * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)nboxes;
-  char *s0 = (char *)cass_scratch(e, bytes + pull.staged() + 256);
+  char *s0 = (char *)cass_scratch(e, bytes + 256);
   if (!s0) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
-  if (int prc = pull.place(e, s0 + bytes)) return prc;
-  std::vector<char> host(state_bytes + 256, 0);
+  if (int prc = pull.place(e, s0 + state_bytes)) return prc;
+  std::vector<char> host(state_bytes, 0);
   size_t off = 0;
   auto take = [&](size_t n) {
     const size_t o = off;
@@ -967,12 +971,12 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
     a.rec_energy = r && r->energy ? pull.at<double>(o.ren) : nullptr;
     a.ln_pacc = r && r->ln_pacc ? pull.at<double>(o.lp) : nullptr;
     a.rec_rng = r && r->rng_state ? pull.at<int64_t>(o.rr) : nullptr;
-    const size_t o_list = state_bytes + (up(kCentre * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)i;
+    const size_t o_list = list_at + (up(kCentre * maxm) + up(sizeof(LiveMol) * maxm)) * (size_t)i;
     a.list = list_cap ? LiveList{nullptr, nullptr, 0}
                       : LiveList{(LiveMol *)(s0 + o_list + up(kCentre * maxm)), (double *)(s0 + o_list), maxm};
   }
   const size_t o_args = take(sizeof(RegrowBoxArgs) * nboxes);
-  if (off > state_bytes) return cass_fail(e, CASS_ERR_STATE, "regrowth state layout exceeds its buffer");
+  if (off != state_bytes) return cass_fail(e, CASS_ERR_STATE, "regrowth state layout differs from its buffer");
   MirrorPull mirrors;
   std::vector<int> ids(nboxes);
   for (int i = 0; i < nboxes; ++i) ids[i] = boxes[i].box;
@@ -987,8 +991,8 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
   if (rc) return rc;
   HIP_TRY(e, hipEventRecord(e->ev1, e->stream));
   if (int mrc = mirrors.queue(e)) return mrc;
-  HIP_TRY(e, hipMemcpyAsync(mirrors.host, s0, off, hipMemcpyDeviceToHost, e->stream));
-  if (int prc = pull.queue(e, mirrors.host + off)) return prc;
+  HIP_TRY(e, hipMemcpyAsync(mirrors.host, s0, off + pull.staged(), hipMemcpyDeviceToHost, e->stream));
+  if (int prc = pull.queue(e)) return prc;
   HIP_TRY(e, hipStreamSynchronize(e->stream));
   mirrors.end(e);
   pull.end(mirrors.host + off);

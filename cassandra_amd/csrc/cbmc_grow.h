@@ -1724,6 +1724,7 @@ __global__ void __launch_bounds__(NT) k_gcmc_chain(const GcmcBoxArgs *__restrict
   // wave 0's registers
   GrowReg G{};
   int nmols = 0, nres = 0, nl = 0, stop = 0;
+  int64_t done = 0;  // moves recorded
   double nb = 0.0, beads = 0.0;
   if (lane < 64) {
     nmols = ufi(vld(a.nmols));
@@ -1908,6 +1909,7 @@ __global__ void __launch_bounds__(NT) k_gcmc_chain(const GcmcBoxArgs *__restrict
       }
     }
     if (lane < 64 && !stop) {
+      done = st + 1;
       wave_sync();
       if (lane == 0) {
         if (a.kind) a.kind[st] = (uint8_t)(del ? 1 : 0);
@@ -1927,6 +1929,11 @@ __global__ void __launch_bounds__(NT) k_gcmc_chain(const GcmcBoxArgs *__restrict
       copy_slots(a.reservoir, reservoir, nres);
     }
     if (lane < nt) a.nbeads[lane] = nb;
+    record_rest(a.kind, done, nsteps);
+    record_rest(a.accepted, done, nsteps);
+    record_rest(a.rec_nmols, done, nsteps);
+    record_rest(a.rec_energy, done, nsteps);
+    record_rest(a.rec_rng, 5 * done, 5 * nsteps);
     if (lane == 0) {
       *a.nmols = nmols;
       *a.nres = stop ? -1 : nres;
@@ -1972,6 +1979,7 @@ __global__ void __launch_bounds__(NT) k_gemc_chain(const GcmcBoxArgs *__restrict
   // wave 0's registers
   GrowReg G{};
   int nm0 = 0, nm1 = 0, nr0 = 0, nr1 = 0, stop = 0;
+  int64_t done = 0;  // moves recorded
   double nb0 = 0.0, nb1 = 0.0, beads = 0.0;
   if (lane < 64) {
     nm0 = ufi(vld(A[0].nmols));
@@ -2252,6 +2260,7 @@ __global__ void __launch_bounds__(NT) k_gemc_chain(const GcmcBoxArgs *__restrict
       }
     }
     if (lane < 64 && !stop) {
+      done = st + 1;
       wave_sync();
       for (int b = 0; b < 2; ++b) {
         const GcmcBoxArgs &a = A[b];
@@ -2276,6 +2285,11 @@ __global__ void __launch_bounds__(NT) k_gemc_chain(const GcmcBoxArgs *__restrict
         copy_slots(a.reservoir, b ? res1 : res0, b ? nr1 : nr0);
       }
       if (lane < nt) a.nbeads[lane] = b ? nb1 : nb0;
+      record_rest(a.kind, done, nsteps);
+      record_rest(a.accepted, done, nsteps);
+      record_rest(a.rec_nmols, done, nsteps);
+      record_rest(a.rec_energy, done, nsteps);
+      record_rest(a.rec_rng, 5 * done, 5 * nsteps);
       if (lane == 0) {
         *a.nmols = b ? nm1 : nm0;
         *a.nres = stop ? -1 : (b ? nr1 : nr0);
@@ -2375,6 +2389,7 @@ __global__ void __launch_bounds__(NT) k_regrow_chain(const RegrowBoxArgs *__rest
   const int nl = ufi(q_nl), natoms = ufi(c.natoms);
   const double beta = a.g.beta;
   int state = 0;
+  int64_t done = 0;  // moves recorded
   for (int64_t st = 0; st < nsteps; ++st) {
     int flive = 0, fdead = 0;
     double xo = 0.0, yo = 0.0, zo = 0.0;  // lane k: atom k as it was
@@ -2497,6 +2512,7 @@ __global__ void __launch_bounds__(NT) k_regrow_chain(const RegrowBoxArgs *__rest
       if (cov2) break;
     }
     if (lane < 64) {
+      done = st + 1;
       wave_sync();
       if (lane == 0) {
         if (a.kind) a.kind[st] = 2;
@@ -2511,6 +2527,11 @@ __global__ void __launch_bounds__(NT) k_regrow_chain(const RegrowBoxArgs *__rest
     wave_sync();
     if (lane < 5) a.rng[lane] = S.rw[lane][G.rpos & (kRing - 1)];
     if (lane < 14) a.energy[lane] = E[lane];
+    record_rest(a.kind, done, nsteps);
+    record_rest(a.accepted, done, nsteps);
+    record_rest(a.rec_energy, done, nsteps);
+    record_rest(a.ln_pacc, done, nsteps);
+    record_rest(a.rec_rng, 5 * done, 5 * nsteps);
     if (lane == 0) *a.status = state == 2 ? 1 : 0;
   }
 }

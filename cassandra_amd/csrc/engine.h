@@ -166,25 +166,26 @@ struct MirrorPull {
   char *dev = nullptr;
 };
 // Per-move records of a chain batch, on their way from the device to the
-// caller's arrays.  Up to kRecordStage bytes of them go through the batch's
-// scratch and pinned staging in one copy; more, from a stream allocation that
-// is given back, are copied straight into the caller's arrays, so that the
-// engine keeps no memory that grows with the moves of a call.
+// caller's arrays.  Up to kRecordStage bytes of them stand behind the batch's
+// states, in its scratch and its pinned staging, and come back in their copy;
+// more, from a stream allocation that is given back, are copied straight into
+// the caller's arrays, so that the engine keeps no memory that grows with the
+// moves of a call.  The kernels write every record of a launch (record_rest).
 constexpr size_t kRecordStage = (size_t)16 << 20;
 struct ChainRecords {
   ~ChainRecords();
   // one array of `bytes` for dst; returns its place for at()
   size_t add(void *dst, size_t bytes);
   size_t staged() const { return total <= kRecordStage ? total : 0; }
-  // zeroed device memory: `room`, with staged() bytes of it, or its own
+  // device memory: `room`, with staged() bytes of it, or its own
   int place(cass_engine *e, char *room);
   template <typename T>
   T *at(size_t off) const {
     return (T *)(dev + off);
   }
-  // queues the copies, through `pinned` where staged; end() after the
-  // synchronisation
-  int queue(cass_engine *e, char *pinned);
+  // queues the copies where the records are not staged; end(), after the
+  // synchronisation, takes those that are from `pinned`
+  int queue(cass_engine *e);
   void end(const char *pinned);
 
  private:

@@ -826,16 +826,11 @@ int ChainRecords::place(cass_engine *e, char *room) {
     }
     owner = e;
   }
-  HIP_TRY(e, hipMemsetAsync(dev, 0, total, e->stream));
   return CASS_OK;
 }
 
-int ChainRecords::queue(cass_engine *e, char *pinned) {
-  if (total == 0) return CASS_OK;
-  if (staged()) {
-    HIP_TRY(e, hipMemcpyAsync(pinned, dev, total, hipMemcpyDeviceToHost, e->stream));
-    return CASS_OK;
-  }
+int ChainRecords::queue(cass_engine *e) {
+  if (staged()) return CASS_OK;
   for (const Part &p : parts)
     if (p.bytes) HIP_TRY(e, hipMemcpyAsync(p.dst, dev + p.off, p.bytes, hipMemcpyDeviceToHost, e->stream));
   return CASS_OK;

@@ -94,6 +94,14 @@ __device__ inline double wave_total(double v) {
                           __builtin_amdgcn_readlane(__double2loint(v), 63));
 }
 
+// Zeroes the records [from, to) of one array (null: none), by the lanes of one
+// wave: what a chain that stops leaves unwritten.
+template <typename T>
+__device__ inline void record_rest(T *p, int64_t from, int64_t to) {
+  if (p)
+    for (int64_t k = from + (threadIdx.x & 63); k < to; k += 64) p[k] = T(0);
+}
+
 // ------------------------------------------------------------- geometry
 __device__ inline void min_image(const BoxDev &b, double &dx, double &dy, double &dz) {
   // minimum_image_separation.f90:35-112: cubic boxes shift by one box length

@@ -616,6 +616,12 @@ __device__ __forceinline__ void nvt_chain_run(const NvtChainArgs &a, int64_t ste
         const NvtOutcome r = nvt_decide(a, red[st & 1], redf[st & 1], nc, rot, uring[pos & (kNvtRing - 1)], en);
         if (r.stop) {
           if (lane == 0) *a.status = 1;
+          const int64_t from = step0 + st, to = step0 + nsteps;
+          record_rest(a.kind, from, to);
+          record_rest(a.accepted, from, to);
+          record_rest(a.energy, from, to);
+          record_rest(a.ln_pacc, from, to);
+          record_rest(a.rng_state, 5 * from, 5 * to);
           break;
         }
         pos += r.drawn;
@@ -1095,13 +1101,13 @@ struct NvtState {
   int status[2];
 };
 
-// The buffers of a batch, laid out over all its chains: first the states, which
-// come back, then the mobile lists and argument tables, then the records.  One
-// copy in, one or two out: with a set of copies per chain the calls themselves
-// outlasted the chains.
+// The buffers of a batch, laid out over all its chains: first the mobile lists
+// and argument tables, then the states, then the records.  One copy in, of all
+// but the records, and one out, of the states and records: with a set of copies
+// per chain the calls themselves outlasted the chains.
 struct NvtBuffers {
   char *dev = nullptr;
-  size_t back = 0, in = 0;  // bytes of the states; with the lists and arguments
+  size_t o_back = 0, in = 0;  // where the states begin; where they end
   size_t o_args = 0;
   std::vector<char> host;   // the first `in` bytes
   ChainRecords rec;
@@ -1114,6 +1120,13 @@ int nvt_buffers(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, NvtB
     off = (off + bytes + 255) & ~(size_t)255;
     return o;
   };
+  for (NvtLaunch &L : Ls)
+    if (!L.host_loop) {
+      L.o_mols = take(sizeof(int) * L.mols.size());
+      if (!L.local) L.o_meta = take(sizeof(int) * e->boxes[L.box].nmols);
+    }
+  B.o_args = take(sizeof(NvtChainArgs) * std::max<size_t>(1, Ls.size()));
+  B.o_back = off;
   const size_t ns = (size_t)nsteps;
   for (NvtLaunch &L : Ls) {
     if (L.host_loop) continue;
@@ -1125,13 +1138,6 @@ int nvt_buffers(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, NvtB
     if (rec && rec->ln_pacc) L.o_lnp = B.rec.add(rec->ln_pacc, sizeof(double) * ns);
     if (rec && rec->rng_state) L.o_rs = B.rec.add(rec->rng_state, sizeof(int64_t) * 5 * ns);
   }
-  B.back = off;
-  for (NvtLaunch &L : Ls)
-    if (!L.host_loop) {
-      L.o_mols = take(sizeof(int) * L.mols.size());
-      if (!L.local) L.o_meta = take(sizeof(int) * e->boxes[L.box].nmols);
-    }
-  B.o_args = take(sizeof(NvtChainArgs) * std::max<size_t>(1, Ls.size()));
   B.in = off;
   B.dev = (char *)cass_scratch(e, off + B.rec.staged() + 256);
   if (!B.dev) return cass_fail(e, CASS_ERR_NOMEM, "scratch");
@@ -1167,11 +1173,12 @@ int nvt_buffers(cass_engine *e, std::vector<NvtLaunch> &Ls, int64_t nsteps, NvtB
 // records, the moved coordinates and centres.
 int nvt_finish(cass_engine *e, std::vector<NvtLaunch> &Ls, NvtBuffers &B, MirrorPull &mirrors) {
   if (int rc = mirrors.queue(e)) return rc;
-  if (B.back) HIP_TRY(e, hipMemcpyAsync(mirrors.host, B.dev, B.back, hipMemcpyDeviceToHost, e->stream));
-  if (int rc = B.rec.queue(e, mirrors.host + B.back)) return rc;
+  const size_t back = B.in - B.o_back + B.rec.staged();
+  if (back) HIP_TRY(e, hipMemcpyAsync(mirrors.host, B.dev + B.o_back, back, hipMemcpyDeviceToHost, e->stream));
+  if (int rc = B.rec.queue(e)) return rc;
   HIP_TRY(e, hipStreamSynchronize(e->stream));
   mirrors.end(e);
-  B.rec.end(mirrors.host + B.back);
+  B.rec.end(mirrors.host + (B.in - B.o_back));
   ++e->gen;
   bool bad = false;
   for (NvtLaunch &L : Ls) {
@@ -1179,7 +1186,7 @@ int nvt_finish(cass_engine *e, std::vector<NvtLaunch> &Ls, NvtBuffers &B, Mirror
     cass_box_state &b = e->boxes[L.box];
     const char *h = mirrors.host;
     NvtState st;
-    std::memcpy(&st, h + L.o_state, sizeof(st));
+    std::memcpy(&st, h + (L.o_state - B.o_back), sizeof(st));
     std::memcpy(L.rng->s, st.rng, sizeof(st.rng));
     L.en->total = st.en[0];
     L.en->inter = st.en[1];
@@ -1218,7 +1225,7 @@ extern "C" int cass_nvt_run_device_batch(cass_engine *e, int32_t nboxes, const i
   for (const NvtLaunch &L : Ls)
     if (!L.host_loop) ids.push_back(L.box);
   MirrorPull mirrors;
-  if ((rc = mirrors.reserve(e, ids, false, B.back + B.rec.staged()))) return rc;
+  if ((rc = mirrors.reserve(e, ids, false, B.in - B.o_back + B.rec.staged()))) return rc;
   // the chains grouped by kernel; every group is one launch per chunk of
   // moves, one workgroup per box.  The argument table holds the groups one
   // after another.

@@ -168,3 +168,41 @@ def test_long_records_within_bounded_staging(entry):
     for k in one:
         assert np.array_equal(one[k], two[k], equal_nan=one[k].dtype == np.float64), k
     assert one["rng"][:, -1].all() and 0 < one["accepted"][:, -100:].sum()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("long", [False, True])
+def test_records_after_a_stop_are_zero(long):
+    """A GCMC chain that runs out of free slots reports it; what it recorded
+    before stands in the caller's arrays, the rest is zero, through the staging
+    and past it."""
+    print(f"[gpu] records after a stop, long={long}", flush=True)
+    from cassandra_amd import abi
+    n, cap = 6, 8
+    steps = 320000 if long else 200
+    sp, system, live = _pentanes(n, cap)
+    eng = E.Engine(system, precision=E.FP64)
+    eng.set_cbmc_species(0, cbmc.pentane_growth(420.0, 4, 4, seed=1)[1])
+    box = eng.add_box(system, live=live)
+    lam = cbmc.de_broglie(sp, 420.0)
+    mu = S.KBOLTZ * 420.0 * (np.log(40 / 30.0 ** 3 * lam ** 3) + 2.0)   # insertions win: the slots fill
+    slots = np.zeros(2 * cap, dtype=np.int32)
+    slots[:n], slots[cap:cap + 2] = np.arange(n), [7, 6]
+    at = slots.ctypes.data
+    p32 = C.POINTER(C.c_int32)
+    gb = abi.CassGcmcBox(box.id, 0, 0, cap, 0.9, mu, lam)
+    st = abi.CassGcmcState()
+    st.rng = E.startup_rng(3, 8, [sp])
+    st.energy = abi.CassEnergy(**box.compute_system_total_energy())
+    st.nmols, st.nres, st.locate, st.reservoir = n, 2, C.cast(at, p32), C.cast(at + 4 * cap, p32)
+    kind, acc = np.full(steps, 9, np.uint8), np.full(steps, 9, np.uint8)
+    nm, en, rr = np.full(steps, 9, np.int32), np.full(steps, 9.0), np.full(5 * steps, 9, np.int64)
+    rec = abi.CassGcmcRecord(*[a.ctypes.data_as(t) for a, t in zip((kind, acc, nm, en, rr), (
+        C.POINTER(C.c_uint8), C.POINTER(C.c_uint8), p32, C.POINTER(C.c_double), C.POINTER(C.c_int64)))])
+    rc = eng.lib.cass_gcmc_run_device(eng.h, 1, C.byref(gb), C.byref(st), steps, C.byref(rec))
+    assert rc == 6   # max_molecules reached
+    done = np.flatnonzero(nm)[-1] + 1
+    assert 0 < done < 200 and nm[done - 1] == cap
+    assert all(np.all(a[done * k:] == 0) for a, k in ((kind, 1), (acc, 1), (nm, 1), (en, 1), (rr, 5)))
+    assert np.all(rr[:5 * done].reshape(-1, 5) != 9) and np.all(nm[:done] >= n)
+    eng.close()
