@@ -255,11 +255,10 @@ constexpr int kAdjList = 512;  // molecule indices held in LDS per pass
 // one ring per site of i, so that the pair terms run on full waves: of the
 // listed molecules' pairs four in ten lie outside the cutoff, and with three
 // sites a molecule a walk of one j per lane left a fifth of the lanes idle.
-// The vector unit's issue rate bounds the kernel (busy four cycles in five):
+// The vector unit's issue rate bounds the kernel (busy three cycles in four):
 // 200 frames of 800 three-site molecules took 2.23 ms with one j per lane and
-// shuffle trees per sum, and take 1.54.  The wave sums are added to LDS slots
-// per site.  Then i's intramolecular pairs,
-// one per lane.  Writes site_out[f][site][6] = (dE/d eps of the site's type,
+// shuffle trees per sum, and take 1.61.  The wave sums are added to LDS slots
+// per site.  Then i's intramolecular pairs, one per lane.  Writes site_out[f][site][6] = (dE/d eps of the site's type,
 // dE/d sigma, dE/d q, force) and emol[f][i], the energy of i's pairs.  vs/qs:
 // per species the intramolecular scale tables (pair_off + ia*n + ja); nj_max:
 // the largest molecule.
@@ -522,8 +521,9 @@ struct AdjCols {
 // two per k vector and site, against the sine and cosine per run and site and
 // the six operations per vector of a walk along the runs (0.65 ms against 2.35
 // ms for 200 frames of 2400 sites and 4117 k vectors).  The y factors are LDS
-// broadcasts, which two signs of n_z share, and bound the kernel.  part[f][split][task][32][lane]: the sums over a share
-// of the sites, so that few frames fill the chip too.
+// broadcasts, which two signs of n_z share, and bound the kernel.
+// part[f][split][task][32][lane]: the sums over a share of the sites, so that
+// few frames fill the chip too.
 __global__ void __launch_bounds__(64 * kSkWaves)
     k_adj_sk(AdjCols A, const double4 *__restrict__ ph, int nsites, int tile, int nsplit, double *__restrict__ part) {
   extern __shared__ cplx tab[];

@@ -424,7 +424,7 @@ static int widom_cbmc(cass_engine *e, int32_t box, int32_t species, int64_t n_in
   const bool lj = lj_growth(e, b, species);
   // One insertion of the parallel mode per workgroup of 4 waves: the LDS
   // holds three of them a CU, and 3001 pentane insertions (kappa 12 / 24) took
-  // 0.77, 0.50, 0.49 and 0.65 ms with 1, 2, 4 and 8 waves.  Insertions in
+  // 0.45, 0.44 and 0.62 ms with 2, 4 and 8 waves.  Insertions in
   // sequence have one CU to themselves: 8 waves.
   const int nt = rng ? 512 : 256;
   const CbmcKernels kt = growth_kernels(e, lj);
@@ -820,12 +820,19 @@ static int gcmc_launch(cass_engine *e, int32_t nboxes, const cass_gcmc_box *boxe
   std::memcpy(host.data() + o_args, args.data(), sizeof(GcmcBoxArgs) * nboxes);
   HIP_TRY(e, hipMemcpyAsync(s0, host.data(), off, hipMemcpyHostToDevice, e->stream));
   HIP_TRY(e, hipEventRecord(e->ev0, e->stream));
-  // 8 waves unless the autotuner picked otherwise: 40 moves of 48 pentane
-  // boxes took 3.9, 2.6, 1.9 and 1.7 ms of kernel with 2, 4, 8 and 16 waves
-  // (16 leave 128 registers a lane, and the kernel then spills)
+  // 8 waves unless the autotuner picked otherwise.  us a move of pentane boxes
+  // (FP64) with 2 / 4 / 8 / 16 waves:
+  //     8 molecules,  48 boxes    59.6 / 50.7 / 45.8 / 47.8
+  //    60 molecules,  48 boxes    87.5 / 68.0 / 56.9 / 54.6
+  //    60 molecules, 300 boxes     203 /  190 /  204 /  201
+  //    60 molecules, 900 boxes     950 /  923 /  958 /  964
+  //   500 molecules,  48 boxes     238 /  159 /  123 /  101
+  //  3000 molecules,   8 boxes     954 /  525 /  343 /  210
+  // and LJ switch, 60 molecules, 48 boxes: 113 / 85 / 69 / 84.  16 waves leave
+  // 128 registers a lane, and the kernels then spill.
   if (nt <= 0) nt = gcmc_block(e) > 0 ? gcmc_block(e) : 512;
   const GcmcBoxArgs *d_args = (const GcmcBoxArgs *)(s0 + o_args);
-  if (gemc) nt = 512;  // 30 transfers of 96 pentane pairs: 3.3 ms with 4 waves, 2.5 ms with 8
+  if (gemc) nt = 512;  // 30 transfers of 96 pentane pairs: 3.0 ms with 4 waves, 2.4 ms with 8
   if (nt != 128 && nt != 256 && nt != 512 && nt != 1024) return cass_fail(e, CASS_ERR_ARG, "workgroup size");
   const CbmcKernels kt = growth_kernels(e, lj);
   const int rc = gemc ? launch_chain(e, kt.gemc, d_args, nboxes / 2, nt, nsteps, list_cap, 2,
@@ -985,7 +992,7 @@ extern "C" int cass_regrow_run_device(cass_engine *e, int32_t nboxes, const cass
   HIP_TRY(e, hipMemcpyAsync(s0, host.data(), off, hipMemcpyHostToDevice, e->stream));
   HIP_TRY(e, hipEventRecord(e->ev0, e->stream));
   const RegrowBoxArgs *d_args = (const RegrowBoxArgs *)(s0 + o_args);
-  const int nt = 512;  // 60 moves of 48 pentane boxes: 6.6 ms with 4 waves, 4.2 ms with 8
+  const int nt = 512;  // 60 moves of 48 pentane boxes: 5.6 ms with 4 waves, 3.8 ms with 8
   const int rc = launch_chain(e, growth_kernels(e, lj).regrow, d_args, nboxes, nt, nsteps, list_cap,
                               1, "k_regrow_chain launch");
   if (rc) return rc;

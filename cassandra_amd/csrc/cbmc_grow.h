@@ -2,17 +2,21 @@
 //
 // One workgroup grows one molecule fragment by fragment as Build_Molecule
 // does (fragment_growth.f90:72-707, Fragment_Order :1317-1446,
-// Fragment_Placement :1449-2132): thread 0 makes the reference's random
-// draws (rranf, random_generators.f90:51-122) and the rigid-body geometry,
-// and the whole workgroup scores every trial of a stage at once -- kappa_ins
+// Fragment_Placement :1449-2132).  Wave 0 keeps the growth's books, a lane per
+// atom, dihedral or trial: the reference's random draws (rranf,
+// random_generators.f90:51-122) in its order, the rigid-body geometry and the
+// selection.  The whole workgroup scores the trials of a stage -- kappa_ins
 // placements of the first fragment, kappa_dih rotations of each further
-// fragment -- against every molecule of the box (lanes split over (trial,
-// molecule)), with the intramolecular and dihedral terms of each trial on
-// one lane.  Two drivers use it:
+// fragment -- a wave per trial, against the molecules of the box in reach.
+// Its drivers:
 //   k_gcmc_chain: one workgroup per box runs that box's whole sequence of
 //     GCMC insertions and deletions (gcmc_driver.f90:90-200,
 //     move_insert.f90:22-424, move_delete.f90:22-416) in one launch, so every
 //     box of a multi-box run advances in the same persistent kernel;
+//   k_gemc_chain: one workgroup per pair of boxes runs its particle transfers
+//     (gemc_driver.f90:91-195, move_mol_swap.f90:22-769);
+//   k_regrow_chain: one workgroup per box runs its Cut_N_Grow moves
+//     (move_regrow.f90:22-510);
 //   k_widom_cbmc: one workgroup per Widom insertion of a grown species
 //     (widom_insert.f90:22-594), or one workgroup walking all insertions on
 //     the reference's single stream.
@@ -1698,10 +1702,10 @@ __device__ __forceinline__ void copy_slots(int *dst, const int *src, int n) {
 // work of one lane was two thirds of it, and scratch traffic of the general
 // pair styles much of the rest: now what can be spread over the lanes of wave
 // 0 is, barriers stand only between stages, and plain LJ species have kernels
-// of their own without scratch.  48 pentane boxes (kappa 12 / 24, up to 233
-// molecules): 179 us a move in the slowest box before, 51 us now, of which 6
-// us a first fragment, 5 us a later one on wave 0, 2.5 us a round of trials
-// and 4 us the full-cutoff sum.
+// of their own without scratch.  40 moves in 48 pentane boxes (kappa 12 / 24,
+// up to 233 molecules): 7.5 ms before, 2.4 ms now, or 188 and 60 us a move of
+// the slowest box; in boxes that have settled 5.7 and 1.4 ms, 143 and 35 us a
+// move.  The vector units of the CUs in use are busy 17 % of the time.
 template <typename P, int NT, bool LJ>
 __global__ void __launch_bounds__(NT) k_gcmc_chain(const GcmcBoxArgs *__restrict__ boxes, int64_t nsteps,
                                                    int list_cap) {
@@ -1953,7 +1957,8 @@ __global__ void __launch_bounds__(NT) k_gcmc_chain(const GcmcBoxArgs *__restrict
 // log(P_forward / P_reverse).  The box_out molecule keeps its re-placed
 // coordinates when rejected, as in the reference.  The pair's boxes are
 // boxes[2 * blockIdx.x] and the next; the generator is the first box's.
-// Waves as in k_gcmc_chain.
+// Waves as in k_gcmc_chain.  30 transfers in 96 pairs of pentane boxes (kappa
+// 12 / 16): 8.1 ms before, 2.4 ms now.
 template <typename P, int NT, bool LJ>
 __global__ void __launch_bounds__(NT) k_gemc_chain(const GcmcBoxArgs *__restrict__ boxes, int64_t nsteps,
                                                    int list_cap) {
@@ -2362,7 +2367,8 @@ __device__ __forceinline__ void cut_regrow_setup(const CbmcSpeciesDev &c, GrowLd
 // energies, the reverse pass over the molecule's own configuration and the
 // acceptance with ln_pfor - ln_prev.  Accepted: the regrown coordinates
 // replace the molecule's; rejected after the reverse pass: its re-placed
-// coordinates do, as in the reference.  Waves as in k_gcmc_chain.
+// coordinates do, as in the reference.  Waves as in k_gcmc_chain.  60 moves
+// in 48 pentane boxes (kappa 16): 6.5 ms before, 3.8 ms now.
 template <typename P, int NT, bool LJ>
 __global__ void __launch_bounds__(NT) k_regrow_chain(const RegrowBoxArgs *__restrict__ boxes, int64_t nsteps,
                                                      int list_cap) {

@@ -41,7 +41,12 @@ struct TopoDev {
 
 // Ewald view.
 // k vectors per segment of the move chains: 2354 vectors make 574 segments of
-// five (82 % filled), about one per lane of eleven waves; four make 723.
+// five (82 % filled), about one per lane of eleven waves; four make 723.  us a
+// move with 3 / 4 / 5 / 6 / 8: 512 waters and 2354 vectors 13.1 / 13.4 / 12.0 /
+// 13.5 / 16.0, 1080 waters 23.7 / 23.2 / 23.2 / 24.7 / 28.0, 27 waters 7.6 / 7.6 /
+// 7.7 / 8.2 / 10.7.  Boxes of many vectors take several rounds of segments
+// either way and would gain from short ones: 17700 vectors 60 / 66 / 72 / 85 /
+// 105, 56500 vectors 215 / 235 / 267 / 305 / 380.
 constexpr int kKSeg = 5;
 
 struct EwaldDev {

@@ -1,4 +1,4 @@
-"""Device CBMC growth (cbmc.hip) against the reference's own runs and the oracle.
+"""Device CBMC growth (cbmc_grow.h) against the reference's own runs and the oracle.
 
 * k_gcmc_chain replays the reference's 2000-move pentane GCMC chain
   (tests/golden/pentane_gcmc_gcmc.npz, written by the reference's

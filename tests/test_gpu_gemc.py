@@ -1,4 +1,4 @@
-"""Device GEMC particle transfers (cbmc.hip::k_gemc_chain) against the
+"""Device GEMC particle transfers (cbmc_grow.h::k_gemc_chain) against the
 reference's own run and the oracle.
 
 * The reference's 2000-transfer pentane GEMC run between a 28 A box of 60
