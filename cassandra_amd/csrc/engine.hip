@@ -1198,9 +1198,9 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
     }
   const int blk = kMaxBlock;
   std::vector<RecomputeBox> rb(nboxes);
-  std::vector<int2> items, kitems_box;
-  std::vector<int4> kitems_mol, kitems_direct;
+  std::vector<int2> items, kitems_box, kitems_mol, kitems_direct;
   int64_t np = 0, nk = 0;
+  std::vector<char> direct;
   int kmols = 0;  // molecules of the Ewald boxes
   for (int i = 0; i < nboxes; ++i)
     if (bs[i]->p.charge_style == CASS_Q_EWALD) kmols += bs[i]->nmols;
@@ -1217,14 +1217,25 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
     r.ew = ewald ? ewald_view(b, row_k0_of(b)) : EwaldDev{};
     r.kblk = ewald ? box_blocks(b.nvecs, b.nmols) : 0;
     r.kparts = ewald ? ewald_parts(b, kmols) : 1;
+    r.kdirect = std::max(1, (b.nvecs + blk - 1) / blk);
     r.kpart_off = nk;
     if (ewald) {
-      if (b.nvecs > 0)
-        for (int m = 0; m < b.nmols; ++m) {
-          const bool direct = ewald_direct(r.ew, b.nmols, e->sp_natoms[b.mol_species[m]]);
-          const int parts = direct ? (b.nvecs + blk - 1) / blk : r.kparts;
-          for (int k = 0; k < parts; ++k) (direct ? kitems_direct : kitems_mol).push_back(make_int4(i, m, k, 0));
-        }
+      // which species take which way first: tests per molecule took 15 us of
+      // a call of 24 boxes of 512
+      bool any = false, all = true;
+      direct.resize(e->nspecies);
+      for (int sp = 0; sp < e->nspecies; ++sp) {
+        direct[sp] = ewald_direct(r.ew, b.nmols, e->sp_natoms[sp]);
+        any = any || direct[sp];
+        all = all && direct[sp];
+      }
+      auto items_of = [&](std::vector<int2> &to, int parts, bool way, bool every) {
+        for (int m = 0; m < b.nmols; ++m)
+          if (every || direct[b.mol_species[m]] == way)
+            for (int k = 0; k < parts; ++k) to.push_back(make_int2(i, m * parts + k));
+      };
+      if (b.nvecs > 0 && !all) items_of(kitems_mol, r.kparts, false, !any);
+      if (b.nvecs > 0 && any) items_of(kitems_direct, r.kdirect, true, all);
       for (int kb = 0; kb < r.kblk; ++kb) kitems_box.push_back(make_int2(i, kb));
       nk += r.kblk;
     }
@@ -1238,8 +1249,8 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
   };
   const size_t o_rb = take(sizeof(RecomputeBox) * std::max(1, nboxes)),
                o_it = take(sizeof(int2) * std::max<size_t>(1, items.size())),
-               o_km = take(sizeof(int4) * std::max<size_t>(1, kitems_mol.size())),
-               o_kd = take(sizeof(int4) * std::max<size_t>(1, kitems_direct.size())),
+               o_km = take(sizeof(int2) * std::max<size_t>(1, kitems_mol.size())),
+               o_kd = take(sizeof(int2) * std::max<size_t>(1, kitems_direct.size())),
                o_kb = take(sizeof(int2) * std::max<size_t>(1, kitems_box.size())),
                o_part = take(2 * sizeof(double) * std::max<int64_t>(1, np)),
                o_pov = take(sizeof(int) * std::max<int64_t>(1, np)),
@@ -1251,10 +1262,10 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
   if (!items.empty())
     HIP_TRY(e, hipMemcpyAsync(s + o_it, items.data(), sizeof(int2) * items.size(), hipMemcpyHostToDevice, e->stream));
   if (!kitems_mol.empty())
-    HIP_TRY(e, hipMemcpyAsync(s + o_km, kitems_mol.data(), sizeof(int4) * kitems_mol.size(), hipMemcpyHostToDevice,
+    HIP_TRY(e, hipMemcpyAsync(s + o_km, kitems_mol.data(), sizeof(int2) * kitems_mol.size(), hipMemcpyHostToDevice,
                               e->stream));
   if (!kitems_direct.empty())
-    HIP_TRY(e, hipMemcpyAsync(s + o_kd, kitems_direct.data(), sizeof(int4) * kitems_direct.size(),
+    HIP_TRY(e, hipMemcpyAsync(s + o_kd, kitems_direct.data(), sizeof(int2) * kitems_direct.size(),
                               hipMemcpyHostToDevice, e->stream));
   if (!kitems_box.empty())
     HIP_TRY(e, hipMemcpyAsync(s + o_kb, kitems_box.data(), sizeof(int2) * kitems_box.size(), hipMemcpyHostToDevice,
@@ -1274,12 +1285,12 @@ extern "C" int cass_total_energy_batch(cass_engine *e, int32_t nboxes, const int
   }
   if (!kitems_mol.empty()) {
     hipLaunchKernelGGL(k_ewald_mol_multi, dim3((unsigned)kitems_mol.size()), dim3(blk), 0, e->stream, d_rb, tv,
-                       (const int4 *)(s + o_km));
+                       (const int2 *)(s + o_km));
     HIP_TRY(e, hipGetLastError());
   }
   if (!kitems_direct.empty()) {
     hipLaunchKernelGGL(k_ewald_direct_multi, dim3((unsigned)kitems_direct.size()), dim3(blk), 0, e->stream, d_rb, tv,
-                       (const int4 *)(s + o_kd));
+                       (const int2 *)(s + o_kd));
     HIP_TRY(e, hipGetLastError());
   }
   if (!kitems_box.empty()) {

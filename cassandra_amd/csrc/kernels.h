@@ -345,7 +345,7 @@ struct RecomputeBox {
   PairConst<double> cd;
   PairConst<float> cf;
   EwaldDev ew;
-  int kblk, kparts;
+  int kblk, kparts, kdirect;  // k blocks; workgroups per molecule of the two ways
   int64_t part_off, kpart_off;
 };
 
@@ -400,8 +400,8 @@ __global__ void k_ewald_box(BoxDev b, EwaldDev ew, double *part);
 template <typename P>
 __global__ void k_total_pairs_multi(const RecomputeBox *boxes, TopoDev tp, const int2 *items, double *part,
                                     int *part_ov);
-__global__ void k_ewald_mol_multi(const RecomputeBox *boxes, TopoDev tp, const int4 *items);
-__global__ void k_ewald_direct_multi(const RecomputeBox *boxes, TopoDev tp, const int4 *items);
+__global__ void k_ewald_mol_multi(const RecomputeBox *boxes, TopoDev tp, const int2 *items);
+__global__ void k_ewald_direct_multi(const RecomputeBox *boxes, TopoDev tp, const int2 *items);
 __global__ void k_ewald_box_multi(const RecomputeBox *boxes, const int2 *items, double *kpart);
 __global__ void k_sum_multi(const RecomputeBox *boxes, const double *kpart, double *out);
 __global__ void k_ewald_move(TopoDev tp, EwaldDev ew, int m, int species, int flag, int n, const double *nxyz,

@@ -414,21 +414,23 @@ __device__ inline void ewald_box_block(const BoxDev &b, const EwaldDev &ew, int 
 
 __global__ void k_ewald_box(BoxDev b, EwaldDev ew, double *part) { ewald_box_block(b, ew, blockIdx.x, part); }
 
-// The two stages over many boxes: items (box, molecule, part), (box, molecule,
-// k block) and (box, k block); a box's k-block terms start at kpart_off in
-// kpart.
+// The two stages over many boxes: items (box, molecule * parts + part), the
+// same with k blocks for parts, and (box, k block); a box's k-block terms start
+// at kpart_off in kpart.
 __global__ void __launch_bounds__(kMaxBlock)
-    k_ewald_mol_multi(const RecomputeBox *__restrict__ boxes, TopoDev tp, const int4 *__restrict__ items) {
-  const int4 it = items[blockIdx.x];
+    k_ewald_mol_multi(const RecomputeBox *__restrict__ boxes, TopoDev tp, const int2 *__restrict__ items) {
+  const int2 it = items[blockIdx.x];
   const RecomputeBox &r = boxes[it.x];
-  ewald_mol_block(r.b, tp, r.ew, it.y, it.z, r.kparts);
+  const int m = it.y / r.kparts;
+  ewald_mol_block(r.b, tp, r.ew, m, it.y - m * r.kparts, r.kparts);
 }
 
 __global__ void k_ewald_direct_multi(const RecomputeBox *__restrict__ boxes, TopoDev tp,
-                                     const int4 *__restrict__ items) {
-  const int4 it = items[blockIdx.x];
+                                     const int2 *__restrict__ items) {
+  const int2 it = items[blockIdx.x];
   const RecomputeBox &r = boxes[it.x];
-  ewald_direct_block(r.b, tp, r.ew, it.y, it.z);
+  const int m = it.y / r.kdirect;
+  ewald_direct_block(r.b, tp, r.ew, m, it.y - m * r.kdirect);
 }
 
 __global__ void k_ewald_box_multi(const RecomputeBox *__restrict__ boxes, const int2 *__restrict__ items,
